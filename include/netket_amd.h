@@ -365,6 +365,15 @@ int64_t nka_rbm_qgt_workspace(const nka_rbm* m, int64_t ns);
 int nka_rbm_qgt(const nka_rbm* m, const int8_t* sigma, const void* tT, int64_t ns, double scale, double shift,
                 double* out, int64_t ldo, void* workspace, void* stream);
 
+/* The same S for an FP64 model (arguments as nka_rbm_qgt, tT FP64): P is +-1 in
+ * int8, Q 55-bit fixed point with a power-of-two scale per row in seven int8
+ * digit planes, and P Q^T exact int32 products on the matrix cores, so C is
+ * rounded once per entry.  At most 2^22 samples (the workspace query returns
+ * 0 for sizes it does not take). */
+int64_t nka_rbm_qgt_f64_workspace(const nka_rbm* m, int64_t ns);
+int nka_rbm_qgt_f64(const nka_rbm* m, const int8_t* sigma, const double* tT, int64_t ns, double scale, double shift,
+                    double* out, int64_t ldo, void* workspace, void* stream);
+
 /* Centred NTK of the RBM without forming its Jacobian: out = scale * O_c O_c^T
  * + shift I + offset 11^T (lower triangle incl. diagonal, FP64, row-major ldo),
  * O_c[s,p] = O[s,p] - mean[p], O as for nka_rbm_contract and t from

@@ -165,10 +165,25 @@ def gram(bufs: JacobianBuffers, shift: float, offset: float = 0.0,
     return out
 
 
-def qgt_structured_available(model, flat) -> bool:
-    """Whether the dense S of ``model`` can be formed from its layer structure
-    (FP32 RBM: spin-pair x activation-pair products)."""
-    return model.kind == "rbm" and flat.dtype == torch.float32
+def qgt_structured_available(model, flat, n_sites: int, n_samples: int) -> bool:
+    """Whether the dense S of ``model`` is formed from its layer structure
+    (RBM: spin-pair x activation-pair products; FP32 models in bf16 planes,
+    FP64 models in exact int8 digit planes).
+
+    The FP64 form holds 7 bytes per activation pair and sample, against the
+    8 bytes per parameter and sample of the Jacobian (their ratio grows like
+    alpha / 2), and a product C of about a quarter of S.  Models that would
+    need more than three Jacobians and one more S (alpha above about 6) keep
+    the Jacobian and its FP64 product, as do batches past the entry point's
+    sample limit."""
+    if model.kind != "rbm":
+        return False
+    if flat.dtype == torch.float32:
+        return True
+    m = model.native(flat, n_sites)
+    need = nat.lib().nka_rbm_qgt_f64_workspace(C.byref(m), n_samples)
+    np_ = model.layout(n_sites)["n_params"]
+    return 0 < need <= 8 * np_ * (3 * _ld(n_samples) + np_) + (64 << 20)
 
 
 def qgt_structured(model, flat, sigma2d: torch.Tensor, tT: torch.Tensor, scale: float, shift: float,
@@ -182,9 +197,10 @@ def qgt_structured(model, flat, sigma2d: torch.Tensor, tT: torch.Tensor, scale: 
     if out is None or out.shape != (np_, np_):
         out = torch.empty((np_, np_), dtype=torch.float64, device=sigma2d.device)
     m = model.native(flat, N)
-    ws = _ops.WORKSPACE.get("rbm_qgt", nat.lib().nka_rbm_qgt_workspace(C.byref(m), n))
+    name = "nka_rbm_qgt" if flat.dtype == torch.float32 else "nka_rbm_qgt_f64"
+    ws = _ops.WORKSPACE.get("rbm_qgt", getattr(nat.lib(), name + "_workspace")(C.byref(m), n))
     with _ops.TIMER.region("qgt_structured"):
-        nat.call("nka_rbm_qgt", C.byref(m), _ops.ptr(sigma2d), _ops.ptr(tT), n, float(scale), float(shift),
+        nat.call(name, C.byref(m), _ops.ptr(sigma2d), _ops.ptr(tT), n, float(scale), float(shift),
                  _ops.ptr(out), out.stride(0), _ops.ptr(ws), _ops.stream())
     return out
 

@@ -1837,14 +1837,24 @@ __global__ void __launch_bounds__(1024) stats_kernel(const double* __restrict__ 
   }
 }
 
-// Copy the lower triangle onto the upper one (row-major, FP64).
-__global__ void symmetrize_kernel(double* __restrict__ a, int64_t n, int64_t lda) {
-  const int64_t total = n * n;
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-       idx += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t i = idx / n, j = idx % n;
-    if (j > i) a[i * lda + j] = a[j * lda + i];
-  }
+// Copy the lower triangle onto the upper one (row-major, FP64): one 64x64 tile
+// of the lower triangle per workgroup, transposed through LDS, so that both
+// the reads and the writes run along rows (an element-wise copy reads the lower
+// triangle down its columns: 0.41 ms at n = 8384).
+constexpr int SY_T = 64;
+__global__ void __launch_bounds__(256) symmetrize_kernel(double* __restrict__ a, int64_t n, int64_t lda) {
+  __shared__ double tile[SY_T][SY_T + 1];
+  int ti, tj;
+  tri_tile(blockIdx.x, ti, tj);
+  const int64_t i0 = (int64_t)ti * SY_T, j0 = (int64_t)tj * SY_T;
+  const int c = threadIdx.x & 63, r0 = threadIdx.x >> 6;
+#pragma unroll
+  for (int r = r0; r < SY_T; r += 4)
+    if (i0 + r < n && j0 + c < n) tile[r][c] = a[(i0 + r) * lda + j0 + c];
+  __syncthreads();
+#pragma unroll
+  for (int r = r0; r < SY_T; r += 4)
+    if (j0 + r < n && i0 + c < n && j0 + r < i0 + c) a[(j0 + r) * lda + i0 + c] = tile[c][r];
 }
 
 // RBM neural tangent kernel on the bf16x3 Gram tiles (called from the NTK
@@ -2394,8 +2404,10 @@ int nka_centre_scale(const double* e, int64_t n, const double* mean, double scal
 int nka_symmetrize_f64(double* a, int64_t n, int64_t lda, void* stream) {
   NKA_CHECK_ARG(n >= 0 && lda >= n && (n == 0 || a), "nka_symmetrize_f64: bad arguments");
   if (n == 0) return NKA_OK;
-  const unsigned g = (unsigned)std::min<int64_t>((n * n + 255) / 256, 65536);
-  hipLaunchKernelGGL(symmetrize_kernel, dim3(g), dim3(256), 0, (hipStream_t)stream, a, n, lda);
+  const int64_t T = (n + SY_T - 1) / SY_T;
+  NKA_CHECK_ARG(T * (T + 1) / 2 < (1LL << 31), "nka_symmetrize_f64: too large");
+  hipLaunchKernelGGL(symmetrize_kernel, dim3((unsigned)(T * (T + 1) / 2)), dim3(256), 0, (hipStream_t)stream, a, n,
+                     lda);
   NKA_CHECK_LAUNCH("nka_symmetrize_f64");
   return NKA_OK;
 }

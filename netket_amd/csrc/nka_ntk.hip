@@ -14,6 +14,7 @@
 // packed spins in the epilogue (the bf16x3 Gram kernel of nka_linalg.hip).
 #include "nka_common.hpp"
 #include "netket_amd.h"
+#include "nka_qgt.hpp"
 
 namespace nka {
 
@@ -175,37 +176,6 @@ void launch_gemm_exact_a(const uint16_t* a, int64_t ma, const uint16_t* bh, cons
 // activations.  The spin side needs no centring: its pair sums are exact
 // integers.
 // ---------------------------------------------------------------------------
-
-// Augmented spin index u in [-1, N) (-1: the constant 1).  Row of P holding
-// s~_u s~_u'.
-__device__ __host__ inline int64_t qgt_spin_row(int u, int v, int N) {
-  if (u == v) return 0;
-  if (u < 0) return 1 + v;
-  if (v < 0) return 1 + u;
-  const int64_t i = u < v ? u : v, k = u < v ? v : u;
-  return 1 + N + k * (k - 1) / 2 + i;
-}
-// Augmented hidden index w in [-1, M).  Row of Q holding t~_w t~_w'.
-__device__ __host__ inline int64_t qgt_hidden_row(int w, int x, int M) {
-  if (w < 0 && x < 0) return 0;
-  if (w < 0) return 1 + x;
-  if (x < 0) return 1 + w;
-  const int64_t j = w < x ? w : x, l = w < x ? x : w;
-  return 1 + M + l * (l + 1) / 2 + j;
-}
-// Largest e with e (e + 1) / 2 <= b.
-__device__ inline int64_t tri_root(int64_t b) {
-  int64_t e = (int64_t)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
-  while ((e + 1) * (e + 2) / 2 <= b) ++e;
-  while (e * (e + 1) / 2 > b) --e;
-  return e;
-}
-// Position of parameter (u, w) in the flat vector, or -1 when it is not one.
-__device__ inline int64_t qgt_param(int u, int w, const nka_rbm& m) {
-  if (u < 0) return (w < 0 || m.bias_off < 0) ? -1 : m.bias_off + w;
-  if (w < 0) return m.visible_off < 0 ? -1 : m.visible_off + u;
-  return m.kernel_off + (int64_t)u * m.n_hidden + w;
-}
 
 // sT (N x ldk int8) = sigma^T as +-1, zero for the padding samples s >= ns.
 __global__ void qgt_spins_t_kernel(const int8_t* __restrict__ sigma, int64_t ns, int N, int64_t ldk,
@@ -409,6 +379,11 @@ __global__ void __launch_bounds__(256) qgt_unpack_kernel(nka_rbm m, const float*
       entry(w, p, cw, up, -1);
     }
   }
+}
+
+void launch_qgt_spins_t(const int8_t* sigma, int64_t ns, int N, int64_t ldk, int8_t* sT, hipStream_t s) {
+  const unsigned g = (unsigned)std::min<int64_t>(((int64_t)N * ldk + 255) / 256, 65536);
+  hipLaunchKernelGGL(qgt_spins_t_kernel, dim3(g), dim3(256), 0, s, sigma, ns, N, ldk, sT);
 }
 
 constexpr int NT_T = 64;
@@ -631,11 +606,7 @@ int nka_rbm_ntk(const nka_rbm* m, const int8_t* sigma, const void* t, int64_t ns
 }
 
 // Workspace of nka_rbm_qgt: transposed spins, P, Q hi and lo, and C.
-static int64_t qgt_ldk(int64_t ns) { return (ns + 63) / 64 * 64; }
-static int64_t qgt_rows_p(const nka_rbm& m) { return 1 + (int64_t)m.n_visible + (int64_t)m.n_visible * (m.n_visible - 1) / 2; }
-static int64_t qgt_rows_q(const nka_rbm& m) { return 1 + (int64_t)m.n_hidden + (int64_t)m.n_hidden * (m.n_hidden + 1) / 2; }
 static int64_t qgt_ldc(const nka_rbm& m) { return (qgt_rows_q(m) + 63) / 64 * 64; }
-static int64_t qgt_round(int64_t b) { return (b + 255) / 256 * 256; }
 
 int64_t nka_rbm_qgt_workspace(const nka_rbm* m, int64_t ns) {
   if (!m || ns <= 0) return 0;
@@ -668,8 +639,7 @@ int nka_rbm_qgt(const nka_rbm* m, const int8_t* sigma, const void* tT, int64_t n
   float* C = (float*)w;
   w += qgt_round(rp * ldc * 4);
   double* cmean = (double*)w;
-  const unsigned g0 = (unsigned)std::min<int64_t>(((int64_t)N * ldk + 255) / 256, 65536);
-  hipLaunchKernelGGL(qgt_spins_t_kernel, dim3(g0), dim3(256), 0, s, sigma, ns, N, ldk, sT);
+  launch_qgt_spins_t(sigma, ns, N, ldk, sT, s);
   hipLaunchKernelGGL(qgt_spin_pairs_kernel, dim3((unsigned)std::min<int64_t>(rp, 65536)), dim3(256), 0, s, sT,
                      ns, N, ldk, rp, P);
   hipLaunchKernelGGL(qgt_hidden_means_kernel, dim3((unsigned)std::min<int64_t>(M, 65536)), dim3(256), 0, s,

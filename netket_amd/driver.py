@@ -246,7 +246,7 @@ class VMC_SR(AbstractVariationalDriver):
         # NTK T from the RBM's structure (FP64, inner sizes n_hidden and n_visible)
         # or from the explicit Jacobian (bf16x3 / FP64 Gram over n_params)
         self.ntk_method = ntk_method
-        # S of an FP32 RBM from its spin-pair x activation-pair structure, or
+        # S of an RBM from its spin-pair x activation-pair structure, or
         # from the explicit Jacobian (bf16x3 / FP64 Gram over n_samples)
         self.qgt_method = qgt_method
         self._old_updates = None
@@ -269,11 +269,11 @@ class VMC_SR(AbstractVariationalDriver):
         proj_reg = self._hyper(self.proj_reg)
         momentum = self._hyper(self.momentum)
         model, flat = vs.model, vs.parameters_flat
-        structured_s = (not self.use_ntk and self.qgt_method == "structured"
-                        and eng.qgt_structured_available(model, flat))
         pc = vs._prepared()
         sig, t = pc["sigma"], pc["t"]
         ns = sig.shape[0]
+        structured_s = (not self.use_ntk and self.qgt_method == "structured"
+                        and eng.qgt_structured_available(model, flat, sig.shape[1], ns))
         need_tT = not self.use_ntk
         tT = eng.prepare(model, flat, sig, row_major=False, transposed=True)[1] if need_tT else None
         S_pre = None

@@ -6,13 +6,15 @@ netket/optimizer/qgt/qgt_jacobian_dense.py:29-161, 251-270) for real
 parameters ("real" mode): O_L = (O - <O>) / sqrt(Ns) with FP64 centring,
 S = O_L^T O_L + diag_shift I.
 
-For FP32 RBMs S is formed from the model's structure without a Jacobian: each
+For RBMs S is formed from the model's structure without a Jacobian: each
 log-derivative is (augmented spin) x (augmented tanh), so O^T O is unpacked
 from the product of the spin-pair and activation-pair tables over the samples
-(nka_rbm_qgt, bf16 matrix cores, FP64 centring).  Other FP32 models store O_L
+(FP32 models: nka_rbm_qgt, bf16 matrix cores, FP64 centring; FP64 models:
+nka_rbm_qgt_f64, exact int8 digit products).  Other FP32 models store O_L
 parameter-major (X = O_L^T, Np x Ns) as a bf16 hi/lo split and form S with
-three BF16 MFMA products per tile (FP32 accumulate); FP64 models keep O_L and
-S in FP64 (FP64 MFMA).  S is built on demand and not kept after a Cholesky
+three BF16 MFMA products per tile (FP32 accumulate); other FP64 models, and
+RBMs with many more hidden than visible units, keep O_L and S in FP64 (FP64
+MFMA).  S is built on demand and not kept after a Cholesky
 solve consumed it.
 """
 
@@ -56,9 +58,10 @@ class QGTJacobianDenseT(LinearOperator):
         self.n_samples = C * L
         sig = s.reshape(C * L, N)
         model, flat = vstate.model, vstate.parameters_flat
-        t, tT = eng.prepare(model, flat, sig, row_major=True, transposed=True)
+        structured = eng.qgt_structured_available(model, flat, N, self.n_samples)
+        t, tT = eng.prepare(model, flat, sig, row_major=not structured, transposed=True)
         self.X = None
-        if eng.qgt_structured_available(model, flat):
+        if structured:
             self._structured = (model, flat, sig, tT)
             self.n_params = model.layout(N)["n_params"]
         else:

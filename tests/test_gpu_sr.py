@@ -572,3 +572,82 @@ def test_vmc_sr_preconditioner_step(gpu):
     g = vs.expect_and_forces_flat(H)[1]  # same cached samples
     dp2 = sr_cg(vs, g)
     assert np.linalg.norm(dp2.cpu().numpy() - ref) <= 1e-3 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("ns,biases,N,alpha", [(1, (True, True), 8, 1),
+                                               (63, (True, False), 16, 2),
+                                               (128, (False, False), 9, 3),
+                                               (129, (False, True), 14, 3),
+                                               (1008, (True, True), 16, 1),
+                                               (4099, (True, True), 33, 2),
+                                               (300, (True, True), 70, 2)])
+def test_rbm_qgt_structured_fp64(gpu, ns, biases, N, alpha):
+    # S of an FP64 RBM from the exact int8 digit products: partial tiles on
+    # both sides, one to many K steps and K slices, odd sample counts, and
+    # (N = 70) a C row past the LDS staging.  Units whose activations are
+    # nearly constant, tiny and saturated take very different row scales.
+    print(f"case rbm_qgt fp64 ns={ns} biases={biases} N={N} alpha={alpha}", flush=True)
+    M = alpha * N
+    model = nk.models.RBM(alpha=alpha, param_dtype=np.float64, use_hidden_bias=biases[0],
+                          use_visible_bias=biases[1])
+    rng = np.random.default_rng(ns + N)
+    lay = model.layout(N)
+    n_par = lay["n_params"]
+    flat = rng.normal(scale=0.3, size=n_par)
+    o, s = lay["kernel"]
+    W = flat[o:o + N * M].reshape(N, M)
+    W[:, 0] *= 1e-6
+    W[:, 1] = 0.0
+    if biases[0]:
+        flat[lay["bias"][0] + 2] = 5.0
+    x = rng.choice(np.array([-1, 1], dtype=np.int8), size=(ns, N))
+    sig = torch.as_tensor(x, device="cuda")
+    fl = torch.as_tensor(flat, device="cuda")
+    assert eng.qgt_structured_available(model, fl, N, ns)
+    _, tT = eng.prepare(model, fl, sig, row_major=False, transposed=True)
+    shift = 1e-2
+    out = torch.full((n_par, n_par), 7.0, dtype=torch.float64, device="cuda")
+    S = eng.qgt_structured(model, fl, sig, tT, 1.0 / ns, shift, out=out).cpu().numpy()
+    p = orbm.RBMParams(flat, N, M, hidden_bias=biases[0], visible_bias=biases[1])
+    Ou = orbm.jacobian(p, x)
+    # the rows of 48 parameters (the special units' among them) in extended
+    # precision: a plain FP64 sum over the samples is less exact than S
+    Ol = Ou.astype(np.longdouble)
+    Ol -= Ol.sum(axis=0) / ns
+    rows = np.unique(np.concatenate([[0, 1, 2, o, o + 1, n_par - 1], rng.integers(0, n_par, 42)]))
+    ref = np.dot(Ol[:, rows].T, Ol) / ns
+    ref[np.arange(len(rows)), rows] += shift
+    # both sides round the activations (2^-53 of |t| <= 1 each), the oracle also
+    # its centred sums: a few units of 2^-53 times the uncentred column norms
+    du = np.sqrt(np.sum(Ou * Ou, axis=0) / ns)
+    bound = 32 * 2.0 ** -53 * np.outer(du[rows], du) + 1e-17
+    keep = np.arange(n_par)[None, :] <= rows[:, None]
+    err = np.abs(S[rows] - ref.astype(np.float64))
+    print(f"max |dS| / bound = {(err / bound)[keep].max():.2e}", flush=True)
+    assert np.all((err <= bound)[keep])
+    up = np.triu_indices(n_par, 1)
+    assert np.all(S[up] == 7.0)
+
+
+def test_rbm_qgt_structured_fp64_nan_activation(gpu):
+    # a unit with a NaN activation makes the entries of its parameters NaN and
+    # leaves the others as they are
+    print("case rbm_qgt fp64 NaN", flush=True)
+    N, ns = 10, 200
+    model = nk.models.RBM(alpha=1, param_dtype=np.float64)
+    rng = np.random.default_rng(4)
+    lay = model.layout(N)
+    fl = torch.as_tensor(rng.normal(scale=0.3, size=lay["n_params"]), device="cuda")
+    sig = torch.as_tensor(rng.choice(np.array([-1, 1], dtype=np.int8), size=(ns, N)), device="cuda")
+    _, tT = eng.prepare(model, fl, sig, row_major=False, transposed=True)
+    ref = eng.qgt_structured(model, fl, sig, tT, 1.0 / ns, 0.0).cpu().numpy()
+    tT[3, 17] = float("nan")
+    S = eng.qgt_structured(model, fl, sig, tT, 1.0 / ns, 0.0).cpu().numpy()
+    o = lay["kernel"][0]
+    hit = np.zeros(lay["n_params"], dtype=bool)
+    hit[lay["bias"][0] + 3] = True
+    hit[o + 3:o + N * N:N] = True
+    lower = np.tril(np.ones_like(S, dtype=bool))
+    either = hit[:, None] | hit[None, :]
+    assert np.all(np.isnan(S[lower & either]))
+    np.testing.assert_array_equal(S[lower & ~either], ref[lower & ~either])
