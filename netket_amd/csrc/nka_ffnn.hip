@@ -34,12 +34,25 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 constexpr int FF_ROWS = 32;      // configurations (or chains) per workgroup
-constexpr int FF_THREADS = 256;
-constexpr int FF_GROUPS = FF_THREADS / FF_ROWS;  // threads per row in the first layer
-constexpr int FF_HPT = 128;      // hidden units per thread: H1 <= FF_GROUPS * FF_HPT
-constexpr int FF_MAXH = FF_GROUPS * FF_HPT;      // 1024
-constexpr int FF_MAXBLK = FF_MAXH / 32;          // column blocks of the second layer
-constexpr int FF_MAXD = 4;                        // differing sites per connected row, fast path
+constexpr int FF_MAXH = 1024;
+// Workgroup sizes.  The second layer is a chain of dependent matrix products
+// per 32-column block; several wavefronts per SIMD cover each other's operand
+// loads (L2 for W2, LDS for the activations), the first layer's gathers and the
+// row sums.  Forward pass: two workgroups of 512 per CU.  Sampler: one of 1024
+// (32 chains per CU are all there is), of 512 where a thread's state does not
+// fit 128 registers (FP64; weighted exchange).  J1-J2 10x10 with layers 100-400-
+// 400 in FP32, against workgroups of 256: the sampler (8192 chains, 700
+// proposals) 42.4 -> 22.0 ms (matrix cores 55% busy), the local energies of 16384
+// samples 23.2 -> 12.5 ms (58%; with the connected elements taken as a list of
+// flipped sites instead of as configurations, 3.0 ms of that).
+constexpr int FF_FWD = 512;
+constexpr int FF_BACK = 256;
+constexpr int FF_MAXBLK = FF_MAXH / 32;  // column blocks of the second layer
+constexpr int FF_MAXD = 4;               // sites a connected configuration differs at (a term acts on at most 4)
+
+// nka_conn.hip
+int launch_conn_list(int op_kind, const void* op, const int8_t* x, int64_t B, int N, int K, void* mels, int* rows,
+                     uint64_t* sites, int* count, hipStream_t s);
 
 template <class T>
 struct FfnnView {
@@ -76,81 +89,79 @@ constexpr int64_t FF_LDS_MAX = 160 * 1024;
 // is applied to every element and its values are summed per row into
 // rowsum[r] (0 <= r < 32) in a fixed order.  part is LDS scratch of
 // 32 * FF_MAXBLK values.  All threads of the workgroup must call it.
-// The 32-column blocks go to the four wavefronts in turn; with rbuf (LDS
+// The 32-column blocks go to the NW wavefronts in turn; with rbuf (LDS
 // scratch of (nblk % 4) * 4 * 1024 values) the nblk % 4 blocks left over
-// after whole rounds are split along K over the four wavefronts instead, and
-// their partial tiles are summed in a fixed order, so every wavefront does the
-// same number of products.
+// after whole rounds of four are split along K into quarters, which go to the
+// next wavefronts in turn, and their partial tiles are summed in a fixed order.
+// Wavefronts w, w + 4, ... share a SIMD, so every SIMD does the same number of
+// products.  The sums' order depends on the sizes alone, not on NW.
 // ---------------------------------------------------------------------------
-template <class Epi>
-__device__ void rows_gemm(const float* As, int lda, int K, int ncols, const float* __restrict__ Bp, int sk,
+template <int NW, class Epi>
+__device__ __forceinline__ void rows_gemm(const float* As, int lda, int K, int ncols, const float* __restrict__ Bp, int sk,
                           int sc, Epi epi, float* part, float* rowsum, float* rbuf = nullptr) {
   const int wid = threadIdx.x >> 6, lane = lane_id();
   const int nblk = (ncols + 31) >> 5;
   const int kh = lane >> 5, lc = lane & 31;
   constexpr int KB = 16;
   // acc += A[:, ka:kb] B(ka:kb, block cb); lane (lc, kh) supplies row lc and
-  // column cb*32 + lc at k = k0 + 2q + kh of each pair of k-rows.  The B
-  // loads run three groups of 16 k-rows ahead of their products (three
-  // register sets in turn; near the end of the range a group reloads the
-  // last full group, unused, so that every load is unconditional).
-  auto mfma_range = [&](floatx16& acc, int cb, int ka, int kb) {
+  // column cb*32 + lc at k = k0 + 2q + kh of each pair of k-rows.  The B loads
+  // run two groups of 16 k-rows ahead of their products (register sets in
+  // turn; one group ahead with four wavefronts per SIMD, which cover the rest);
+  // near the end of the range a group reloads the last full group, unused, so
+  // that every load is unconditional.  The lane's part of the address is one
+  // 32-bit offset, the k-row's part a scalar.
+  const __amdgpu_buffer_rsrc_t Bs = __builtin_amdgcn_make_buffer_rsrc((void*)Bp, 0, K * ncols * 4, 0x00020000);
+  auto mfma_range = [&](floatx16& acc, int cb, int ka, int kb) __attribute__((always_inline)) {
     const int col = cb * 32 + lc;
     const bool cok = col < ncols;
-    const int colc = cok ? col : ncols - 1;
-    const uint32_t boff = (uint32_t)colc * (uint32_t)sc + (uint32_t)kh * (uint32_t)sk;
-    const uint32_t s2 = 2u * (uint32_t)sk;
+    const int boff = ((cok ? col : ncols - 1) * sc + kh * sk) * 4;
     const int kend = ka + (kb - ka) / KB * KB;
+    const float* arow = As + lc * lda + kh;
+    constexpr int NB = NW >= 16 ? 2 : 3;
     int k = ka;
-    auto loadB = [&](int kk0, float* bv) {
+    auto loadB = [&](int kk0, float (&bv)[KB / 2]) __attribute__((always_inline)) {
       const int kc = kk0 < kend ? kk0 : kend - KB;
-      const uint32_t kn = (uint32_t)kc * (uint32_t)sk + boff;
 #pragma unroll
-      for (int q = 0; q < KB / 2; ++q) bv[q] = Bp[kn + (uint32_t)q * s2];
+      for (int q = 0; q < KB / 2; ++q)
+        bv[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(Bs, boff, (kc + 2 * q) * sk * 4, 0));
     };
-    auto group = [&](int kk0, const float* bv) {
+    auto group = [&](int kk0, const float (&bv)[KB / 2]) __attribute__((always_inline)) {
       float a[KB / 2];
 #pragma unroll
-      for (int q = 0; q < KB / 2; ++q) a[q] = As[lc * lda + kk0 + 2 * q + kh];
+      for (int q = 0; q < KB / 2; ++q) a[q] = arow[kk0 + 2 * q];
 #pragma unroll
       for (int q = 0; q < KB / 2; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], bv[q], acc, 0, 0, 0);
     };
     if (kend > ka) {
-      float b0[KB / 2], b1[KB / 2], b2[KB / 2];
-      loadB(k, b0);
-      loadB(k + KB, b1);
-      while (true) {
-        loadB(k + 2 * KB, b2);
-        __builtin_amdgcn_sched_barrier(0);
-        group(k, b0);
-        k += KB;
-        if (k >= kend) break;
-        loadB(k + 2 * KB, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        group(k, b1);
-        k += KB;
-        if (k >= kend) break;
-        loadB(k + 2 * KB, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        group(k, b2);
-        k += KB;
-        if (k >= kend) break;
+      float bv[NB][KB / 2];
+#pragma unroll
+      for (int i = 0; i < NB - 1; ++i) loadB(k + i * KB, bv[i]);
+      while (k < kend) {
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+          loadB(k + (NB - 1) * KB, bv[(i + NB - 1) % NB]);
+          __builtin_amdgcn_sched_barrier(0);
+          group(k, bv[i]);
+          k += KB;
+          if (k >= kend) break;
+        }
       }
     }
     for (; k < kb; k += 2) {
       const int kk = k + kh;
       const float av = kk < kb ? As[lc * lda + kk] : 0.0f;
-      const float bv = (kk < kb && cok) ? Bp[(uint32_t)kk * (uint32_t)sk + (uint32_t)col * (uint32_t)sc] : 0.0f;
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
+      const float bw = (kk < kb && cok) ? Bp[(uint32_t)kk * (uint32_t)sk + (uint32_t)col * (uint32_t)sc] : 0.0f;
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bw, acc, 0, 0, 0);
     }
   };
-  // element e of lane l is (row (e/4)*8 + (l/32)*4 + e%4, col l%32)
-  auto finish = [&](const floatx16& acc, int cb) {
+  // element e of lane l is (row (e/4)*8 + (l/32)*4 + e%4, col l%32); elements
+  // 4 q .. 4 q + 3 of block cb
+  auto finish = [&](const float (&acc)[4], int q, int cb) __attribute__((always_inline)) {
     const int col = cb * 32 + lc;
     const bool cok = col < ncols;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int row = (e >> 2) * 8 + kh * 4 + (e & 3);
+    for (int e = 0; e < 4; ++e) {
+      const int row = q * 8 + kh * 4 + e;
       float v = cok ? epi(row, col, acc[e]) : 0.0f;
 #pragma unroll
       for (int off = 16; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -159,37 +170,43 @@ __device__ void rows_gemm(const float* As, int lda, int K, int ncols, const floa
   };
   const int rem = rbuf ? (nblk & 3) : 0;
   const int nfull = nblk - rem;
-  for (int cb = wid; cb < nfull; cb += 4) {
+  for (int cb = wid; cb < nfull; cb += NW) {
     floatx16 acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
     mfma_range(acc, cb, 0, K);
-    finish(acc, cb);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float aq[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
+      finish(aq, q, cb);
+    }
   }
   if (rem > 0) {
-    // K quarters rounded up to whole groups; wavefront w takes quarter w
+    // K quarters rounded up to whole groups
     const int kq = ((K + 3) / 4 + KB - 1) / KB * KB;
-    const int k0 = min(K, wid * kq), k1 = min(K, k0 + kq);
-    for (int j = 0; j < rem; ++j) {
+    for (int u = (wid + NW - nfull % NW) % NW; u < 4 * rem; u += NW) {
+      const int k0 = min(K, (u & 3) * kq), k1 = min(K, k0 + kq);
       floatx16 acc;
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-      mfma_range(acc, nfull + j, k0, k1);
-      float* dst = rbuf + (j * 4 + wid) * 1024;
+      mfma_range(acc, nfull + (u >> 2), k0, k1);
+      float* dst = rbuf + u * 1024;
 #pragma unroll
       for (int e = 0; e < 16; ++e) dst[e * 64 + lane] = acc[e];
     }
     __syncthreads();
-    if (wid < rem) {
-      floatx16 acc;
+    // the sums of four elements per wavefront in turn
+    for (int u = wid; u < 4 * rem; u += NW) {
+      const int j = u >> 2, q = u & 3;
+      float acc[4];
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
+      for (int e = 0; e < 4; ++e) {
         float t = 0.0f;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) t += rbuf[(wid * 4 + w) * 1024 + e * 64 + lane];
+        for (int w = 0; w < 4; ++w) t += rbuf[(j * 4 + w) * 1024 + (4 * q + e) * 64 + lane];
         acc[e] = t;
       }
-      finish(acc, nfull + wid);
+      finish(acc, q, nfull + j);
     }
   }
   __syncthreads();
@@ -201,12 +218,14 @@ __device__ void rows_gemm(const float* As, int lda, int K, int ncols, const floa
   __syncthreads();
 }
 
-template <class Epi>
-__device__ void rows_gemm(const double* As, int lda, int K, int ncols, const double* __restrict__ Bp, int sk,
+template <int NW, class Epi>
+__device__ __forceinline__ void rows_gemm(const double* As, int lda, int K, int ncols, const double* __restrict__ Bp, int sk,
                           int sc, Epi epi, double* part, double* rowsum, double* rbuf = nullptr) {
+  constexpr int G = NW * 64 / FF_ROWS;  // threads per row
+  static_assert(G <= FF_MAXBLK, "one partial sum per thread of a row");
   const int r = threadIdx.x & 31, g = threadIdx.x >> 5;
   double s = 0.0;
-  for (int c = g; c < ncols; c += FF_GROUPS) {
+  for (int c = g; c < ncols; c += G) {
     double z = 0.0;
     for (int k = 0; k < K; ++k) z += As[r * lda + k] * Bp[(int64_t)k * sk + (int64_t)c * sc];
     s += epi(r, c, z);
@@ -215,7 +234,7 @@ __device__ void rows_gemm(const double* As, int lda, int K, int ncols, const dou
   __syncthreads();
   if (threadIdx.x < FF_ROWS) {
     double t = 0.0;
-    for (int q = 0; q < FF_GROUPS; ++q) t += part[threadIdx.x * FF_MAXBLK + q];
+    for (int q = 0; q < G; ++q) t += part[threadIdx.x * FF_MAXBLK + q];
     rowsum[threadIdx.x] = t;
   }
   __syncthreads();
@@ -231,31 +250,30 @@ __device__ inline T theta1_full(const FfnnView<T>& v, const int8_t* x, int a) {
 
 // ---------------------------------------------------------------------------
 // Batched forward pass.  MODE 0: rows are configurations x[r]; theta1 from
-// scratch (optionally stored to th_out).  MODE 1: rows r = (s, k) of
-// connected configurations xp[r] of sample s = r / K, taken from the list
-// ridx[0 .. *rcount) (the rows with a nonzero matrix element); theta1 is the
-// sample's theta1 (th_base[s]) plus 2 x'_i W1[i] for every site where x'
+// scratch (optionally stored to th_out).  MODE 1: the connected
+// configurations of the list ridx, rsites [0 .. *rcount) (the nonzero matrix
+// elements; row r = s K + k belongs to sample s); theta1 is the sample's theta1
+// (th_base[s]) plus 2 x'_i W1[i] for the sites i, in ascending order, where x'
 // differs from x[s].  Outputs log psi per row (MODE 1: at the row's own
 // index); g2_out (rows x H2), when set, receives tanh(z2).
 // ---------------------------------------------------------------------------
 template <class T, int MODE>
-__global__ void __launch_bounds__(FF_THREADS) ffnn_forward_kernel(nka_ffnn m, const int8_t* __restrict__ xr,
-                                                                 const int8_t* __restrict__ xs, int Kc,
+__global__ void __launch_bounds__(FF_FWD) ffnn_forward_kernel(nka_ffnn m, const int8_t* __restrict__ xr, int Kc,
                                                                  const T* __restrict__ th_base, int64_t rows,
                                                                  T* __restrict__ logpsi, T* __restrict__ th_out,
                                                                  T* __restrict__ g2_out, const int* __restrict__ ridx,
+                                                                 const uint64_t* __restrict__ rsites,
                                                                  const int* __restrict__ rcount) {
   extern __shared__ unsigned char smem[];
+  constexpr int FWD_G = FF_FWD / FF_ROWS;  // threads per row in the first layer
   const FfnnView<T> v = ffnn_view<T>(m);
   const int N = v.N, H1 = v.H1, H2 = v.H2;
   const int lda = lda_of(H1);
   T* hA = (T*)smem;                                   // 32 x lda
   T* part = hA + FF_ROWS * lda;                        // 32 x FF_MAXBLK
   T* rowsum = part + FF_ROWS * FF_MAXBLK;              // 32
-  int* dsite = (int*)(rowsum + FF_ROWS);               // 32 x (FF_MAXD + 1): count, sites
-  int8_t* xl = (int8_t*)(dsite + FF_ROWS * (FF_MAXD + 1));  // 32 x N (+ 32 x N base rows)
-  int8_t* xb = xl + FF_ROWS * N;
-  T* rbuf = sizeof(T) == 4 ? (T*)(smem + ffpad((int64_t)(xb - (int8_t*)smem) + (int64_t)FF_ROWS * N)) : nullptr;
+  int8_t* xl = (int8_t*)(rowsum + FF_ROWS);            // 32 x N (MODE 0)
+  T* rbuf = sizeof(T) == 4 ? (T*)(smem + ffpad((int64_t)(xl - (int8_t*)smem) + (int64_t)FF_ROWS * N)) : nullptr;
   const int64_t r0 = (int64_t)blockIdx.x * FF_ROWS;
   // MODE 1: tile rows r0 .. r0+31 of the row list; the grid covers the
   // longest possible list, so tiles past its end leave at once
@@ -266,60 +284,66 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_forward_kernel(nka_ffnn m, co
     if (cr >= nrows) return -1;
     return MODE == 1 ? (int64_t)ridx[cr] : cr;
   };
-  for (int idx = threadIdx.x; idx < FF_ROWS * N; idx += FF_THREADS) {
-    const int r = idx / N, i = idx % N;
-    const int64_t gr = row_of(r);
-    xl[idx] = gr >= 0 ? xr[gr * N + i] : (int8_t)1;
-    if (MODE == 1) xb[idx] = gr >= 0 ? xs[(gr / Kc) * N + i] : (int8_t)1;
-  }
-  __syncthreads();
-  if (MODE == 1) {
-    // the sites where row r differs from its sample, ascending; a count of
-    // -1 marks a row with more than FF_MAXD of them (full scan below)
-    if (threadIdx.x < FF_ROWS) {
-      const int rr = threadIdx.x;
-      int cnt = 0;
-      for (int i = 0; i < N; ++i)
-        if (xl[rr * N + i] != xb[rr * N + i]) {
-          if (cnt < FF_MAXD) dsite[rr * (FF_MAXD + 1) + 1 + cnt] = i;
-          ++cnt;
-        }
-      dsite[rr * (FF_MAXD + 1)] = cnt <= FF_MAXD ? cnt : -1;
+  const int r = threadIdx.x / FWD_G, g = threadIdx.x % FWD_G;
+  const int64_t gr = row_of(r);
+  if (MODE == 0) {
+    for (int idx = threadIdx.x; idx < FF_ROWS * N; idx += FF_FWD) {
+      const int64_t ri = row_of(idx / N);
+      xl[idx] = ri >= 0 ? xr[ri * N + idx % N] : (int8_t)1;
     }
     __syncthreads();
-  }
-  const int r = threadIdx.x / FF_GROUPS, g = threadIdx.x % FF_GROUPS;
-  const int64_t gr = row_of(r);
-  int nd = 0, ds[FF_MAXD];
-  T sg[FF_MAXD];
-  if (MODE == 1) {
-    nd = dsite[r * (FF_MAXD + 1)];
+    for (int a = g; a < H1; a += FWD_G) {
+      const T t = theta1_full<T>(v, xl + r * N, a);
+      if (th_out && gr >= 0) th_out[gr * H1 + a] = t;
+      hA[r * lda + a] = log_cosh<T>(t);
+    }
+  } else {
+    // rows past the end of the list take its last row's place (not stored)
+    const int64_t cr = min<int64_t>(r0 + r, nrows - 1);
+    const uint64_t code = rsites[cr];
+    const T* base = th_base + (int64_t)((uint32_t)ridx[cr] / (uint32_t)Kc) * H1;
+    int nd = 0, ds[FF_MAXD];
+    T sg[FF_MAXD];
 #pragma unroll
     for (int d = 0; d < FF_MAXD; ++d) {
-      ds[d] = d < nd ? dsite[r * (FF_MAXD + 1) + 1 + d] : 0;
-      sg[d] = xl[r * N + ds[d]] > 0 ? (T)2 : (T)-2;
+      const uint32_t c = (uint32_t)(code >> (16 * d)) & 0xffffu;
+      const bool any = c != 0xffffu;
+      nd += any;
+      ds[d] = any ? (int)(c & 0x7fffu) : 0;
+      sg[d] = c & 0x8000u ? (T)2 : (T)-2;
     }
-  }
-  for (int a = g; a < H1; a += FF_GROUPS) {
-    T t;
-    if (MODE == 0) {
-      t = theta1_full<T>(v, xl + r * N, a);
-      if (th_out && gr >= 0) th_out[gr * H1 + a] = t;
+    if (nd <= 2) {
+      // every connected row of an Ising or two-site operator: a batch of
+      // units' loads in flight at a time
+      constexpr int LB = 8;
+      const T* w0 = v.W1 + (int64_t)ds[0] * H1;
+      const T* w1 = v.W1 + (int64_t)ds[1] * H1;
+      for (int ab = g; ab < H1; ab += LB * FWD_G) {
+        T t[LB], u0[LB], u1[LB];
+#pragma unroll
+        for (int q = 0; q < LB; ++q) {
+          const int a = min(ab + q * FWD_G, H1 - 1);
+          t[q] = base[a];
+          u0[q] = w0[a];
+          u1[q] = w1[a];
+        }
+#pragma unroll
+        for (int q = 0; q < LB; ++q) {
+          const int a = ab + q * FWD_G;
+          if (nd > 0) t[q] += sg[0] * u0[q];
+          if (nd > 1) t[q] += sg[1] * u1[q];
+          if (a < H1) hA[r * lda + a] = log_cosh<T>(t[q]);
+        }
+      }
     } else {
-      t = gr >= 0 ? th_base[(gr / Kc) * H1 + a] : (T)0;
-      if (nd >= 0) {
-        // same terms in the same (ascending) order as the full scan
+      for (int a = g; a < H1; a += FWD_G) {
+        T t = base[a];
 #pragma unroll
         for (int d = 0; d < FF_MAXD; ++d)
           if (d < nd) t += sg[d] * v.W1[(int64_t)ds[d] * H1 + a];
-      } else {
-        const int8_t* x1 = xl + r * N;
-        const int8_t* x0 = xb + r * N;
-        for (int i = 0; i < N; ++i)
-          if (x1[i] != x0[i]) t += (x1[i] > 0 ? (T)2 : (T)-2) * v.W1[(int64_t)i * H1 + a];
+        hA[r * lda + a] = log_cosh<T>(t);
       }
     }
-    hA[r * lda + a] = log_cosh<T>(t);
   }
   __syncthreads();
   const T* W2 = v.W2;
@@ -329,7 +353,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_forward_kernel(nka_ffnn m, co
     if (g2_out && r0 + rr < rows) g2_out[(r0 + rr) * H2 + c] = tanh_t<T>(zz);
     return log_cosh<T>(zz);
   };
-  rows_gemm(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
+  rows_gemm<FF_FWD / 64>(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
   if (threadIdx.x < FF_ROWS) {
     const int64_t go = row_of(threadIdx.x);
     if (go >= 0) logpsi[go] = rowsum[threadIdx.x];
@@ -340,31 +364,12 @@ template <class T>
 inline size_t forward_lds(const nka_ffnn& m) {
   return ffpad((size_t)FF_ROWS * lda_of(m.n_hidden1) * sizeof(T)) +
          ffpad((size_t)FF_ROWS * FF_MAXBLK * sizeof(T)) + ffpad(FF_ROWS * sizeof(T)) +
-         ffpad((size_t)FF_ROWS * (FF_MAXD + 1) * sizeof(int)) + ffpad((size_t)2 * FF_ROWS * m.n_visible) +
+         ffpad((size_t)FF_ROWS * m.n_visible) +
          (sizeof(T) == 4 ? split_scratch_bytes(m.n_hidden2) : 0);
 }
 
-// List of the connected rows with a nonzero matrix element (only those enter
-// the local energy; the reduction below skips the others).  Slots are taken by
-// one atomic add per wavefront, so the list order varies between runs, but
-// every row's log psi is formed from that row alone, so the results do not.
 __global__ void ffnn_zero_count_kernel(int* __restrict__ count) {
   if (threadIdx.x == 0) count[0] = 0;
-}
-
-template <class M>
-__global__ void __launch_bounds__(256) ffnn_compact_rows_kernel(const M* __restrict__ mels, int64_t rows,
-                                                                int* __restrict__ ridx, int* __restrict__ count) {
-  const int lane = lane_id();
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < rows; base += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t r = base + threadIdx.x;
-    const bool nz = r < rows && mels[r] != (M)0;
-    const uint64_t bal = __ballot(nz);
-    int slot0 = 0;
-    if (lane == 0 && bal) slot0 = atomicAdd(count, (int)__popcll(bal));
-    slot0 = __shfl(slot0, 0, 64);
-    if (nz) ridx[slot0 + (int)__popcll(bal & ((1ull << lane) - 1ull))] = (int)r;
-  }
 }
 
 // eloc[s] = sum_k mel[s,k] exp(lp[s,k] - lp0[s]) (FP64); one wavefront per sample
@@ -390,7 +395,7 @@ __global__ void ffnn_eloc_reduce_kernel(const M* __restrict__ mels, const T* __r
 // gradient with respect to theta1 (a second tile product with B = W2^T).
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ void __launch_bounds__(FF_THREADS) ffnn_backprop_kernel(nka_ffnn m, const T* __restrict__ th1,
+__global__ void __launch_bounds__(FF_BACK) ffnn_backprop_kernel(nka_ffnn m, const T* __restrict__ th1,
                                                                   const T* __restrict__ g2, int64_t rows,
                                                                   T* __restrict__ h1_out, T* __restrict__ d1_out) {
   extern __shared__ unsigned char smem[];
@@ -401,11 +406,11 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_backprop_kernel(nka_ffnn m, c
   T* part = gA + FF_ROWS * ldg;
   T* rowsum = part + FF_ROWS * FF_MAXBLK;
   const int64_t r0 = (int64_t)blockIdx.x * FF_ROWS;
-  for (int idx = threadIdx.x; idx < FF_ROWS * H2; idx += FF_THREADS) {
+  for (int idx = threadIdx.x; idx < FF_ROWS * H2; idx += FF_BACK) {
     const int r = idx / H2, c = idx % H2;
     gA[r * ldg + c] = r0 + r < rows ? g2[(r0 + r) * H2 + c] : (T)0;
   }
-  for (int idx = threadIdx.x; idx < FF_ROWS * H1; idx += FF_THREADS) {
+  for (int idx = threadIdx.x; idx < FF_ROWS * H1; idx += FF_BACK) {
     const int r = idx / H1, a = idx % H1;
     if (r0 + r < rows) h1_out[(r0 + r) * H1 + a] = log_cosh<T>(th1[(r0 + r) * H1 + a]);
   }
@@ -415,7 +420,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_backprop_kernel(nka_ffnn m, c
     if (r0 + rr < rows) d1_out[(r0 + rr) * H1 + a] = u * tanh_t<T>(th1[(r0 + rr) * H1 + a]);
     return (T)0;
   };
-  rows_gemm(gA, ldg, H2, H1, W2, 1, H2, epi, part, rowsum);
+  rows_gemm<FF_BACK / 64>(gA, ldg, H2, H1, W2, 1, H2, epi, part, rowsum);
 }
 
 template <class T>
@@ -729,13 +734,15 @@ struct FfSweepArgs {
 
 constexpr int FF_MAXCL = 16;  // cluster slots per lane: n_clusters <= 1024
 
-template <class T, int HPT>
-__global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m, FfSweepArgs sa,
+template <class T, int NT, int HPT, bool WEIGHTED>
+__global__ void __launch_bounds__(NT) ffnn_metropolis_kernel(nka_ffnn m, FfSweepArgs sa,
                                                                     int8_t* __restrict__ sigma, T* __restrict__ log_prob,
                                                                     int8_t* __restrict__ samples,
                                                                     T* __restrict__ lp_samples,
                                                                     int64_t* __restrict__ n_accepted) {
   extern __shared__ unsigned char smem[];
+  constexpr int GR = NT / FF_ROWS;                // threads per chain
+  constexpr int CPW = FF_ROWS / (NT / 64);        // chains whose proposals a wavefront draws
   const FfnnView<T> v = ffnn_view<T>(m);
   const int N = v.N, H1 = v.H1, H2 = v.H2;
   const int lda = lda_of(H1);
@@ -754,7 +761,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
   // bit set (word w, bit b: cluster 64 w + b) and their count, the clusters,
   // and for every site the clusters that contain it (other site, cluster)
   const bool exch = sa.rule == NKA_RULE_EXCHANGE;
-  const bool fast_exch = exch && !sa.weights;
+  const bool fast_exch = exch && !WEIGHTED;
   const int ncl = fast_exch ? sa.n_clusters : 0;
   const int NWc = (ncl + 63) / 64;
   unsigned char* xb = smem + ffpad((int64_t)((unsigned char*)xs - smem) + (int64_t)FF_ROWS * N);
@@ -769,19 +776,19 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
   T* rbuf = sizeof(T) == 4 ? (T*)(smem + ffpad((int64_t)((unsigned char*)(pnew + FF_ROWS) - smem))) : nullptr;
   const int tid = threadIdx.x, wid = tid >> 6, lane = lane_id();
   const int c0 = blockIdx.x * FF_ROWS;
-  const int cr = tid / FF_GROUPS, g = tid % FF_GROUPS;   // chain row and unit group of this thread
+  const int cr = tid / GR, g = tid % GR;   // chain row and unit group of this thread
   const int chain = c0 + cr;
 
-  for (int idx = tid; idx < FF_ROWS * N; idx += FF_THREADS) {
+  for (int idx = tid; idx < FF_ROWS * N; idx += NT) {
     const int r = idx / N, i = idx % N;
     xs[idx] = (c0 + r < sa.C) ? sigma[(int64_t)(c0 + r) * N + i] : (int8_t)1;
   }
   if (tid < FF_ROWS) nacc[tid] = 0;
   if (fast_exch) {
-    for (int i = tid; i <= N; i += FF_THREADS) adj_off[i] = 0;
-    for (int i = tid; i < 2 * ncl; i += FF_THREADS) cls[i] = sa.clusters[i];
+    for (int i = tid; i <= N; i += NT) adj_off[i] = 0;
+    for (int i = tid; i < 2 * ncl; i += NT) cls[i] = sa.clusters[i];
     __syncthreads();
-    for (int c = tid; c < ncl; c += FF_THREADS) {
+    for (int c = tid; c < ncl; c += NT) {
       atomicAdd(&adj_off[cls[2 * c] + 1], 1);
       atomicAdd(&adj_off[cls[2 * c + 1] + 1], 1);
     }
@@ -789,8 +796,8 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
     if (tid == 0)
       for (int i = 0; i < N; ++i) adj_off[i + 1] += adj_off[i];
     __syncthreads();
-    for (int i = tid; i < N; i += FF_THREADS) adj_pos[i] = adj_off[i];
-    for (int idx = tid; idx < FF_ROWS * NWc; idx += FF_THREADS) {
+    for (int i = tid; i < N; i += NT) adj_pos[i] = adj_off[i];
+    for (int idx = tid; idx < FF_ROWS * NWc; idx += NT) {
       const int r = idx / NWc, w = idx % NWc;
       uint64_t bits = 0;
       for (int b = 0; b < 64; ++b) {
@@ -800,7 +807,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
       dmask[idx] = bits;
     }
     __syncthreads();
-    for (int c = tid; c < ncl; c += FF_THREADS) {
+    for (int c = tid; c < ncl; c += NT) {
       const int u = cls[2 * c], w = cls[2 * c + 1];
       int at = atomicAdd(&adj_pos[u], 1);
       adj_t[at] = w;
@@ -819,7 +826,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
   T th[HPT];
 #pragma unroll
   for (int j = 0; j < HPT; ++j) {
-    const int a = g + FF_GROUPS * j;
+    const int a = g + GR * j;
     th[j] = a < H1 ? theta1_full<T>(v, xs + cr * N, a) : (T)0;
     if (a < H1) hA[cr * lda + a] = log_cosh<T>(th[j]);
   }
@@ -827,15 +834,16 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
   const T* W2 = v.W2;
   const T* b2 = v.b2;
   auto epi = [=](int, int c, T z) { return log_cosh<T>(z + (b2 ? b2[c] : (T)0)); };
-  rows_gemm(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
+  rows_gemm<NT / 64>(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
   const T pw = (T)sa.machine_pow;
   if (tid < FF_ROWS) lp[tid] = pw * rowsum[tid];
 
   // cluster slots of this lane (weighted exchange rule): cl = lane + 64 r
-  const int RS = exch ? (sa.n_clusters + 63) / 64 : 0;
-  int cu[FF_MAXCL], cv[FF_MAXCL];
+  const int RS = WEIGHTED ? (sa.n_clusters + 63) / 64 : 0;
+  constexpr int SLOTS = WEIGHTED ? FF_MAXCL : 1;
+  int cu[SLOTS], cv[SLOTS];
 #pragma unroll
-  for (int r = 0; r < FF_MAXCL; ++r) {
+  for (int r = 0; r < SLOTS; ++r) {
     const int cl = lane + 64 * r;
     const bool ok = r < RS && cl < sa.n_clusters;
     cu[r] = ok ? sa.clusters[2 * cl] : -1;
@@ -851,57 +859,60 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
   const int n_sweeps = sa.n_discard + sa.chain_length;
   for (int sw = 0; sw < n_sweeps; ++sw) {
     for (int p = 0; p < sa.sweep_size; ++p, ++q) {
-      if (!exch || fast_exch) {
-        // proposals of chains 8w .. 8w+7 by lanes 0..7 of wavefront w.  An
-        // exchange picks the k-th set bit of the chain's differing-cluster
-        // set; swapping the two (different) spins of that cluster flips the
-        // state of every other cluster at either site, so the count after the
-        // move follows from the sites' clusters alone
-        if (lane < FF_ROWS / 4) {
-          const int r = wid * (FF_ROWS / 4) + lane;
-          const int ch = c0 + r;
-          const u32x4 rnd = philox4x32_10({(uint32_t)q, (uint32_t)(q >> 32), (uint32_t)ch, TAG_METROPOLIS},
-                                          sa.k0, sa.k1);
-          const int8_t* x = xs + r * N;
-          int s0 = 0, s1 = 0, nf = 1, nn = 0;
-          T corr = (T)0;
-          if (!exch) {
-            s0 = (int)bounded(rnd.x, (uint32_t)N);
-          } else {
-            const int nd = ndiff[r];
-            nf = 0;
-            if (nd > 0) {
-              int k = (int)bounded(rnd.x, (uint32_t)nd);
-              const uint64_t* dm = dmask + r * NWc;
-              int w = 0;
-              uint64_t word = dm[0];
-              int cnt = __popcll(word);
-              while (k >= cnt && w + 1 < NWc) {
-                k -= cnt;
-                ++w;
-                word = dm[w];
-                cnt = __popcll(word);
-              }
-              if (k < cnt) {
-                const int c = 64 * w + kth_set_bit(word, k);
-                s0 = cls[2 * c];
-                s1 = cls[2 * c + 1];
-                nf = 2;
-                const int8_t x0 = x[s0], x1 = x[s1];
-                int delta = 0;
-                for (int e = adj_off[s0]; e < adj_off[s0 + 1]; ++e) {
-                  const int t = adj_t[e];
-                  if (t != s0 && t != s1) delta += x[t] != x0 ? -1 : 1;
-                }
-                for (int e = adj_off[s1]; e < adj_off[s1 + 1]; ++e) {
-                  const int t = adj_t[e];
-                  if (t != s0 && t != s1) delta += x[t] != x1 ? -1 : 1;
-                }
-                nn = nd + delta;
-                corr = log_t<T>((T)nd) - log_t<T>((T)nn);
-              }
+      if constexpr (!WEIGHTED) {
+        // proposals of chains CPW w .. by wavefront w, 64 / CPW lanes each.  An
+        // exchange picks the k-th set bit of the chain's differing-cluster set
+        // (the lanes count a word each); swapping the two (different) spins of
+        // that cluster flips the state of every other cluster at either site, so
+        // the count after the move follows from the sites' clusters alone (one
+        // per lane)
+        constexpr int LPC = 64 / CPW;
+        static_assert(LPC >= FF_MAXCL, "a lane per word of the differing-cluster set");
+        const int sl = lane % LPC;
+        const int r = wid * CPW + lane / LPC;
+        const int ch = c0 + r;
+        const u32x4 rnd = philox4x32_10({(uint32_t)q, (uint32_t)(q >> 32), (uint32_t)ch, TAG_METROPOLIS},
+                                        sa.k0, sa.k1);
+        const int8_t* x = xs + r * N;
+        int s0 = 0, s1 = 0, nf = 1, nn = 0;
+        T corr = (T)0;
+        if (!exch) {
+          s0 = (int)bounded(rnd.x, (uint32_t)N);
+        } else {
+          const int nd = ndiff[r];
+          const int k = nd > 0 ? (int)bounded(rnd.x, (uint32_t)nd) : 0;
+          const uint64_t word = sl < NWc ? dmask[r * NWc + sl] : 0ull;
+          const int cnt = __popcll(word);
+          int inc = cnt;  // inclusive prefix sum over the chain's words
+#pragma unroll
+          for (int o = 1; o < FF_MAXCL; o <<= 1) {
+            const int u = __shfl_up(inc, o, LPC);
+            if (sl >= o) inc += u;
+          }
+          const uint64_t hit = (__ballot(nd > 0 && inc - cnt <= k && k < inc) >> (lane - sl)) & ((1ull << LPC) - 1ull);
+          nf = hit ? 2 : 0;
+          const int w = hit ? (int)__builtin_ctzll(hit) : 0;
+          const uint64_t wsel = ((uint64_t)(uint32_t)__shfl((int)(word >> 32), w, LPC) << 32) |
+                                (uint32_t)__shfl((int)(uint32_t)word, w, LPC);
+          const int below = __shfl(inc - cnt, w, LPC);
+          int delta = 0;
+          if (hit) {
+            const int c = 64 * w + kth_set_bit(wsel, k - below);
+            s0 = cls[2 * c];
+            s1 = cls[2 * c + 1];
+            const int8_t x0 = x[s0], x1 = x[s1];
+            const int e0 = adj_off[s0], n0 = adj_off[s0 + 1] - e0, e1 = adj_off[s1], n1 = adj_off[s1 + 1] - e1;
+            for (int e = sl; e < n0 + n1; e += LPC) {
+              const int t = adj_t[e < n0 ? e0 + e : e1 + e - n0];
+              if (t != s0 && t != s1) delta += x[t] != (e < n0 ? x0 : x1) ? -1 : 1;
             }
           }
+#pragma unroll
+          for (int o = LPC / 2; o >= 1; o >>= 1) delta += __shfl_xor(delta, o, LPC);
+          nn = nd + delta;
+          if (hit) corr = log_t<T>((T)nd) - log_t<T>((T)nn);
+        }
+        if (sl == 0) {
           psite[2 * r] = s0;
           psite[2 * r + 1] = s1;
           pnf[r] = nf;
@@ -909,96 +920,48 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
           pu[r] = uniform01<T>(rnd);
           pnew[r] = nn;
         }
-      } else
-      // weighted exchange: proposals of chains 8w .. 8w+7, one at a time per wavefront
-      for (int cc = 0; cc < FF_ROWS / 4; ++cc) {
-        const int r = wid * (FF_ROWS / 4) + cc;
+      } else {
+      // weighted exchange: the wavefront's proposals one at a time
+      for (int cc = 0; cc < CPW; ++cc) {
+        const int r = wid * CPW + cc;
         const int ch = c0 + r;
         const u32x4 rnd = philox4x32_10({(uint32_t)q, (uint32_t)(q >> 32), (uint32_t)ch, TAG_METROPOLIS},
                                         sa.k0, sa.k1);
         const int8_t* x = xs + r * N;
-        int s0 = 0, s1 = 0, nf = 1;
+        int s0 = 0, s1 = 0, nf = 0;
         T corr = (T)0;
-        if (!exch) {
-          s0 = (int)bounded(uniform_value<uint32_t>(rnd.x), (uint32_t)N);
-        } else if (sa.weights) {
-          // weighted choice among the differing clusters (as the RBM sampler)
-          uint32_t wd[FF_MAXCL];
-          uint32_t tot = 0;
+        // weighted choice among the differing clusters (as the RBM sampler)
+        uint32_t wd[SLOTS];
+        uint32_t tot = 0;
 #pragma unroll
-          for (int rr = 0; rr < FF_MAXCL; ++rr) {
-            const bool d = rr < RS && cu[rr] >= 0 && x[cu[rr]] != x[cv[rr]];
-            wd[rr] = d ? sa.weights[lane + 64 * rr] : 0u;
-            if (rr < RS) tot += wave_sum_u32(wd[rr]);
-          }
-          tot = uniform_value<uint32_t>(tot);
-          if (tot == 0) {
-            nf = 0;
-          } else {
-            const uint32_t k = bounded(uniform_value<uint32_t>(rnd.x), tot);
-            int sel = uniform_value<int>(weighted_pick<FF_MAXCL>(wd, RS, k));
-            if (sel < 0 || sel >= sa.n_clusters) sel = 0;  // unreachable: k < tot
-            cluster_sites<FF_MAXCL>(cu, cv, sel, s0, s1);
-            nf = 2;
-            uint32_t tot_new = 0;
+        for (int rr = 0; rr < SLOTS; ++rr) {
+          const bool d = rr < RS && cu[rr] >= 0 && x[cu[rr]] != x[cv[rr]];
+          wd[rr] = d ? sa.weights[lane + 64 * rr] : 0u;
+          if (rr < RS) tot += wave_sum_u32(wd[rr]);
+        }
+        tot = uniform_value<uint32_t>(tot);
+        if (tot != 0) {
+          const uint32_t k = bounded(uniform_value<uint32_t>(rnd.x), tot);
+          int sel = uniform_value<int>(weighted_pick<SLOTS>(wd, RS, k));
+          if (sel < 0 || sel >= sa.n_clusters) sel = 0;  // unreachable: k < tot
+          cluster_sites<SLOTS>(cu, cv, sel, s0, s1);
+          nf = 2;
+          uint32_t tot_new = 0;
 #pragma unroll
-            for (int rr = 0; rr < FF_MAXCL; ++rr) {
-              if (rr < RS) {
-                bool d = false;
-                if (cu[rr] >= 0) {
-                  const int ua = cu[rr], ub = cv[rr];
-                  const int8_t xa = ua == s0 ? x[s1] : (ua == s1 ? x[s0] : x[ua]);
-                  const int8_t xb = ub == s0 ? x[s1] : (ub == s1 ? x[s0] : x[ub]);
-                  d = xa != xb;
-                }
-                tot_new += wave_sum_u32(d ? sa.weights[lane + 64 * rr] : 0u);
-              }
-            }
-            tot_new = uniform_value<uint32_t>(tot_new);
-            corr = uniform_value<T>(log_t<T>((T)tot) - log_t<T>((T)tot_new));
-          }
-        } else {
-          uint64_t bal[FF_MAXCL];
-          int n_diff = 0;
-#pragma unroll
-          for (int rr = 0; rr < FF_MAXCL; ++rr) {
-            const bool d = rr < RS && cu[rr] >= 0 && x[cu[rr]] != x[cv[rr]];
-            bal[rr] = __ballot(d);
-            n_diff += __popcll(bal[rr]);
-          }
-          n_diff = uniform_value<int>(n_diff);
-          if (n_diff == 0) {
-            nf = 0;
-          } else {
-            int k = (int)bounded(uniform_value<uint32_t>(rnd.x), (uint32_t)n_diff);
-            int sel = -1;
-#pragma unroll
-            for (int rr = 0; rr < FF_MAXCL; ++rr) {
-              if (sel < 0 && rr < RS) {
-                const int cnt = __popcll(bal[rr]);
-                if (k < cnt) sel = rr * 64 + kth_set_bit(bal[rr], k);
-                else k -= cnt;
-              }
-            }
-            sel = uniform_value<int>(sel);
-            if (sel < 0 || sel >= sa.n_clusters) sel = 0;  // unreachable: k < n_diff
-            cluster_sites<FF_MAXCL>(cu, cv, sel, s0, s1);
-            nf = 2;
-            int n_new = 0;
-#pragma unroll
-            for (int rr = 0; rr < FF_MAXCL; ++rr) {
+          for (int rr = 0; rr < SLOTS; ++rr) {
+            if (rr < RS) {
               bool d = false;
-              if (rr < RS && cu[rr] >= 0) {
+              if (cu[rr] >= 0) {
                 const int ua = cu[rr], ub = cv[rr];
                 const int8_t xa = ua == s0 ? x[s1] : (ua == s1 ? x[s0] : x[ua]);
                 const int8_t xb = ub == s0 ? x[s1] : (ub == s1 ? x[s0] : x[ub]);
                 d = xa != xb;
               }
-              n_new += __popcll(__ballot(d));
+              tot_new += wave_sum_u32(d ? sa.weights[lane + 64 * rr] : 0u);
             }
-            n_new = uniform_value<int>(n_new);
-            corr = uniform_value<T>(log_t<T>((T)n_diff) - log_t<T>((T)n_new));
           }
+          tot_new = uniform_value<uint32_t>(tot_new);
+          corr = uniform_value<T>(log_t<T>((T)tot) - log_t<T>((T)tot_new));
         }
         if (lane == 0) {
           psite[2 * r] = s0;
@@ -1008,12 +971,13 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
           pu[r] = uniform01<T>(rnd);
         }
       }
+      }
       __syncthreads();
       // theta1' and h1' of every chain
       T thn[HPT];
       {
-        // at most two flipped sites; their W1 rows are read with every load
-        // of the thread's units in flight (no loop over the flips per unit)
+        // at most two flipped sites; the loads of their W1 rows for a batch of
+        // units are in flight together
         const int nf = pnf[cr];
         const int8_t* x = xs + cr * N;
         const int s0 = nf > 0 ? psite[2 * cr] : 0;
@@ -1021,23 +985,36 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
         // x'_site = -x_site: theta1 gains (x' - x) W1 = -2 x W1
         const T c0 = x[s0] > 0 ? (T)-2 : (T)2;
         const T c1 = x[s1] > 0 ? (T)-2 : (T)2;
-        const T* w0 = v.W1 + (int64_t)s0 * H1;
-        const T* w1 = v.W1 + (int64_t)s1 * H1;
+        const T* w0 = v.W1 + (int64_t)s0 * H1 + g;
+        const T* w1 = v.W1 + (int64_t)s1 * H1 + g;
+        // units left from this thread's first one; opaque, so that the bound
+        // checks are made here and not kept in registers over the sweep
+        int left = H1 - g;
+        asm volatile("" : "+v"(left));
+        constexpr int LB = HPT < 8 ? HPT : 8;   // loads in flight: 2 LB
 #pragma unroll
-        for (int j = 0; j < HPT; ++j) {
-          const int a = g + FF_GROUPS * j;
-          T t = th[j];
-          if (a < H1) {
-            const T u0 = w0[a], u1 = w1[a];
-            if (nf > 0) t += c0 * u0;
-            if (nf > 1) t += c1 * u1;
-            hA[cr * lda + a] = log_cosh<T>(t);
+        for (int jb = 0; jb < HPT; jb += LB) {
+          T u0[LB], u1[LB];
+#pragma unroll
+          for (int j = 0; j < LB; ++j) {
+            u0[j] = u1[j] = (T)0;
+            if (GR * (jb + j) < left) {
+              u0[j] = w0[GR * (jb + j)];
+              u1[j] = w1[GR * (jb + j)];
+            }
           }
-          thn[j] = t;
+#pragma unroll
+          for (int j = 0; j < LB; ++j) {
+            T t = th[jb + j];
+            if (nf > 0) t += c0 * u0[j];
+            if (nf > 1) t += c1 * u1[j];
+            if (GR * (jb + j) < left) hA[cr * lda + g + GR * (jb + j)] = log_cosh<T>(t);
+            thn[jb + j] = t;
+          }
         }
       }
       __syncthreads();
-      rows_gemm(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
+      rows_gemm<NT / 64>(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
       if (tid < FF_ROWS) {
         const int r = tid;
         int acc = 0;
@@ -1062,14 +1039,14 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
         for (int j = 0; j < HPT; ++j) th[j] = thn[j];
         if (fast_exch) {
           // every other cluster at the two exchanged sites changes state; the
-          // chain's FF_GROUPS threads share its clusters
+          // chain's GR threads share its clusters
           const int s0 = psite[2 * cr], s1 = psite[2 * cr + 1];
           unsigned long long* dm = (unsigned long long*)(dmask + cr * NWc);
-          for (int e = adj_off[s0] + g; e < adj_off[s0 + 1]; e += FF_GROUPS) {
+          for (int e = adj_off[s0] + g; e < adj_off[s0 + 1]; e += GR) {
             const int t = adj_t[e], c = adj_c[e];
             if (t != s0 && t != s1) atomicXor(&dm[c >> 6], 1ull << (c & 63));
           }
-          for (int e = adj_off[s1] + g; e < adj_off[s1 + 1]; e += FF_GROUPS) {
+          for (int e = adj_off[s1] + g; e < adj_off[s1 + 1]; e += GR) {
             const int t = adj_t[e], c = adj_c[e];
             if (t != s0 && t != s1) atomicXor(&dm[c >> 6], 1ull << (c & 63));
           }
@@ -1079,7 +1056,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
     }
     if (sw >= sa.n_discard) {
       const int t = sw - sa.n_discard;
-      for (int idx = tid; idx < FF_ROWS * N; idx += FF_THREADS) {
+      for (int idx = tid; idx < FF_ROWS * N; idx += NT) {
         const int r = idx / N, i = idx % N;
         if (c0 + r < sa.C) samples[((int64_t)(c0 + r) * sa.chain_length + t) * N + i] = xs[idx];
       }
@@ -1088,7 +1065,7 @@ __global__ void __launch_bounds__(FF_THREADS) ffnn_metropolis_kernel(nka_ffnn m,
     }
     __syncthreads();
   }
-  for (int idx = tid; idx < FF_ROWS * N; idx += FF_THREADS) {
+  for (int idx = tid; idx < FF_ROWS * N; idx += NT) {
     const int r = idx / N, i = idx % N;
     if (c0 + r < sa.C) sigma[(int64_t)(c0 + r) * N + i] = xs[idx];
   }
@@ -1117,27 +1094,27 @@ static void allow_lds(K kernel, int64_t bytes) {
     (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-template <class T, int HPT>
+template <class T, int NT, int HPT, bool WEIGHTED>
 static void launch_ffnn_sweep(const nka_ffnn& m, const FfSweepArgs& sa, int8_t* sigma, void* lp, int8_t* smp,
                               void* lps, int64_t* nacc, hipStream_t s) {
   const unsigned g = (unsigned)((sa.C + FF_ROWS - 1) / FF_ROWS);
   const int ncl = (sa.rule == NKA_RULE_EXCHANGE && !sa.weights) ? sa.n_clusters : 0;
   const size_t lds = metropolis_lds<T>(m, ncl);
-  allow_lds(ffnn_metropolis_kernel<T, HPT>, (int64_t)lds);
-  hipLaunchKernelGGL((ffnn_metropolis_kernel<T, HPT>), dim3(g), dim3(FF_THREADS), lds, s, m, sa, sigma, (T*)lp,
+  allow_lds(ffnn_metropolis_kernel<T, NT, HPT, WEIGHTED>, (int64_t)lds);
+  hipLaunchKernelGGL((ffnn_metropolis_kernel<T, NT, HPT, WEIGHTED>), dim3(g), dim3(NT), lds, s, m, sa, sigma, (T*)lp,
                      smp, (T*)lps, nacc);
 }
 
-template <class T>
+// HPT: first-layer units per thread
+template <class T, int NT, bool WEIGHTED>
 static void dispatch_ffnn_sweep(const nka_ffnn& m, const FfSweepArgs& sa, int8_t* sigma, void* lp, int8_t* smp,
                                 void* lps, int64_t* nacc, hipStream_t s) {
-  const int need = (m.n_hidden1 + FF_GROUPS - 1) / FF_GROUPS;
-  if (need <= 8) launch_ffnn_sweep<T, 8>(m, sa, sigma, lp, smp, lps, nacc, s);
-  else if (need <= 16) launch_ffnn_sweep<T, 16>(m, sa, sigma, lp, smp, lps, nacc, s);
-  else if (need <= 32) launch_ffnn_sweep<T, 32>(m, sa, sigma, lp, smp, lps, nacc, s);
-  else if (need <= 56) launch_ffnn_sweep<T, 56>(m, sa, sigma, lp, smp, lps, nacc, s);
-  else if (need <= 64) launch_ffnn_sweep<T, 64>(m, sa, sigma, lp, smp, lps, nacc, s);
-  else launch_ffnn_sweep<T, 128>(m, sa, sigma, lp, smp, lps, nacc, s);
+  constexpr int MAXH = FF_MAXH / (NT / FF_ROWS);
+  const int need = (m.n_hidden1 + NT / FF_ROWS - 1) / (NT / FF_ROWS);
+  if (need <= MAXH / 8) launch_ffnn_sweep<T, NT, MAXH / 8, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
+  else if (need <= MAXH / 4) launch_ffnn_sweep<T, NT, MAXH / 4, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
+  else if (need <= MAXH / 2) launch_ffnn_sweep<T, NT, MAXH / 2, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
+  else launch_ffnn_sweep<T, NT, MAXH, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
 }
 
 static int check_model(const nka_ffnn* m, const char* who) {
@@ -1166,8 +1143,8 @@ static void launch_forward0(const nka_ffnn& m, const int8_t* x, int64_t rows, T*
   if (rows <= 0) return;
   const unsigned g = (unsigned)((rows + FF_ROWS - 1) / FF_ROWS);
   allow_lds(ffnn_forward_kernel<T, 0>, (int64_t)forward_lds<T>(m));
-  hipLaunchKernelGGL((ffnn_forward_kernel<T, 0>), dim3(g), dim3(FF_THREADS), forward_lds<T>(m), s, m, x,
-                     (const int8_t*)nullptr, 1, (const T*)nullptr, rows, lp, th, g2, (const int*)nullptr,
+  hipLaunchKernelGGL((ffnn_forward_kernel<T, 0>), dim3(g), dim3(FF_FWD), forward_lds<T>(m), s, m, x, 1,
+                     (const T*)nullptr, rows, lp, th, g2, (const int*)nullptr, (const uint64_t*)nullptr,
                      (const int*)nullptr);
 }
 
@@ -1189,8 +1166,7 @@ static int op_rows(int op_kind, const void* op, int N, int* K, int* mel_dtype) {
 // bytes per sample of the local-energy workspace
 static int64_t eloc_bytes_per_sample(const nka_ffnn& m, int K) {
   const int64_t ts = m.dtype == NKA_F32 ? 4 : 8;
-  return ffpad((int64_t)K * m.n_visible) + (int64_t)K * 8 + (int64_t)K * ts + (int64_t)m.n_hidden1 * ts + ts +
-         (int64_t)K * 4 + 4;
+  return (int64_t)K * 8 + (int64_t)K * 8 + (int64_t)K * ts + (int64_t)m.n_hidden1 * ts + ts + (int64_t)K * 4 + 4;
 }
 
 template <class T>
@@ -1211,7 +1187,7 @@ static int ffnn_eloc_impl(const nka_ffnn& m, int op_kind, const void* op, const 
     p += ffpad(bytes);
     return q;
   };
-  int8_t* xp = (int8_t*)take(chunk * K * N);
+  uint64_t* rsites = (uint64_t*)take(chunk * K * 8);
   void* mels = take(chunk * K * 8);
   T* lp = (T*)take(chunk * K * sizeof(T));
   T* th = (T*)take(chunk * H1 * sizeof(T));
@@ -1223,28 +1199,19 @@ static int ffnn_eloc_impl(const nka_ffnn& m, int op_kind, const void* op, const 
     const int64_t cs = std::min<int64_t>(chunk, n - s0);
     const int8_t* x = sigma + s0 * N;
     T* lp0 = log_psi ? log_psi + s0 : lp0own;
-    int st;
-    if (op_kind == NKA_OP_ISING) {
-      const nka_ising* o = (const nka_ising*)op;
-      st = nka_ising_conn(x, cs, N, o->edges, o->n_edges, o->h, o->J, o->mel_dtype, K, xp, mels, s);
-    } else {
-      st = nka_localop_conn(x, cs, N, (const nka_localop*)op, xp, mels, nullptr, s);
-    }
+    // the nonzero matrix elements only: slots are taken by one atomic add per
+    // sample, so the list order varies between runs, but every row's log psi is
+    // formed from that row alone, so the results do not
+    hipLaunchKernelGGL(ffnn_zero_count_kernel, dim3(1), dim3(64), 0, s, rcount);
+    int st = launch_conn_list(op_kind, op, x, cs, N, K, mels, ridx, rsites, rcount, s);
     if (st) return st;
     launch_forward0<T>(m, x, cs, lp0, th, nullptr, s);
     const int64_t rows = cs * K;
     const unsigned g = (unsigned)((rows + FF_ROWS - 1) / FF_ROWS);
-    hipLaunchKernelGGL(ffnn_zero_count_kernel, dim3(1), dim3(64), 0, s, rcount);
-    const unsigned gc = (unsigned)std::min<int64_t>((rows + 255) / 256, 8192);
-    if (md == NKA_F32)
-      hipLaunchKernelGGL((ffnn_compact_rows_kernel<float>), dim3(gc), dim3(256), 0, s, (const float*)mels, rows,
-                         ridx, rcount);
-    else
-      hipLaunchKernelGGL((ffnn_compact_rows_kernel<double>), dim3(gc), dim3(256), 0, s, (const double*)mels, rows,
-                         ridx, rcount);
     allow_lds(ffnn_forward_kernel<T, 1>, (int64_t)forward_lds<T>(m));
-    hipLaunchKernelGGL((ffnn_forward_kernel<T, 1>), dim3(g), dim3(FF_THREADS), forward_lds<T>(m), s, m, xp, x, K,
-                       (const T*)th, rows, lp, (T*)nullptr, (T*)nullptr, (const int*)ridx, (const int*)rcount);
+    hipLaunchKernelGGL((ffnn_forward_kernel<T, 1>), dim3(g), dim3(FF_FWD), forward_lds<T>(m), s, m,
+                       (const int8_t*)nullptr, K, (const T*)th, rows, lp, (T*)nullptr, (T*)nullptr, (const int*)ridx,
+                       (const uint64_t*)rsites, (const int*)rcount);
     const unsigned gr = (unsigned)((cs + 3) / 4);
     if (md == NKA_F32)
       hipLaunchKernelGGL((ffnn_eloc_reduce_kernel<T, float>), dim3(gr), dim3(256), 0, s, (const float*)mels,
@@ -1380,10 +1347,15 @@ int nka_ffnn_metropolis(const nka_ffnn* m, int rule, const int32_t* clusters, in
   NKA_CHECK_ARG(lds <= FF_LDS_MAX, "nka_ffnn_metropolis: %d clusters need %lld bytes of LDS (max %lld)",
                 n_clusters, (long long)lds, (long long)FF_LDS_MAX);
   hipStream_t s = (hipStream_t)stream;
-  if (m->dtype == NKA_F32)
-    dispatch_ffnn_sweep<float>(*m, sa, sigma, log_prob, samples, log_prob_samples, n_accepted, s);
+  const bool weighted = sa.rule == NKA_RULE_EXCHANGE && sa.weights;
+  if (m->dtype == NKA_F32 && !weighted)
+    dispatch_ffnn_sweep<float, 1024, false>(*m, sa, sigma, log_prob, samples, log_prob_samples, n_accepted, s);
+  else if (m->dtype == NKA_F32)
+    dispatch_ffnn_sweep<float, 512, true>(*m, sa, sigma, log_prob, samples, log_prob_samples, n_accepted, s);
+  else if (!weighted)
+    dispatch_ffnn_sweep<double, 512, false>(*m, sa, sigma, log_prob, samples, log_prob_samples, n_accepted, s);
   else
-    dispatch_ffnn_sweep<double>(*m, sa, sigma, log_prob, samples, log_prob_samples, n_accepted, s);
+    dispatch_ffnn_sweep<double, 512, true>(*m, sa, sigma, log_prob, samples, log_prob_samples, n_accepted, s);
   NKA_CHECK_LAUNCH("nka_ffnn_metropolis");
   return NKA_OK;
 }
@@ -1408,12 +1380,12 @@ int nka_ffnn_prepare(const nka_ffnn* m, const int8_t* sigma, int64_t ns, void* h
   if (m->dtype == NKA_F32) {
     launch_forward0<float>(*m, sigma, ns, (float*)lp, (float*)th, (float*)g2, s);
     allow_lds(ffnn_backprop_kernel<float>, (int64_t)backprop_lds<float>(*m));
-    hipLaunchKernelGGL((ffnn_backprop_kernel<float>), dim3(g), dim3(FF_THREADS), backprop_lds<float>(*m), s, *m,
+    hipLaunchKernelGGL((ffnn_backprop_kernel<float>), dim3(g), dim3(FF_BACK), backprop_lds<float>(*m), s, *m,
                        (const float*)th, (const float*)g2, ns, (float*)h1, (float*)d1);
   } else {
     launch_forward0<double>(*m, sigma, ns, (double*)lp, (double*)th, (double*)g2, s);
     allow_lds(ffnn_backprop_kernel<double>, (int64_t)backprop_lds<double>(*m));
-    hipLaunchKernelGGL((ffnn_backprop_kernel<double>), dim3(g), dim3(FF_THREADS), backprop_lds<double>(*m), s, *m,
+    hipLaunchKernelGGL((ffnn_backprop_kernel<double>), dim3(g), dim3(FF_BACK), backprop_lds<double>(*m), s, *m,
                        (const double*)th, (const double*)g2, ns, (double*)h1, (double*)d1);
   }
   NKA_CHECK_LAUNCH("nka_ffnn_prepare");

@@ -264,3 +264,63 @@ def test_vmc_sr_ffnn_tfim_converges(gpu):
     rel = abs(tail - e0) / abs(e0)
     print(f"E(last 20) = {tail:.6f} E0 = {e0:.6f} rel {rel:.2e}", flush=True)
     assert rel < 5e-3
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("N,H1,H2", [(9, 17, 33), (21, 130, 65), (12, 31, 97)])
+def test_local_energy_terms_of_one_to_four_sites(gpu, N, H1, H2, dtype):
+    # connected configurations that differ at up to four sites, more than one
+    # slab of 64 terms, rows with several elements per term, and second layers
+    # of 2, 3 and 4 column blocks (0 to 3 left over after whole rounds of four)
+    # with inner sizes that are not whole groups of 16
+    print(f"case ffnn eloc mixed terms N={N} H=({H1},{H2}) {np.dtype(dtype)}", flush=True)
+    rng = np.random.default_rng(N)
+    hi = nk.hilbert.Spin(0.5, N=N)
+    ops, aon = [], []
+    for k in range(72):
+        ns = 1 + k % 4
+        m = rng.normal(size=(2**ns, 2**ns)) * (rng.random((2**ns, 2**ns)) < 0.3)
+        ops.append(m + m.T + np.diag(rng.normal(size=2**ns)))
+        aon.append(sorted(rng.choice(N, ns, replace=False).tolist()))
+    H = nk.operator.LocalOperator(hi, ops, aon, constant=0.25)
+    terms = dict(zip([tuple(a) for a in H.acting_on], H.operators))
+    model, flat, p = _model(N, H1, H2, dtype, 3, 0.1)
+    x = rng.choice(np.array([-1, 1], dtype=np.int8), size=(67, N))
+    e, lp = eng.local_energies(model, flat, H, torch.as_tensor(x, device="cuda"), log_psi=True)
+    ref = of.local_energy(p, x, lambda z: O.local_conn(z, terms, constant=0.25))
+    tol = 1e-10 if dtype == np.float64 else 1e-4
+    np.testing.assert_allclose(e.cpu().numpy(), ref, rtol=tol, atol=tol * np.abs(ref).max())
+    np.testing.assert_allclose(lp.cpu().numpy(), of.log_psi(p, x), rtol=0,
+                               atol=_rtol(dtype) * np.abs(of.log_psi(p, x)).max())
+
+
+@pytest.mark.parametrize("rule", ["local", "exchange", "exchange-weighted"])
+@pytest.mark.parametrize("H1,H2,n_chains", [(20, 40, 5), (128, 70, 33), (257, 97, 64), (700, 33, 32)])
+def test_fp32_chains_carry_their_own_log_prob(gpu, rule, H1, H2, n_chains):
+    # every instance of the FP32 sampler (4 to 32 first-layer units per thread),
+    # second layers with 1 to 3 column blocks left over, partial chain groups:
+    # the chains' log-probabilities are those of their final configurations,
+    # and a second run from the same state repeats them bit for bit
+    print(f"case ffnn fp32 sampler {rule} H=({H1},{H2}) chains={n_chains}", flush=True)
+    N = 12
+    model, flat, p = _model(N, H1, H2, np.float32, 7, 0.1)
+    g = nk.graph.Chain(N)
+    if rule == "local":
+        sa = nk.sampler.MetropolisLocal(nk.hilbert.Spin(0.5, N=N), n_chains=n_chains)
+    else:
+        sa = nk.sampler.MetropolisExchange(nk.hilbert.Spin(0.5, N=N, total_sz=0), graph=g, d_max=2,
+                                           probabilities=[0.4, 1.0] if rule.endswith("weighted") else None,
+                                           n_chains=n_chains)
+    out = []
+    for _ in range(2):
+        st = sa.init_state(model, flat, seed=5)
+        samples, st = sa.sample_fused(model, flat, st, 2, 6)
+        out.append(samples.cpu().numpy())
+    np.testing.assert_array_equal(out[0], out[1])
+    assert st.n_accepted > 0
+    x = st.sigma.cpu().numpy()
+    np.testing.assert_array_equal(x, out[0][:, -1])
+    if rule != "local":
+        assert np.all(x.sum(axis=1) == 0)
+    ref = 2 * of.log_psi(p, x)
+    np.testing.assert_allclose(st.log_prob.cpu().numpy(), ref, rtol=0, atol=2e-5 * np.abs(ref).max())
