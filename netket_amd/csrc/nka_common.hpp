@@ -48,6 +48,35 @@ enum : uint32_t {
   TAG_RANDSTATE = 0x52414E44u,   // "RAND"
 };
 
+// The draws of a run of proposals of one chain, shared out over the LPC lanes
+// that work on it (groups of LPC lanes of a wavefront: one chain each): lane l
+// makes the draw of proposal base + l, so the ten rounds (40 quarter-rate integer
+// products, about 850 cycles of a SIMD) are issued once per LPC proposals instead
+// of once per proposal.  q has to be the same in every lane.
+template <int LPC>
+struct DrawBlock {
+  uint64_t base;
+  u32x4 r;
+
+  __device__ inline void refill(uint64_t q, uint32_t c, uint32_t k0, uint32_t k1) {
+    base = q;
+    const uint64_t ql = q + (uint64_t)(threadIdx.x & (LPC - 1));
+    r = philox4x32_10({(uint32_t)ql, (uint32_t)(ql >> 32), c, TAG_METROPOLIS}, k0, k1);
+  }
+  // The first three words of proposal q's draw, in every lane of the group.
+  __device__ inline u32x4 at(uint64_t q, uint32_t c, uint32_t k0, uint32_t k1) {
+    if (q - base >= (uint64_t)LPC) refill(q, c, k0, k1);
+    const int i = (int)(q - base);
+    if constexpr (LPC == NKA_WAVE) {
+      return {(uint32_t)__builtin_amdgcn_readlane((int)r.x, i), (uint32_t)__builtin_amdgcn_readlane((int)r.y, i),
+              (uint32_t)__builtin_amdgcn_readlane((int)r.z, i), 0u};
+    } else {
+      return {(uint32_t)__shfl((int)r.x, i, LPC), (uint32_t)__shfl((int)r.y, i, LPC),
+              (uint32_t)__shfl((int)r.z, i, LPC), 0u};
+    }
+  }
+};
+
 // Uniform in [0, 1) from the top 24 bits (float) or 53 bits (double).
 template <class T> __device__ inline T uniform01(const u32x4& r);
 template <> __device__ inline float uniform01<float>(const u32x4& r) {
@@ -77,9 +106,36 @@ template <> __device__ inline double log_cosh<double>(double x) {
   return ax + log1p(exp(-2.0 * ax)) - 0.69314718055994530942;
 }
 
+// exp(x) in FP64 for the amplitude ratios: x = n ln2 + r with |r| <= ln2 / 2,
+// the Taylor series of e^r to r^13 (remainder below 2^-57 of the sum) in even
+// and odd halves, then a power of two.  |x| is limited to 800, past which the
+// result is 0 or infinity anyway; a NaN stays one.  About 20 instructions
+// against about 40 of the library's.
+__device__ inline double exp_f64(double x) {
+  x = x < -800.0 ? -800.0 : (x > 800.0 ? 800.0 : x);
+  const double n = rint(x * 1.4426950408889634);
+  double r = fma(n, -0x1.62e42fefa39efp-1, x);
+  r = fma(n, -0x1.abc9e3b39803fp-56, r);
+  const double q = r * r;
+  double e = 1.0 / 479001600.0, o = 1.0 / 6227020800.0;
+  e = fma(e, q, 1.0 / 3628800.0);
+  o = fma(o, q, 1.0 / 39916800.0);
+  e = fma(e, q, 1.0 / 40320.0);
+  o = fma(o, q, 1.0 / 362880.0);
+  e = fma(e, q, 1.0 / 720.0);
+  o = fma(o, q, 1.0 / 5040.0);
+  e = fma(e, q, 1.0 / 24.0);
+  o = fma(o, q, 1.0 / 120.0);
+  e = fma(e, q, 0.5);
+  o = fma(o, q, 1.0 / 6.0);
+  e = fma(e, q, 1.0);
+  o = fma(o, q, 1.0);
+  return ldexp(fma(o, r, e), (int)n);
+}
+
 template <class T> __device__ inline T exp_t(T x);
 template <> __device__ inline float exp_t<float>(float x) { return __expf(x); }
-template <> __device__ inline double exp_t<double>(double x) { return exp(x); }
+template <> __device__ inline double exp_t<double>(double x) { return exp_f64(x); }
 
 template <class T> __device__ inline T log_t(T x);
 template <> __device__ inline float log_t<float>(float x) { return logf(x); }
@@ -113,6 +169,73 @@ template <> __device__ inline float wave_sum<float>(float v) {
   v += dpp_f32<0x142, 0xa, 0xf>(v);  // row_bcast:15
   v += dpp_f32<0x143, 0xc, 0xf>(v);  // row_bcast:31
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// Lane permutations that stay in the VALU: DPP inside a row of 16 lanes (quads,
+// mirrored half-rows and rows; once the lanes of a quad or half-row agree, a
+// mirror is an exchange with the other one) and the row swaps of gfx950.
+template <int CTRL>
+__device__ inline float dpp_perm(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ inline double dpp_perm(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
+}
+constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppHalfMirror = 0x141, kDppMirror = 0x140;
+
+// a <- rows (a0, b0, a2, b2), b <- rows (a1, b1, a3, b3) of 16 lanes.
+__device__ inline void swap_rows16(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ inline void swap_rows16(double& a, double& b) {
+  const auto l = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(a), (uint32_t)__double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane16_swap((uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b), false, false);
+  a = __hiloint2double((int)h[0], (int)l[0]);
+  b = __hiloint2double((int)h[1], (int)l[1]);
+}
+// a <- lanes (a 0-31, b 0-31), b <- lanes (a 32-63, b 32-63).
+__device__ inline void swap_halves(float& a, float& b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  a = __uint_as_float(r[0]);
+  b = __uint_as_float(r[1]);
+}
+__device__ inline void swap_halves(double& a, double& b) {
+  const auto l = __builtin_amdgcn_permlane32_swap((uint32_t)__double2loint(a), (uint32_t)__double2loint(b), false, false);
+  const auto h = __builtin_amdgcn_permlane32_swap((uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b), false, false);
+  a = __hiloint2double((int)h[0], (int)l[0]);
+  b = __hiloint2double((int)h[1], (int)l[1]);
+}
+
+// Sum (product) over the 16 lanes of a row, in every lane of it.
+template <class T>
+__device__ inline T row_sum(T v) {
+  v += dpp_perm<kDppXor1>(v);
+  v += dpp_perm<kDppXor2>(v);
+  v += dpp_perm<kDppHalfMirror>(v);
+  v += dpp_perm<kDppMirror>(v);
+  return v;
+}
+template <class T>
+__device__ inline T row_prod(T v) {
+  v *= dpp_perm<kDppXor1>(v);
+  v *= dpp_perm<kDppXor2>(v);
+  v *= dpp_perm<kDppHalfMirror>(v);
+  v *= dpp_perm<kDppMirror>(v);
+  return v;
+}
+template <> __device__ inline double wave_sum<double>(double v) {
+  v = row_sum(v);
+  double w = v;
+  swap_rows16(v, w);
+  v += w;
+  w = v;
+  swap_halves(v, w);
+  return v + w;
 }
 
 __device__ inline int lane_id() { return (int)(threadIdx.x & (NKA_WAVE - 1)); }

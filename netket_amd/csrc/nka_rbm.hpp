@@ -30,12 +30,23 @@ struct HiddenState {
   T th[JL];  // theta_j
   T lc[JL];  // log_cosh(theta_j)
 };
+// FP64: sum_j log_cosh(theta_j) = sum_j |theta_j| + log prod_j (1 + e^{-2|theta_j|})
+// - n log 2, so a lane keeps one logarithm for all its units and a proposal costs
+// one exponential per unit and one logarithm per lane.
+template <int JL>
+struct HiddenState<double, JL> {
+  double th[JL];
+  double lg;    // log of the product of 1 + e^{-2|theta_j|} over this lane's units (at most 2^64)
+  double nln2;  // number of this lane's units times log 2
+};
 
 // theta_j = b_j + sum_i s_i W_ij for this lane's hidden units.
 template <class T, int JL>
 __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, const T* W,
                                      const T* bias, int N, int M) {
   const int lane = lane_id();
+  T prod = (T)1;
+  int live = 0;
 #pragma unroll
   for (int jj = 0; jj < JL; ++jj) {
     const int j = lane + NKA_WAVE * jj;
@@ -47,11 +58,20 @@ __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, co
         acc += (xs[i] > 0) ? w : -w;
       }
       h.th[jj] = acc;
-      h.lc[jj] = log_cosh<T>(acc);
+      if constexpr (sizeof(T) == 4) {
+        h.lc[jj] = log_cosh<T>(acc);
+      } else {
+        prod = fma(prod, exp_f64(-2.0 * fabs(acc)), prod);
+        ++live;
+      }
     } else {
       h.th[jj] = (T)0;
-      h.lc[jj] = (T)0;
+      if constexpr (sizeof(T) == 4) h.lc[jj] = (T)0;
     }
+  }
+  if constexpr (sizeof(T) == 8) {
+    h.lg = log(prod);
+    h.nln2 = 0.69314718055994530942 * (double)live;
   }
 }
 
@@ -60,7 +80,11 @@ template <class T, int JL>
 __device__ inline T sum_log_cosh(const HiddenState<T, JL>& h) {
   T s = (T)0;
 #pragma unroll
-  for (int jj = 0; jj < JL; ++jj) s += h.lc[jj];
+  for (int jj = 0; jj < JL; ++jj) {
+    if constexpr (sizeof(T) == 4) s += h.lc[jj];
+    else s += fabs(h.th[jj]);
+  }
+  if constexpr (sizeof(T) == 8) s += h.lg - h.nln2;
   return wave_sum(s);
 }
 
@@ -74,14 +98,15 @@ __device__ inline T visible_term(const int8_t* xs, const T* a, int N) {
 }
 
 // Change of log psi when the spins at sites[0..nf) flip sign.  Fills the new
-// theta and log_cosh values into nth / nlc so a caller that accepts the move
-// can commit them without recomputation.
+// theta and log_cosh values (FP64: nlc[0], the lane's logarithm) into nth / nlc
+// so a caller that accepts the move can commit them without recomputation.
 template <class T, int JL>
 __device__ inline T flip_delta(const HiddenState<T, JL>& h, const int8_t* xs, const T* W,
                                const T* a, int N, int M, const int* sites, int nf, T* nth,
                                T* nlc) {
   const int lane = lane_id();
   T part = (T)0;
+  T prod = (T)1;
 #pragma unroll
   for (int jj = 0; jj < JL; ++jj) {
     const int j = lane + NKA_WAVE * jj;
@@ -93,14 +118,23 @@ __device__ inline T flip_delta(const HiddenState<T, JL>& h, const int8_t* xs, co
         d += (xs[s] > 0) ? -2 * w : 2 * w;
       }
       const T t = h.th[jj] + d;
-      const T l = log_cosh<T>(t);
       nth[jj] = t;
-      nlc[jj] = l;
-      part += l - h.lc[jj];
+      if constexpr (sizeof(T) == 4) {
+        const T l = log_cosh<T>(t);
+        nlc[jj] = l;
+        part += l - h.lc[jj];
+      } else {
+        prod = fma(prod, exp_f64(-2.0 * fabs(t)), prod);
+        part += fabs(t) - fabs(h.th[jj]);
+      }
     } else {
       nth[jj] = (T)0;
-      nlc[jj] = (T)0;
+      if constexpr (sizeof(T) == 4) nlc[jj] = (T)0;
     }
+  }
+  if constexpr (sizeof(T) == 8) {
+    nlc[0] = log(prod);
+    part += nlc[0] - h.lg;
   }
   T delta = wave_sum(part);
   if (a) {
@@ -110,6 +144,17 @@ __device__ inline T flip_delta(const HiddenState<T, JL>& h, const int8_t* xs, co
     }
   }
   return delta;
+}
+
+// The state after the move of flip_delta.
+template <class T, int JL>
+__device__ inline void commit_flip(HiddenState<T, JL>& h, const T* nth, const T* nlc) {
+#pragma unroll
+  for (int jj = 0; jj < JL; ++jj) {
+    h.th[jj] = nth[jj];
+    if constexpr (sizeof(T) == 4) h.lc[jj] = nlc[jj];
+  }
+  if constexpr (sizeof(T) == 8) h.lg = nlc[0];
 }
 
 template <class T>

@@ -15,7 +15,7 @@
 // The wavefront keeps theta_j and log_cosh(theta_j) of its chain in registers
 // (64 hidden units per register slot) and the spins in LDS, so a proposal
 // reads only the W rows of the flipped sites.
-#include "nka_rbm.hpp"
+#include "nka_sampler.hpp"
 
 namespace nka {
 
@@ -55,20 +55,6 @@ __global__ void random_states_kernel(int8_t* __restrict__ sigma, int C, int N, i
 // ---------------------------------------------------------------------------
 // Sweeps
 // ---------------------------------------------------------------------------
-constexpr int kMaxClusterSlots = 16;  // clusters per lane: n_clusters <= 1024
-
-struct SweepArgs {
-  int rule;
-  const int32_t* clusters;
-  int n_clusters;
-  const uint32_t* weights;      // exchange: integer weight per cluster (NULL: uniform)
-  int C, sweep_size, n_discard, chain_length;
-  double machine_pow;
-  uint32_t k0, k1;
-  uint64_t counter;
-  const uint64_t* counter_dev;  // when set, the counter is read from device memory
-};
-
 template <class T, int JL, bool STAGE>
 __device__ __forceinline__ void rbm_metropolis_kernel_body(const nka_rbm& m, const SweepArgs& sa, int8_t* __restrict__ sigma, T* __restrict__ log_prob, int8_t* __restrict__ samples, T* __restrict__ lp_samples, int64_t* __restrict__ n_accepted, int bx) {
   extern __shared__ unsigned char smem[];
@@ -118,18 +104,15 @@ __device__ __forceinline__ void rbm_metropolis_kernel_body(const nka_rbm& m, con
   }
   T nth[JL], nlc[JL];
   const int n_sweeps = sa.n_discard + sa.chain_length;
-  // the draw of the next proposal is computed one proposal ahead, so its
+  // the draw of the next proposal is read one proposal ahead, so its
   // latency overlaps the current proposal's reductions
-  u32x4 rnd_next = philox4x32_10({(uint32_t)q, (uint32_t)(q >> 32), (uint32_t)c, TAG_METROPOLIS},
-                                 sa.k0, sa.k1);
+  DrawBlock<NKA_WAVE> draws;
+  draws.refill(q, (uint32_t)c, sa.k0, sa.k1);
+  u32x4 rnd_next = draws.at(q, (uint32_t)c, sa.k0, sa.k1);
   for (int sw = 0; sw < n_sweeps; ++sw) {
     for (int p = 0; p < sa.sweep_size; ++p, ++q) {
       const u32x4 rnd = rnd_next;
-      {
-        const uint64_t qn = q + 1;
-        rnd_next = philox4x32_10({(uint32_t)qn, (uint32_t)(qn >> 32), (uint32_t)c, TAG_METROPOLIS},
-                                 sa.k0, sa.k1);
-      }
+      rnd_next = draws.at(q + 1, (uint32_t)c, sa.k0, sa.k1);
       int sites[2];
       int nf;
       T corr = (T)0;
@@ -242,11 +225,7 @@ __device__ __forceinline__ void rbm_metropolis_kernel_body(const nka_rbm& m, con
         const T u = uniform_value<T>(uniform01<T>(rnd));
         const bool acc = u < exp_t<T>(pw * delta + corr);
         if (acc) {
-#pragma unroll
-          for (int jj = 0; jj < JL; ++jj) {
-            h.th[jj] = nth[jj];
-            h.lc[jj] = nlc[jj];
-          }
+          commit_flip<T, JL>(h, nth, nlc);
           if (lane == 0) {
             for (int f = 0; f < nf; ++f) xs[sites[f]] = (int8_t)(-xs[sites[f]]);
           }
@@ -442,7 +421,7 @@ __global__ void __launch_bounds__(256) rbm_metropolis_wide_kernel_batched(const 
 }
 
 // ---------------------------------------------------------------------------
-// Several chains per wavefront.  For small RBMs (M <= 8 * 64/G hidden units)
+// Several FP32 chains per wavefront (FP64: nka_sampler64.hip).  For small RBMs (M <= 8 * 64/G hidden units)
 // a proposal's arithmetic is a few hundred instructions that the per-proposal
 // overhead (random draw, cluster bookkeeping, reduction, acceptance) would
 // dominate on a wavefront per chain.  Here the wavefront holds G chains, one
@@ -454,44 +433,12 @@ __global__ void __launch_bounds__(256) rbm_metropolis_wide_kernel_batched(const 
 // add the same two operands, so every lane of a group holds the identical sum.
 // Same random streams, rules and acceptance as rbm_metropolis_kernel.
 // ---------------------------------------------------------------------------
-template <int CTRL>
-__device__ inline float dpp_perm_f32(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-template <int CTRL>
-__device__ inline double dpp_perm_f64(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)(b & 0xffffffffLL), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, false);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-template <int CTRL, class T> __device__ inline T dpp_perm(T v);
-template <> __device__ inline float dpp_perm<0xb1, float>(float v) { return dpp_perm_f32<0xb1>(v); }
-template <> __device__ inline float dpp_perm<0x4e, float>(float v) { return dpp_perm_f32<0x4e>(v); }
-template <> __device__ inline float dpp_perm<0x141, float>(float v) { return dpp_perm_f32<0x141>(v); }
-template <> __device__ inline float dpp_perm<0x140, float>(float v) { return dpp_perm_f32<0x140>(v); }
-template <> __device__ inline double dpp_perm<0xb1, double>(double v) { return dpp_perm_f64<0xb1>(v); }
-template <> __device__ inline double dpp_perm<0x4e, double>(double v) { return dpp_perm_f64<0x4e>(v); }
-template <> __device__ inline double dpp_perm<0x141, double>(double v) { return dpp_perm_f64<0x141>(v); }
-template <> __device__ inline double dpp_perm<0x140, double>(double v) { return dpp_perm_f64<0x140>(v); }
-
-// Sum over the LPC lanes of this lane's group (LPC = 16 or 32), in every lane.
 // log of a small positive integer count: hardware log2 for FP32, log for FP64.
 template <class T> __device__ inline T log_fast(T x);
 template <> __device__ inline float log_fast<float>(float x) {
   return 0.69314718055994531f * __builtin_amdgcn_logf(x);
 }
 template <> __device__ inline double log_fast<double>(double x) { return log(x); }
-
-template <int LPC, class T>
-__device__ inline T group_sum(T v) {
-  v += dpp_perm<0xb1, T>(v);    // quad_perm [1,0,3,2]
-  v += dpp_perm<0x4e, T>(v);    // quad_perm [2,3,0,1]
-  v += dpp_perm<0x141, T>(v);   // row_half_mirror: quads 0 <-> 1 of each half-row
-  v += dpp_perm<0x140, T>(v);   // row_mirror: half-rows 0 <-> 1 of each row
-  if (LPC == 32) v += __shfl_xor(v, 16, NKA_WAVE);
-  return v;
-}
 
 template <class T, int G, int JG, int RSG, bool STAGE>
 __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& m, const SweepArgs& sa, int8_t* __restrict__ sigma, T* __restrict__ log_prob, int8_t* __restrict__ samples, T* __restrict__ lp_samples, int64_t* __restrict__ n_accepted, int bx) {
@@ -573,16 +520,13 @@ __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& 
         (uint64_t)uniform_value<uint32_t>((uint32_t)cd);
   }
   const int n_sweeps = sa.n_discard + sa.chain_length;
-  u32x4 rnd_next = philox4x32_10({(uint32_t)q, (uint32_t)(q >> 32), (uint32_t)c, TAG_METROPOLIS},
-                                 sa.k0, sa.k1);
+  DrawBlock<LPC> draws;
+  draws.refill(q, (uint32_t)c, sa.k0, sa.k1);
+  u32x4 rnd_next = draws.at(q, (uint32_t)c, sa.k0, sa.k1);
   for (int sw = 0; sw < n_sweeps; ++sw) {
     for (int p = 0; p < sa.sweep_size; ++p, ++q) {
       const u32x4 rnd = rnd_next;
-      {
-        const uint64_t qn = q + 1;
-        rnd_next = philox4x32_10({(uint32_t)qn, (uint32_t)(qn >> 32), (uint32_t)c, TAG_METROPOLIS},
-                                 sa.k0, sa.k1);
-      }
+      rnd_next = draws.at(q + 1, (uint32_t)c, sa.k0, sa.k1);
       int s0, s1 = 0, nf;
       T corr = (T)0;
       bool valid = true;
@@ -590,52 +534,10 @@ __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& 
         s0 = (int)bounded(rnd.x, (uint32_t)N);
         nf = 1;
       } else {
-        // differing clusters of this group's chain as a bit set in cluster
-        // order: cluster cl = gl + LPC * r is bit cl % 64 of word cl / 64
-        constexpr int NW = (RSG * LPC + 63) / 64;
-        uint64_t word[NW];
-        int8_t xu[RSG], xv[RSG];
-#pragma unroll
-        for (int w = 0; w < NW; ++w) word[w] = 0;
-#pragma unroll
-        for (int r = 0; r < RSG; ++r) {
-          xu[r] = cu[r] >= 0 ? xs[cu[r]] : (int8_t)0;
-          xv[r] = cu[r] >= 0 ? xs[cv[r]] : (int8_t)0;
-          const uint64_t gbits = (__ballot(xu[r] != xv[r]) >> (g * LPC)) & GMASK;
-          word[(LPC * r) / 64] |= gbits << ((LPC * r) % 64);
-        }
-        int n_diff = 0;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) n_diff += __popcll(word[w]);
-        valid = n_diff > 0;
-        int k = (int)bounded(rnd.x, (uint32_t)max(n_diff, 1));
-        int sel = 0;
-        bool found = false;
-#pragma unroll
-        for (int w = 0; w < NW; ++w) {
-          const int cnt = __popcll(word[w]);
-          if (!found && k < cnt) {
-            sel = 64 * w + kth_set_bit(word[w], k);
-            found = true;
-          } else if (!found) {
-            k -= cnt;
-          }
-        }
-        if (!valid || sel >= sa.n_clusters) sel = 0;
-        s0 = cl_s[2 * sel];
-        s1 = cl_s[2 * sel + 1];
+        int n_diff, n_new;
+        valid = group_exchange<LPC, RSG>(xs, cl_s, sa.n_clusters, cu, cv, g, rnd.x, s0, s1, n_diff, n_new);
         nf = 2;
-        // differing clusters after the swap (sigma'_u = sigma_v, sigma'_v = sigma_u)
-        const int8_t y0 = xs[s0], y1 = xs[s1];
-        int n_new = 0;
-#pragma unroll
-        for (int r = 0; r < RSG; ++r) {
-          const int a = cu[r], bb = cv[r];
-          const int8_t xa = a == s0 ? y1 : (a == s1 ? y0 : xu[r]);
-          const int8_t xb = bb == s0 ? y1 : (bb == s1 ? y0 : xv[r]);
-          n_new += __popcll((__ballot(a >= 0 && xa != xb) >> (g * LPC)) & GMASK);
-        }
-        corr = valid ? log_fast<T>((T)n_diff) - log_fast<T>((T)max(n_new, 1)) : (T)0;
+        corr = valid ? log_fast<T>((T)n_diff) - log_fast<T>((T)n_new) : (T)0;
       }
       // change of log psi with the new theta / log_cosh kept for a commit
       const int8_t x0 = xs[s0], x1 = xs[s1];
@@ -720,7 +622,7 @@ __global__ void advance_counter_kernel(uint64_t* __restrict__ c, uint64_t inc) {
 }
 
 // compute units of the current device (queried once per process)
-static int device_cus() {
+int device_cus() {
   static int cus = 0;
   if (cus == 0) {
     int dev = 0, n = 0;
@@ -803,8 +705,9 @@ template <int JL, class T>
 static void launch_sweep(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, T* lp, int8_t* smp,
                          T* lps, int64_t* nacc, const nka_sweep_job* jobs, int n_jobs, hipStream_t s) {
   const int waves = 4;
-  const int G = pick_group<T>(m, sa, waves);
-  if (G) {
+  if constexpr (sizeof(T) == 8) {
+    if (launch_group64(m, sa, sigma, lp, smp, lps, nacc, jobs, n_jobs, s)) return;
+  } else if (const int G = pick_group<T>(m, sa, waves)) {
     const int lpc = NKA_WAVE / G;
     const int need = (m.n_hidden + lpc - 1) / lpc;
     const int jg = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;

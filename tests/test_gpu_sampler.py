@@ -169,3 +169,42 @@ def test_mcstate_sample_shapes_and_reset(gpu):
     assert s2 is not s1
     acc = vs.sampler_state.acceptance
     assert 0.0 < acc <= 1.0
+
+
+@pytest.mark.parametrize("rule,N,alpha,n_chains,power", [
+    ("local", 16, 1, 5, 2.0),        # 16 units: four chains per wavefront, one unit a lane
+    ("local", 17, 1, 7, 1.0),        # 17 units: two chains; another machine power
+    ("exchange", 12, 5, 9, 2.0),     # 60 units, the last lanes without a second one
+    ("exchange", 16, 16, 3, 3.0),    # 256 units, the most of the grouped kernel
+    ("local", 100, 1, 33, 2.0),      # W of 80 KB: one workgroup of eight wavefronts per CU
+    ("local", 10, 30, 4, 2.0),       # 300 units: one chain per wavefront
+    ("exchange", 8, 40, 4, 1.0),
+])
+def test_fp64_chains_identical_to_oracle_over_sizes(gpu, rule, N, alpha, n_chains, power):
+    # 12 sweeps of 9 proposals cross the runs of 16, 32 and 64 draws shared out
+    # over a chain's lanes
+    print(f"case fp64 chains {rule} N={N} M={alpha * N} chains={n_chains} power={power}", flush=True)
+    model, flat, p = _model(N, alpha, np.float64, 11, 0.6 / np.sqrt(alpha * N))
+    if rule == "local":
+        sa = nk.sampler.MetropolisLocal(nk.hilbert.Spin(0.5, N=N), n_chains=n_chains, sweep_size=9,
+                                        machine_pow=power)
+        clusters = None
+    else:
+        sa = nk.sampler.MetropolisExchange(nk.hilbert.Spin(0.5, N=N, total_sz=0), graph=nk.graph.Chain(N),
+                                           n_chains=n_chains, sweep_size=9, machine_pow=power)
+        clusters = sa.rule.clusters
+    st = sa.init_state(model, flat, seed=21)
+    sigma0 = st.sigma.cpu().numpy().copy()
+    counter0 = st.counter
+    (samples, lps), st = sa.sample_fused(model, flat, st, 4, 8, return_log_probabilities=True)
+    ref, ref_sigma, ref_acc = osamp.metropolis(p, sigma0, rule=rule, clusters=clusters, n_discard=4,
+                                               chain_length=8, sweep_size=9, seed=21, counter=counter0,
+                                               machine_pow=power)
+    np.testing.assert_array_equal(samples.cpu().numpy(), ref)
+    np.testing.assert_array_equal(st.sigma.cpu().numpy(), ref_sigma)
+    np.testing.assert_array_equal(st.n_accepted_proc.cpu().numpy(), ref_acc)
+    # log psi is a sum of N M + M terms rounded to 2^-53 of their size
+    lp_ref = power * orbm.log_psi(p, ref.reshape(-1, N)).reshape(n_chains, 8)
+    tol = 1e-12 * np.abs(lp_ref).max()
+    np.testing.assert_allclose(lps.cpu().numpy(), lp_ref, rtol=0, atol=tol)
+    np.testing.assert_allclose(st.log_prob.cpu().numpy(), lp_ref[:, -1], rtol=0, atol=tol)
