@@ -105,6 +105,9 @@ __device__ __forceinline__ bool group_exchange(const int8_t* xs, const int32_t* 
 // or the rule does not fit it.
 bool launch_group64(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, double* lp, int8_t* smp, double* lps,
                     int64_t* nacc, const nka_sweep_job* jobs, int n_jobs, hipStream_t s);
+// FP32 local-rule sweeps with W in the caches (nka_sampler_wide.hip).
+void launch_wide(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, float* lp, int8_t* smp, float* lps,
+                 int64_t* nacc, const nka_sweep_job* jobs, int n_jobs, hipStream_t s);
 int device_cus();
 
 }  // namespace nka

@@ -208,3 +208,26 @@ def test_fp64_chains_identical_to_oracle_over_sizes(gpu, rule, N, alpha, n_chain
     tol = 1e-12 * np.abs(lp_ref).max()
     np.testing.assert_allclose(lps.cpu().numpy(), lp_ref, rtol=0, atol=tol)
     np.testing.assert_allclose(st.log_prob.cpu().numpy(), lp_ref[:, -1], rtol=0, atol=tol)
+
+
+@pytest.mark.parametrize("N,alpha,n_chains,sweep", [(130, 1, 5, 131), (150, 3, 9, 70), (200, 16, 4, 33)])
+def test_wide_model_chains_carry_their_own_log_prob(gpu, N, alpha, n_chains, sweep):
+    # W past LDS, unit counts that are no multiple of a wavefront (130 and 450:
+    # the last slots partly or wholly past the end) or fill 50 slots exactly
+    # (3200), odd sweeps (the two row buffers swap roles between sweeps): the
+    # running log-probability is that of the final configuration, and a second
+    # run repeats the chains
+    print(f"case wide sampler N={N} M={alpha * N} chains={n_chains} sweep={sweep}", flush=True)
+    model, flat, p = _model(N, alpha, np.float32, 13, 0.3 / np.sqrt(alpha * N))
+    sa = nk.sampler.MetropolisLocal(nk.hilbert.Spin(0.5, N=N), n_chains=n_chains, sweep_size=sweep)
+    out = []
+    for _ in range(2):
+        st = sa.init_state(model, flat, seed=3)
+        samples, st = sa.sample_fused(model, flat, st, 2, 5)
+        out.append(samples.cpu().numpy())
+    np.testing.assert_array_equal(out[0], out[1])
+    np.testing.assert_array_equal(st.sigma.cpu().numpy(), out[0][:, -1])
+    assert st.n_accepted > 0
+    ref = 2 * orbm.log_psi(p, st.sigma.cpu().numpy())
+    # 7 sweeps of accumulated FP32 steps
+    np.testing.assert_allclose(st.log_prob.cpu().numpy(), ref, rtol=0, atol=1e-4 * np.abs(ref).max())
