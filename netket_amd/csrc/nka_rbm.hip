@@ -11,6 +11,8 @@
 //                       (netket/jax/_jacobian/logic.py:356-373)
 #include "nka_rbm.hpp"
 
+#include <type_traits>
+
 namespace nka {
 
 // ---------------------------------------------------------------------------
@@ -53,6 +55,172 @@ __device__ inline double load_mel(const void* p, int64_t i, int dtype) {
   return dtype == NKA_F64 ? ((const double*)p)[i] : (double)((const float*)p)[i];
 }
 
+// Wavefronts per workgroup of the local energies: a staged FP64 W is shared by as
+// many as the registers of a CU hold (16 of up to 128, 8 of up to 256).
+template <class T, int JL, bool STAGE>
+constexpr int eloc_waves = sizeof(T) == 8 && STAGE && JL < 16 ? (JL <= 4 ? 16 : 8) : 4;
+
+// Up to 64 connected elements of one sample, one per lane: the sites that flip
+// (16 bits each, site | (x'_site > 0) << 15, 0xffff for none, in order), the matrix
+// element, and the change of the visible term (FP32: per site, added in order;
+// FP64: va[0], the sites' sum).
+template <class T>
+struct ElocEntry {
+  uint32_t s01, s23;
+  double mel;
+  T va[4];
+};
+
+// sum mel exp(log psi(x') - log psi(x)) over the entries of the lanes in
+// `mask`, added to E of the lanes of the four rows (E of a row's lanes agree).
+//
+// Four elements at a time: every lane forms its units' contribution to each, the
+// four sums share the cross-lane steps (a row of 16 lanes ends with one
+// element's), and one exponential per row serves all four.  FP32: the units'
+// log_cosh differences, summed over the lanes in the order 1, 2, 4, ..., 32.
+// FP64: sum |t| - |theta| and the product of (1 + e^{-2|t|}) / (1 + e^{-2|theta|})
+// (at most 2^960 over the lanes; with more than 15 units per lane, its logarithm),
+// one exponential per unit.
+//
+// Bound by the vector units (78% busy in FP64).  Heisenberg, 64 sites, 128 units,
+// 16384 samples, FP64: 0.17 ms; an element at a time, each with its own reduction
+// over the wavefront, its logarithms and W from the cache, 0.46 ms.  FP32: 0.12 and
+// 0.40 ms.
+template <class T, int JL>
+__device__ __forceinline__ void eloc_quads(uint64_t mask, const ElocEntry<T>& en, const HiddenState<T, JL>& h,
+                                           double rpr, const T* W, int M, bool visible, double& E) {
+  constexpr bool F64 = sizeof(T) == 8, LOG = F64 && JL > 15;
+  const int lane = lane_id(), row = lane >> 4;
+  while (mask) {
+    int l[4], n = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      if (mask) {
+        l[k] = __builtin_ctzll(mask);
+        mask &= mask - 1;
+        n = k + 1;
+      } else {
+        l[k] = l[0];
+      }
+    }
+    T part[4], rat[4];
+    uint32_t nmax = 1;
+    auto element = [&](int le, T& pe, T& re) __attribute__((always_inline)) {
+      const uint32_t s01 = (uint32_t)__builtin_amdgcn_readlane((int)en.s01, le);
+      const uint32_t s23 = (uint32_t)__builtin_amdgcn_readlane((int)en.s23, le);
+      T d[JL];
+#pragma unroll
+      for (int jj = 0; jj < JL; ++jj) d[jj] = (T)0;
+      auto flip = [&](uint32_t c, uint32_t nth) __attribute__((always_inline)) {
+        if (c == 0xffffu) return;
+        nmax = nmax > nth ? nmax : nth;
+        const T* w = W + (size_t)(c & 0x7fffu) * M + lane;
+        const T g = c & 0x8000u ? (T)2 : (T)-2;
+#pragma unroll
+        for (int jj = 0; jj < JL; ++jj) d[jj] += lane + NKA_WAVE * jj < M ? g * w[NKA_WAVE * jj] : (T)0;
+      };
+      flip(s01 & 0xffffu, 1);
+      flip(s01 >> 16, 2);
+      if (s23 != 0xffffffffu) {
+        flip(s23 & 0xffffu, 3);
+        flip(s23 >> 16, 4);
+      }
+      T A = (T)0, P = (T)1;
+#pragma unroll
+      for (int jj = 0; jj < JL; ++jj) {
+        const T t = h.th[jj] + d[jj];
+        if constexpr (F64) {
+          A += fabs(t) - fabs(h.th[jj]);
+          P = fma(P, exp_f64(-2.0 * fabs(t)), P);
+        } else {
+          A += lane + NKA_WAVE * jj < M ? log_cosh<T>(t) - h.lc[jj] : (T)0;
+        }
+      }
+      pe = A;
+      re = P * (T)rpr;
+      if constexpr (LOG) pe += log(re);
+    };
+    // unrolled while four elements' loads and exponentials fit in 128 registers
+    if constexpr (JL <= (F64 ? 2 : 4)) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) element(l[k], part[k], rat[k]);
+    } else {
+      // one element at a time; the registers of four are not there
+#pragma unroll
+      for (int k = 0; k < 4; ++k) part[k] = rat[k] = (T)0;
+#pragma unroll 1
+      for (int k = 0; k < 4; ++k) {
+        T pe, re;
+        const int le = l[0];
+        element(le, pe, re);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          l[i] = l[i + 1];
+          part[i] = part[i + 1];
+          rat[i] = rat[i + 1];
+        }
+        l[3] = le;
+        part[3] = pe;
+        rat[3] = re;
+      }
+    }
+    int el;
+    T tot, prod = (T)1;
+    if constexpr (F64) {
+      auto sum4 = [](double (&v)[4]) {
+        swap_halves(v[0], v[1]);
+        swap_halves(v[2], v[3]);
+        double x = v[0] + v[1], y = v[2] + v[3];
+        swap_rows16(x, y);
+        return row_sum(x + y);
+      };
+      tot = sum4(part);
+      if constexpr (!LOG) {
+        swap_halves(rat[0], rat[1]);
+        swap_halves(rat[2], rat[3]);
+        double x = rat[0] * rat[1], y = rat[2] * rat[3];
+        swap_rows16(x, y);
+        prod = row_prod(x * y);
+      }
+      el = (row >> 1) | ((row & 1) << 1);
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) part[k] = row_sum(part[k]);
+      swap_rows16(part[0], part[1]);
+      swap_rows16(part[2], part[3]);
+      T x = part[0] + part[1], y = part[2] + part[3];
+      swap_halves(x, y);
+      tot = x + y;
+      el = row;
+    }
+    const int src = el == 0 ? l[0] : el == 1 ? l[1] : el == 2 ? l[2] : l[3];
+    if constexpr (!F64) {
+      if (visible) {
+        tot += __shfl(en.va[0], src);
+        if (nmax > 1) tot += __shfl(en.va[1], src);
+        if (nmax > 2) {
+          tot += __shfl(en.va[2], src);
+          tot += __shfl(en.va[3], src);
+        }
+      }
+    }
+    const double mel = __shfl(en.mel, src);
+    double term;
+    if constexpr (F64) {
+      if (visible) tot += __shfl(en.va[0], src);
+      if (__any(fabs(tot) > 600.0)) {  // halves: finite wherever the whole is
+        const double hx = exp_f64(0.5 * tot);
+        term = mel * (hx * prod * hx);
+      } else {
+        term = mel * (exp_f64(tot) * prod);
+      }
+    } else {
+      term = mel * (double)exp_t<T>(tot);
+    }
+    if (el < n) E += term;
+  }
+}
+
 template <class T, int JL, bool STAGE>
 __device__ __forceinline__ void rbm_eloc_body(const nka_rbm& m, const OpArgs& op, const int8_t* __restrict__ sigma,
                                               int64_t n, double* __restrict__ eloc, T* __restrict__ log_psi,
@@ -78,77 +246,115 @@ __device__ __forceinline__ void rbm_eloc_body(const nka_rbm& m, const OpArgs& op
       const T lp = sum_log_cosh<T, JL>(h) + visible_term<T>(xs, v.a, N);
       if (lane == 0) log_psi[b] = lp;
     }
-    T nth[JL], nlc[JL];
-    double E = 0.0;
+    double rpr = 1.0;
+    if constexpr (sizeof(T) == 8) {
+      // a unit past the last has t = 0, a factor of two of its own
+      int dead = 0;
+#pragma unroll
+      for (int jj = 0; jj < JL; ++jj) dead += lane + NKA_WAVE * jj < M ? 0 : 1;
+      rpr = ldexp(1.0 / h.pr, -dead);
+    }
+    auto visible = [&](ElocEntry<T>& en) {
+      double sum = 0.0;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const uint32_t c = (k < 2 ? en.s01 : en.s23) >> (16 * (k & 1)) & 0xffffu;
+        en.va[k] = (T)0;
+        if (v.a && c != 0xffffu) en.va[k] = c & 0x8000u ? 2 * v.a[c & 0x7fffu] : -2 * v.a[c & 0x7fffu];
+        if constexpr (sizeof(T) == 8) sum += en.va[k];
+      }
+      if constexpr (sizeof(T) == 8) en.va[0] = sum;
+    };
+    double diag = 0.0, E = 0.0;
     if (op.kind == NKA_OP_ISING) {
       const nka_ising& is = op.ising;
       int zz = 0;
       for (int e = lane; e < is.n_edges; e += NKA_WAVE)
         zz += (xs[is.edges[2 * e]] == xs[is.edges[2 * e + 1]]) ? 1 : -1;
-      zz = wave_sum(zz);
+      zz = (int)wave_sum_u32((uint32_t)zz);
       // mel of row 0 is J * (integer sum) in the operator dtype
-      const double diag =
-          is.mel_dtype == NKA_F64 ? is.J * (double)zz : (double)((float)is.J * (float)zz);
-      E += diag;
+      diag = is.mel_dtype == NKA_F64 ? is.J * (double)zz : (double)((float)is.J * (float)zz);
       if (is.h != 0.0) {
         const double mh = is.mel_dtype == NKA_F64 ? -is.h : (double)(-(float)is.h);
-        for (int r = 0; r < N; ++r) {
-          const int sites[1] = {r};
-          const T d = flip_delta<T, JL>(h, xs, W, v.a, N, M, sites, 1, nth, nlc);
-          E += mh * (double)exp_t<T>(d);
+        for (int r0 = 0; r0 < N; r0 += NKA_WAVE) {
+          const int r = r0 + lane;
+          ElocEntry<T> en;
+          en.s01 = 0xffff0000u | (r < N ? (uint32_t)r | (xs[r] > 0 ? 0u : 0x8000u) : 0xffffu);
+          en.s23 = 0xffffffffu;
+          en.mel = mh;
+          visible(en);
+          eloc_quads<T, JL>(__ballot(r < N), en, h, rpr, W, M, v.a != nullptr, E);
         }
       }
     } else {
       const nka_localop& lo = op.local;
       // diagonal: constant + sum over terms of the selected row's diagonal element
       double dpart = 0.0;
-      for (int t = lane; t < lo.n_ops; t += NKA_WAVE) {
-        const int ns = lo.op_nsites[t];
-        int r = 0;
-        for (int k = 0; k < ns; ++k) r = 2 * r + (xs[lo.op_sites[4 * t + k]] < 0 ? 1 : 0);
-        dpart += load_mel(lo.row_diag, lo.op_row_off[t] + r, lo.mel_dtype);
-      }
-      const double diag = lo.constant + wave_sum(dpart);
-      if (lo.nonzero_diagonal && fabs(diag) > lo.mel_cutoff) E += diag;
-      for (int t = 0; t < lo.n_ops; ++t) {
-        const int ns = lo.op_nsites[t];
-        int st[4];
-        int r = 0;
-        for (int k = 0; k < ns; ++k) {
-          st[k] = lo.op_sites[4 * t + k];
-          r = 2 * r + (xs[st[k]] < 0 ? 1 : 0);
+      for (int t0 = 0; t0 < lo.n_ops; t0 += NKA_WAVE) {
+        const int t = t0 + lane;
+        int ns = 0, r = 0, nc = 0, off = 0;
+        int st[4] = {0, 0, 0, 0};
+        if (t < lo.n_ops) {
+          ns = lo.op_nsites[t];
+          for (int k = 0; k < ns; ++k) {
+            st[k & 3] = lo.op_sites[4 * t + k];
+            r = 2 * r + (xs[st[k & 3]] < 0 ? 1 : 0);
+          }
+          const int row = lo.op_row_off[t] + r;
+          dpart += load_mel(lo.row_diag, row, lo.mel_dtype);
+          nc = lo.row_nconn[row];
+          off = lo.row_conn_off[row];
         }
-        r = uniform_value<int>(r);
-        const int row = lo.op_row_off[t] + r;
-        const int nc = lo.row_nconn[row];
-        const int off = lo.row_conn_off[row];
-        for (int c = 0; c < nc; ++c) {
-          const int nidx = lo.conn_newidx[off + c];
-          int fl[4];
-          int nf = 0;
-          for (int k = 0; k < ns; ++k)
-            if ((((nidx ^ r) >> (ns - 1 - k)) & 1) != 0) fl[nf++] = st[k];
-          const T d = flip_delta<T, JL>(h, xs, W, v.a, N, M, fl, nf, nth, nlc);
-          E += load_mel(lo.conn_mel, off + c, lo.mel_dtype) * (double)exp_t<T>(d);
+        for (int c = 0; __any(c < nc); ++c) {
+          ElocEntry<T> en;
+          en.s01 = en.s23 = 0xffffffffu;
+          en.mel = 0.0;
+          if (c < nc) {
+            const int nidx = lo.conn_newidx[off + c];
+            uint64_t code = ~0ull;
+#pragma unroll
+            for (int k = 3; k >= 0; --k) {
+              if (k < ns) {
+                const int now = (nidx >> (ns - 1 - k)) & 1, was = (r >> (ns - 1 - k)) & 1;
+                if (now != was) code = (code << 16) | (uint64_t)((uint32_t)st[k] | (now ? 0u : 0x8000u));
+              }
+            }
+            en.s01 = (uint32_t)code;
+            en.s23 = (uint32_t)(code >> 32);
+            en.mel = load_mel(lo.conn_mel, off + c, lo.mel_dtype);
+          }
+          visible(en);
+          eloc_quads<T, JL>(__ballot(c < nc), en, h, rpr, W, M, v.a != nullptr, E);
         }
       }
+      const double dsum = lo.constant + wave_sum(dpart);
+      if (lo.nonzero_diagonal && fabs(dsum) > lo.mel_cutoff) diag = dsum;
     }
-    if (lane == 0) eloc[b] = E;
+    // the four rows' sums
+    double w = E;
+    swap_rows16(E, w);
+    E += w;
+    w = E;
+    swap_halves(E, w);
+    E += w;
+    if (lane == 0) eloc[b] = diag + E;
     wave_lds_sync();
   }
 }
 
 template <class T, int JL, bool STAGE>
-__global__ void __launch_bounds__(256) rbm_eloc_kernel(nka_rbm m, OpArgs op, const int8_t* __restrict__ sigma,
-                                                       int64_t n, double* __restrict__ eloc,
-                                                       T* __restrict__ log_psi) {
+__global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64)) rbm_eloc_kernel(nka_rbm m, OpArgs op,
+                                                                               const int8_t* __restrict__ sigma,
+                                                                               int64_t n, double* __restrict__ eloc,
+                                                                               T* __restrict__ log_psi) {
   rbm_eloc_body<T, JL, STAGE>(m, op, sigma, n, eloc, log_psi, blockIdx.x, gridDim.x);
 }
 
 // The local energies of a batch of jobs of one shape (Ising operators on the
 // same lattice, each with its own couplings): blockIdx.y selects the job.
 template <class T, int JL, bool STAGE>
-__global__ void __launch_bounds__(256) rbm_eloc_kernel_batched(const nka_eloc_job* __restrict__ jobs, int64_t n) {
+__global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64)) rbm_eloc_kernel_batched(
+    const nka_eloc_job* __restrict__ jobs, int64_t n) {
   const nka_eloc_job& j = jobs[blockIdx.y];
   OpArgs op{};
   op.kind = NKA_OP_ISING;
@@ -581,11 +787,24 @@ template <int JL, class T>
 static void launch_eloc(const nka_rbm& m, const OpArgs& op, const int8_t* sigma, int64_t n,
                         double* eloc, T* lp, hipStream_t s, const nka_eloc_job* jobs = nullptr,
                         int n_jobs = 0) {
-  const int waves = 4;
-  const bool stage = stage_fits<T>(m, waves);
-  const size_t lds = (stage ? pad16((size_t)m.n_visible * m.n_hidden * sizeof(T)) : 0) +
-                     waves * pad16(m.n_visible);
-  const unsigned g = grid_for(n, waves, 2048);
+  // W in LDS: FP32 up to 64 KB; FP64 up to 156 KB, one workgroup per CU.  Each
+  // workgroup stages W once, so a large W gets only the workgroups that run at once
+  // (FP64, 64 sites x 256 units, 8192 samples: 0.18 ms; with W from the cache 0.27 ms).
+  constexpr bool F64 = sizeof(T) == 8;
+  constexpr int sw = eloc_waves<T, JL, true>;
+  const size_t wb = pad16((size_t)m.n_visible * m.n_hidden * sizeof(T));
+  const bool stage = F64 ? wb + sw * pad16(m.n_visible) <= 156 * 1024 : stage_fits<T>(m, sw);
+  const int waves = stage ? sw : 4;
+  const size_t lds = (stage ? wb : 0) + waves * pad16(m.n_visible);
+  const unsigned g = grid_for(n, waves, F64 && stage && lds > 32 * 1024 ? 256 : 2048);
+  if constexpr (F64) {
+    if (stage && lds > 64 * 1024) {
+      (void)hipFuncSetAttribute((const void*)rbm_eloc_kernel<T, JL, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds);
+      (void)hipFuncSetAttribute((const void*)rbm_eloc_kernel_batched<T, JL, true>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    }
+  }
   if (jobs) {
     // fewer blocks per job when the batch fills the device anyway
     const unsigned gb = std::max<unsigned>(1, std::min<unsigned>(g, (unsigned)((4096 + n_jobs - 1) / n_jobs)));
@@ -616,99 +835,165 @@ static void launch_eloc_f64(const nka_rbm& m, const OpArgs& op, const int8_t* sg
 }
 
 // theta = sigma W + b for models whose W does not fit in LDS, as a tiled
-// matrix product: 64 samples x 64 hidden units per workgroup, K = N in steps
-// of 16 through LDS (sigma as exact +-1), so W is read once per 64 samples
-// instead of once per sample.  FP32 on v_mfma_f32_32x32x2f32 (one 32x32
-// block per wave), FP64 on v_mfma_f64_16x16x4f64 (2x2 blocks per wave).
-// The epilogue writes t = tanh(theta) to t (ns, M) and/or tT (M, ns).
+// matrix product without operand staging: 128 units x 128 samples per workgroup,
+// 64 x 64 per wavefront (W^T as the row operand, so that a lane's results are
+// samples side by side and the transposed output is written in whole lines).
+// FP32 on v_mfma_f32_32x32x2f32, FP64 on v_mfma_f64_16x16x4f64, k ascending.  The W
+// fragments come straight from the caches (16 bytes of it per product at most, 32
+// sites' loads in flight; rows past the last site read zero), the spins from a bit
+// set per sample in LDS.  The epilogue writes t = tanh(theta) to t (ns, M) and/or
+// tT (M, ns); RAW: theta itself to tT.
+// Bound by the matrix cores: FP32, 32768 samples x 400 sites x 3200 units, RAW,
+// 0.76 ms with its packed spins made by spin_bits_kernel (0.02 ms; 110 TFLOP/s, of
+// 149 for a large product), 1.18 ms as a product with both operands staged and the
+// samples as rows, 1.09 ms with every workgroup packing its own spins, which is
+// how the calls without a workspace run.
 typedef float ffx16 __attribute__((ext_vector_type(16)));
-constexpr int PG_T = 64, PG_K = 16;
+constexpr int PG_T = 128, PG_K = 1024;    // samples, units; sites whose spins are in LDS at once
+
+// bits[w][sample]: bit k of word w = (x_{32 w + k} > 0); 64 samples x 64 sites
+// per workgroup, a sample's 64 sites per load.
+__global__ void __launch_bounds__(256) spin_bits_kernel(const int8_t* __restrict__ sigma, int64_t ns, int N,
+                                                        uint32_t* __restrict__ bits) {
+  __shared__ uint32_t w[2][64];
+  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t s0 = (int64_t)blockIdx.x * 64;
+  const int k = blockIdx.y * 64 + lane;
+  const int8_t* col = sigma + min(k, N - 1);
+#pragma unroll 8
+  for (int r = wid; r < 64; r += 4) {
+    const uint64_t up = __ballot(k < N && col[min(s0 + r, ns - 1) * N] > 0);
+    if (lane < 2) w[lane][r] = (uint32_t)(up >> (32 * lane));
+  }
+  __syncthreads();
+  const int word = 2 * blockIdx.y + wid;
+  if (wid < 2 && 32 * word < N && s0 + lane < ns) bits[(int64_t)word * ns + s0 + lane] = w[wid][lane];
+}
 
 template <class T, bool RAW>
-__global__ void __launch_bounds__(256) rbm_prepare_gemm_kernel(nka_rbm m, const int8_t* __restrict__ sigma,
-                                                               int64_t ns, T* __restrict__ t, T* __restrict__ tT) {
-  __shared__ T sA[PG_T][PG_K + 1];
-  __shared__ T sB[PG_K][PG_T + 1];
+__global__ void __launch_bounds__(256, sizeof(T) == 8 ? 1 : 3) rbm_theta_kernel(
+    nka_rbm m, const int8_t* __restrict__ sigma, const uint32_t* __restrict__ bits, int64_t ns, T* __restrict__ t,
+    T* __restrict__ tT) {
+  __shared__ uint32_t sbits[PG_K / 32 * PG_T];  // [word][sample]: bit k % 32 of word k / 32 = (x_k > 0)
+  constexpr bool F64 = sizeof(T) == 8;
+  constexpr int E = F64 ? 16 : 32;        // block edge
+  constexpr int KS = F64 ? 4 : 2;         // sites per product
+  constexpr int NB = 64 / E;              // blocks per wavefront edge
+  constexpr int ACC = F64 ? 4 : 16;
+  using acc_t = typename std::conditional<F64, ddx4, ffx16>::type;
   const RbmView<T> v = rbm_view<T>(m);
   const int N = v.N, M = v.M;
   const int64_t s0 = (int64_t)blockIdx.x * PG_T;
   const int j0 = blockIdx.y * PG_T;
-  const int tid = threadIdx.x, wid = tid >> 6, lane = lane_id();
-  const int wm = (wid >> 1) * 32, wn = (wid & 1) * 32;
-  ffx16 accf;
-  ddx4 accd[2][2];
+  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
+  const int wu = (wid >> 1) * 64, ws = (wid & 1) * 64;
+  const bool active = s0 + ws < ns && j0 + wu < (RAW ? (M + 63) / 64 * 64 : M);
+  const int lc = lane % E, kh = lane / E;
+  int woff[NB];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) accf[e] = 0.0f;
+  for (int a = 0; a < NB; ++a) woff[a] = (kh * M + min(j0 + wu + a * E + lc, M - 1)) * (int)sizeof(T);
+  acc_t acc[NB][NB];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < NB; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) accd[a][b] = (ddx4){0.0, 0.0, 0.0, 0.0};
-  for (int k0 = 0; k0 < N; k0 += PG_K) {
-    __syncthreads();
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int idx = tid + it * 256;
-      const int r = idx >> 4, kc = idx & 15;            // A: 64 rows x 16 k
-      const int kk = k0 + kc;
-      T va = (T)0;
-      if (s0 + r < ns && kk < N) va = sigma[(s0 + r) * N + kk] > 0 ? (T)1 : (T)-1;
-      sA[r][kc] = va;
-      const int kr = idx >> 6, c = idx & 63;            // B: 16 k x 64 cols
-      T vb = (T)0;
-      if (k0 + kr < N && j0 + c < M) vb = v.W[(int64_t)(k0 + kr) * M + j0 + c];
-      sB[kr][c] = vb;
-    }
-    __syncthreads();
-    if constexpr (sizeof(T) == 4) {
+      for (int e = 0; e < ACC; ++e) acc[a][b][e] = (T)0;
+  constexpr int KB = 8;                   // sites per batch of W loads
+  constexpr int Q = KB / KS;
+  T wv[2][Q][NB];
+  auto load = [&](const __amdgpu_buffer_rsrc_t Wb, int k0, T (&w)[Q][NB]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int k = 0; k < PG_K; k += 2) {
-        const float a = sA[wm + (lane & 31)][k + (lane >> 5)];
-        const float b = sB[k + (lane >> 5)][wn + (lane & 31)];
-        accf = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, accf, 0, 0, 0);
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int a = 0; a < NB; ++a) {
+        const int soff = (k0 + q * KS) * M * (int)sizeof(T);
+        if constexpr (F64) {
+          const auto x = __builtin_amdgcn_raw_buffer_load_b64(Wb, woff[a], soff, 0);
+          w[q][a] = __builtin_bit_cast(double, x);
+        } else {
+          w[q][a] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(Wb, woff[a], soff, 0));
+        }
       }
-    } else {
+  };
+  auto group = [&](int k0, const uint32_t (&word)[NB], const T (&w)[Q][NB]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int k = 0; k < PG_K; k += 4) {
-        double av[2], bv[2];
+    for (int q = 0; q < Q; ++q) {
+      T sg[NB];
 #pragma unroll
-        for (int a = 0; a < 2; ++a) av[a] = sA[wm + a * 16 + (lane & 15)][k + (lane >> 4)];
+      for (int b = 0; b < NB; ++b) sg[b] = (word[b] >> ((k0 & 31) + q * KS + kh)) & 1u ? (T)1 : (T)-1;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) bv[b] = sB[k + (lane >> 4)][wn + b * 16 + (lane & 15)];
+      for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int a = 0; a < 2; ++a)
-#pragma unroll
-          for (int b = 0; b < 2; ++b)
-            accd[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], accd[a][b], 0, 0, 0);
-      }
-    }
-  }
-  // RAW: theta itself into tT, with the columns up to the next multiple of 64
-  // (zero beyond M) written too
-  const int Mp = (M + PG_T - 1) / PG_T * PG_T;
-  auto store = [&](int64_t sr, int j, T th) {
-    if (RAW) {
-      if (sr < ns && j < Mp) tT[(int64_t)j * ns + sr] = j < M ? th + (v.b ? v.b[j] : (T)0) : (T)0;
-    } else if (sr < ns && j < M) {
-      const T tv = tanh_t<T>(th + (v.b ? v.b[j] : (T)0));
-      if (t) t[sr * M + j] = tv;
-      if (tT) tT[(int64_t)j * ns + sr] = tv;
+        for (int b = 0; b < NB; ++b) {
+          if constexpr (F64) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[q][a], sg[b], acc[a][b], 0, 0, 0);
+          else acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[q][a], sg[b], acc[a][b], 0, 0, 0);
+        }
     }
   };
-  if constexpr (sizeof(T) == 4) {
-    // element e of lane l: row (e/4)*8 + (l/32)*4 + e%4, col l%32
+  for (int c0 = 0; c0 < N; c0 += PG_K) {
+    const int nk = min(PG_K, N - c0);
+    if (c0) __syncthreads();
+    if (RAW) {
+      const int nwc = (nk + 31) >> 5;
+      for (int e = tid; e < nwc * PG_T; e += 256)
+        sbits[e] = bits[(int64_t)(c0 / 32 + e / PG_T) * ns + min(s0 + e % PG_T, ns - 1)];
+    } else {
+      // 64 sites of a sample per load, one per lane; eight loads in flight
+      for (int k = 0; k < nk; k += 64) {
+        const bool in = k + lane < nk;
+        const int8_t* col = sigma + c0 + (in ? k + lane : 0);
+#pragma unroll 8
+        for (int r = wid; r < PG_T; r += 4) {
+          const uint64_t up = __ballot(in && s0 + r < ns && col[min(s0 + r, ns - 1) * N] > 0);
+          if (lane < 2) sbits[((k >> 5) + lane) * PG_T + r] = (uint32_t)(up >> (32 * lane));
+        }
+      }
+    }
+    __syncthreads();
+    if (!active) continue;
+    const __amdgpu_buffer_rsrc_t Wb = __builtin_amdgcn_make_buffer_rsrc(
+        (void*)(v.W + (size_t)c0 * M), 0, nk * M * (int)sizeof(T), 0x00020000);
+    load(Wb, 0, wv[0]);
+    for (int k1 = 0; k1 < nk; k1 += 32) {
+      uint32_t word[NB];
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      store(s0 + wm + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3), j0 + wn + (lane & 31), (T)accf[e]);
-  } else {
-    // element e of lane l in a 16x16 block: row l/16 + 4e, col l%16
+      for (int b = 0; b < NB; ++b) word[b] = sbits[(k1 >> 5) * PG_T + ws + b * E + lc];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          store(s0 + wm + a * 16 + (lane >> 4) + 4 * e, j0 + wn + b * 16 + (lane & 15), (T)accd[a][b][e]);
+      for (int g = 0; g < 32 / KB; ++g) {
+        load(Wb, k1 + (g + 1) * KB, wv[(g + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
+        group(g * KB, word, wv[g & 1]);
+      }
+    }
   }
+  if (!active) return;
+  // element e of lane l: FP32 row (e/4)*8 + (l/32)*4 + e%4, FP64 row l/16 + 4e;
+  // col (sample) l % E.  RAW also writes the rows up to the next multiple of 64
+  // (zero beyond M).
+  const int Mp = (M + 63) / 64 * 64;
+#pragma unroll
+  for (int a = 0; a < NB; ++a)
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      const int64_t sr = s0 + ws + b * E + lc;
+#pragma unroll
+      for (int e = 0; e < ACC; ++e) {
+        const int j = j0 + wu + a * E + (F64 ? kh + 4 * e : (e >> 2) * 8 + kh * 4 + (e & 3));
+        const T th = acc[a][b][e] + (v.b && j < M ? v.b[j] : (T)0);
+        if (RAW) {
+          if (sr < ns && j < Mp) tT[(int64_t)j * ns + sr] = j < M ? th : (T)0;
+        } else if (sr < ns && j < M) {
+          const T tv = tanh_t<T>(th);
+          if (t) t[sr * M + j] = tv;
+          if (tT) tT[(int64_t)j * ns + sr] = tv;
+        }
+      }
+    }
+}
+
+static dim3 theta_grid(int64_t ns, int units) {
+  return dim3((unsigned)((ns + PG_T - 1) / PG_T), (unsigned)((units + PG_T - 1) / PG_T));
 }
 
 template <int JL, class T>
@@ -717,8 +1002,8 @@ static void launch_prepare(const nka_rbm& m, const int8_t* sigma, int64_t ns, T*
   const int waves = 4;
   const bool stage = stage_fits<T>(m, waves);
   if (!stage) {
-    dim3 grid((unsigned)((ns + PG_T - 1) / PG_T), (unsigned)((m.n_hidden + PG_T - 1) / PG_T));
-    hipLaunchKernelGGL((rbm_prepare_gemm_kernel<T, false>), grid, dim3(256), 0, s, m, sigma, ns, t, tT);
+    hipLaunchKernelGGL((rbm_theta_kernel<T, false>), theta_grid(ns, m.n_hidden), dim3(256), 0, s,
+                       m, sigma, (const uint32_t*)nullptr, ns, t, tT);
     return;
   }
   const size_t lds = (stage ? pad16((size_t)m.n_visible * m.n_hidden * sizeof(T)) : 0) +
@@ -871,24 +1156,36 @@ __global__ void __launch_bounds__(256) ising_flip_tile_kernel(
   }
 }
 
-__global__ void __launch_bounds__(256) ising_flip_finish_kernel(const float* __restrict__ part,
-                                                                const double* __restrict__ diag,
-                                                                int64_t ns, int N, int n_jt, double mh,
-                                                                double* __restrict__ eloc,
-                                                                float* __restrict__ log_psi) {
-  const int64_t s = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (s >= ns) return;
-  double E = diag[s];
-  for (int i = 0; i < N; ++i) {
+// 64 samples per workgroup, the sites shared out over 16 wavefronts (one thread
+// per sample walking every site kept 2% of the chip's loads in flight: 1.94 ms
+// at 32768 x 400 x 13 partial sums, 0.68 GB).
+__global__ void __launch_bounds__(1024, 8) ising_flip_finish_kernel(const float* __restrict__ part,
+                                                                 const double* __restrict__ diag,
+                                                                 int64_t ns, int N, int n_jt, double mh,
+                                                                 double* __restrict__ eloc,
+                                                                 float* __restrict__ log_psi) {
+  __shared__ double red[16][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t s = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t sc = min(s, ns - 1);
+  auto total = [&](int i) {
+    const float* p = part + (int64_t)i * ns + sc;
+    const int64_t step = (int64_t)(N + 1) * ns;
     double d = 0.0;
-    for (int jt = 0; jt < n_jt; ++jt) d += (double)part[((int64_t)jt * (N + 1) + i) * ns + s];
-    E += mh * exp(d);
-  }
-  eloc[s] = E;
-  if (log_psi) {
-    double l = 0.0;
-    for (int jt = 0; jt < n_jt; ++jt) l += (double)part[((int64_t)jt * (N + 1) + N) * ns + s];
-    log_psi[s] = (float)l;
+#pragma unroll 7
+    for (int jt = 0; jt < n_jt; ++jt) d += (double)p[jt * step];
+    return d;
+  };
+  double E = 0.0;
+  for (int i = w; i < N; i += 16) E += mh * exp_f64(total(i));
+  red[w][lane] = E;
+  __syncthreads();
+  if (w == 0 && s < ns) {
+    E = diag[s];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) E += red[k][lane];
+    eloc[s] = E;
+    if (log_psi) log_psi[s] = (float)total(N);
   }
 }
 
@@ -941,13 +1238,16 @@ static int ising_tiled_eloc(const nka_rbm& m, const nka_ising& is, const int8_t*
   const size_t bits_lds = (size_t)(N + 31) / 32 * 64 * sizeof(uint32_t);
   for (int64_t c0 = 0; c0 < n; c0 += chunk) {
     const int64_t nc = min(chunk, n - c0);
-    dim3 gg((unsigned)((nc + PG_T - 1) / PG_T), (unsigned)(tl.Mp / PG_T));
-    hipLaunchKernelGGL((rbm_prepare_gemm_kernel<float, true>), gg, dim3(256), 0, s, m, sigma + c0 * N,
-                       nc, (float*)nullptr, thT);
+    // the packed spins are read before `part` is first written
+    uint32_t* bits = (uint32_t*)part;
+    hipLaunchKernelGGL(spin_bits_kernel, dim3((unsigned)((nc + 63) / 64), (unsigned)((N + 63) / 64)), dim3(256), 0, s,
+                       sigma + c0 * N, nc, N, bits);
+    hipLaunchKernelGGL((rbm_theta_kernel<float, true>), theta_grid(nc, tl.Mp), dim3(256), 0, s, m,
+                       (const int8_t*)nullptr, bits, nc, (float*)nullptr, thT);
     dim3 gf((unsigned)((nc + 63) / 64), (unsigned)tl.n_jt);
     hipLaunchKernelGGL(ising_flip_tile_kernel, gf, dim3(256), bits_lds, s, thT, Wp, sigma + c0 * N, nc, N,
                        tl.Mp, v.a, is, log_psi ? 1 : 0, part, diag);
-    hipLaunchKernelGGL(ising_flip_finish_kernel, dim3((unsigned)((nc + 255) / 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL(ising_flip_finish_kernel, dim3((unsigned)((nc + 63) / 64)), dim3(1024), 0, s,
                        part, diag, nc, N, tl.n_jt, mh, eloc + c0, log_psi ? log_psi + c0 : nullptr);
   }
   return NKA_OK;

@@ -36,7 +36,8 @@ struct HiddenState {
 template <int JL>
 struct HiddenState<double, JL> {
   double th[JL];
-  double lg;    // log of the product of 1 + e^{-2|theta_j|} over this lane's units (at most 2^64)
+  double pr;    // product of 1 + e^{-2|theta_j|} over this lane's units (at most 2^64)
+  double lg;    // its logarithm
   double nln2;  // number of this lane's units times log 2
 };
 
@@ -70,6 +71,7 @@ __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, co
     }
   }
   if constexpr (sizeof(T) == 8) {
+    h.pr = prod;
     h.lg = log(prod);
     h.nln2 = 0.69314718055994530942 * (double)live;
   }

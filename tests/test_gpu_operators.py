@@ -194,3 +194,76 @@ def test_local_energy_ising_tiled(gpu, lattice, alpha, scale, bias, n):
         nat.call("nka_rbm_local_energy", C.byref(m), kind, op_ptr, _ops.ptr(xt), n, _ops.ptr(e2), None,
                  None, 0, _ops.stream())
     del keep
+
+
+@pytest.mark.parametrize("kind,N,M,dtype", [
+    ("mixed", 9, 63, np.float64), ("mixed", 9, 70, np.float32),     # one to four sites flip; lanes without a unit
+    ("mixed", 9, 129, np.float64), ("mixed", 9, 255, np.float32),
+    ("ising", 71, 65, np.float64), ("ising", 130, 64, np.float32),  # more than 64 elements per sample
+    ("heis", 34, 260, np.float64),                                  # 71 KB of W in LDS
+    ("heis", 34, 598, np.float64),                                  # W beyond LDS, up to ten units per lane
+    ("ising", 16, 1056, np.float64), ("heis", 16, 1100, np.float64),  # logarithms per lane, W in LDS and not
+    ("heis", 20, 1100, np.float32), ("heis", 8, 3000, np.float32),
+])
+def test_local_energy_sizes(gpu, kind, N, M, dtype):
+    print(f"case eloc sizes {kind} N={N} M={M} {np.dtype(dtype)}", flush=True)
+    from netket_amd import _engine as eng
+    model, flat, p = _rbm_state(N, (M + 0.5) / N, dtype, 40 + M, scale=1.6 / np.sqrt(M))
+    assert p.W.shape == (N, M)
+    x = _states(N, 150, 41, n_down=N // 2)
+    hi = nk.hilbert.Spin(0.5, N=N)
+    if kind == "ising":
+        op = nk.operator.Ising(hi, nk.graph.Chain(N), h=0.9, J=1.1)
+        conn = lambda xx: O.ising_conn(xx, op.edges, 0.9, 1.1)
+    else:
+        if kind == "heis":
+            op = nk.operator.Heisenberg(hi, nk.graph.Chain(N))
+        else:
+            rng = np.random.default_rng(42)
+            op = nk.operator.LocalOperator(hi, constant=0.5)
+            for k in (1, 2, 3, 4, 4, 2):
+                s = [int(v) for v in rng.choice(N, size=k, replace=False)]
+                m = rng.normal(size=(2**k, 2**k))
+                m[np.abs(m) < 0.7] = 0
+                op += nk.operator.LocalOperator(hi, [m + m.T], [s])
+        terms = _terms(op)
+        conn = lambda xx: O.local_conn(xx, terms, constant=float(op.constant))
+    e, lp = eng.local_energies(model, flat, op, torch.as_tensor(x, device="cuda"), log_psi=True)
+    ref = orbm.local_energy(p, x, conn)
+    tol = 1e-10 if dtype == np.float64 else 1e-5
+    np.testing.assert_allclose(e.cpu().numpy(), ref, rtol=tol, atol=tol * np.abs(ref).max())
+    np.testing.assert_allclose(lp.cpu().numpy(), orbm.log_psi(p, x), rtol=tol, atol=tol)
+
+
+@pytest.mark.parametrize("N,M,n", [(1040, 70, 35), (1025, 20, 2)])
+def test_local_energy_ising_tiled_many_sites(gpu, N, M, n):
+    # spins beyond the first 1024 sites are packed in a second pass
+    print(f"case eloc ising tiled N={N} M={M}", flush=True)
+    from netket_amd import _engine as eng
+    model, flat, p = _rbm_state(N, (M + 0.5) / N, np.float32, 50, scale=0.02)
+    op = nk.operator.Ising(nk.hilbert.Spin(0.5, N=N), nk.graph.Chain(N), h=0.8, J=0.9, dtype=np.float32)
+    x = _states(N, n, 51)
+    ref = orbm.local_energy(p, x, lambda xx: O.ising_conn(xx, op.edges, 0.8, 0.9, np.float32))
+    e = eng.local_energies(model, flat, op, torch.as_tensor(x, device="cuda")).cpu().numpy()
+    np.testing.assert_allclose(e, ref, rtol=1e-5, atol=1e-5 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("N,M,ns,dtype", [(130, 127, 1, np.float32), (130, 129, 129, np.float32),
+                                          (1056, 66, 65, np.float32), (70, 130, 127, np.float64),
+                                          (1037, 17, 200, np.float64)])
+def test_activations_of_wide_models(gpu, N, M, ns, dtype):
+    # W beyond LDS: the tiled product, at the edges of its tiles and of its passes over the sites
+    print(f"case activations N={N} M={M} ns={ns} {np.dtype(dtype)}", flush=True)
+    import ctypes as C
+    from netket_amd import _native as nat, _ops
+    model, flat, p = _rbm_state(N, (M + 0.5) / N, dtype, 60, scale=0.5 / np.sqrt(N))
+    x = _states(N, ns, 61)
+    xt = torch.as_tensor(x, device="cuda")
+    t = torch.empty((ns, M), dtype=flat.dtype, device="cuda")
+    tT = torch.empty((M, ns), dtype=flat.dtype, device="cuda")
+    m = model.native(flat, N)
+    nat.call("nka_rbm_prepare", C.byref(m), _ops.ptr(xt), ns, _ops.ptr(t), _ops.ptr(tT), _ops.stream())
+    ref = np.tanh(x.astype(np.float64) @ p.W + p.b)
+    tol = 1e-13 if dtype == np.float64 else 1e-5  # sums of up to 1056 terms of about 0.02, |theta| < 3
+    np.testing.assert_allclose(t.cpu().numpy(), ref, rtol=0, atol=tol)
+    np.testing.assert_array_equal(tT.cpu().numpy(), t.cpu().numpy().T)
