@@ -15,6 +15,7 @@
 // nka_gemv_f64, nka_check_finite, nka_sgd_update, nka_centre_scale, nka_stats_moments
 //                  vector helpers of the step.
 #include "nka_common.hpp"
+#include "nka_panel.hpp"
 #include "netket_amd.h"
 #include <mutex>
 
@@ -22,7 +23,6 @@ namespace nka {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef double doublex4 __attribute__((ext_vector_type(4)));
 
 // Map a linear block id onto the lower-triangular tile pair (ti >= tj).
 __device__ inline void tri_tile(int64_t b, int& ti, int& tj) {
@@ -777,723 +777,6 @@ __global__ void __launch_bounds__(256) gemm_big_reduce_kernel(const double* __re
   }
 }
 
-// ---------------------------------------------------------------------------
-// Cholesky building blocks (block size 64).
-// ---------------------------------------------------------------------------
-constexpr int CH_NB = 64;
-
-constexpr int CH_LT = CH_NB + 2;  // LDS row stride of the transposed factor (16-byte rows)
-constexpr int TS_LD = CH_NB + 1;  // LDS row stride of a 64x64 block (doubles)
-constexpr int PF_ROWS = 16;  // rows of the panel per wavefront
-
-// Lane `src`'s value of v in every lane (src a compile-time constant after
-// unrolling).
-__device__ inline double readlane_f64(double v, int src) {
-  const int lo = __builtin_amdgcn_readlane(__double2loint(v), src);
-  const int hi = __builtin_amdgcn_readlane(__double2hiint(v), src);
-  return __hiloint2double(hi, lo);
-}
-
-// 1/sqrt(a) from the hardware estimate (about 2^-23 relative error) refined by
-// two Newton-Raphson steps y <- y + y (1/2 - (a/2) y^2), each of which squares
-// the relative error.
-__device__ inline double rsqrt_refined(double a) {
-  const double h = 0.5 * a;
-  double y = __builtin_amdgcn_rsq(a);
-  y = fma(y, fma(-(h * y), y, 0.5), y);
-  y = fma(y, fma(-(h * y), y, 0.5), y);
-  return y;
-}
-
-// Bounded wait of a wavefront for an LDS flag of its own workgroup set by
-// another wavefront (workgroup-scope acquire; every lane of the setter stores
-// the flag, so each lane's earlier LDS accesses are released).  The setter
-// always runs to its publication, so the wait ends; past the bound the
-// factorisation is reported as failed at this step (*info = k0 + 1) and the
-// wavefront goes on.  A factorisation already reported as failed (*info set,
-// possibly by another workgroup of the launch, after which a wavefront that
-// read it at its start has left) ends the wait too: its result is discarded.
-constexpr int64_t kLdsSpinLimit = 1LL << 24;
-__device__ inline void lds_wait(const int* flag, int32_t* info, int64_t k0) {
-  int64_t spins = 0;
-  while (__builtin_amdgcn_readfirstlane(__hip_atomic_load(const_cast<int*>(flag), __ATOMIC_ACQUIRE,
-                                                          __HIP_MEMORY_SCOPE_WORKGROUP)) == 0) {
-    __builtin_amdgcn_s_sleep(1);
-    ++spins;
-    // (a normal wait ends within a few hundred polls, before *info is read)
-    if (spins > 4096 && (spins & 255) == 0 &&
-        __builtin_amdgcn_readfirstlane(__hip_atomic_load(info, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0)
-      break;
-    if (spins > kLdsSpinLimit) {
-      if ((threadIdx.x & 63) == 0) atomicCAS(info, 0, (int32_t)(k0 + 1));
-      break;
-    }
-  }
-}
-
-// Publish an LDS flag of the workgroup (every lane stores it).
-__device__ inline void lds_publish(int* flag) {
-  __hip_atomic_store(flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-}
-
-// Factor a 64x64 block held in LDS (Ab, row-major, zeros above the diagonal)
-// in place with one wavefront, lane i = row i, by 16-column sub-panels:
-//  * sub-panel p (columns 16p..16p+15, rows 16p..63) is factored
-//    right-looking with the 16 values of each row in registers; at step j the
-//    pivot a_jj is read from its lane with v_readlane and the column entries
-//    a_cj of the sub-panel's rows c are broadcast through LDS (colbuf), and
-//    the update is a_ic -= L_ij L_cj = a_ij a_cj / a_jj, with 1/sqrt(a_jj)
-//    from the hardware estimate and two Newton steps;
-//  * the block's remaining lower part (rows and columns >= 16(p+1)) then
-//    receives the rank-16 update on FP64 MFMA (v_mfma_f64_16x16x4).
-// On return Ab holds L (exact zeros above the diagonal) and yv[j] = 1/L_jj.
-// With `done` (LDS, zeroed beforehand), done[p] is set with a workgroup-scope
-// release once columns 16p..16p+15 of L and their yv entries are final.
-// With `ready`, the blocks right of the first sub-panel are written by other
-// wavefronts during its factorisation: ready[0..2] are awaited before they
-// are first touched (the rank-16 update after sub-panel 0).
-// A non-positive or non-finite pivot is replaced by 1 so the factor
-// completes; the return value is then the first failing column + 1 + k0
-// (0 when every pivot is positive).
-__device__ __forceinline__ int factor_block_wave(double* Ab, double* colbuf, double* yv, int lane,
-                                                 int64_t k0, int* done = nullptr,
-                                                 const int* ready = nullptr, int32_t* info = nullptr) {
-  int bad = 0;
-#pragma unroll
-  for (int p = 0; p < 4; ++p) {
-    double x[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) x[q] = Ab[lane * TS_LD + 16 * p + q];
-    double ajj_next = readlane_f64(x[0], 16 * p);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int jj = 16 * p + j;
-      // the pivot comes from v_readlane values (the critical path), the
-      // rest of the column through LDS while the reciprocal square root is
-      // formed
-      colbuf[lane] = x[j];
-      const double ajj = ajj_next;
-      double a1 = 0.0, b1 = 0.0;
-      if (j < 15) {
-        a1 = readlane_f64(x[j], jj + 1);
-        b1 = readlane_f64(x[j + 1], jj + 1);
-      }
-      wave_lds_sync();
-      double cj[16];
-#pragma unroll
-      for (int q = j + 1; q < 16; ++q) cj[q] = colbuf[16 * p + q];
-      const bool ok = (ajj > 0.0) && isfinite(ajj);
-      if (!ok && bad == 0) bad = (int)(k0 + jj + 1);
-      const double piv = ok ? ajj : 1.0;
-      const double y = rsqrt_refined(piv);
-      // the next pivot: lane jj + 1 forms x[j+1] - (x[j] y^2) x[j] below with
-      // these same operations (one rounding for the multiply-subtract), so
-      // the value is the one that lane holds after this step
-      const double yy = y * y;
-      if (j < 15) ajj_next = fma(-(a1 * yy), a1, b1);
-      // every lane scales and updates: in rows jj and above the entries
-      // changed lie above the diagonal, which no later pivot or column
-      // broadcast reads and the write-back below replaces by zeros; row jj
-      // holds a_jj itself (the value the pivot was formed from)
-      const double sij = x[j] * yy;
-      x[j] *= y;
-      if (!ok && lane == jj) x[j] = piv * y;
-      if (lane == jj) yv[jj] = y;
-#pragma unroll
-      for (int q = j + 1; q < 16; ++q) x[q] -= sij * cj[q];
-      wave_lds_sync();
-    }
-#pragma unroll
-    for (int q = 0; q < 16; ++q) Ab[lane * TS_LD + 16 * p + q] = (16 * p + q <= lane) ? x[q] : 0.0;
-    wave_lds_sync();
-    // columns 16p..16p+15 of L and yv[16p..16p+15] are final from here on
-    // (the update below writes only later columns)
-    if (done != nullptr) lds_publish(&done[p]);
-    if (p == 0 && ready != nullptr) {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) lds_wait(&ready[i], info, k0);
-    }
-    // rank-16 update of the lower blocks (bi, bj), p < bj <= bi < 4
-#pragma unroll
-    for (int bi = p + 1; bi < 4; ++bi)
-#pragma unroll
-      for (int bj = p + 1; bj <= bi; ++bj) {
-        doublex4 acc = (doublex4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int kb = 0; kb < 16; kb += 4) {
-          const int kk = 16 * p + kb + (lane >> 4);
-          const double av = Ab[(bi * 16 + (lane & 15)) * TS_LD + kk];
-          const double bv = Ab[(bj * 16 + (lane & 15)) * TS_LD + kk];
-          acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
-        }
-        // element e of lane l is (row l/16 + 4e, col l%16) of the 16x16 block
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const int r = bi * 16 + (lane >> 4) + 4 * e, c = bj * 16 + (lane & 15);
-          Ab[r * TS_LD + c] -= acc[e];
-        }
-      }
-    wave_lds_sync();
-  }
-  return bad;
-}
-
-constexpr int MI_LD = 17;               // row stride of a 16x16 inverse block (doubles)
-constexpr int MI_SZ = 16 * MI_LD;       // one inverse block
-
-// Mi = L_pp^{-1} for the 16x16 diagonal sub-block p of L (Ls, row-major LDS;
-// rdiag[j] = 1/L_jj), stored row-major with row stride MI_LD.  One wavefront:
-// lane k (< 16) forms column k by forward substitution; lanes 16.. repeat the
-// work of lane & 15 and do not store.
-__device__ __forceinline__ void invert_diag16_wave(const double* Ls, const double* rdiag, double* Mi, int p,
-                                                   int lane) {
-  const int k = lane & 15;
-  double m[16];
-#pragma unroll
-  for (int i = 0; i < 16; ++i) m[i] = (i == k) ? 1.0 : 0.0;
-#pragma unroll
-  for (int j = 0; j < 16; ++j) {
-    m[j] *= rdiag[16 * p + j];
-#pragma unroll
-    for (int i = j + 1; i < 16; ++i) m[i] -= Ls[(16 * p + i) * TS_LD + 16 * p + j] * m[j];
-  }
-  if (lane < 16) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) Mi[i * MI_LD + k] = m[i];
-  }
-}
-
-// Block p of the solve of 16 rows of X (LDS, row-major) in place,
-// X <- X L^{-T}, with one wavefront on FP64 MFMA (v_mfma_f64_16x16x4, one
-// 16x16 accumulator): X_p -= X_{<p} L_{p,<p}^T, then X_p <- X_p (L_pp^{-1})^T
-// with the inverse of the diagonal sub-block (Mi + p * MI_SZ, from
-// invert_diag16_wave).  Ls = L (row-major, LDS).  Blocks must be applied in
-// order p = 0..3; columns 16p.. of L's rows 16p..16p+15 must be final.
-__device__ __forceinline__ void solve_block16_wave(const double* Ls, const double* Mi, double* X, int p,
-                                                   int lane) {
-  const int row = lane & 15;
-  if (p > 0) {
-    // X[:, 16p..16p+16) -= X[:, 0..16p) L[16p..16p+16, 0..16p)^T
-    doublex4 acc = (doublex4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int kb = 0; kb < 16 * p; kb += 4) {
-      const int kk = kb + (lane >> 4);
-      const double av = X[row * TS_LD + kk];
-      const double bv = Ls[(16 * p + row) * TS_LD + kk];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
-    }
-    // element e of lane l is (row l/16 + 4e, col l%16)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) X[((lane >> 4) + 4 * e) * TS_LD + 16 * p + row] -= acc[e];
-    wave_lds_sync();
-  }
-  // X_p <- X_p Mi_p^T: operand B[k][n] = Mi_p[n][k]
-  doublex4 acc = (doublex4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int kb = 0; kb < 16; kb += 4) {
-    const int kk = kb + (lane >> 4);
-    const double av = X[row * TS_LD + 16 * p + kk];
-    const double bv = Mi[p * MI_SZ + row * MI_LD + kk];
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
-  }
-  wave_lds_sync();  // every lane's operand reads of X_p precede the writes
-#pragma unroll
-  for (int e = 0; e < 4; ++e) X[((lane >> 4) + 4 * e) * TS_LD + 16 * p + row] = acc[e];
-  wave_lds_sync();
-}
-
-// Wavefronts 1-3 while wavefront 0 factors the diagonal block with
-// done = pflags[0..3]: wavefront p+1 inverts sub-block p (p < 3) of L11 once
-// it is published and announces the inverse in pflags[4+p]; every one of them
-// then applies block p of the solve to its 16-row strips (w - 1, and 3 for
-// wavefront 1).  Block 3 follows once the factor is done; the operations and
-// their order are those of applying blocks 0..3 one after another.
-__device__ __forceinline__ void solve_during_factor(const double* Ls, const double* rdiag, double* Mi,
-                                                    double (*Xs)[PF_ROWS * TS_LD], int* pflags, int w,
-                                                    int lane, int32_t* info, int64_t k0) {
-#pragma unroll
-  for (int p = 0; p < 3; ++p) {
-    if (w == p + 1) {
-      lds_wait(&pflags[p], info, k0);
-      invert_diag16_wave(Ls, rdiag, Mi + p * MI_SZ, p, lane);
-      lds_publish(&pflags[4 + p]);
-    }
-    lds_wait(&pflags[4 + p], info, k0);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int s = w - 1 + 3 * t;
-      if (s < 4) solve_block16_wave(Ls, Mi, Xs[s], p, lane);
-    }
-  }
-}
-
-// Factor the diagonal block A[k0:k0+nb, k0:k0+nb] in place (lower triangle)
-// with one wavefront; used for the last block, which has no rows below it.
-// The factor (64x64 row-major, identity padding past nb, zeros above the
-// diagonal) is also written to `slot`, where the inversion kernel reads it.
-// A non-positive or non-finite pivot sets *info (first failing column + 1).
-__global__ void __launch_bounds__(64) potf2_kernel(double* __restrict__ A, int64_t lda, int64_t n,
-                                                   int64_t k0, double* __restrict__ slot,
-                                                   int32_t* __restrict__ info) {
-  if (*info != 0) return;
-  __shared__ double Ab[CH_NB * TS_LD];   // the block, row-major
-  __shared__ double colbuf[CH_NB];
-  __shared__ double yv[CH_NB];
-  const int lane = threadIdx.x;
-  const int nb = (int)min<int64_t>(CH_NB, n - k0);
-  if (nb == CH_NB) {
-    // lane = column; all 64 row loads are issued before the first LDS store
-    const double* pc = A + k0 * lda + k0 + lane;
-    double v[CH_NB];
-#pragma unroll
-    for (int r = 0; r < CH_NB; ++r) v[r] = pc[r * lda];
-#pragma unroll
-    for (int r = 0; r < CH_NB; ++r) Ab[r * TS_LD + lane] = lane <= r ? v[r] : 0.0;
-  } else {
-    for (int idx = lane; idx < CH_NB * CH_NB; idx += 64) {
-      const int r = idx >> 6, c = idx & 63;
-      double v = (r == c) ? 1.0 : 0.0;
-      if (r < nb && c < nb && c <= r) v = A[(k0 + r) * lda + k0 + c];
-      Ab[r * TS_LD + c] = v;
-    }
-  }
-  wave_lds_sync();
-  const int bad = factor_block_wave(Ab, colbuf, yv, lane, k0);
-#pragma unroll 16
-  for (int r = 0; r < nb; ++r) {
-    const double v = Ab[r * TS_LD + lane];
-    if (lane < nb && lane <= r) A[(k0 + r) * lda + k0 + lane] = v;
-  }
-#pragma unroll
-  for (int r = 0; r < CH_NB; ++r) slot[r * CH_NB + lane] = Ab[r * TS_LD + lane];
-  if (lane == 0 && bad) atomicCAS(info, 0, bad);
-}
-
-// One 64-column step of the factorisation for a block with rows below it:
-// factor the diagonal block A[k0:k0+64, k0:k0+64] and solve the rows below,
-// L21 = A21 L11^{-T}, in place.  Every workgroup (four wavefronts of 16 rows,
-// 64 rows) reads the diagonal block and factors it in LDS itself (wavefront
-// 0), so the solve needs no second launch and no exchange through global
-// memory.  Workgroup 0 writes L11 to `slot` (64x64 row-major) and reports a
-// failed pivot in *info; L11 reaches A's diagonal block in the inversion
-// kernel at the end, since a workgroup that starts late still reads the
-// unfactored block from A.  All global loads of a workgroup are issued before
-// its first LDS store.  Rows past n re-read the last row and are not stored.
-
-__global__ void __launch_bounds__(256) panel_factor_kernel(double* __restrict__ A, int64_t lda, int64_t n,
-                                                           int64_t k0, double* __restrict__ slot,
-                                                           int32_t* __restrict__ info) {
-  if (*info != 0) return;
-  __shared__ double Ls[CH_NB * TS_LD];           // the diagonal block, then L11 (row-major)
-  __shared__ double colbuf[CH_NB];
-  __shared__ double rdiag[CH_NB];
-  __shared__ double Xs[4][PF_ROWS * TS_LD];      // 16 rows per wavefront
-  __shared__ double Mi[4 * MI_SZ];               // inverses of L11's diagonal 16x16 blocks
-  __shared__ int pflags[8];                      // sub-panels factored, inverses ready
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  double* X = Xs[w];
-  if (tid < 8) pflags[tid] = 0;                  // ordered by the barrier below
-  const int64_t r0 = k0 + CH_NB + (int64_t)blockIdx.x * (4 * PF_ROWS) + PF_ROWS * w;
-  {
-    // wavefront w reads rows 16w..16w+15 of the diagonal block and its own
-    // 16 rows, lanes along the columns
-    double vd[PF_ROWS], v[PF_ROWS];
-    const double* pd = A + (k0 + PF_ROWS * w) * lda + k0 + lane;
-#pragma unroll
-    for (int r = 0; r < PF_ROWS; ++r) vd[r] = pd[r * lda];
-#pragma unroll
-    for (int r = 0; r < PF_ROWS; ++r) v[r] = A[min<int64_t>(r0 + r, n - 1) * lda + k0 + lane];
-#pragma unroll
-    for (int r = 0; r < PF_ROWS; ++r) {
-      const int R = PF_ROWS * w + r;
-      Ls[R * TS_LD + lane] = lane <= R ? vd[r] : 0.0;
-    }
-#pragma unroll
-    for (int r = 0; r < PF_ROWS; ++r) X[r * TS_LD + lane] = v[r];
-  }
-  __syncthreads();
-  // wavefront 0 factors the diagonal block while wavefronts 1-3 solve blocks
-  // 0..2 of the four strips as its sub-panels are published
-  if (w == 0) {
-    const int bad = factor_block_wave(Ls, colbuf, rdiag, lane, k0, pflags);
-    if (blockIdx.x == 0 && lane == 0 && bad) atomicCAS(info, 0, bad);
-  } else {
-    solve_during_factor(Ls, rdiag, Mi, Xs, pflags, w, lane, info, k0);
-  }
-  __syncthreads();
-  if (blockIdx.x == 0) {
-    // wavefront w writes rows 16w..16w+15 of L11 (zeros above the diagonal)
-    // to the slot; A's diagonal block is left unchanged here because other
-    // workgroups of this launch may still be reading it
-#pragma unroll
-    for (int r = 0; r < PF_ROWS; ++r) {
-      const int R = PF_ROWS * w + r;
-      slot[R * CH_NB + lane] = Ls[R * TS_LD + lane];
-    }
-  }
-  // the last diagonal sub-block's inverse, then block 3 of each strip
-  if (w == 0) invert_diag16_wave(Ls, rdiag, Mi + 3 * MI_SZ, 3, lane);
-  __syncthreads();
-  solve_block16_wave(Ls, Mi, X, 3, lane);
-#pragma unroll
-  for (int r = 0; r < PF_ROWS; ++r) {
-    if (r0 + r < n) A[(r0 + r) * lda + k0 + lane] = X[r * TS_LD + lane];
-  }
-}
-
-// Update of the panel columns to the right of a 64-column step:
-// C[i][j] -= sum_{k<64} P[i][k] P[j][k] for i < rest, j < cols, where
-// P = A[k0+64.., k0..k0+64) holds the solved rows and C = A[k0+64.., k0+64..).
-// One 64x64 tile per workgroup.  The operand tiles and the C tile are read
-// with every load in flight (one memory latency per tile); the product runs on
-// 4 waves of 32x32 (2x2 v_mfma_f64_16x16x4) out of LDS in two K halves.
-// Rows and columns past the edge re-read the last valid one and are not stored.
-constexpr int PU_LD = 33;  // doubles per row of a 64x32 LDS half tile
-
-// One 64x64 tile of C - Pa Pb^T with K = 64: rows i0.. of Pa (clamped to ra
-// rows) against rows j0.. of Pb (clamped to rb rows) as the columns, C read at
-// C[(i0 + r) * lda + j0 + c] with the same clamps.  out[x][y][e] is element
-// (wm + 16x + l/16 + 4e, wn + 16y + l%16) of the tile, wave (wm, wn) of the
-// 2 x 2 wave grid.  All threads of the workgroup call it.
-__device__ __forceinline__ void pu_tile(const double* __restrict__ Pa, const double* __restrict__ Pb,
-                                        const double* __restrict__ C, int64_t lda, int64_t i0, int64_t j0,
-                                        int64_t ra, int64_t rb, double* sA, double* sB,
-                                        double out[2][2][4]) {
-  const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
-  const int wm = (wid >> 1) * 32, wn = (wid & 1) * 32;
-  // operand loads: wave w reads rows w, w+4, ... with lanes along k
-  double va[16], vb[16], vc[2][2][4];
-#pragma unroll
-  for (int it = 0; it < 16; ++it) {
-    const int r = wid + 4 * it;
-    va[it] = Pa[min<int64_t>(i0 + r, ra - 1) * lda + lane];
-    vb[it] = Pb[min<int64_t>(j0 + r, rb - 1) * lda + lane];
-  }
-  // C in the MFMA output layout: element e of lane l in a 16x16 block is
-  // (row l/16 + 4e, col l%16)
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t gi = min<int64_t>(i0 + wm + x * 16 + (lane >> 4) + 4 * e, ra - 1);
-        const int64_t gj = min<int64_t>(j0 + wn + y * 16 + (lane & 15), rb - 1);
-        vc[x][y][e] = C[gi * lda + gj];
-      }
-  doublex4 acc[2][2];
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = (doublex4){0.0, 0.0, 0.0, 0.0};
-  __syncthreads();  // the staging buffers may still be read by an earlier tile
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (h) __syncthreads();
-    if ((lane >> 5) == h) {
-#pragma unroll
-      for (int it = 0; it < 16; ++it) {
-        const int r = wid + 4 * it;
-        sA[r * PU_LD + (lane & 31)] = va[it];
-        sB[r * PU_LD + (lane & 31)] = vb[it];
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int ks = 0; ks < 32; ks += 4) {
-      const int kq = ks + (lane >> 4);
-      double av[2], bv[2];
-#pragma unroll
-      for (int x = 0; x < 2; ++x) av[x] = sA[(wm + x * 16 + (lane & 15)) * PU_LD + kq];
-#pragma unroll
-      for (int y = 0; y < 2; ++y) bv[y] = sB[(wn + y * 16 + (lane & 15)) * PU_LD + kq];
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-#pragma unroll
-        for (int y = 0; y < 2; ++y)
-          acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x], bv[y], acc[x][y], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) out[x][y][e] = vc[x][y][e] - acc[x][y][e];
-}
-
-// Block (bi, bj) of the previous step's rank-64 update of the diagonal block,
-// C - P P^T with K = 64, from P's rows staged in Pd (64 rows, stride TS_LD)
-// and the block's C values cv in the accumulator layout; written to Ls with
-// zeros above the diagonal.  The sums run in ascending K steps of 4, the
-// order of pu_tile.  One wavefront.
-__device__ __forceinline__ void diag_block_update(const double* Pd, double* Ls, int bi, int bj,
-                                                  const double cv[4], int lane) {
-  doublex4 acc = (doublex4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-  for (int kb = 0; kb < CH_NB; kb += 4) {
-    const int kk = kb + (lane >> 4);
-    const double av = Pd[(16 * bi + (lane & 15)) * TS_LD + kk];
-    const double bv = Pd[(16 * bj + (lane & 15)) * TS_LD + kk];
-    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av, bv, acc, 0, 0, 0);
-  }
-  // element e of lane l is (row l/16 + 4e, col l%16) of the block
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int R = 16 * bi + (lane >> 4) + 4 * e, c = 16 * bj + (lane & 15);
-    Ls[R * TS_LD + c] = c <= R ? cv[e] - acc[e] : 0.0;
-  }
-}
-
-// The lower blocks of the diagonal block right of its first 16 columns,
-// (1,1) (2,1) | (2,2) (3,1) | (3,2) (3,3), two for each of wavefronts 1-3.
-__device__ inline int rest_bi(int w, int t) { return w == 1 ? 1 + t : (w == 2 ? 2 + t : 3); }
-__device__ inline int rest_bj(int w, int t) { return w == 1 ? 1 : (w == 2 ? 2 - t : 2 + t); }
-
-// The previous step's update of the diagonal block (P rows 0..63, which must
-// all be valid rows) for its first 16 columns, which the factorisation needs
-// first: wavefront w updates block (w, 0).  P's rows are staged in Pd, the
-// zeros above the diagonal are written, and wavefronts 1-3 also load the C
-// values of their two further blocks into cr (applied by diag_block_update
-// during the factorisation of the first sub-panel).  All threads of the
-// workgroup call it; it ends with a barrier.
-__device__ __forceinline__ void diag_col0_update(const double* __restrict__ P, const double* __restrict__ C,
-                                                 int64_t lda, double* Pd, double* Ls, double cr[2][4]) {
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  double vb[16], c0[4];
-#pragma unroll
-  for (int it = 0; it < 16; ++it) vb[it] = P[(int64_t)(w + 4 * it) * lda + lane];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) c0[e] = C[(int64_t)(16 * w + (lane >> 4) + 4 * e) * lda + (lane & 15)];
-  if (w > 0) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int bi = rest_bi(w, t), bj = rest_bj(w, t);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-        cr[t][e] = C[(int64_t)(16 * bi + (lane >> 4) + 4 * e) * lda + 16 * bj + (lane & 15)];
-    }
-  }
-#pragma unroll
-  for (int it = 0; it < 16; ++it) Pd[(w + 4 * it) * TS_LD + lane] = vb[it];
-  // rows 16w..16w+15 right of their diagonal sub-block hold zeros
-  if (lane >= 16 * (w + 1)) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) Ls[(16 * w + r) * TS_LD + lane] = 0.0;
-  }
-  __syncthreads();
-  diag_block_update(Pd, Ls, w, 0, c0, lane);
-  __syncthreads();
-}
-
-// Rows 16s..16s+15 of the tile of rows i0.. of C - P P^T (K = 64; P rows
-// i0.. clamped to ra rows, against P rows 0..63 staged in Pd), for one
-// wavefront: out[y][e] is element ((l/16) + 4e, 16y + l%16) of the 16-row
-// strip, lane l.  The A operand is read from global memory in the MFMA's
-// layout; the sums run in the order of pu_tile.
-__device__ __forceinline__ void own_strip_update(const double* __restrict__ P, const double* __restrict__ C,
-                                                 int64_t lda, int64_t i0, int64_t ra, int s, const double* Pd,
-                                                 double out[4][4]) {
-  const int lane = threadIdx.x & 63;
-  double av[16], cv[4][4];
-  const double* pa = P + min<int64_t>(i0 + 16 * s + (lane & 15), ra - 1) * lda + (lane >> 4);
-#pragma unroll
-  for (int q = 0; q < 16; ++q) av[q] = pa[4 * q];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const double* pc = C + min<int64_t>(i0 + 16 * s + (lane >> 4) + 4 * e, ra - 1) * lda + (lane & 15);
-#pragma unroll
-    for (int y = 0; y < 4; ++y) cv[y][e] = pc[16 * y];
-  }
-#pragma unroll
-  for (int y = 0; y < 4; ++y) {
-    doublex4 acc = (doublex4){0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-      const double bv = Pd[(16 * y + (lane & 15)) * TS_LD + 4 * q + (lane >> 4)];
-      acc = __builtin_amdgcn_mfma_f64_16x16x4f64(av[q], bv, acc, 0, 0, 0);
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) out[y][e] = cv[y][e] - acc[e];
-  }
-}
-
-// C[i][j] -= sum_{k<64} Pa[i][k] Pb[j][k] over a grid of 64x64 tiles, stored
-// for i < rest, j < cols.
-__device__ __forceinline__ void pu_store_tile(const double* Pa, const double* Pb, double* C, int64_t lda,
-                                              int64_t tile, int64_t tiles_n, int64_t rest, int64_t cols,
-                                              double* sA, double* sB) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const int wm = (wid >> 1) * 32, wn = (wid & 1) * 32;
-  const int64_t i0 = (tile / tiles_n) * 64, j0 = (tile % tiles_n) * 64;
-  double out[2][2][4];
-  pu_tile(Pa, Pb, C, lda, i0, j0, rest, cols, sA, sB, out);
-#pragma unroll
-  for (int x = 0; x < 2; ++x)
-#pragma unroll
-    for (int y = 0; y < 2; ++y)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int64_t gi = i0 + wm + x * 16 + (lane >> 4) + 4 * e;
-        const int64_t gj = j0 + wn + y * 16 + (lane & 15);
-        if (gi < rest && gj < cols) C[gi * lda + gj] = out[x][y][e];
-      }
-}
-
-__global__ void __launch_bounds__(256) panel_update_kernel(double* __restrict__ A, int64_t lda, int64_t k0,
-                                                           int64_t rest, int64_t cols, int64_t tiles_n,
-                                                           int64_t n_tiles, const int32_t* __restrict__ info) {
-  if (*info != 0) return;
-  __shared__ double sA[CH_NB * PU_LD];
-  __shared__ double sB[CH_NB * PU_LD];
-  const int64_t bid = xcd_remap(blockIdx.x, gridDim.x);
-  if (bid >= n_tiles) return;
-  const double* P = A + (k0 + CH_NB) * lda + k0;
-  double* C = A + (k0 + CH_NB) * lda + k0 + CH_NB;
-  pu_store_tile(P, P, C, lda, bid, tiles_n, rest, cols, sA, sB);
-}
-
-// One 64-column step k0 of a panel after its first, in one launch with two
-// roles.  Workgroups [0, n_factor) work as panel_factor_kernel, except that
-// the previous step's rank-64 update of this step's columns is applied here:
-// to the diagonal block's first 16 columns by all four wavefronts before the
-// factorisation, to its further lower blocks and to the workgroup's own 64
-// rows by wavefronts 1-3 while wavefront 0 factors (same sums, in the same
-// order, as the panel update's tiles).  The other workgroups apply the previous step's update to
-// the panel's columns right of this step (panel_update_kernel's tiles, shifted
-// by 64 columns).  The roles write disjoint columns and read only what earlier
-// launches wrote, so the panel update no longer sits between two steps.
-__global__ void __launch_bounds__(256, 2) panel_step_kernel(double* __restrict__ A, int64_t lda, int64_t n,
-                                                         int64_t k0, int64_t n_factor, int64_t cols_b,
-                                                         int64_t tiles_n_b, double* __restrict__ slot,
-                                                         int32_t* __restrict__ info) {
-  if (*info != 0) return;
-  __shared__ double Ls[CH_NB * TS_LD];           // the diagonal block, then L11 (row-major)
-  __shared__ double colbuf[CH_NB];
-  __shared__ double rdiag[CH_NB];
-  __shared__ double Xs[4][PF_ROWS * TS_LD];      // 16 rows per wavefront
-  __shared__ double Mi[4 * MI_SZ];               // inverses of L11's diagonal 16x16 blocks
-  // LDS flags: [0..3] sub-panels factored, [4..6] their inverses, [8..10]
-  // the diagonal block's further blocks updated and [12..14] the own strips
-  // updated (wavefronts 1-3)
-  __shared__ int pflags[16];
-  double* sA = Ls;                               // staging of the update tiles (before Ls is filled)
-  double* sB = &Xs[0][0];
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63;
-  const int64_t kp = k0 - CH_NB;                 // the previous step
-  const double* P = A + k0 * lda + kp;           // rows k0.. of the previous step's columns
-  const int64_t rest_p = n - k0;                 // rows of P
-  if ((int64_t)blockIdx.x >= n_factor) {
-    const int64_t tile = (int64_t)blockIdx.x - n_factor;
-    // columns k0 + 64 .. of the panel: B operand rows k0 + 64 ..
-    pu_store_tile(P, P + CH_NB * lda, A + k0 * lda + k0 + CH_NB, lda, tile, tiles_n_b, rest_p, cols_b, sA, sB);
-    return;
-  }
-  // diagonal block (rows and columns k0 .. k0+63) first: the launch has rows
-  // below this step, so rest_p > 64 and P rows 0..63 are valid.  P rows
-  // 0..63 are staged in the Xs region, which the factorisation does not use.
-  double* Pd = &Xs[0][0];
-  const double* Ck = A + k0 * lda + k0;
-  if (tid < 16) pflags[tid] = 0;                 // ordered by the barriers below
-  double cr[2][4];
-  diag_col0_update(P, Ck, lda, Pd, Ls, cr);
-  double* X = Xs[w];
-  const int64_t own0 = CH_NB + (int64_t)blockIdx.x * (4 * PF_ROWS);   // relative to k0
-  const int64_t r0 = k0 + own0 + PF_ROWS * w;
-  // wavefront 0 factors the diagonal block; meanwhile wavefronts 1-3 update
-  // its further lower blocks (awaited before the factor first touches them),
-  // update this workgroup's 16-row strips (w - 1, and 3 for wavefront 1) in
-  // registers, store them once none of them reads Pd any more, and solve
-  // their blocks 0..2 as the factor publishes its sub-panels
-  if (w == 0) {
-    const int bad = factor_block_wave(Ls, colbuf, rdiag, lane, k0, pflags, &pflags[8], info);
-    if (blockIdx.x == 0 && lane == 0 && bad) atomicCAS(info, 0, bad);
-  } else {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) diag_block_update(Pd, Ls, rest_bi(w, t), rest_bj(w, t), cr[t], lane);
-    lds_publish(&pflags[7 + w]);
-    double ow[2][4][4];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int s = w - 1 + 3 * t;
-      if (s < 4) own_strip_update(P, Ck, lda, own0, rest_p, s, Pd, ow[t]);
-    }
-    lds_publish(&pflags[11 + w]);
-#pragma unroll
-    for (int i = 12; i < 15; ++i) lds_wait(&pflags[i], info, k0);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      const int s = w - 1 + 3 * t;
-      if (s < 4) {
-#pragma unroll
-        for (int y = 0; y < 4; ++y)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) Xs[s][((lane >> 4) + 4 * e) * TS_LD + 16 * y + (lane & 15)] = ow[t][y][e];
-      }
-    }
-    wave_lds_sync();
-    solve_during_factor(Ls, rdiag, Mi, Xs, pflags, w, lane, info, k0);
-  }
-  __syncthreads();  // the factor and blocks 0..2 of every strip are done
-  if (blockIdx.x == 0) {
-#pragma unroll
-    for (int r = 0; r < PF_ROWS; ++r) {
-      const int R = PF_ROWS * w + r;
-      slot[R * CH_NB + lane] = Ls[R * TS_LD + lane];
-    }
-  }
-  if (w == 0) invert_diag16_wave(Ls, rdiag, Mi + 3 * MI_SZ, 3, lane);
-  __syncthreads();
-  solve_block16_wave(Ls, Mi, X, 3, lane);
-#pragma unroll
-  for (int r = 0; r < PF_ROWS; ++r) {
-    if (r0 + r < n) A[(r0 + r) * lda + k0 + lane] = X[r * TS_LD + lane];
-  }
-}
-
-// inv_b = L_bb^{-1} for every 64x64 diagonal block b of the factor; one
-// wavefront per block.  The factored block is read from its slot in `inv`
-// (row-major, identity padding, zeros above the diagonal), copied into A's
-// diagonal block, and replaced by its inverse (row-major): lane k computes
-// column k by substitution with the block's columns broadcast from LDS.
-__global__ void __launch_bounds__(64) trtri_blocks_kernel(double* __restrict__ A, int64_t lda, int64_t n,
-                                                          double* __restrict__ inv,
-                                                          const int32_t* __restrict__ info) {
-  if (*info != 0) return;
-  __shared__ double LT[CH_NB * CH_LT];
-  __shared__ double rdiag[CH_NB];
-  const int k = threadIdx.x;
-  const int64_t k0 = (int64_t)blockIdx.x * CH_NB;
-  const int nb = (int)min<int64_t>(CH_NB, n - k0);
-  double* blk = inv + (int64_t)blockIdx.x * CH_NB * CH_NB;
-  {
-    // lane = column; all row loads in flight before the stores
-    double v[CH_NB];
-#pragma unroll
-    for (int r = 0; r < CH_NB; ++r) v[r] = blk[r * CH_NB + k];
-#pragma unroll
-    for (int r = 0; r < CH_NB; ++r) LT[k * CH_LT + r] = v[r];
-#pragma unroll
-    for (int r = 0; r < CH_NB; ++r)
-      if (r < nb && k < nb && k <= r) A[(k0 + r) * lda + k0 + k] = v[r];
-  }
-  wave_lds_sync();
-  rdiag[k] = 1.0 / LT[k * CH_LT + k];
-  wave_lds_sync();
-  double x[CH_NB];
-#pragma unroll
-  for (int r = 0; r < CH_NB; ++r) x[r] = (r == k) ? 1.0 : 0.0;
-#pragma unroll
-  for (int m = 0; m < CH_NB; ++m) {
-    const double xm = x[m] * rdiag[m];
-    x[m] = xm;
-#pragma unroll
-    for (int r = m + 1; r < CH_NB; ++r) x[r] -= xm * LT[m * CH_LT + r];
-  }
-#pragma unroll
-  for (int r = 0; r < CH_NB; ++r) blk[r * CH_NB + k] = x[r];
-}
-
 // Zero n 32-bit words (a fill kernel rather than a memset node, so that a
 // captured graph replays it correctly).
 __global__ void zero_u32_kernel(uint32_t* __restrict__ p, int64_t n) {
@@ -1510,17 +793,13 @@ __global__ void zero_u32_kernel(uint32_t* __restrict__ p, int64_t n) {
 // that exceeds the spin bound sets *err and the workgroup proceeds (the
 // result is then invalid and reported as such by the caller).
 //
-// The solved entries are their own flags: the output vector is filled with
-// kUnsolved before the launch, each entry is written once, as a 64-bit
-// atomic store, and a reader polls the entries it needs with 64-bit atomic
-// loads until none holds kUnsolved.  One memory round trip per dependency,
-// and no ordering between different entries is needed.  kUnsolved is a
-// signalling NaN, which arithmetic never returns; a value with its bit
-// pattern would be published as the default NaN all the same.
+// The solved entries are their own flags: the output vector holds kUnsolved
+// before the launch, each entry is written once, as a 64-bit atomic store, and a
+// reader polls the entries it needs with 64-bit atomic loads until none holds
+// kUnsolved.  One memory round trip per dependency, and no ordering between
+// different entries is needed.
 // ---------------------------------------------------------------------------
 constexpr int64_t kSpinLimit = 1LL << 26;
-constexpr uint64_t kUnsolved = 0x7FF4D15EA5E0F00DULL;
-constexpr uint64_t kDefaultNaN = 0x7FF8000000000000ULL;
 
 // The entry *p (lanes with active), polled with relaxed agent-scope loads
 // (they read the L2 copy); inactive lanes get 0.  Wave-uniform loop.
@@ -1545,130 +824,152 @@ __device__ inline void publish_entry(double* p, double v) {
   __hip_atomic_store((uint64_t*)p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-__global__ void fill_unsolved_kernel(uint64_t* __restrict__ p, int64_t n) {
-  for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n;
-       k += (int64_t)gridDim.x * blockDim.x)
-    p[k] = kUnsolved;
+// a b += y_c L[c], c = 0..15, y_c that of lane c of the lane's row of 16 (two sums).
+__device__ __forceinline__ void row_dot16(double& a, double& b, double y, const double (&L)[16]) {
+#define NKA_ROW_FMAC(acc, n, c) "v_fmac_f64_dpp %" #acc ", %2, %" #n " row_newbcast:" #c " row_mask:0xf bank_mask:0xf\n\t"
+  // (two wait states between the write of y and its DPP reads)
+  asm("s_nop 1\n\t"
+      NKA_ROW_FMAC(0, 3, 0) NKA_ROW_FMAC(1, 4, 1) NKA_ROW_FMAC(0, 5, 2) NKA_ROW_FMAC(1, 6, 3)
+      NKA_ROW_FMAC(0, 7, 4) NKA_ROW_FMAC(1, 8, 5) NKA_ROW_FMAC(0, 9, 6) NKA_ROW_FMAC(1, 10, 7)
+      NKA_ROW_FMAC(0, 11, 8) NKA_ROW_FMAC(1, 12, 9) NKA_ROW_FMAC(0, 13, 10) NKA_ROW_FMAC(1, 14, 11)
+      NKA_ROW_FMAC(0, 15, 12) NKA_ROW_FMAC(1, 16, 13) NKA_ROW_FMAC(0, 17, 14) NKA_ROW_FMAC(1, 18, 15)
+      : "+v"(a), "+v"(b)
+      : "v"(y), "v"(L[0]), "v"(L[1]), "v"(L[2]), "v"(L[3]), "v"(L[4]), "v"(L[5]), "v"(L[6]), "v"(L[7]), "v"(L[8]),
+        "v"(L[9]), "v"(L[10]), "v"(L[11]), "v"(L[12]), "v"(L[13]), "v"(L[14]), "v"(L[15]));
+#undef NKA_ROW_FMAC
+}
+// Sum over the four rows of lanes, in every one.
+__device__ __forceinline__ double sum_rows(double v) {
+  double w = v;
+  swap_rows16(v, w);
+  v += w;
+  w = v;
+  swap_halves(v, w);
+  return v + w;
 }
 
-// forward: y_k = inv_kk (b_k - sum_{j<k} L_kj y_j); block kb = blockIdx.x.
-// Each wave walks its share of the blocks j < k from the oldest (finished
-// first) to the newest, so only the last tile waits on the chain; the tiles
-// of L and the inverse block are loaded before any wait.
-__global__ void __launch_bounds__(256) trsv_fwd_lookback(const double* __restrict__ A, int64_t lda, int64_t n,
-                                                         const double* __restrict__ inv,
-                                                         const double* __restrict__ b, double* y,
-                                                         const int32_t* __restrict__ info, int32_t* err) {
-  if (*info != 0) return;
-  __shared__ double part[4][CH_NB];
-  __shared__ double t[CH_NB];
-  __shared__ double xs[4][CH_NB];
-  __shared__ double Xs[CH_NB * (CH_NB + 1)];
-  const int kb = blockIdx.x;
-  const int64_t k0 = (int64_t)kb * CH_NB;
-  const int nb = (int)min<int64_t>(CH_NB, n - k0);
-  const int wid = threadIdx.x / 64, r = lane_id();
-  const double* invk = inv + (int64_t)kb * CH_NB * CH_NB;
-#pragma unroll
-  for (int it = 0; it < CH_NB * CH_NB / 256; ++it) {
-    const int idx = threadIdx.x + it * 256;
-    Xs[(idx >> 6) * (CH_NB + 1) + (idx & 63)] = invk[idx];
-  }
-  const double bk = (wid == 0 && r < nb) ? b[k0 + r] : 0.0;
-  // rows past nb re-read the last row; their sums are never used
-  const double* arow = A + (k0 + min(r, nb - 1)) * lda;
-  // four interleaved partial sums: the dependent chain of each 64-term dot
-  // product is 16 FMAs instead of 64 (it is on the critical path of the solve)
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int jb = wid; jb < kb; jb += 4) {
-    const int64_t j0 = (int64_t)jb * CH_NB;
-    double Lrow[CH_NB];
-#pragma unroll
-    for (int c = 0; c < CH_NB; ++c) Lrow[c] = arow[j0 + c];
-    // block jb < kb is a full block: y[j0 + lane] is in bounds
-    xs[wid][r] = poll_entry(y + j0 + r, true, err);
-    wave_lds_sync();
-#pragma unroll
-    for (int c = 0; c < CH_NB; ++c) acc[c & 3] += Lrow[c] * xs[wid][c];
-    wave_lds_sync();
-  }
-  part[wid][r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
-  __syncthreads();
-  if (wid == 0) {
-    t[r] = (r < nb) ? bk - (part[0][r] + part[1][r] + part[2][r] + part[3][r]) : 0.0;
-    wave_lds_sync();
-    // inv_kk is lower triangular (zeros above the diagonal)
-    double sp[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int c = 0; c < CH_NB; ++c) sp[c & 3] += Xs[r * (CH_NB + 1) + c] * t[c];
-    const double s = (sp[0] + sp[1]) + (sp[2] + sp[3]);
-    if (r < nb) publish_entry(y + k0 + r, s);
-  }
-}
-
-// backward: x_k = inv_kk^T (y_k - sum_{j>k} L_jk^T x_j); workgroup w owns block
-// kb = nblk - 1 - w so that dependencies point to smaller workgroup ids.  Each
-// wave walks its blocks j > k from the farthest (finished first) down to k+1.
-__global__ void __launch_bounds__(256) trsv_bwd_lookback(const double* __restrict__ A, int64_t lda, int64_t n,
-                                                         const double* __restrict__ inv,
-                                                         const double* __restrict__ y, double* x,
-                                                         const int32_t* __restrict__ info, int32_t* err) {
-  if (*info != 0) return;
-  __shared__ double part[4][CH_NB];
-  __shared__ double t[CH_NB];
-  __shared__ double xs[4][CH_NB];
-  __shared__ double Xs[CH_NB * (CH_NB + 1)];
+// Both solves.  Workgroup k (block kb) of four wavefronts, 16 rows of the block
+// each; lane l has row l % 16 and a quarter of the columns, and the entries of the
+// solution reach it from the lanes of its row of 16, so that neither LDS nor a
+// barrier lies between an entry's arrival and the next block's.
+//
+//   x_k = inv_kk (b_k - sum_j L_kj x_j) = s_k - (inv_kk L_k,prev) x_prev
+//
+// The product W = inv_kk L_k,prev is formed ahead of time on the matrix cores, and
+// s_k, which takes all blocks but the last to come, while that one is being solved:
+// what is left in the chain per block is one memory round trip and 16 FMAs.
+// Bound by that chain: 29 + 28 us at 27 blocks and 147 + 141 at 131 (1.1 us a
+// block), against 40 + 46 and 203 + 237 with the block's sums and its inverse's
+// product taken through LDS after the last entry's arrival.
+//
+// forward (BWD false): L y = b from block 0 up; b's entries become unsolved ones
+// (the next launch fills them with x).  Backward: L^T x = y from the last block
+// down; y's entries become unsolved again, for another solve with the factor.
+template <bool BWD>
+__global__ void __launch_bounds__(256, 2) trsv_lookback(const double* __restrict__ A, int64_t lda, int64_t n,
+                                                        const double* __restrict__ inv, double* rhs, double* out,
+                                                        const int32_t* __restrict__ info, int32_t* err) {
+  __shared__ double ts[CH_NB];
   const int nblk = gridDim.x;
-  const int kb = nblk - 1 - blockIdx.x;
+  const int kb = BWD ? nblk - 1 - (int)blockIdx.x : (int)blockIdx.x;
   const int64_t k0 = (int64_t)kb * CH_NB;
   const int nb = (int)min<int64_t>(CH_NB, n - k0);
-  const int wid = threadIdx.x / 64, r = lane_id();
+  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, i = lane & 15, g = lane >> 4;
+  const int r = 16 * w + i;             // row of the block
+  const int rc = min(r, nb - 1);        // rows past nb re-read the last; their sums are never used
+  if (*info != 0) {
+    // a failed factorisation leaves NaN in the solution, as LAPACK-based cho_solve
+    // does on a matrix that is not positive definite
+    if (BWD && tid < nb) out[k0 + tid] = __longlong_as_double((long long)kDefaultNaN);
+    return;
+  }
   const double* invk = inv + (int64_t)kb * CH_NB * CH_NB;
+  const int m = BWD ? nblk - 1 - kb : kb;      // blocks before this one
+  // the t-th of them, in the order in which they are solved
+  auto first = [&](int t) { return (int64_t)(BWD ? nblk - 1 - t : t) * CH_NB; };
+  // a lane's columns (BWD: rows) of a tile: pairs, so that four lanes read 64 bytes
+  auto col = [&](int c) { return 8 * (c >> 1) + 2 * g + (c & 1); };
+  double iv[16], W[16], rk = 0.0;
+  if constexpr (BWD) {
 #pragma unroll
-  for (int it = 0; it < CH_NB * CH_NB / 256; ++it) {
-    const int idx = threadIdx.x + it * 256;
-    Xs[(idx >> 6) * (CH_NB + 1) + (idx & 63)] = invk[idx];
+    for (int c = 0; c < 16; ++c) iv[c] = invk[col(c) * CH_NB + r];
+  } else {
+    load_k_pairs(invk + r * CH_NB, 0, lane, iv);
   }
-  const double yk = (wid == 0 && r < nb) ? y[k0 + r] : 0.0;
-  // columns past nb re-read the last column; their sums are never used
-  const int64_t col = k0 + min(r, nb - 1);
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};   // interleaved partial sums, as in the forward solve
-  for (int jb = nblk - 1 - wid; jb > kb; jb -= 4) {
-    const int64_t j0 = (int64_t)jb * CH_NB;
+  if (r < nb) rk = rhs[k0 + r];
+  if (m > 0) {
+    const int64_t j0 = first(m - 1);
     const int mb = (int)min<int64_t>(CH_NB, n - j0);
-    // column r of the tile L[j0:j0+mb, k0:k0+nb] (coalesced over r); rows
-    // past mb re-read the last row and meet a zero entry of x below
-    double Lcol[CH_NB];
 #pragma unroll
-    for (int c = 0; c < CH_NB; ++c) Lcol[c] = A[(j0 + min(c, mb - 1)) * lda + col];
-    xs[wid][r] = poll_entry(x + j0 + r, r < mb, err);
-    wave_lds_sync();
+    for (int cb = 0; cb < 4; ++cb) {
+      double a[16];
+      if constexpr (BWD) {
+        load_k_pairs(A + (j0 + min(16 * cb + i, mb - 1)) * lda + k0, 0, lane, a);
+      } else {
 #pragma unroll
-    for (int c = 0; c < CH_NB; ++c) acc[c & 3] += Lcol[c] * xs[wid][c];
-    wave_lds_sync();
+        for (int q = 0; q < 16; ++q) a[q] = A[(k0 + min(col(q), nb - 1)) * lda + j0 + 16 * cb + i];
+      }
+      doublex4 acc = (doublex4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int q = 0; q < 16; ++q) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], iv[q], acc, 0, 0, 0);
+      // element e is W[r][16 cb + 4 e + g]
+#pragma unroll
+      for (int e = 0; e < 4; ++e) W[4 * cb + e] = acc[e];
+    }
   }
-  part[wid][r] = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+  auto load = [&](int t, double (&L)[16]) __attribute__((always_inline)) {
+    const int64_t j0 = first(t);
+    if constexpr (BWD) {
+      // rows past the matrix re-read the last one and meet a zero entry of x
+      const int mb = (int)min<int64_t>(CH_NB, n - j0);
+#pragma unroll
+      for (int c = 0; c < 16; ++c) L[c] = A[(j0 + min(col(c), mb - 1)) * lda + k0 + rc];
+    } else {
+      load_k_pairs(A + (k0 + rc) * lda + j0, 0, lane, L);
+    }
+  };
+  // the tiles of four blocks in flight; the last block is left for W
+  double L[4][16];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    if (u + 1 < m) load(u, L[u]);
+  const int cl = 8 * (i >> 1) + 2 * g + (i & 1);  // the entry that lane l holds for a tile
+  double s0 = 0.0, s1 = 0.0;
+  for (int t0 = 0; t0 + 1 < m; t0 += 4) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (t0 + u + 1 >= m) break;
+      const int64_t j = first(t0 + u) + cl;
+      const double x = poll_entry(out + j, j < n, err);
+      row_dot16(s0, s1, x, L[u]);
+      if (t0 + u + 5 < m) load(t0 + u + 4, L[u]);
+    }
+  }
+  const double tr = r < nb ? rk - sum_rows(s0 + s1) : 0.0;
+  if (g == 0) ts[r] = tr;
   __syncthreads();
-  if (wid == 0) {
-    t[r] = (r < nb) ? yk - (part[0][r] + part[1][r] + part[2][r] + part[3][r]) : 0.0;
-    wave_lds_sync();
-    // column r of inv_kk (zeros above the diagonal)
-    double sp[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-    for (int c = 0; c < CH_NB; ++c) sp[c & 3] += Xs[c * (CH_NB + 1) + r] * t[c];
-    const double s = (sp[0] + sp[1]) + (sp[2] + sp[3]);
-    if (r < nb) publish_entry(x + k0 + r, s);
+  s0 = s1 = 0.0;
+  row_dot16(s0, s1, ts[cl], iv);
+  double v = sum_rows(s0 + s1);
+  if (g == 0 && r < nb) ((uint64_t*)rhs)[k0 + r] = kUnsolved;
+  if (m > 0) {
+    const int64_t j = first(m - 1) + 4 * i + g;   // W's order of columns
+    const double x = poll_entry(out + j, j < n, err);
+    s0 = s1 = 0.0;
+    row_dot16(s0, s1, x, W);
+    v -= sum_rows(s0 + s1);
   }
-}
-
-// A failed factorisation leaves NaN in the solution, as LAPACK-based
-// cho_solve does on a non-positive-definite matrix.
-__global__ void nan_on_info_kernel(double* __restrict__ x, int64_t n, const int32_t* __restrict__ info,
-                                   const int32_t* __restrict__ err) {
-  if (*info == 0 && *err == 0) return;
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    x[i] = __longlong_as_double(0x7FF8000000000000LL);
+  if (g == 0 && r < nb) publish_entry(out + k0 + r, v);
+  if (BWD && kb == 0) {
+    // the last block to be solved: a wait that ran out anywhere leaves NaN
+    __syncthreads();
+    const bool failed = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    __syncthreads();
+    if (failed) {
+      for (int64_t q = tid; q < n; q += 256) out[q] = __longlong_as_double((long long)kDefaultNaN);
+      if (tid == 0) *err = 0;
+    }
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -2078,49 +1379,45 @@ static inline double* ws_split(void* ws, int64_t n, int64_t nblk) {
 // the trailing products' split tail tiles (nullptr / 0: no split).
 static void potrf_run(double* a, int64_t n, int64_t lda, void* workspace, double* split, int64_t n_split,
                       int32_t* info, hipStream_t s) {
+  static_assert(sizeof(PanelLds) <= 80 * 1024, "two workgroups per CU");
+  (void)hipFuncSetAttribute((const void*)panel_step_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)sizeof(PanelLds));
+  (void)hipFuncSetAttribute((const void*)panel_step_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)sizeof(PanelLds));
   double* inv = ws_inv(workspace);
   const int64_t nblk = (n + CH_NB - 1) / CH_NB;
-  // panel widths measured best on MI355X: (768, 768) below n = 16384 (at
-  // n = 4096, 8384 and 12288: 2.02, 6.64 and 15.1 ms, against 2.06, 6.94 and
-  // 15.8 ms with (512, 512)); (4096, 512) from n = 16384 (30.8 ms at 16384,
-  // 200 ms at 32768)
+  // Panel widths.  Up to n = 5000 as few panels as can be of at most 2048 columns:
+  // the steps' own updates (K = 64) are cheaper there than a product and the sum of
+  // its slices (whole solves at n = 960, 1680, 2600, 4096: 276, 510, 863, 1707 us,
+  // against 345, 595, 971, 1800 us with panels of 768).  Then 768 (6000, 8384,
+  // 12288: 3.37, 6.55, 15.8 ms, against 3.43, 6.70, 16.2 with 512 and 3.38, 6.65,
+  // 15.9 with 1024), and (4096, 512) from 16384 (32.4 ms there against 33.0 with 768).
   const bool large = n >= 16384;
-  const int64_t NB0 = large ? 4096 : 768, NB1 = large ? 512 : 768;
+  const int64_t few = (n + 2047) / 2048, one = ((n + few - 1) / few + CH_NB - 1) / CH_NB * CH_NB;
+  const int64_t NB0 = large ? 4096 : n <= 5000 ? one : 768, NB1 = large ? 512 : NB0;
   for (int64_t K0 = 0; K0 < n; K0 += NB0) {
     const int64_t n0 = std::min<int64_t>(NB0, n - K0);
     for (int64_t K1 = K0; K1 < K0 + n0; K1 += NB1) {
       const int64_t n1 = std::min<int64_t>(NB1, K0 + n0 - K1);
-      // 64-column steps.  The first step of the panel factors its columns as
-      // the trailing updates left them.  A later step runs as one two-role
-      // launch: the previous step's update of this step's columns fused into
-      // the factorisation, and its update of the columns further right beside
-      // it.  The last block of the matrix (no rows below) takes the separate
-      // update and the one-wavefront factor.
+      // 64-column steps, one launch each.  The first step of the panel factors
+      // its columns as the trailing updates left them; a later one applies the
+      // previous step's update to its columns itself, and to the columns further
+      // right beside it.
       for (int64_t k0 = K1; k0 < K1 + n1; k0 += CH_NB) {
-        const int64_t nb = std::min<int64_t>(CH_NB, n - k0);
-        const int64_t rest = n - k0 - nb;
+        const int nb = (int)std::min<int64_t>(CH_NB, n - k0);
+        const int64_t rest = std::max<int64_t>(n - k0 - CH_NB, 0);
         double* slot = inv + (k0 / CH_NB) * CH_NB * CH_NB;
-        if (rest <= 0) {
-          if (k0 > K1) {
-            const int64_t kp = k0 - CH_NB, rest_p = n - k0, cols_p = K1 + n1 - k0;
-            const int64_t tm = (rest_p + 63) / 64, tn = (cols_p + 63) / 64;
-            hipLaunchKernelGGL(panel_update_kernel, dim3(grid_mult8(tm * tn)), dim3(256), 0, s, a, lda, kp,
-                               rest_p, cols_p, tn, tm * tn, info);
-          }
-          hipLaunchKernelGGL(potf2_kernel, dim3(1), dim3(64), 0, s, a, lda, n, k0, slot, info);
-          continue;
-        }
-        // rows below imply nb == 64
-        const unsigned grid = (unsigned)((rest + 4 * PF_ROWS - 1) / (4 * PF_ROWS));
+        const int strips = rest <= 256 * 48 ? 3 : 4;
+        const int64_t nf = std::max<int64_t>((rest + 16 * strips - 1) / (16 * strips), 1);
         if (k0 == K1) {
-          hipLaunchKernelGGL(panel_factor_kernel, dim3(grid), dim3(256), 0, s, a, lda, n, k0, slot, info);
+          hipLaunchKernelGGL(panel_step_kernel<false>, dim3((unsigned)nf), dim3(512), sizeof(PanelLds), s, a, lda, n,
+                             k0, nb, strips, (int)nf, (int64_t)0, 1, slot, info);
         } else {
-          // the previous step's update of the columns right of this step
-          const int64_t cols_b = K1 + n1 - (k0 + CH_NB);
-          const int64_t tm = (n - k0 + 63) / 64, tn = cols_b > 0 ? (cols_b + 63) / 64 : 0;
-          const int64_t tiles_b = cols_b > 0 ? tm * tn : 0;
-          hipLaunchKernelGGL(panel_step_kernel, dim3((unsigned)(grid + tiles_b)), dim3(256), 0, s, a, lda, n,
-                             k0, (int64_t)grid, cols_b, tn, slot, info);
+          const int64_t cols_b = std::max<int64_t>(K1 + n1 - (k0 + CH_NB), 0);
+          const int64_t tn = std::max<int64_t>((cols_b + 63) / 64, 1);
+          const int64_t tiles_b = cols_b > 0 ? (rest + 127) / 128 * tn : 0;
+          hipLaunchKernelGGL(panel_step_kernel<true>, dim3((unsigned)(nf + tiles_b)), dim3(512), sizeof(PanelLds), s,
+                             a, lda, n, k0, nb, strips, (int)nf, cols_b, (int)tn, slot, info);
         }
       }
       // update of the outer panel's columns right of this NB1-column panel
@@ -2144,7 +1441,8 @@ static void potrf_run(double* a, int64_t n, int64_t lda, void* workspace, double
       gemm_big_launch(l21, lda, l21, lda, a22, lda, rest2, rest2, n0, -1.0, 1.0, 1, info, s, split, n_split);
     }
   }
-  hipLaunchKernelGGL(trtri_blocks_kernel, dim3((unsigned)nblk), dim3(64), 0, s, a, lda, n, inv, info);
+  hipLaunchKernelGGL(trtri_blocks_kernel, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, ws_vec(workspace, nblk),
+                     (int32_t*)(ws_flags(workspace, n, nblk) + nblk), info);
 }
 
 int nka_potrf_f64(double* a, int64_t n, int64_t lda, void* workspace, int32_t* info,
@@ -2164,19 +1462,10 @@ static void potrs_run(const double* a, int64_t n, int64_t lda, void* ws, double*
   const int64_t nblk = (n + CH_NB - 1) / CH_NB;
   const double* inv = ws_inv(ws);
   double* y = ws_vec(ws, nblk);
-  uint32_t* flags = ws_flags(ws, n, nblk);
-  int32_t* err = (int32_t*)(flags + nblk);
-  const unsigned gf = (unsigned)std::min<int64_t>((n + 255) / 256, 256);
-  hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, (uint32_t*)err, (int64_t)1);
-  hipLaunchKernelGGL(fill_unsolved_kernel, dim3(gf), dim3(256), 0, s, (uint64_t*)y, n);
-  hipLaunchKernelGGL(trsv_fwd_lookback, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, b, y,
-                     info, err);
-  // b has been read: it now receives x, entry by entry
-  hipLaunchKernelGGL(fill_unsolved_kernel, dim3(gf), dim3(256), 0, s, (uint64_t*)b, n);
-  hipLaunchKernelGGL(trsv_bwd_lookback, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, y, b,
-                     info, err);
-  hipLaunchKernelGGL(nan_on_info_kernel, dim3((unsigned)std::min<int64_t>((n + 255) / 256, 1024)),
-                     dim3(256), 0, s, b, n, info, err);
+  int32_t* err = (int32_t*)(ws_flags(ws, n, nblk) + nblk);
+  // (y and err are as the factorisation or the last solve left them: unsolved, 0)
+  hipLaunchKernelGGL(trsv_lookback<false>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, b, y, info, err);
+  hipLaunchKernelGGL(trsv_lookback<true>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, y, b, info, err);
 }
 
 int nka_potrs_f64(const double* a, int64_t n, int64_t lda, const void* workspace, double* b,

@@ -651,3 +651,50 @@ def test_rbm_qgt_structured_fp64_nan_activation(gpu):
     either = hit[:, None] | hit[None, :]
     assert np.all(np.isnan(S[lower & either]))
     np.testing.assert_array_equal(S[lower & ~either], ref[lower & ~either])
+
+
+@pytest.mark.parametrize("n,lda", [(2, 2), (15, 17), (16, 16), (17, 17), (48, 49), (63, 64), (65, 65), (80, 81),
+                                   (111, 112), (112, 112), (113, 113), (129, 130), (176, 176), (177, 180),
+                                   (256, 257), (321, 321), (2050, 2051), (5056, 5057)])
+def test_cholesky_step_edges(gpu, n, lda):
+    # edges of the 16-row strips, 64-column steps, workgroups (48 rows below the diagonal block, 128 beside
+    # it) and panels; several solves with one factor
+    print(f"case cholesky step n={n} lda={lda}", flush=True)
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, n))
+    A = torch.as_tensor(X, device="cuda")
+    A = (A @ A.T) / n + 0.1 * torch.eye(n, dtype=torch.float64, device="cuda")
+    buf = torch.full((n, lda), float("nan"), dtype=torch.float64, device="cuda")
+    a = buf[:, :n]
+    a.copy_(torch.tril(A))  # the lower triangle is all that is read
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ws = _ops.potrf_(a, info)
+    assert int(info.item()) == 0
+    # condition below 50: |dL| <= a few n eps cond |L|, 5e-11 at n = 5056
+    Lref = np.linalg.cholesky(A.cpu().numpy())
+    L = np.tril(a.cpu().numpy())
+    assert np.abs(L - Lref).max() < 1e-10 * np.abs(Lref).max()
+    for seed in (1, 2, 3):
+        b = torch.as_tensor(np.random.default_rng(seed).normal(size=n), device="cuda")
+        x = b.clone()
+        _ops.potrs_(a, ws, x, info)
+        assert (A @ x - b).abs().max().item() < 1e-10 * b.abs().max().item()
+    if lda > n:
+        assert torch.isnan(buf[:, n:]).all()
+
+
+@pytest.mark.parametrize("n,k", [(1, 0), (70, 15), (70, 16), (70, 63), (70, 64), (200, 40), (200, 127), (200, 199),
+                                 (900, 771)])
+@pytest.mark.parametrize("value", [-1.0, 0.0, float("nan"), float("inf")])
+def test_cholesky_first_failing_column(gpu, n, k, value):
+    print(f"case cholesky failing column n={n} k={k} {value}", flush=True)
+    a = torch.eye(n, dtype=torch.float64, device="cuda") * 2.0
+    a[k, k] = value
+    if k + 3 < n:
+        a[k + 3, k + 3] = -1.0   # a later one is not reported
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ws = _ops.potrf_(a, info)
+    assert int(info.item()) == k + 1
+    x = torch.ones(n, dtype=torch.float64, device="cuda")
+    _ops.potrs_(a, ws, x, info)
+    assert torch.isnan(x).all()
