@@ -544,22 +544,30 @@ __global__ void __launch_bounds__(256) gemm_nt_f64_kernel(const double* a, int64
 }
 
 // ---------------------------------------------------------------------------
-// Large FP64 NT GEMM for the trailing updates: C = beta C + alpha A B^T on a
-// 128x128 tile per workgroup, 4 waves of 64x64 (4x4 v_mfma_f64_16x16x4
-// blocks, 16 accumulators per wave), K step 16.  The next K tile is loaded
-// into registers while the current one is multiplied out of LDS; the LDS
+// FP64 NT GEMM for K a multiple of 16: C = beta C + alpha A B^T (+ shift on the
+// diagonal) on a T x T tile per workgroup, T = 128 (4 waves of 64x64, 4x4
+// v_mfma_f64_16x16x4 blocks, two workgroups per CU) or 64, K step 16, LDS tiles in
+// two buffers.  The tile after the next is loaded into registers and the
+// next one stored to the other buffer while the current one is multiplied; the
 // tiles are k-major so a fragment read is 16 consecutive rows.  lower_only
 // skips tiles above the diagonal and elements with j > i.  A, B and C must
-// not overlap.
+// not overlap.  Bound by the matrix cores: 73.9 TFLOP/s at 16384^2 x 4096 and 69.4
+// at 8192^2 x 768 (68.7 and 58.9 with one buffer, two barriers per K step and the
+// requests in front of the products; the peak is 78.6).
 // ---------------------------------------------------------------------------
 constexpr int G2_T = 128;
 constexpr int G2_K = 16;
-constexpr int G2_LD = G2_T + 4;   // doubles per k row of an LDS tile
+// LDS tile of T rows, k-major: row k starts at (T + 16) k (+ 16 from k = 8 on)
+// doubles, so that the two k rows that half a wavefront reads fall into different
+// banks, and so do the two (k, k + 8) that it writes.
+template <int T>
+__device__ constexpr int g2_row(int k) { return k * (T + 16) + (k >= 8 ? 16 : 0); }
+constexpr int g2_tile(int T) { return G2_K * (T + 16) + 16; }
 
-template <bool VEC>
+template <int T, bool VEC, bool SPLIT>
 __device__ __forceinline__ void gemm_big_tile(const double* __restrict__ a, int64_t lda, const double* __restrict__ b,
                                      int64_t ldb, double* __restrict__ c, int64_t ldc, int64_t m, int64_t n,
-                                     int64_t K, double alpha, double beta, int lower_only, int64_t tiles_n,
+                                     int64_t K, double alpha, double beta, double shift, int lower_only, int64_t tiles_n,
                                      int64_t bid, double* sA, double* sB, double* __restrict__ wout) {
   int ti, tj;
   if (lower_only) {
@@ -568,73 +576,104 @@ __device__ __forceinline__ void gemm_big_tile(const double* __restrict__ a, int6
     ti = (int)(bid / tiles_n);
     tj = (int)(bid % tiles_n);
   }
-  const int64_t i0 = (int64_t)ti * G2_T, j0 = (int64_t)tj * G2_T;
+  constexpr int NB = T / 32;            // 16x16 blocks per wavefront and direction
+  constexpr int PER = 2 * NB;           // values per thread, operand and K tile
+  const int64_t i0 = (int64_t)ti * T, j0 = (int64_t)tj * T;
   const int tid = threadIdx.x, wid = tid / 64, lane = lane_id();
-  const int wm = (wid >> 1) * 64, wn = (wid & 1) * 64;
-  // global -> register mapping: thread t loads row t/2, k = (t%2)*8 .. +8 of
-  // each operand.  Rows past the edge re-read the last row (K is a multiple
-  // of 16, so every load is in bounds); their products are never stored.
-  const int lr = tid >> 1, lk = (tid & 1) * 8;
+  const int wm = (wid >> 1) * (T / 2), wn = (wid & 1) * (T / 2);
+  // global -> register mapping: 16 / PER threads per row, PER values of k each.
+  // Rows past the edge re-read the last row (K is a multiple of 16, so every load
+  // is in bounds); their products are never stored.
+  const int lr = tid / (16 / PER), lk = (tid % (16 / PER)) * PER;
   const double* pa = a + min<int64_t>(i0 + lr, m - 1) * lda + lk;
   const double* pb = b + min<int64_t>(j0 + lr, n - 1) * ldb + lk;
-  double ra[8], rb[8];
-  auto load = [&](int64_t k0) {
+  double ra[PER], rb[PER];
+  // request q (< 2 PER) of a tile: 16 bytes (VEC; q < PER) or 8
+  auto load_one = [&](int64_t k0, int q) __attribute__((always_inline)) {
     if (VEC) {
-#pragma unroll
-      for (int q = 0; q < 8; q += 2) {
-        const double2 va = *reinterpret_cast<const double2*>(pa + k0 + q);
-        const double2 vb = *reinterpret_cast<const double2*>(pb + k0 + q);
-        ra[q] = va.x; ra[q + 1] = va.y;
-        rb[q] = vb.x; rb[q + 1] = vb.y;
+      if (q >= PER) return;
+      const int h = q % (PER / 2);
+      const double2 v = *reinterpret_cast<const double2*>((q < PER / 2 ? pa : pb) + k0 + 2 * h);
+      if (q < PER / 2) {
+        ra[2 * h] = v.x;
+        ra[2 * h + 1] = v.y;
+      } else {
+        rb[2 * h] = v.x;
+        rb[2 * h + 1] = v.y;
       }
+    } else if (q < PER) {
+      ra[q % PER] = pa[k0 + q % PER];
     } else {
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        ra[q] = pa[k0 + q];
-        rb[q] = pb[k0 + q];
-      }
+      rb[q % PER] = pb[k0 + q % PER];
     }
   };
-  doublex4 acc[4][4];
+  auto load = [&](int64_t k0) __attribute__((always_inline)) {
 #pragma unroll
-  for (int x = 0; x < 4; ++x)
+    for (int q = 0; q < 2 * PER; ++q) load_one(k0, q);
+  };
+  doublex4 acc[NB][NB];
 #pragma unroll
-    for (int y = 0; y < 4; ++y) acc[x][y] = (doublex4){0.0, 0.0, 0.0, 0.0};
+  for (int x = 0; x < NB; ++x)
+#pragma unroll
+    for (int y = 0; y < NB; ++y) acc[x][y] = (doublex4){0.0, 0.0, 0.0, 0.0};
+  constexpr int TILE = g2_tile(T);
+  double* wa = sA + g2_row<T>(lk) + lr;
+  double* wb = sB + g2_row<T>(lk) + lr;
+  auto store = [&](int q, int buf) __attribute__((always_inline)) {  // q < PER: A, else B (lk + PER <= 8 or >= 8)
+    if (q < PER) wa[buf * TILE + (q % PER) * (T + 16)] = ra[q % PER];
+    else wb[buf * TILE + (q % PER) * (T + 16)] = rb[q % PER];
+  };
   load(0);
+#pragma unroll
+  for (int q = 0; q < 2 * PER; ++q) store(q, 0);
+  load(min<int64_t>(G2_K, K - G2_K));
+  const double* fa = sA + (lane >> 4) * (T + 16) + wm + (lane & 15);
+  const double* fb = sB + (lane >> 4) * (T + 16) + wn + (lane & 15);
+  double fr[2][2 * NB];  // the fragments of a product group and the next
+  auto frag = [&](int ks, int q, int buf) __attribute__((always_inline)) {
+    fr[ks & 1][q] = q < NB ? fa[buf * TILE + g2_row<T>(4 * ks) + 16 * q] : fb[buf * TILE + g2_row<T>(4 * ks) + 16 * (q - NB)];
+  };
+  int buf = 0;
   for (int64_t k0 = 0; k0 < K; k0 += G2_K) {
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      sA[(lk + q) * G2_LD + lr] = ra[q];
-      sB[(lk + q) * G2_LD + lr] = rb[q];
+    for (int q = 0; q < 2 * NB; ++q) frag(0, q, buf);
+    // one memory request (T = 64: two) behind each product: the next group's
+    // fragments, then the next tile's stores to the other buffer and the loads of the
+    // one after it (past the last tile it is loaded and stored again, and not read)
+    const int64_t kn = min<int64_t>(k0 + 2 * G2_K, K - G2_K);
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+#pragma unroll
+      for (int t = 0; t < NB * NB; ++t) {
+        const int x = t / NB, y = t % NB;
+        acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(fr[ks & 1][x], fr[ks & 1][NB + y], acc[x][y], 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4 / NB; ++u) {
+          const int q = t * (4 / NB) + u;  // < 4 NB
+          if (q < 2 * NB) {
+            if (ks < 3) frag(ks + 1, q, buf);
+          } else if (ks < 2) {
+            store(2 * NB * ks + q - 2 * NB, buf ^ 1);
+          } else {
+            load_one(kn, 2 * NB * (ks - 2) + q - 2 * NB);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
-    __syncthreads();
-    if (k0 + G2_K < K) load(k0 + G2_K);
-#pragma unroll
-    for (int ks = 0; ks < G2_K; ks += 4) {
-      const int kq = ks + (lane >> 4);
-      double av[4], bv[4];
-#pragma unroll
-      for (int x = 0; x < 4; ++x) av[x] = sA[kq * G2_LD + wm + x * 16 + (lane & 15)];
-#pragma unroll
-      for (int y = 0; y < 4; ++y) bv[y] = sB[kq * G2_LD + wn + y * 16 + (lane & 15)];
-#pragma unroll
-      for (int x = 0; x < 4; ++x)
-#pragma unroll
-        for (int y = 0; y < 4; ++y)
-          acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[x], bv[y], acc[x][y], 0, 0, 0);
-    }
+    buf ^= 1;
   }
   // element e of lane l in a 16x16 block is (row l/16 + 4e, col l%16)
-  if (wout) {
-    // partial product of a K slice: the raw 128x128 tile, row-major
+  if constexpr (SPLIT) {
+    // partial product of a K slice: the raw tile, row-major
 #pragma unroll
-    for (int x = 0; x < 4; ++x)
+    for (int x = 0; x < NB; ++x)
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
+      for (int y = 0; y < NB; ++y)
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          wout[(wm + x * 16 + (lane >> 4) + 4 * e) * G2_T + wn + y * 16 + (lane & 15)] = acc[x][y][e];
+          wout[(wm + x * 16 + (lane >> 4) + 4 * e) * T + wn + y * 16 + (lane & 15)] = acc[x][y][e];
     return;
   }
   // C is read in batches of one 16-row block (16 values per lane) before
@@ -644,21 +683,21 @@ __device__ __forceinline__ void gemm_big_tile(const double* __restrict__ a, int6
   // Interior tiles (inside C and, for lower_only, below the diagonal) take
   // unpredicated loads and stores, which keep each store's data in its own
   // registers; edge tiles check every element.
-  const bool interior = i0 + G2_T <= m && j0 + G2_T <= n && (!lower_only || j0 + G2_T <= i0);
+  const bool interior = i0 + T <= m && j0 + T <= n && (!lower_only || j0 + T <= i0);
 #pragma unroll
-  for (int xb = 0; xb < 4; ++xb) {
-    double cv[1][4][4];
+  for (int xb = 0; xb < NB; ++xb) {
+    double cv[1][NB][4];
 #pragma unroll
     for (int x = 0; x < 1; ++x)
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
+      for (int y = 0; y < NB; ++y)
 #pragma unroll
         for (int e = 0; e < 4; ++e) cv[x][y][e] = 0.0;
     if (beta != 0.0) {
 #pragma unroll
       for (int x = 0; x < 1; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y)
+        for (int y = 0; y < NB; ++y)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int64_t gi = i0 + wm + (xb + x) * 16 + (lane >> 4) + 4 * e;
@@ -669,14 +708,14 @@ __device__ __forceinline__ void gemm_big_tile(const double* __restrict__ a, int6
 #pragma unroll
     for (int x = 0; x < 1; ++x)
 #pragma unroll
-      for (int y = 0; y < 4; ++y)
+      for (int y = 0; y < NB; ++y)
 #pragma unroll
         for (int e = 0; e < 4; ++e) cv[x][y][e] = alpha * acc[xb + x][y][e] + beta * cv[x][y][e];
     if (interior) {
 #pragma unroll
       for (int x = 0; x < 1; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y)
+        for (int y = 0; y < NB; ++y)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
             c[(i0 + wm + (xb + x) * 16 + (lane >> 4) + 4 * e) * ldc + j0 + wn + y * 16 + (lane & 15)] = cv[x][y][e];
@@ -684,12 +723,13 @@ __device__ __forceinline__ void gemm_big_tile(const double* __restrict__ a, int6
 #pragma unroll
       for (int x = 0; x < 1; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y)
+        for (int y = 0; y < NB; ++y)
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int64_t gi = i0 + wm + (xb + x) * 16 + (lane >> 4) + 4 * e;
             const int64_t gj = j0 + wn + y * 16 + (lane & 15);
-            if (gi < m && gj < n && (!lower_only || gj <= gi)) c[gi * ldc + gj] = cv[x][y][e];
+            if (gi < m && gj < n && (!lower_only || gj <= gi))
+              c[gi * ldc + gj] = gi == gj ? cv[x][y][e] + shift : cv[x][y][e];
           }
     }
   }
@@ -702,27 +742,29 @@ __device__ __forceinline__ void gemm_big_tile(const double* __restrict__ a, int6
 // C updated.  SPLIT = true: unit u is slice u % S (kc columns of K) of tile
 // n_main + u / S, whose raw product goes to work + u * 128 * 128 for
 // gemm_big_reduce_kernel.
-template <bool VEC, bool SPLIT>
-__global__ void __launch_bounds__(256, 2) gemm_nt_f64_big_kernel(const double* __restrict__ a, int64_t lda,
+template <int T, bool VEC, bool SPLIT>
+__global__ void __launch_bounds__(256, T == 128 ? 2 : 3) gemm_nt_f64_big_kernel(const double* __restrict__ a, int64_t lda,
                                                               const double* __restrict__ b, int64_t ldb,
                                                               double* __restrict__ c, int64_t ldc, int64_t m,
                                                               int64_t n, int64_t K, double alpha, double beta,
-                                                              int lower_only, int64_t tiles_n,
+                                                              double shift, int lower_only, int64_t tiles_n,
                                                               int64_t n_units, int64_t n_main, int S,
                                                               int64_t kc, double* __restrict__ work,
                                                               const int32_t* info) {
   if (info && *info != 0) return;
-  __shared__ double sA[G2_K * G2_LD];
-  __shared__ double sB[G2_K * G2_LD];
+  extern __shared__ __align__(16) unsigned char smem[];
+  double* sA = (double*)smem;  // two tiles of each operand
+  double* sB = sA + 2 * g2_tile(T);
   const int64_t G = gridDim.x;
   for (int64_t u = xcd_remap(blockIdx.x, G); u < n_units; u += G) {
     if (!SPLIT) {
-      gemm_big_tile<VEC>(a, lda, b, ldb, c, ldc, m, n, K, alpha, beta, lower_only, tiles_n, u, sA, sB, nullptr);
+      gemm_big_tile<T, VEC, false>(a, lda, b, ldb, c, ldc, m, n, K, alpha, beta, shift, lower_only, tiles_n, u, sA, sB,
+                                nullptr);
     } else {
       const int64_t tile = n_main + u / S;
       const int64_t kb = (u % S) * kc, kl = min<int64_t>(kc, K - kb);
-      gemm_big_tile<VEC>(a + kb, lda, b + kb, ldb, c, ldc, m, n, kl, alpha, beta, lower_only, tiles_n, tile,
-                         sA, sB, work + u * (int64_t)(G2_T * G2_T));
+      gemm_big_tile<T, VEC, true>(a + kb, lda, b + kb, ldb, c, ldc, m, n, kl, alpha, beta, 0.0, lower_only, tiles_n, tile,
+                               sA, sB, work + u * (int64_t)(G2_T * G2_T));
     }
     __syncthreads();
   }
@@ -1266,14 +1308,14 @@ constexpr int64_t kMaxSplitUnits = 1024;
 static void gemm_big_launch(const double* a, int64_t lda, const double* b, int64_t ldb, double* c,
                             int64_t ldc, int64_t m, int64_t n, int64_t k, double alpha, double beta,
                             int lower, const int32_t* info, hipStream_t s, double* work = nullptr,
-                            int64_t work_units = 0) {
+                            int64_t work_units = 0, double shift = 0.0) {
   if (m <= 0 || n <= 0) return;
-  if (k % G2_K != 0) {
-    gemm_launch(a, lda, b, ldb, c, ldc, m, n, k, alpha, beta, 0.0, lower, info, s);
+  if (k % G2_K != 0 || k == 0) {
+    gemm_launch(a, lda, b, ldb, c, ldc, m, n, k, alpha, beta, shift, lower, info, s);
     return;
   }
-  const int64_t tm = (m + G2_T - 1) / G2_T, tn = (n + G2_T - 1) / G2_T;
-  const int64_t tiles = lower ? tm * (tm + 1) / 2 : tm * tn;
+  int64_t tm = (m + G2_T - 1) / G2_T, tn = (n + G2_T - 1) / G2_T;
+  int64_t tiles = lower ? tm * (tm + 1) / 2 : tm * tn;
   const int64_t slots = big_gemm_slots();
   const int64_t n_main = (tiles / slots) * slots;
   const int64_t tail = tiles - n_main;
@@ -1286,26 +1328,38 @@ static void gemm_big_launch(const double* a, int64_t lda, const double* b, int64
   }
   const int64_t kc = S > 1 ? ((k + S - 1) / S + G2_K - 1) / G2_K * G2_K : k;
   if (S > 1) S = (int)((k + kc - 1) / kc);  // slices actually needed with kc columns each
-  const int64_t main_tiles = S > 1 ? n_main : tiles;
+  int64_t main_tiles = S > 1 ? n_main : tiles;
+  // 64x64 tiles where their rounds over the chip are cheaper: a round of 128x128
+  // tiles takes 1.88 us per K step, one of 64x64 tiles 0.56 (0.74 if it is the only
+  // one).  X X^T of 1008 x 8384, 2560 x 8384, 4096 x 8384: 376, 1191, 2626 us with
+  // 64x64 tiles, 980, 1042, 2981 with 128x128.  In place of slices and their sum
+  // only for one round and K up to 1024 (solves at n = 5500 and 6500: 2.63 and 3.64
+  // ms against 2.69 and 3.70): a longer single sum doubles the solve's error.
+  const int64_t t64 = lower ? ((m + 63) / 64) * ((m + 63) / 64 + 1) / 2 : ((m + 63) / 64) * ((n + 63) / 64);
+  const int64_t r64 = (t64 + slots / 2 - 1) / (slots / 2), r128 = (tiles + slots / 2 - 1) / (slots / 2);
+  const bool small = 3 * r64 < 10 * r128 && (S == 1 || (r64 == 1 && k <= 1024));
+  if (small) {
+    tm = (m + 63) / 64;
+    tn = (n + 63) / 64;
+    main_tiles = t64;
+    S = 1;
+  }
   const bool vec = ((uintptr_t)a % 16 == 0) && ((uintptr_t)b % 16 == 0) && lda % 2 == 0 && ldb % 2 == 0;
+  const int lds = 4 * g2_tile(small ? 64 : 128) * (int)sizeof(double);
+  auto launch = [&](auto kernel, int64_t units, int64_t first, int slices, int64_t width) {
+    (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    hipLaunchKernelGGL(kernel, dim3(grid_mult8(units)), dim3(256), lds, s, a, lda, b, ldb, c, ldc, m, n, k, alpha, beta,
+                       shift, lower, tn, units, first, slices, width, work, info);
+  };
   if (main_tiles > 0) {
-    const unsigned grid = grid_mult8(main_tiles);
-    if (vec)
-      hipLaunchKernelGGL((gemm_nt_f64_big_kernel<true, false>), dim3(grid), dim3(256), 0, s, a, lda, b, ldb, c,
-                         ldc, m, n, k, alpha, beta, lower, tn, main_tiles, (int64_t)0, 1, k, work, info);
-    else
-      hipLaunchKernelGGL((gemm_nt_f64_big_kernel<false, false>), dim3(grid), dim3(256), 0, s, a, lda, b, ldb,
-                         c, ldc, m, n, k, alpha, beta, lower, tn, main_tiles, (int64_t)0, 1, k, work, info);
+    if (small && vec) launch(gemm_nt_f64_big_kernel<64, true, false>, main_tiles, 0, 1, k);
+    else if (small) launch(gemm_nt_f64_big_kernel<64, false, false>, main_tiles, 0, 1, k);
+    else if (vec) launch(gemm_nt_f64_big_kernel<128, true, false>, main_tiles, 0, 1, k);
+    else launch(gemm_nt_f64_big_kernel<128, false, false>, main_tiles, 0, 1, k);
   }
   if (S > 1) {
-    const int64_t su = tail * S;
-    const unsigned grid = grid_mult8(su);
-    if (vec)
-      hipLaunchKernelGGL((gemm_nt_f64_big_kernel<true, true>), dim3(grid), dim3(256), 0, s, a, lda, b, ldb, c,
-                         ldc, m, n, k, alpha, beta, lower, tn, su, main_tiles, S, kc, work, info);
-    else
-      hipLaunchKernelGGL((gemm_nt_f64_big_kernel<false, true>), dim3(grid), dim3(256), 0, s, a, lda, b, ldb,
-                         c, ldc, m, n, k, alpha, beta, lower, tn, su, main_tiles, S, kc, work, info);
+    if (vec) launch(gemm_nt_f64_big_kernel<128, true, true>, tail * S, main_tiles, S, kc);
+    else launch(gemm_nt_f64_big_kernel<128, false, true>, tail * S, main_tiles, S, kc);
   }
   if (S > 1)
     hipLaunchKernelGGL(gemm_big_reduce_kernel, dim3((unsigned)(tail * 4)), dim3(256), 0, s, work, c, ldc, m, n,
@@ -1315,7 +1369,7 @@ static void gemm_big_launch(const double* a, int64_t lda, const double* b, int64
 int nka_syrk_f64(const double* x, int64_t n, int64_t k, int64_t ldx, double alpha, double beta,
                  double shift, double* c, int64_t ldc, void* stream) {
   NKA_CHECK_ARG(n >= 0 && k >= 0 && ldx >= k && ldc >= n, "nka_syrk_f64: bad sizes");
-  gemm_launch(x, ldx, x, ldx, c, ldc, n, n, k, alpha, beta, shift, 1, nullptr, (hipStream_t)stream);
+  gemm_big_launch(x, ldx, x, ldx, c, ldc, n, n, k, alpha, beta, 1, nullptr, (hipStream_t)stream, nullptr, 0, shift);
   NKA_CHECK_LAUNCH("nka_syrk_f64");
   return NKA_OK;
 }

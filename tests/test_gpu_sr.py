@@ -698,3 +698,34 @@ def test_cholesky_first_failing_column(gpu, n, k, value):
     x = torch.ones(n, dtype=torch.float64, device="cuda")
     _ops.potrs_(a, ws, x, info)
     assert torch.isnan(x).all()
+
+
+@pytest.mark.parametrize("n,k,pad", [(1, 16, 0), (63, 16, 1), (64, 32, 0), (65, 48, 3), (127, 16, 2), (129, 160, 0),
+                                     (300, 1000, 0), (300, 1024, 1), (1280, 64, 0), (1281, 48, 1), (2300, 32, 0),
+                                     (2700, 32, 2)])
+def test_gram_fp64_tiles(gpu, n, k, pad):
+    # both tile sizes, their edges, K below and above a K step, and row strides that rule out 16-byte loads
+    print(f"case fp64 gram n={n} k={k} pad={pad}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    buf = torch.randn(n, k + pad, dtype=torch.float64, device="cuda", generator=g)
+    c0 = torch.randn(n, n + 1, dtype=torch.float64, device="cuda", generator=g)
+    for alpha, beta, shift in ((1.0, 0.0, 0.25), (-0.5, 1.0, 0.0)):
+        c = c0.clone()
+        nat.call("nka_syrk_f64", _ops.ptr(buf), n, k, k + pad, alpha, beta, shift, _ops.ptr(c), n + 1, _ops.stream())
+        x = buf[:, :k]
+        ref = alpha * (x @ x.T) + beta * c0[:, :n] + shift * torch.eye(n, dtype=torch.float64, device="cuda")
+        # k terms of variance one: k eps, and a wide margin for the order
+        assert torch.tril(c[:, :n] - ref).abs().max().item() < 1e-13 * k
+        assert torch.equal(torch.triu(c[:, :n], 1), torch.triu(c0[:, :n], 1)) and torch.equal(c[:, n], c0[:, n])
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 16), (65, 130, 16), (300, 7, 48), (1000, 2000, 64), (3000, 3001, 32)])
+def test_gemm_fp64_tiles(gpu, m, n, k):
+    print(f"case fp64 gemm {m}x{n}x{k}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    a = torch.randn(m, k, dtype=torch.float64, device="cuda", generator=g)
+    b = torch.randn(n, k, dtype=torch.float64, device="cuda", generator=g)
+    c0 = torch.randn(m, n, dtype=torch.float64, device="cuda", generator=g)
+    c = c0.clone()
+    nat.call("nka_gemm_nt_f64", _ops.ptr(a), k, _ops.ptr(b), k, _ops.ptr(c), n, m, n, k, -1.0, 1.0, _ops.stream())
+    assert (c - (c0 - a @ b.T)).abs().max().item() < 1e-13 * k
