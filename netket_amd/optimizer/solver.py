@@ -63,9 +63,8 @@ def _system(A, b):
     raise TypeError(f"unsupported linear operator {type(A).__name__}")
 
 
-def _chol_solve(sys_, b: torch.Tensor):
-    a = sys_.lower()
-    n = a.shape[0]
+def _chol_solve(a: torch.Tensor, b: torch.Tensor):
+    """Solve with ``a`` (lower triangle valid), which is overwritten by its factor."""
     info = torch.zeros(1, dtype=torch.int32, device=a.device)
     ws = _ops.potrf_(a, info)
     x = b.clone()
@@ -75,8 +74,13 @@ def _chol_solve(sys_, b: torch.Tensor):
 
 def cholesky(A, b, *, lower: bool = False, x0=None):
     """Cholesky factorisation and solve (netket/optimizer/solver/solvers.py:241-270)."""
+    if isinstance(A, torch.Tensor):
+        # nothing keeps the system once it is solved, so one copy of the matrix is enough
+        # (of n = 32768, 2.5 ms each at 8.6 GB)
+        a = torch.empty(A.shape, dtype=torch.float64, device=A.device).copy_(A)
+        return _chol_solve(a, b.to(torch.float64).contiguous())[0], None
     sys_, bf, unflat = _system(A, b)
-    x, _ = _chol_solve(sys_, bf)
+    x, _ = _chol_solve(sys_.lower(), bf)
     return unflat(x), None
 
 
@@ -145,7 +149,7 @@ def cholesky_with_fallback(A, b, *, rtol: float = 1e-14, rtol_smooth: float = 1e
     sys_, bf, unflat = _system(A, b)
     flag = torch.zeros(1, dtype=torch.int32, device=bf.device)
     _ops.check_finite(bf, flag)
-    x, info = _chol_solve(sys_, bf)
+    x, info = _chol_solve(sys_.lower(), bf)
     _ops.check_finite(x, flag)
     _ops.select_on_flag(flag, None, x)
     fb = DeviceFallback(flag, lambda: pinv_smooth(sys_, bf, rtol=rtol, rtol_smooth=rtol_smooth)[0])
