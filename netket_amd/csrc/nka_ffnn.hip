@@ -42,8 +42,8 @@ constexpr int FF_MAXH = 1024;
 // (32 chains per CU are all there is), of 512 where a thread's state does not
 // fit 128 registers (FP64; weighted exchange).  J1-J2 10x10 with layers 100-400-
 // 400 in FP32, against workgroups of 256: the sampler (8192 chains, 700
-// proposals) 42.4 -> 22.0 ms (matrix cores 55% busy), the local energies of 16384
-// samples 23.2 -> 12.5 ms (58%; with the connected elements taken as a list of
+// proposals) 42.4 -> 20.3 ms (matrix products 60% of it), the local energies of 16384
+// samples 23.2 -> 12.5 ms (58%; the rest is vector work and its latencies; with the connected elements taken as a list of
 // flipped sites instead of as configurations, 3.0 ms of that).
 constexpr int FF_FWD = 512;
 constexpr int FF_BACK = 256;
@@ -96,100 +96,116 @@ constexpr int64_t FF_LDS_MAX = 160 * 1024;
 // Wavefronts w, w + 4, ... share a SIMD, so every SIMD does the same number of
 // products.  The sums' order depends on the sizes alone, not on NW.
 // ---------------------------------------------------------------------------
+// acc += A[:, ka:kb] B(ka:kb, block cb); lane (lc, kh) supplies row lc and
+// column cb*32 + lc at k = k0 + 2q + kh of each pair of k-rows.  The B loads
+// run NB - 1 groups of 16 k-rows ahead of their products (register sets in
+// turn; one group ahead with four wavefronts per SIMD, which cover the rest);
+// near the end of the range a group reloads the last full group, unused, so
+// that every load is unconditional.  The lane's part of the address is one
+// 32-bit offset, the k-row's part a scalar.
+constexpr int FF_KB = 16;
+template <int NB>
+__device__ __forceinline__ void rows_mfma(floatx16& acc, const float* As, int lda, int K, int ncols,
+                                          const float* __restrict__ Bp, int sk, int sc, int cb, int ka, int kb) {
+  constexpr int KB = FF_KB;
+  const int lane = lane_id(), kh = lane >> 5, lc = lane & 31;
+  const __amdgpu_buffer_rsrc_t Bs = __builtin_amdgcn_make_buffer_rsrc((void*)Bp, 0, K * ncols * 4, 0x00020000);
+  const int col = cb * 32 + lc;
+  const bool cok = col < ncols;
+  const int boff = ((cok ? col : ncols - 1) * sc + kh * sk) * 4;
+  const int kend = ka + (kb - ka) / KB * KB;
+  const float* arow = As + lc * lda + kh;
+  int k = ka;
+  auto loadB = [&](int kk0, float (&bv)[KB / 2]) __attribute__((always_inline)) {
+    const int kc = kk0 < kend ? kk0 : kend - KB;
+#pragma unroll
+    for (int q = 0; q < KB / 2; ++q)
+      bv[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(Bs, boff, (kc + 2 * q) * sk * 4, 0));
+  };
+  auto group = [&](int kk0, const float (&bv)[KB / 2]) __attribute__((always_inline)) {
+    float a[KB / 2];
+#pragma unroll
+    for (int q = 0; q < KB / 2; ++q) a[q] = arow[kk0 + 2 * q];
+#pragma unroll
+    for (int q = 0; q < KB / 2; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], bv[q], acc, 0, 0, 0);
+  };
+  if (kend > ka) {
+    float bv[NB][KB / 2];
+#pragma unroll
+    for (int i = 0; i < NB - 1; ++i) loadB(k + i * KB, bv[i]);
+    while (k < kend) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i) {
+        loadB(k + (NB - 1) * KB, bv[(i + NB - 1) % NB]);
+        __builtin_amdgcn_sched_barrier(0);
+        group(k, bv[i]);
+        k += KB;
+        if (k >= kend) break;
+      }
+    }
+  }
+  for (; k < kb; k += 2) {
+    const int kk = k + kh;
+    const float av = kk < kb ? As[lc * lda + kk] : 0.0f;
+    const float bw = (kk < kb && cok) ? Bp[(uint32_t)kk * (uint32_t)sk + (uint32_t)col * (uint32_t)sc] : 0.0f;
+    acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bw, acc, 0, 0, 0);
+  }
+}
+
+// Sums over the columns of block cb of epi of elements 4 q .. 4 q + 3 (element e
+// of lane l is (row (e/4)*8 + (l/32)*4 + e%4, col l%32)) to part: over lanes 16,
+// 8, 4, 2, 1 apart in turn, two elements sharing the steps within rows of lanes.
+// Vector instructions only, and few: an FP32 matrix product holds the SIMD's vector
+// unit for its whole 64 cycles, so whatever else runs there adds to the time (the
+// sampler of the J1-J2 lattice with shuffles through LDS 22.0 ms, this 20.3 ms).
+template <class Epi>
+__device__ __forceinline__ void rows_finish(const float (&acc)[4], int q, int cb, int ncols, Epi epi, float* part) {
+  const int lane = lane_id(), kh = lane >> 5, lc = lane & 31;
+  const int col = cb * 32 + lc;
+  const bool cok = col < ncols;
+  float v[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = cok ? epi(q * 8 + kh * 4 + e, col, acc[e]) : 0.0f;
+#pragma unroll
+  for (int e = 0; e < 4; e += 2) {
+    swap_rows16(v[e], v[e + 1]);
+    float s = v[e] + v[e + 1];  // rows of lanes 0 and 2: element e, 1 and 3: e + 1
+    s += dpp_perm<0x128>(s);    // row_ror:8, 4, 2, 1
+    s += dpp_perm<0x124>(s);
+    s += dpp_perm<0x122>(s);
+    s += dpp_perm<0x121>(s);
+    if ((lane & 15) == 0) part[(q * 8 + kh * 4 + e + (lane >> 4 & 1)) * FF_MAXBLK + cb] = s;
+  }
+}
+
 template <int NW, class Epi>
 __device__ __forceinline__ void rows_gemm(const float* As, int lda, int K, int ncols, const float* __restrict__ Bp, int sk,
                           int sc, Epi epi, float* part, float* rowsum, float* rbuf = nullptr) {
   const int wid = threadIdx.x >> 6, lane = lane_id();
   const int nblk = (ncols + 31) >> 5;
-  const int kh = lane >> 5, lc = lane & 31;
-  constexpr int KB = 16;
-  // acc += A[:, ka:kb] B(ka:kb, block cb); lane (lc, kh) supplies row lc and
-  // column cb*32 + lc at k = k0 + 2q + kh of each pair of k-rows.  The B loads
-  // run two groups of 16 k-rows ahead of their products (register sets in
-  // turn; one group ahead with four wavefronts per SIMD, which cover the rest);
-  // near the end of the range a group reloads the last full group, unused, so
-  // that every load is unconditional.  The lane's part of the address is one
-  // 32-bit offset, the k-row's part a scalar.
-  const __amdgpu_buffer_rsrc_t Bs = __builtin_amdgcn_make_buffer_rsrc((void*)Bp, 0, K * ncols * 4, 0x00020000);
-  auto mfma_range = [&](floatx16& acc, int cb, int ka, int kb) __attribute__((always_inline)) {
-    const int col = cb * 32 + lc;
-    const bool cok = col < ncols;
-    const int boff = ((cok ? col : ncols - 1) * sc + kh * sk) * 4;
-    const int kend = ka + (kb - ka) / KB * KB;
-    const float* arow = As + lc * lda + kh;
-    constexpr int NB = NW >= 16 ? 2 : 3;
-    int k = ka;
-    auto loadB = [&](int kk0, float (&bv)[KB / 2]) __attribute__((always_inline)) {
-      const int kc = kk0 < kend ? kk0 : kend - KB;
-#pragma unroll
-      for (int q = 0; q < KB / 2; ++q)
-        bv[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(Bs, boff, (kc + 2 * q) * sk * 4, 0));
-    };
-    auto group = [&](int kk0, const float (&bv)[KB / 2]) __attribute__((always_inline)) {
-      float a[KB / 2];
-#pragma unroll
-      for (int q = 0; q < KB / 2; ++q) a[q] = arow[kk0 + 2 * q];
-#pragma unroll
-      for (int q = 0; q < KB / 2; ++q) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[q], bv[q], acc, 0, 0, 0);
-    };
-    if (kend > ka) {
-      float bv[NB][KB / 2];
-#pragma unroll
-      for (int i = 0; i < NB - 1; ++i) loadB(k + i * KB, bv[i]);
-      while (k < kend) {
-#pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          loadB(k + (NB - 1) * KB, bv[(i + NB - 1) % NB]);
-          __builtin_amdgcn_sched_barrier(0);
-          group(k, bv[i]);
-          k += KB;
-          if (k >= kend) break;
-        }
-      }
-    }
-    for (; k < kb; k += 2) {
-      const int kk = k + kh;
-      const float av = kk < kb ? As[lc * lda + kk] : 0.0f;
-      const float bw = (kk < kb && cok) ? Bp[(uint32_t)kk * (uint32_t)sk + (uint32_t)col * (uint32_t)sc] : 0.0f;
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bw, acc, 0, 0, 0);
-    }
-  };
-  // element e of lane l is (row (e/4)*8 + (l/32)*4 + e%4, col l%32); elements
-  // 4 q .. 4 q + 3 of block cb
-  auto finish = [&](const float (&acc)[4], int q, int cb) __attribute__((always_inline)) {
-    const int col = cb * 32 + lc;
-    const bool cok = col < ncols;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int row = q * 8 + kh * 4 + e;
-      float v = cok ? epi(row, col, acc[e]) : 0.0f;
-#pragma unroll
-      for (int off = 16; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-      if (lc == 0) part[row * FF_MAXBLK + cb] = v;
-    }
-  };
+  constexpr int NB = NW >= 16 ? 2 : 3;
   const int rem = rbuf ? (nblk & 3) : 0;
   const int nfull = nblk - rem;
   for (int cb = wid; cb < nfull; cb += NW) {
     floatx16 acc;
 #pragma unroll
     for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-    mfma_range(acc, cb, 0, K);
+    rows_mfma<NB>(acc, As, lda, K, ncols, Bp, sk, sc, cb, 0, K);
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
       const float aq[4] = {acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]};
-      finish(aq, q, cb);
+      rows_finish(aq, q, cb, ncols, epi, part);
     }
   }
   if (rem > 0) {
     // K quarters rounded up to whole groups
-    const int kq = ((K + 3) / 4 + KB - 1) / KB * KB;
+    const int kq = ((K + 3) / 4 + FF_KB - 1) / FF_KB * FF_KB;
     for (int u = (wid + NW - nfull % NW) % NW; u < 4 * rem; u += NW) {
       const int k0 = min(K, (u & 3) * kq), k1 = min(K, k0 + kq);
       floatx16 acc;
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-      mfma_range(acc, nfull + (u >> 2), k0, k1);
+      rows_mfma<NB>(acc, As, lda, K, ncols, Bp, sk, sc, nfull + (u >> 2), k0, k1);
       float* dst = rbuf + u * 1024;
 #pragma unroll
       for (int e = 0; e < 16; ++e) dst[e * 64 + lane] = acc[e];
@@ -206,7 +222,7 @@ __device__ __forceinline__ void rows_gemm(const float* As, int lda, int K, int n
         for (int w = 0; w < 4; ++w) t += rbuf[(j * 4 + w) * 1024 + (4 * q + e) * 64 + lane];
         acc[e] = t;
       }
-      finish(acc, q, nfull + j);
+      rows_finish(acc, q, nfull + j, ncols, epi, part);
     }
   }
   __syncthreads();
