@@ -106,31 +106,46 @@ template <> __device__ inline double log_cosh<double>(double x) {
   return ax + log1p(exp(-2.0 * ax)) - 0.69314718055994530942;
 }
 
+// a b + k with the constant k in scalar registers: as a plain fma the compiler
+// copies a constant from vector registers in front of every step of a polynomial.
+__device__ __forceinline__ double fma_const(double a, double b, double k) {
+  double r;
+  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(k));
+  return r;
+}
+
 // exp(x) in FP64 for the amplitude ratios: x = n ln2 + r with |r| <= ln2 / 2,
 // the Taylor series of e^r to r^13 (remainder below 2^-57 of the sum) in even
 // and odd halves, then a power of two.  |x| is limited to 800, past which the
 // result is 0 or infinity anyway; a NaN stays one.  About 20 instructions
 // against about 40 of the library's.
-__device__ inline double exp_f64(double x) {
-  x = x < -800.0 ? -800.0 : (x > 800.0 ? 800.0 : x);
+__device__ __forceinline__ double exp_f64_limited(double x) {
   const double n = rint(x * 1.4426950408889634);
   double r = fma(n, -0x1.62e42fefa39efp-1, x);
   r = fma(n, -0x1.abc9e3b39803fp-56, r);
   const double q = r * r;
   double e = 1.0 / 479001600.0, o = 1.0 / 6227020800.0;
-  e = fma(e, q, 1.0 / 3628800.0);
-  o = fma(o, q, 1.0 / 39916800.0);
-  e = fma(e, q, 1.0 / 40320.0);
-  o = fma(o, q, 1.0 / 362880.0);
-  e = fma(e, q, 1.0 / 720.0);
-  o = fma(o, q, 1.0 / 5040.0);
-  e = fma(e, q, 1.0 / 24.0);
-  o = fma(o, q, 1.0 / 120.0);
+  e = fma_const(e, q, 1.0 / 3628800.0);
+  o = fma_const(o, q, 1.0 / 39916800.0);
+  e = fma_const(e, q, 1.0 / 40320.0);
+  o = fma_const(o, q, 1.0 / 362880.0);
+  e = fma_const(e, q, 1.0 / 720.0);
+  o = fma_const(o, q, 1.0 / 5040.0);
+  e = fma_const(e, q, 1.0 / 24.0);
+  o = fma_const(o, q, 1.0 / 120.0);
   e = fma(e, q, 0.5);
-  o = fma(o, q, 1.0 / 6.0);
+  o = fma_const(o, q, 1.0 / 6.0);
   e = fma(e, q, 1.0);
   o = fma(o, q, 1.0);
   return ldexp(fma(o, r, e), (int)n);
+}
+__device__ __forceinline__ double exp_f64(double x) {
+  return exp_f64_limited(x < -800.0 ? -800.0 : (x > 800.0 ? 800.0 : x));
+}
+// exp(-2 |t|)
+__device__ __forceinline__ double exp_m2abs(double t) {
+  const double x = -2.0 * fabs(t);
+  return exp_f64_limited(x < -800.0 ? -800.0 : x);
 }
 
 template <class T> __device__ inline T exp_t(T x);
@@ -176,12 +191,12 @@ template <> __device__ inline float wave_sum<float>(float v) {
 // mirror is an exchange with the other one) and the row swaps of gfx950.
 template <int CTRL>
 __device__ inline float dpp_perm(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), CTRL, 0xf, 0xf, true));
 }
 template <int CTRL>
 __device__ inline double dpp_perm(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
   return __hiloint2double(hi, lo);
 }
 constexpr int kDppXor1 = 0xb1, kDppXor2 = 0x4e, kDppHalfMirror = 0x141, kDppMirror = 0x140;

@@ -131,7 +131,7 @@ __device__ __forceinline__ void eloc_quads(uint64_t mask, const ElocEntry<T>& en
         const T t = h.th[jj] + d[jj];
         if constexpr (F64) {
           A += fabs(t) - fabs(h.th[jj]);
-          P = fma(P, exp_f64(-2.0 * fabs(t)), P);
+          P = fma(P, exp_m2abs(t), P);
         } else {
           A += lane + NKA_WAVE * jj < M ? log_cosh<T>(t) - h.lc[jj] : (T)0;
         }
@@ -140,8 +140,9 @@ __device__ __forceinline__ void eloc_quads(uint64_t mask, const ElocEntry<T>& en
       re = P * (T)rpr;
       if constexpr (LOG) pe += log(re);
     };
-    // unrolled while four elements' loads and exponentials fit in 128 registers
-    if constexpr (JL <= (F64 ? 2 : 4)) {
+    // unrolled while four elements' loads and exponentials fit in 128 registers (FP64,
+    // 32 sites x 96 units: 65 us rolled, 74 unrolled with spills)
+    if constexpr (JL <= (F64 ? 1 : 4)) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) element(l[k], part[k], rat[k]);
     } else {

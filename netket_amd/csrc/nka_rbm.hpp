@@ -62,7 +62,7 @@ __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, co
       if constexpr (sizeof(T) == 4) {
         h.lc[jj] = log_cosh<T>(acc);
       } else {
-        prod = fma(prod, exp_f64(-2.0 * fabs(acc)), prod);
+        prod = fma(prod, exp_m2abs(acc), prod);
         ++live;
       }
     } else {
@@ -126,7 +126,7 @@ __device__ inline T flip_delta(const HiddenState<T, JL>& h, const int8_t* xs, co
         nlc[jj] = l;
         part += l - h.lc[jj];
       } else {
-        prod = fma(prod, exp_f64(-2.0 * fabs(t)), prod);
+        prod = fma(prod, exp_m2abs(t), prod);
         part += fabs(t) - fabs(h.th[jj]);
       }
     } else {

@@ -18,9 +18,9 @@
 // Bound by the FP64 issue rate with many chains, by the serial latency of a
 // proposal (about 800 cycles) with few.  Measured, against one exponential and
 // one log1p of the library per unit and a draw per proposal: 4096 chains, 64
-// sites, 128 hidden units, exchange, 576 proposals: 5.22 -> 0.85 ms (W, 64 KB, now
+// sites, 128 hidden units, exchange, 576 proposals: 5.22 -> 0.81 ms (W, 64 KB, now
 // staged in LDS as well); 16 chains, 16 sites and units, local rule, 1264
-// proposals: 0.91 -> 0.45 ms.
+// proposals: 0.91 -> 0.36 ms (two proposals per step, see below).
 #include "nka_sampler.hpp"
 
 namespace nka {
@@ -77,7 +77,7 @@ __device__ __forceinline__ void group64_body(const nka_rbm& m, const SweepArgs& 
         acc += (xs[i] > 0) ? w : -w;
       }
       th[jj] = acc;
-      P0 = fma(P0, exp_f64(-2.0 * fabs(acc)), P0);
+      P0 = fma(P0, exp_m2abs(acc), P0);
     }
   }
   P0 = group_prod<LPC>(P0);
@@ -154,7 +154,7 @@ __device__ __forceinline__ void group64_body(const nka_rbm& m, const SweepArgs& 
       for (int jj = 0; jj < JG; ++jj) {
         t[jj] = th[jj] + d[jj];
         A += fabs(t[jj]) - fabs(th[jj]);
-        P = fma(P, exp_f64(-2.0 * fabs(t[jj])), P);
+        P = fma(P, exp_m2abs(t[jj]), P);
       }
       A = group_sum<LPC>(A) + vis;
       P = group_prod<LPC>(P);
@@ -222,6 +222,201 @@ __global__ void __launch_bounds__(512) rbm_metropolis_group64_kernel_batched(con
                                  j.n_accepted, blockIdx.x);
 }
 
+// Local rule with few chains: two proposals per step.
+//
+// One chain per wavefront.  While proposal q is tested (lanes 0-15), q + 1 is
+// tested for both outcomes of q (lanes 16-31: q rejected; 32-47: q accepted), each
+// with the operations that it would see one after the other; the two decisions are
+// then taken together.  The serial chain of a test (W row, exponentials, product,
+// comparison) is what bounds few chains, and it is paid once per two proposals.  The
+// spins are bits in a register (lane l: sites 32 l ..), so that no LDS round trip
+// lies between a decision and the next test.
+// 16 chains, 16 sites and units, 1264 proposals: 0.36 ms, against 0.46 one at a time.
+template <int JG>
+__device__ __forceinline__ void pair64_body(const nka_rbm& m, const SweepArgs& sa, int8_t* __restrict__ sigma,
+                                            double* __restrict__ log_prob, int8_t* __restrict__ samples,
+                                            double* __restrict__ lp_samples, int64_t* __restrict__ n_accepted, int bx) {
+  constexpr int LPC = 16;
+  extern __shared__ unsigned char smem[];
+  const RbmView<double> v = rbm_view<double>(m);
+  const int N = v.N, M = v.M;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / NKA_WAVE), waves = blockDim.x / NKA_WAVE;
+  const int lane = lane_id(), e = lane >> 4, gl = lane & 15;
+  const double* W = (const double*)smem;
+  double* a_s = (double*)(smem + pad16((size_t)N * M * sizeof(double)));
+  for (int i = threadIdx.x; i < N; i += blockDim.x) a_s[i] = v.a ? v.a[i] : 0.0;
+  stage_w<double>((double*)smem, v.W, N, M);  // ends with a workgroup barrier
+  const int c = bx * waves + wid;
+  if (c >= sa.C) return;
+
+  uint32_t xb = 0;
+  for (int i0 = 0; i0 < N; i0 += NKA_WAVE) {
+    const uint64_t up = __ballot(i0 + lane < N && sigma[(int64_t)c * N + min(i0 + lane, N - 1)] > 0);
+    if (lane == i0 / 32) xb = (uint32_t)up;
+    if (lane == i0 / 32 + 1) xb = (uint32_t)(up >> 32);
+  }
+  auto spin_up = [&](int i) { return ((uint32_t)__builtin_amdgcn_readlane((int)xb, i >> 5) >> (i & 31)) & 1u; };
+  // unit gl + 16 jj (a slot past the last holds 1e300, as above)
+  double th[JG], P0 = 1.0;
+  int jo[JG];
+#pragma unroll
+  for (int jj = 0; jj < JG; ++jj) {
+    const int j = gl + LPC * jj;
+    th[jj] = 1e300;
+    jo[jj] = min(j, M - 1);
+    if (j < M) {
+      double acc = v.b ? v.b[j] : 0.0;
+      for (int i = 0; i < N; ++i) {
+        const double w = W[(size_t)i * M + j];
+        acc += spin_up(i) ? w : -w;
+      }
+      th[jj] = acc;
+      P0 = fma(P0, exp_m2abs(acc), P0);
+    }
+  }
+  P0 = group_prod<LPC>(P0);
+  const double pw = sa.machine_pow;
+  auto log_prob_now = [&]() {
+    double part = 0.0;
+#pragma unroll
+    for (int jj = 0; jj < JG; ++jj) part += gl + LPC * jj < M ? fabs(th[jj]) : 0.0;
+    for (int i0 = 0; i0 < N; i0 += LPC) {
+      const int i = i0 + gl;
+      const uint32_t w = (uint32_t)__shfl((int)xb, min(i, N - 1) >> 5);
+      part += i < N ? ((w >> (i & 31)) & 1u ? a_s[i] : -a_s[i]) : 0.0;
+    }
+    return pw * (group_sum<LPC>(part) + log_call(P0) - 0.69314718055994530942 * (double)M);
+  };
+
+  int64_t nacc = 0;
+  uint64_t q = sa.counter;
+  if (sa.counter_dev) {
+    const uint64_t cd = *sa.counter_dev;
+    q = ((uint64_t)uniform_value<uint32_t>((uint32_t)(cd >> 32)) << 32) |
+        (uint64_t)uniform_value<uint32_t>((uint32_t)cd);
+  }
+  DrawBlock<NKA_WAVE> draws;
+  draws.refill(q, (uint32_t)c, sa.k0, sa.k1);
+  // the next two proposals' draws, sites, W rows and visible biases
+  u32x4 r0n, r1n;
+  int s0n, s1n;
+  double w0n[JG], w1n[JG], a0n, a1n;
+  auto fetch = [&]() __attribute__((always_inline)) {
+    r0n = draws.at(q, (uint32_t)c, sa.k0, sa.k1);
+    r1n = draws.at(q + 1, (uint32_t)c, sa.k0, sa.k1);
+    s0n = __builtin_amdgcn_readfirstlane((int)bounded(r0n.x, (uint32_t)N));
+    s1n = __builtin_amdgcn_readfirstlane((int)bounded(r1n.x, (uint32_t)N));
+    a0n = a_s[s0n];
+    a1n = a_s[s1n];
+#pragma unroll
+    for (int jj = 0; jj < JG; ++jj) {
+      w0n[jj] = W[s0n * M + jo[jj]];
+      w1n[jj] = W[s1n * M + jo[jj]];
+    }
+  };
+  fetch();
+  const int n_sweeps = sa.n_discard + sa.chain_length;
+  for (int sw = 0; sw < n_sweeps; ++sw) {
+    for (int p = 0; p < sa.sweep_size; p += 2) {
+      const bool two = p + 1 < sa.sweep_size;
+      const u32x4 rnd = e == 0 ? r0n : r1n;
+      const int s0 = s0n, s1 = s1n;
+      // x' - x of a site; the second site's after the first was accepted
+      const double f0 = spin_up(s0) ? -2.0 : 2.0, f1 = spin_up(s1) ? -2.0 : 2.0;
+      const double f1a = s0 == s1 ? -f1 : f1;
+      const double fe = e == 2 ? f1a : f1;
+      const double vis = e == 0 ? f0 * a0n : fe * a1n;
+      double A = 0.0, P = 1.0, u[JG], w1[JG];
+#pragma unroll
+      for (int jj = 0; jj < JG; ++jj) {
+        u[jj] = th[jj] + f0 * w0n[jj];
+        w1[jj] = w1n[jj];
+        const double from = e == 2 ? u[jj] : th[jj];
+        const double t = e == 0 ? u[jj] : from + fe * w1[jj];
+        A += fabs(t) - fabs(from);
+        P = fma(P, exp_m2abs(t), P);
+      }
+      q += two ? 2 : 1;
+      fetch();
+      A = group_sum<LPC>(A) + vis;
+      P = group_prod<LPC>(P);
+      auto lane_value = [](double x, int l) {
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                                __builtin_amdgcn_readlane(__double2loint(x), l));
+      };
+      const double Pq = lane_value(P, 0);
+      const double Pe = e == 2 ? Pq : P0;
+      double lhs = Pe * Pe, rhs = P * P, x = 2.0 * A;
+      if (pw != 2.0) {
+        lhs = rhs = 1.0;
+        x = pw * (A + log_call(P / Pe));
+      }
+      const uint64_t acc = __ballot(uniform01<double>(rnd) * lhs < exp_f64(x) * rhs);
+      const bool acc0 = acc & 1ull;
+      const bool acc1 = two && (acc >> (acc0 ? 32 : 16) & 1ull);
+      if (acc0) {
+#pragma unroll
+        for (int jj = 0; jj < JG; ++jj) th[jj] = u[jj];
+        P0 = Pq;
+        xb ^= lane == s0 >> 5 ? 1u << (s0 & 31) : 0u;
+        ++nacc;
+      }
+      if (acc1) {
+        const double f = acc0 ? f1a : f1;
+#pragma unroll
+        for (int jj = 0; jj < JG; ++jj) th[jj] += f * w1[jj];
+        P0 = lane_value(P, acc0 ? 32 : 16);
+        xb ^= lane == s1 >> 5 ? 1u << (s1 & 31) : 0u;
+        ++nacc;
+      }
+    }
+    if (sw >= sa.n_discard) {
+      const int k = sw - sa.n_discard;
+      int8_t* dst = samples + ((int64_t)c * sa.chain_length + k) * N;
+      for (int i0 = 0; i0 < N; i0 += NKA_WAVE) {
+        const int i = i0 + lane;
+        const uint32_t w = (uint32_t)__shfl((int)xb, min(i, N - 1) >> 5);
+        if (i < N) dst[i] = (w >> (i & 31)) & 1u ? (int8_t)1 : (int8_t)-1;
+      }
+      if (lp_samples) {
+        const double lp = log_prob_now();
+        if (lane == 0) lp_samples[(int64_t)c * sa.chain_length + k] = lp;
+      }
+    }
+  }
+  const double lp = log_prob_now();
+  for (int i0 = 0; i0 < N; i0 += NKA_WAVE) {
+    const int i = i0 + lane;
+    const uint32_t w = (uint32_t)__shfl((int)xb, min(i, N - 1) >> 5);
+    if (i < N) sigma[(int64_t)c * N + i] = (w >> (i & 31)) & 1u ? (int8_t)1 : (int8_t)-1;
+  }
+  if (lane == 0) {
+    log_prob[c] = lp;
+    n_accepted[c] += nacc;
+  }
+}
+
+template <int JG>
+__global__ void __launch_bounds__(256) rbm_metropolis_pair64_kernel(nka_rbm m, SweepArgs sa, int8_t* __restrict__ sigma,
+                                                                    double* __restrict__ log_prob,
+                                                                    int8_t* __restrict__ samples,
+                                                                    double* __restrict__ lp_samples,
+                                                                    int64_t* __restrict__ n_accepted) {
+  pair64_body<JG>(m, sa, sigma, log_prob, samples, lp_samples, n_accepted, blockIdx.x);
+}
+template <int JG>
+__global__ void __launch_bounds__(256) rbm_metropolis_pair64_kernel_batched(const nka_sweep_job* __restrict__ jobs,
+                                                                            SweepArgs sa) {
+  const nka_sweep_job& j = jobs[blockIdx.y];
+  SweepArgs s = sa;
+  s.k0 = (uint32_t)j.seed;
+  s.k1 = (uint32_t)(j.seed >> 32);
+  s.counter = j.counter;
+  s.counter_dev = j.counter_dev;
+  pair64_body<JG>(j.model, s, j.sigma, (double*)j.log_prob, j.samples, (double*)j.log_prob_samples, j.n_accepted,
+                  blockIdx.x);
+}
+
 struct Group64 {
   const nka_rbm& m;
   const SweepArgs& sa;
@@ -254,6 +449,19 @@ struct Group64 {
   void allow(K kernel) const {
     if (lds > 64 * 1024)
       (void)hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  }
+  template <int JG>
+  void pair() const {
+    const unsigned g = (unsigned)((sa.C + waves - 1) / waves);
+    if (jobs) {
+      allow(rbm_metropolis_pair64_kernel_batched<JG>);
+      hipLaunchKernelGGL((rbm_metropolis_pair64_kernel_batched<JG>), dim3(g, n_jobs), dim3(64 * waves), lds, s, jobs,
+                         sa);
+    } else {
+      allow(rbm_metropolis_pair64_kernel<JG>);
+      hipLaunchKernelGGL((rbm_metropolis_pair64_kernel<JG>), dim3(g), dim3(64 * waves), lds, s, m, sa, sigma, lp, smp,
+                         lps, nacc);
+    }
   }
   template <int G, int JG>
   void rule() const {
@@ -290,6 +498,21 @@ static size_t group64_lds(const nka_rbm& m, const SweepArgs& sa, int waves, int 
 bool launch_group64(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, double* lp, int8_t* smp, double* lps,
                     int64_t* nacc, const nka_sweep_job* jobs, int n_jobs, hipStream_t s) {
   if (sa.weights) return false;
+  // two proposals per step while every chain has a SIMD of its own and its units fit
+  // four a lane (16 units: 1.30x at 16 chains, 1.16x at 1024, 0.97x at 2048; 64
+  // units: 1.07x, 1.01x, 0.75x)
+  const int64_t chains = (int64_t)sa.C * (jobs ? n_jobs : 1);
+  if (sa.rule == NKA_RULE_LOCAL && m.n_hidden <= 64 && m.n_visible <= 32 * NKA_WAVE && chains <= 4 * device_cus()) {
+    const size_t lds = pad16((size_t)m.n_visible * m.n_hidden * sizeof(double)) +
+                       pad16((size_t)m.n_visible * sizeof(double));
+    if (lds <= 156 * 1024) {
+      const Group64 k{m, sa, sigma, lp, smp, lps, nacc, jobs, n_jobs, 4, lds, s};
+      if (m.n_hidden <= 16) k.pair<1>();
+      else if (m.n_hidden <= 32) k.pair<2>();
+      else k.pair<4>();
+      return true;
+    }
+  }
   const bool four = m.n_hidden <= 16 || (m.n_hidden <= 128 && (int64_t)sa.C >= (int64_t)4 * 8 * device_cus());
   for (int G : {4, 2}) {
     if (G == 4 && !four) continue;

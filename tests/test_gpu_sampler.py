@@ -231,3 +231,34 @@ def test_wide_model_chains_carry_their_own_log_prob(gpu, N, alpha, n_chains, swe
     ref = 2 * orbm.log_psi(p, st.sigma.cpu().numpy())
     # 7 sweeps of accumulated FP32 steps
     np.testing.assert_allclose(st.log_prob.cpu().numpy(), ref, rtol=0, atol=1e-4 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("N,M,n_chains,sweep,power", [
+    (16, 16, 3, 16, 2.0),        # two proposals per step
+    (16, 16, 1030, 9, 2.0),      # more chains than SIMDs: one at a time
+    (3, 5, 4, 7, 2.0),           # three sites: both proposals of a step often flip the same one
+    (2, 64, 2, 5, 1.0),
+    (33, 33, 5, 33, 2.0),        # odd sweeps end with a single proposal; spins in two words
+    (70, 20, 2, 3, 2.0),
+    (1100, 17, 2, 40, 2.0),      # W of 150 KB, spins over 35 lanes
+])
+def test_fp64_local_chains_two_proposals_per_step(gpu, N, M, n_chains, sweep, power):
+    print(f"case fp64 pairs N={N} M={M} chains={n_chains} sweep={sweep} power={power}", flush=True)
+    model, flat, p = _model(N, (M + 0.5) / N, np.float64, 12, 0.7 / np.sqrt(M))
+    assert p.W.shape == (N, M)
+    sa = nk.sampler.MetropolisLocal(nk.hilbert.Spin(0.5, N=N), n_chains=n_chains, sweep_size=sweep,
+                                    machine_pow=power)
+    st = sa.init_state(model, flat, seed=23)
+    sigma0 = st.sigma.cpu().numpy().copy()
+    counter0 = st.counter
+    (samples, lps), st = sa.sample_fused(model, flat, st, 3, 4, return_log_probabilities=True)
+    ref, ref_sigma, ref_acc = osamp.metropolis(p, sigma0, rule="local", clusters=None, n_discard=3,
+                                               chain_length=4, sweep_size=sweep, seed=23, counter=counter0,
+                                               machine_pow=power)
+    np.testing.assert_array_equal(samples.cpu().numpy(), ref)
+    np.testing.assert_array_equal(st.sigma.cpu().numpy(), ref_sigma)
+    np.testing.assert_array_equal(st.n_accepted_proc.cpu().numpy(), ref_acc)
+    lp_ref = power * orbm.log_psi(p, ref.reshape(-1, N)).reshape(n_chains, 4)
+    tol = 1e-12 * np.abs(lp_ref).max()
+    np.testing.assert_allclose(lps.cpu().numpy(), lp_ref, rtol=0, atol=tol)
+    np.testing.assert_allclose(st.log_prob.cpu().numpy(), lp_ref[:, -1], rtol=0, atol=tol)
