@@ -325,7 +325,7 @@ constexpr int kExactAMIA = 3, kExactAMIB = 2;
 constexpr int kExactAChunk = 16;
 
 template <int MIA, int MIB>
-__global__ void __launch_bounds__(256, 1) gemm_exact_a_kernel(const uint16_t* __restrict__ a, int64_t ma,
+__global__ void __launch_bounds__(256, MIA * MIB == 1 ? 4 : 1) gemm_exact_a_kernel(const uint16_t* __restrict__ a, int64_t ma,
                                                            const uint16_t* __restrict__ bh,
                                                            const uint16_t* __restrict__ bl, int64_t nb,
                                                            int64_t K, int64_t ldk, float* __restrict__ c,
@@ -1217,21 +1217,46 @@ bool launch_gram_rbm(const uint16_t* xh, const uint16_t* xl, int64_t n, int64_t 
   return true;
 }
 
-// The two-layer network's tangent kernel on the bf16x3 Gram tiles (called from
-// the network's NTK entry point): H, G and D from the split h1, g2 and d1
-// (hi + lo planes, n rows each), X from the packed spins.  Returns false when
-// the spins do not fit the epilogue.
+// Workgroups of the 128-tile kernel resident at once (two per CU), from the
+// device's CU count (queried once per process for the current device).
+static int64_t big_gemm_slots() {
+  static int64_t slots = 0;
+  if (slots == 0) {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
+      slots = 2 * (int64_t)cus;
+    else
+      slots = 512;
+  }
+  return slots;
+}
+
 // C = A (Bh + Bl)^T (FP32) for an exact single-plane A; K and ldk multiples
 // of 8, operands 16-byte aligned (checked by the caller).
 void launch_gemm_exact_a(const uint16_t* a, int64_t ma, const uint16_t* bh, const uint16_t* bl, int64_t nb,
                          int64_t K, int64_t ldk, float* c, int64_t ldc, hipStream_t s) {
+  if (ma == 0 || nb == 0) return;
   constexpr int TA = 64 * kExactAMIA, TB = 64 * kExactAMIB;
   const int64_t tm = (ma + TA - 1) / TA, tn = (nb + TB - 1) / TB;
-  if (tm == 0 || tn == 0) return;
-  hipLaunchKernelGGL((gemm_exact_a_kernel<kExactAMIA, kExactAMIB>), dim3(grid_mult8(tm * tn)), dim3(256), 0, s, a,
-                     ma, bh, bl, nb, K, ldk, c, ldc, tm, tm * tn);
+  // A round of 192x128 tiles over the chip takes 1.6 us per K slab of 64, 64x64 tiles
+  // 0.2 + 0.35 per tile and CU (0.65 at least): the small ones where they are
+  // fewer.  Same sums.  Whole dense S at 36 sites x 36 units, 6912 samples (121
+  // tiles of 64x64): 138 us against 231; 48 x 96, 4096 (1387): 292 against 367; 64 x
+  // 64 (1089): 223 against 218.
+  const int64_t sm = (ma + 63) / 64, sn = (nb + 63) / 64, cus = big_gemm_slots() / 2;
+  if (sm * sn + 128 < 1180 * ((tm * tn + cus - 1) / cus))
+    hipLaunchKernelGGL((gemm_exact_a_kernel<1, 1>), dim3(grid_mult8(sm * sn)), dim3(256), 0, s, a, ma, bh, bl, nb, K,
+                       ldk, c, ldc, sm, sm * sn);
+  else
+    hipLaunchKernelGGL((gemm_exact_a_kernel<kExactAMIA, kExactAMIB>), dim3(grid_mult8(tm * tn)), dim3(256), 0, s, a,
+                       ma, bh, bl, nb, K, ldk, c, ldc, tm, tm * tn);
 }
 
+// The two-layer network's tangent kernel on the bf16x3 Gram tiles (called from
+// the network's NTK entry point): H, G and D from the split h1, g2 and d1
+// (hi + lo planes, n rows each), X from the packed spins.  Returns false when
+// the spins do not fit the epilogue.
 bool launch_gram_ffnn(const uint16_t* h1h, const uint16_t* h1l, int64_t K0, int64_t ld0, const uint16_t* g2h,
                       const uint16_t* g2l, int64_t K1, int64_t ld1, const uint16_t* d1h, const uint16_t* d1l,
                       int64_t K2, int64_t ld2, int64_t n, const uint32_t* bits, int nw, int N, const double* v,
@@ -1281,22 +1306,6 @@ static int gemm_launch(const double* a, int64_t lda, const double* b, int64_t ld
   return NKA_OK;
 }
 
-// The 128-tile kernel needs K to be a multiple of its K step; other shapes
-// take the 64-tile kernel.
-// Workgroups of the 128-tile kernel resident at once (two per CU), from the
-// device's CU count (queried once per process for the current device).
-static int64_t big_gemm_slots() {
-  static int64_t slots = 0;
-  if (slots == 0) {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
-      slots = 2 * (int64_t)cus;
-    else
-      slots = 512;
-  }
-  return slots;
-}
 
 // Tail-split workspace of the 128-tile GEMM: at most kMaxSplitUnits raw tiles.
 constexpr int64_t kMaxSplitUnits = 1024;
