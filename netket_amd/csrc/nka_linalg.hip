@@ -303,34 +303,170 @@ constexpr int kGramRbmWT = 64;
 
 // ---------------------------------------------------------------------------
 // C = A (Bh + Bl)^T in FP32 (ma x nb), K contiguous in both operands (row
-// stride ldk, zero beyond the true K).  A is one bf16 plane whose entries
-// bf16 holds exactly (products of +-1 spins, 0 and 1); B is split into two
-// bf16 planes.  Each fragment pair therefore takes two products instead of
-// the Gram's three, and A's LDS slab is a single plane.  Four waves of
-// 32 MIA x 32 MIB (v_mfma_f32_32x32x16_bf16) make a 64 MIA x 64 MIB tile;
-// K step, slab prefetch and fragment layout are the Gram kernel's.  Tiles are
-// numbered down the columns (the ma side fastest), so the workgroups that
-// share a B column panel (the larger operand) sit on one XCD and read it
-// through one L2.
+// stride ldk, a multiple of 64; K too, zero beyond the true K).  A is one bf16
+// plane whose entries bf16 holds exactly (products of +-1 spins, 0 and 1); B
+// is split into two bf16 planes.  Each fragment pair therefore takes two
+// products (v_mfma_f32_32x32x16_bf16) instead of the Gram's three, and A's LDS
+// slab is a single plane.  Tiles are numbered down the columns (the ma side
+// fastest), so the workgroups that share a B column panel (the larger operand)
+// sit on one XCD and read it through one L2.
 // The FP32 accumulation inside the MFMA rounds with a bias (the error of a
 // plain sum over 16384 samples grows like the number of accumulations times
 // 2^-24, not like its square root), so the products are accumulated on the
-// matrix cores for kExactAChunk K steps (128 accumulations) at a time and each
-// chunk is added into a separate FP32 total with round-to-nearest vector adds.
-// 192 x 128 tiles (3 x 2 blocks of 32 x 32 per wave) leave the registers for
-// that total; the single-plane operand takes the 192-row side, so a K step
-// reads 7 fragments per 12 products from LDS.
+// matrix cores for 64 kExactAChunk samples (128 accumulations) at a time and
+// each chunk is added into a separate FP32 total with round-to-nearest vector
+// adds.  Both kernels take the products of an entry in the same order.
 // ---------------------------------------------------------------------------
-constexpr int kExactAMIA = 3, kExactAMIB = 2;
 constexpr int kExactAChunk = 16;
+constexpr int kExactAMIA = 3, kExactAMIB = 2;  // 32 x 32 blocks per wavefront
+constexpr int kExactAK = 32;                   // samples per K step
+constexpr int kExactABuf = 4;                  // K steps held in LDS
 
-template <int MIA, int MIB>
-__global__ void __launch_bounds__(256, MIA * MIB == 1 ? 4 : 1) gemm_exact_a_kernel(const uint16_t* __restrict__ a, int64_t ma,
+// 192 x 128 tiles, four wavefronts of 96 x 64, one workgroup per CU: the
+// accumulators and totals take 192 registers, and a sub-step of 16 samples
+// reads 7 fragments from LDS for 12 products.  Operands go from global memory
+// straight into LDS, three K steps ahead; one request (an LDS read of the other
+// sub-step's fragments, or a load of a later step) stands behind each product.
+// A row's four 16-byte chunks of a K step are stored in the order
+// chunk ^ (row / 4 % 4): fragment reads (32 consecutive rows, one chunk) are
+// free of bank conflicts over the 64 banks.  Bound by the matrix cores.
+// 2081 x 8385 x 16384: 1.24 ms (0.92 PFLOP/s executed, a library bf16 product
+// reaches 1.09), 1.42 with the slab prefetched into registers and one buffer.
+// Whole dense S there 1.80 -> 1.57 ms; the whole SR step, whose FP64 products
+// then run at a lower clock, 8.25 -> 8.18 ms.
+// ldk < 2^26, so that 16 rows lie within a buffer descriptor's offsets.
+__global__ void __launch_bounds__(256, 1) gemm_exact_a_kernel(const uint16_t* __restrict__ a, int64_t ma,
                                                            const uint16_t* __restrict__ bh,
-                                                           const uint16_t* __restrict__ bl, int64_t nb,
-                                                           int64_t K, int64_t ldk, float* __restrict__ c,
-                                                           int64_t ldc, int64_t tiles_m, int64_t n_tiles_total) {
-  constexpr int TA = 64 * MIA, TB = 64 * MIB;
+                                                           const uint16_t* __restrict__ bl, int64_t nb, int64_t K,
+                                                           int64_t ldk, float* __restrict__ c, int64_t ldc,
+                                                           int64_t tiles_m, int64_t n_tiles_total) {
+  constexpr int MIA = kExactAMIA, MIB = kExactAMIB, TA = 64 * MIA, TB = 64 * MIB;
+  constexpr int ROWB = 2 * kExactAK, BYTES = (TA + 2 * TB) * ROWB;  // a row's and a K step's bytes
+  constexpr int LOADS = BYTES / 1024 / 4;                           // 16-row loads per wavefront and K step
+  constexpr int AHEAD = kExactABuf - 1;                             // K steps in flight ahead of the products
+  static_assert(ROWB == 64 && BYTES % 4096 == 0, "whole loads per wavefront");
+  __shared__ __attribute__((aligned(1024))) uint8_t smem[kExactABuf][BYTES];
+  const int64_t bid = xcd_remap(blockIdx.x, gridDim.x);
+  if (bid >= n_tiles_total) return;
+  const int64_t i0 = (bid % tiles_m) * TA, j0 = (bid / tiles_m) * TB;
+  const int tid = threadIdx.x, wid = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int wm = (wid >> 1) * 32 * MIA, wn = (wid & 1) * 32 * MIB;
+  const int64_t steps = K / kExactAK;
+
+  // Each of the wavefront's loads covers 16 rows of A or of one plane of B: a
+  // buffer descriptor of those rows (rows past the operand's end read as zero),
+  // and for this lane row lane / 4 and the chunk that belongs in slot lane % 4.
+  __amdgpu_buffer_rsrc_t src[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int row = (wid * LOADS + i) * 16;  // first row in the stacked tile (A, B hi, B lo)
+    const int b = row - TA;
+    const int64_t first = row < TA ? i0 + row : j0 + b % TB, rows = row < TA ? ma : nb;
+    const uint16_t* base = row < TA ? a : b < TB ? bh : bl;
+    const int64_t left = min<int64_t>(max<int64_t>(rows - first, 0), 16);
+    const uint64_t addr = (uint64_t)(base + (left > 0 ? first : 0) * ldk);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)addr);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)(addr >> 32));
+    src[i] = __builtin_amdgcn_make_buffer_rsrc((void*)(((uint64_t)hi << 32) | lo), 0,
+                                               __builtin_amdgcn_readfirstlane((int)(2 * left * ldk)), 0x00020000);
+  }
+  // (row / 4) % 4 of the stacked row is that of the row among the 16
+  const int voff = (lane >> 2) * 2 * (int)ldk + (((lane & 3) ^ ((lane >> 4) & 3)) * 16);
+  auto issue = [&](int buf, int64_t t, int i) __attribute__((always_inline)) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        src[i], (__attribute__((address_space(3))) void*)&smem[buf][(wid * LOADS + i) * 1024], 16, voff,
+        (int)(t * ROWB), 0, 0);
+  };
+  floatx16 acc[MIA][MIB], tot[MIA][MIB];
+#pragma unroll
+  for (int x = 0; x < MIA; ++x)
+#pragma unroll
+    for (int y = 0; y < MIB; ++y)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[x][y][e] = tot[x][y][e] = 0.0f;
+
+  // fragment f (A blocks, B lo, B hi) of sub-step ks of the step in `buf`
+  const int fr = lane & 31, sw = (fr >> 2) & 3;
+  const int foff[2] = {fr * ROWB + ((lane >> 5) ^ sw) * 16, fr * ROWB + ((2 + (lane >> 5)) ^ sw) * 16};
+  auto frag = [&](int buf, int ks, int f) __attribute__((always_inline)) {
+    const int y = f - MIA;
+    const int row = f < MIA ? wm + f * 32 : TA + (y < MIB ? TB + y * 32 : (y - MIB) * 32) + wn;
+    return *(const bf16x8*)(smem[buf] + row * ROWB + foff[ks]);
+  };
+  // Two phases of 12 products per K step: a phase multiplies one sub-step's
+  // fragments while it reads the other's (the next step's first ones in phase 1)
+  // and issues its share of the loads of the step AHEAD.  (The last steps are
+  // requested again past the end: the count of loads in flight is the same at
+  // every step.)
+  constexpr int NF = MIA + 2 * MIB, NP = 2 * MIA * MIB, SPLIT = NP - NF;
+  static_assert(SPLIT >= 0 && LOADS >= SPLIT && LOADS - SPLIT <= NP, "requests fit behind the products");
+  bf16x8 fg[2][NF];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+    for (int k = 0; k < LOADS; ++k) issue(i, min<int64_t>(i, steps - 1), k);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((AHEAD - 1) * LOADS) : "memory");
+#pragma unroll
+  for (int f = 0; f < NF; ++f) fg[0][f] = frag(0, 0, f);
+  int buf = 0;
+  for (int64_t t = 0; t < steps; ++t) {
+    if (t != 0 && t % (64 / kExactAK * kExactAChunk) == 0) {
+#pragma unroll
+      for (int x = 0; x < MIA; ++x)
+#pragma unroll
+        for (int y = 0; y < MIB; ++y)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) {
+            tot[x][y][e] += acc[x][y][e];
+            acc[x][y][e] = 0.0f;
+          }
+    }
+    const int next = (buf + 1) % kExactABuf, into = (buf + AHEAD) % kExactABuf;
+    const int64_t tl = min<int64_t>(t + AHEAD, steps - 1);
+#pragma unroll
+    for (int ph = 0; ph < 2; ++ph) {
+      if (ph == 1)
+        // this wavefront's loads of step t + 1 have landed and its reads of step t
+        // are done; after the barrier that holds for all four
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((AHEAD - 2) * LOADS + SPLIT) : "memory");
+#pragma unroll
+      for (int q = 0; q < NP; ++q) {
+        // small products first
+        const int x = q / MIB % MIA, y = q % MIB, pl = q / (MIA * MIB);
+        acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fg[ph][x], fg[ph][MIA + pl * MIB + y], acc[x][y], 0, 0, 0);
+        if (q < NF) fg[ph ^ 1][q] = ph == 0 ? frag(buf, 1, q) : frag(next, 0, q);
+        if (ph == 0 && q >= NF) issue(into, tl, q - NF);
+        if (ph == 1 && q >= NP - (LOADS - SPLIT)) issue(into, tl, SPLIT + q - (NP - (LOADS - SPLIT)));
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    buf = next;
+  }
+  // no load may be in flight into LDS when the workgroup ends
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // element e of lane l in a 32x32 block is (row (e/4)*8 + (l/32)*4 + e%4, col l%32)
+#pragma unroll
+  for (int x = 0; x < MIA; ++x)
+#pragma unroll
+    for (int y = 0; y < MIB; ++y)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int64_t gi = i0 + wm + x * 32 + (e / 4) * 8 + (lane >> 5) * 4 + (e & 3);
+        const int64_t gj = j0 + wn + y * 32 + (lane & 31);
+        if (gi < ma && gj < nb) c[gi * ldc + gj] = tot[x][y][e] + acc[x][y][e];
+      }
+}
+
+// 64 x 64 tiles (a 32 x 32 block per wavefront, four workgroups per CU) for
+// products whose large tiles would leave CUs idle.  K step, slab prefetch and
+// fragment layout are the Gram kernel's.
+__global__ void __launch_bounds__(256, 4) gemm_exact_a_small_kernel(const uint16_t* __restrict__ a, int64_t ma,
+                                                                 const uint16_t* __restrict__ bh,
+                                                                 const uint16_t* __restrict__ bl, int64_t nb,
+                                                                 int64_t K, int64_t ldk, float* __restrict__ c,
+                                                                 int64_t ldc, int64_t tiles_m,
+                                                                 int64_t n_tiles_total) {
+  constexpr int MIA = 1, MIB = 1, TA = 64 * MIA, TB = 64 * MIB;
   constexpr int NITA = TA * GB_CPR / 256, NITB = TB * GB_CPR / 256;
   constexpr int NIT = NITA > NITB ? NITA : NITB;
   __shared__ __attribute__((aligned(16))) uint16_t sA[TA * GB_LD];
@@ -1243,23 +1379,23 @@ static int64_t big_gemm_slots() {
 }
 
 // C = A (Bh + Bl)^T (FP32) for an exact single-plane A; K and ldk multiples
-// of 8, operands 16-byte aligned (checked by the caller).
+// of 64, operands 16-byte aligned (checked by the caller).
 void launch_gemm_exact_a(const uint16_t* a, int64_t ma, const uint16_t* bh, const uint16_t* bl, int64_t nb,
                          int64_t K, int64_t ldk, float* c, int64_t ldc, hipStream_t s) {
   if (ma == 0 || nb == 0) return;
   constexpr int TA = 64 * kExactAMIA, TB = 64 * kExactAMIB;
   const int64_t tm = (ma + TA - 1) / TA, tn = (nb + TB - 1) / TB;
-  // A round of 192x128 tiles over the chip takes 1.6 us per K slab of 64, 64x64 tiles
+  // A round of 192x128 tiles over the chip takes 1.05 us per K slab of 64, 64x64 tiles
   // 0.2 + 0.35 per tile and CU (0.65 at least): the small ones where they are
   // fewer.  Same sums.  Whole dense S at 36 sites x 36 units, 6912 samples (121
-  // tiles of 64x64): 138 us against 231; 48 x 96, 4096 (1387): 292 against 367; 64 x
-  // 64 (1089): 223 against 218.
+  // tiles of 64x64): 136 us against 165; 36 x 72, 4096 (462): 140 against 152;
+  // 48 x 96, 4096 (1387, two rounds): 300 against 300; 64 x 64, 4096 (1089): 228 against 190.
   const int64_t sm = (ma + 63) / 64, sn = (nb + 63) / 64, cus = big_gemm_slots() / 2;
-  if (sm * sn + 128 < 1180 * ((tm * tn + cus - 1) / cus))
-    hipLaunchKernelGGL((gemm_exact_a_kernel<1, 1>), dim3(grid_mult8(sm * sn)), dim3(256), 0, s, a, ma, bh, bl, nb, K,
+  if (sm * sn + 146 < 768 * ((tm * tn + cus - 1) / cus) || ldk >= 1 << 26)
+    hipLaunchKernelGGL(gemm_exact_a_small_kernel, dim3(grid_mult8(sm * sn)), dim3(256), 0, s, a, ma, bh, bl, nb, K,
                        ldk, c, ldc, sm, sm * sn);
   else
-    hipLaunchKernelGGL((gemm_exact_a_kernel<kExactAMIA, kExactAMIB>), dim3(grid_mult8(tm * tn)), dim3(256), 0, s, a,
+    hipLaunchKernelGGL(gemm_exact_a_kernel, dim3(grid_mult8(tm * tn)), dim3(256), 0, s, a,
                        ma, bh, bl, nb, K, ldk, c, ldc, tm, tm * tn);
 }
 

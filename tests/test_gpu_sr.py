@@ -192,6 +192,14 @@ def test_rbm_qgt_structured(gpu, ns, biases, N, alpha):
     assert np.all(S[up] == 7.0)
 
 
+@pytest.mark.parametrize("ns", [40, 1025, 2100])
+def test_rbm_qgt_structured_large_tiles(gpu, ns):
+    # 192 x 128 tiles with a remainder on both sides (2081 = 10 * 192 + 161 =
+    # 16 * 128 + 33 rows): fewer K steps than are loaded ahead, and sums past
+    # one and two accumulation chunks
+    test_rbm_qgt_structured(gpu, ns, (True, True), 64, 1)
+
+
 def test_rbm_qgt_structured_large_mean_activations(gpu):
     # hidden biases of 2 put every tanh near 0.96 with a small spread, so
     # E[t_j t_l] is far larger than S's entries: the activations are centred
