@@ -468,12 +468,12 @@ def roofline_for(stage: str, mean_ms: float):
                 "mean_ms": mean_ms}
     if stage == "local_energy":
         u = unit_utilisation("rbm_eloc_kernel")
-        return {"bound": "salu", "achieved": u.get("salu_issue") if u else None, "peak": 1.0,
-                "unit": "fraction of scalar-unit cycles issuing SALU (counters)",
-                "frac": u.get("salu_issue") if u else None, "valu_busy": u.get("valu_busy") if u else None,
+        return {"bound": "valu", "achieved": u.get("valu_busy") if u else None, "peak": 1.0,
+                "unit": "fraction of SIMD cycles issuing VALU (counters)",
+                "frac": u.get("valu_busy") if u else None, "salu_issue": u.get("salu_issue") if u else None,
                 "traffic": measured_traffic("rbm_eloc_kernel"), "kernel": "rbm_eloc_kernel",
-                "per_launch": "16384 samples x 64 bonds; the walk over the operator tables (one scalar lookup chain "
-                              "per bond) keeps the scalar unit the busiest, W is in LDS",
+                "per_launch": "16384 samples x 64 bonds; the log-cosh sums of the connected elements, four at a "
+                              "time, keep the vector units the busiest, W is in LDS",
                 "mean_ms": mean_ms}
     return None
 
@@ -549,8 +549,7 @@ def measured_traffic_per_call(kernels, per_call_kernel: str):
     return int(total / calls)
 
 
-POTRF_KERNELS = ("panel_step_kernel", "gemm_nt_f64_big_kernel", "panel_factor_kernel", "gemm_big_reduce_kernel",
-                 "trtri_blocks_kernel", "potf2_kernel", "panel_update_kernel")
+POTRF_KERNELS = ("panel_step_kernel", "gemm_nt_f64_big_kernel", "gemm_big_reduce_kernel", "trtri_blocks_kernel")
 QGT_KERNELS = ("qgt_spins_t_kernel", "qgt_spin_pairs_kernel", "qgt_hidden_means_kernel", "qgt_hidden_pairs_kernel",
                "gemm_exact_a_kernel", "qgt_unpack_kernel")
 
@@ -648,7 +647,7 @@ def main():
     # roofline of the dominant stage (the Cholesky factorisation of S); the
     # other stages are listed beside it
     roof = roofline_for("potrf", stages["potrf"]["mean_ms"])
-    roof["traffic"] = measured_traffic_per_call(POTRF_KERNELS, "potf2_kernel")
+    roof["traffic"] = measured_traffic_per_call(POTRF_KERNELS, "trtri_blocks_kernel")
     others = {k: roofline_for(k, stages[k]["mean_ms"]) for k in ("qgt_structured", "metropolis", "local_energy")
               if k in stages}
     if others.get("qgt_structured"):

@@ -416,15 +416,18 @@ int nka_gemv_f64(const double* a, int64_t lda, int64_t m, int64_t n, int trans, 
 
 /* Cholesky factorisation A = L L^T of the lower triangle in place (FP64),
  * cho_factor of netket/optimizer/solver/solvers.py:241-270.  workspace holds
- * nka_potrf_workspace(n) bytes (inverses of the diagonal blocks).  info (one
+ * nka_potrf_workspace(n) bytes (inverses of the diagonal blocks, and the
+ * solves' buffers in their starting state).  info (one
  * device int32) is 0 on success, or j+1 for the first non-positive or
  * non-finite pivot j; later kernels of the same call skip their work then. */
 int64_t nka_potrf_workspace(int64_t n);
 int nka_potrf_f64(double* a, int64_t n, int64_t lda, void* workspace, int32_t* info,
                   void* stream);
 
-/* cho_solve: b <- A^{-1} b from the factor of nka_potrf_f64 (same workspace);
- * b is set to NaN when the factorisation failed (info != 0). */
+/* cho_solve: b <- A^{-1} b from the factor of nka_potrf_f64 (same workspace, as
+ * nka_potrf_f64 or the last nka_potrs_f64 left it; its solve buffers are used
+ * and left in their starting state, so solves from one workspace are ordered,
+ * never concurrent); b is set to NaN when the factorisation failed (info != 0). */
 int nka_potrs_f64(const double* a, int64_t n, int64_t lda, const void* workspace, double* b,
                   const int32_t* info, void* stream);
 
