@@ -71,6 +71,36 @@ struct ElocEntry {
   T va[4];
 };
 
+// (1 + a)(1 + b) - 1
+__device__ __forceinline__ double prod_less_one(double a, double b) { return fma(a, b, a + b); }
+
+// The product of v over the wavefront, in every lane; `rest` becomes the sum of the
+// lanes' relative residuals and of those of the product's own roundings.
+__device__ inline void wave_prod_rest(double& v, double& rest) {
+  auto step = [&](double w, double wr) __attribute__((always_inline)) {
+    const double p = v * w;
+    rest += wr + fma(v, w, -p) * __builtin_amdgcn_rcp(p);
+    v = p;
+  };
+  step(dpp_perm<kDppXor1>(v), dpp_perm<kDppXor1>(rest));
+  step(dpp_perm<kDppXor2>(v), dpp_perm<kDppXor2>(rest));
+  step(dpp_perm<kDppHalfMirror>(v), dpp_perm<kDppHalfMirror>(rest));
+  step(dpp_perm<kDppMirror>(v), dpp_perm<kDppMirror>(rest));
+  double a = v, b = v, ar = rest, br = rest;
+  swap_rows16(a, b);
+  swap_rows16(ar, br);
+  v = a;
+  rest = ar;
+  step(b, br);
+  a = b = v;
+  ar = br = rest;
+  swap_halves(a, b);
+  swap_halves(ar, br);
+  v = a;
+  rest = ar;
+  step(b, br);
+}
+
 // sum mel exp(log psi(x') - log psi(x)) over the entries of the lanes in
 // `mask`, added to E of the lanes of the four rows (E of a row's lanes agree).
 //
@@ -78,12 +108,13 @@ struct ElocEntry {
 // four sums share the cross-lane steps (a row of 16 lanes ends with one
 // element's), and one exponential per row serves all four.  FP32: the units'
 // log_cosh differences, summed over the lanes in the order 1, 2, 4, ..., 32.
-// FP64: sum |t| - |theta| and the product of (1 + e^{-2|t|}) / (1 + e^{-2|theta|})
-// (at most 2^960 over the lanes; with more than 15 units per lane, its logarithm),
-// one exponential per unit.
+// FP64: sum |t| - |theta| and the product of 1 + e^{-2|t|} over the lanes (at most
+// 2^960; kept less one, so that no factor is rounded at size one) times `rpr`, the
+// sample's 1 / prod (1 + e^{-2|theta|}); with more than 15 units per lane `rpr` is the
+// lane's and the logarithms of the lanes' quotients are added.  One exponential per unit.
 //
 // Bound by the vector units (78% busy in FP64).  Heisenberg, 64 sites, 128 units,
-// 16384 samples, FP64: 0.17 ms; an element at a time, each with its own reduction
+// 16384 samples, FP64: 0.18 ms; an element at a time, each with its own reduction
 // over the wavefront, its logarithms and W from the cache, 0.46 ms.  FP32: 0.12 and
 // 0.40 ms.
 template <class T, int JL>
@@ -125,20 +156,21 @@ __device__ __forceinline__ void eloc_quads(uint64_t mask, const ElocEntry<T>& en
         flip(s23 & 0xffffu, 3);
         flip(s23 >> 16, 4);
       }
-      T A = (T)0, P = (T)1;
+      T A = (T)0, Z = (T)0;
 #pragma unroll
       for (int jj = 0; jj < JL; ++jj) {
         const T t = h.th[jj] + d[jj];
         if constexpr (F64) {
           A += fabs(t) - fabs(h.th[jj]);
-          P = fma(P, exp_m2abs(t), P);
+          const T e = exp_m2abs(t);
+          Z = jj == 0 ? e : prod_less_one(Z, e);
         } else {
           A += lane + NKA_WAVE * jj < M ? log_cosh<T>(t) - h.lc[jj] : (T)0;
         }
       }
       pe = A;
-      re = P * (T)rpr;
-      if constexpr (LOG) pe += log(re);
+      re = Z;
+      if constexpr (LOG) pe += log(fma(Z, rpr, rpr));
     };
     // unrolled while four elements' loads and exponentials fit in 128 registers (FP64,
     // 32 sites x 96 units: 65 us rolled, 74 unrolled with spills)
@@ -179,9 +211,14 @@ __device__ __forceinline__ void eloc_quads(uint64_t mask, const ElocEntry<T>& en
       if constexpr (!LOG) {
         swap_halves(rat[0], rat[1]);
         swap_halves(rat[2], rat[3]);
-        double x = rat[0] * rat[1], y = rat[2] * rat[3];
+        double x = prod_less_one(rat[0], rat[1]), y = prod_less_one(rat[2], rat[3]);
         swap_rows16(x, y);
-        prod = row_prod(x * y);
+        x = prod_less_one(x, y);
+        x = prod_less_one(x, dpp_perm<kDppXor1>(x));
+        x = prod_less_one(x, dpp_perm<kDppXor2>(x));
+        x = prod_less_one(x, dpp_perm<kDppHalfMirror>(x));
+        x = prod_less_one(x, dpp_perm<kDppMirror>(x));
+        prod = fma(x, rpr, rpr);
       }
       el = (row >> 1) | ((row & 1) << 1);
     } else {
@@ -247,13 +284,25 @@ __device__ __forceinline__ void rbm_eloc_body(const nka_rbm& m, const OpArgs& op
       const T lp = sum_log_cosh<T, JL>(h) + visible_term<T>(xs, v.a, N);
       if (lane == 0) log_psi[b] = lp;
     }
-    double rpr = 1.0;
+    double rpr = 1.0, rest = 0.0;
     if constexpr (sizeof(T) == 8) {
-      // a unit past the last has t = 0, a factor of two of its own
-      int dead = 0;
+      // a unit past the last: no change moves it, and its factor is one
 #pragma unroll
-      for (int jj = 0; jj < JL; ++jj) dead += lane + NKA_WAVE * jj < M ? 0 : 1;
-      rpr = ldexp(1.0 / h.pr, -dead);
+      for (int jj = 0; jj < JL; ++jj)
+        if (lane + NKA_WAVE * jj >= M) h.th[jj] = 1e300;
+      // `rest`: what the roundings of the lanes' 1 / pr and of their product leave out,
+      // relative.  It is common to all elements of the sample, so it would not average
+      // out of their sum.  Error of a sum of flips, 10 sites x 20 units and 64 x 128:
+      // 1.5e-16 and 2.4e-16; 4.0e-16 and 7.4e-16 without it and with the factors rounded
+      // at size one; 2.6e-16 and 5.9e-16 as sums of log_cosh differences.
+      const double inv = 1.0 / h.pr;
+      rest = fma(-h.pr, inv, 1.0) - h.pe * inv;
+      rpr = inv;
+      if constexpr (JL <= 15) {
+        wave_prod_rest(rpr, rest);
+      } else {
+        rest = wave_sum(rest);
+      }
     }
     auto visible = [&](ElocEntry<T>& en) {
       double sum = 0.0;
@@ -338,6 +387,7 @@ __device__ __forceinline__ void rbm_eloc_body(const nka_rbm& m, const OpArgs& op
     w = E;
     swap_halves(E, w);
     E += w;
+    if constexpr (sizeof(T) == 8) E = isfinite(E) ? fma(E, rest, E) : E;
     if (lane == 0) eloc[b] = diag + E;
     wave_lds_sync();
   }

@@ -37,6 +37,7 @@ template <int JL>
 struct HiddenState<double, JL> {
   double th[JL];
   double pr;    // product of 1 + e^{-2|theta_j|} over this lane's units (at most 2^64)
+  double pe;    // what its roundings left out
   double lg;    // its logarithm
   double nln2;  // number of this lane's units times log 2
 };
@@ -46,7 +47,7 @@ template <class T, int JL>
 __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, const T* W,
                                      const T* bias, int N, int M) {
   const int lane = lane_id();
-  T prod = (T)1;
+  T prod = (T)1, left = (T)0;
   int live = 0;
 #pragma unroll
   for (int jj = 0; jj < JL; ++jj) {
@@ -62,7 +63,9 @@ __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, co
       if constexpr (sizeof(T) == 4) {
         h.lc[jj] = log_cosh<T>(acc);
       } else {
-        prod = fma(prod, exp_m2abs(acc), prod);
+        const T e = exp_m2abs(acc), next = fma(prod, e, prod);
+        left = fma(left, e, left) + fma(prod, e, prod - next);
+        prod = next;
         ++live;
       }
     } else {
@@ -72,6 +75,7 @@ __device__ inline void compute_theta(HiddenState<T, JL>& h, const int8_t* xs, co
   }
   if constexpr (sizeof(T) == 8) {
     h.pr = prod;
+    h.pe = left;
     h.lg = log(prod);
     h.nln2 = 0.69314718055994530942 * (double)live;
   }

@@ -164,7 +164,8 @@ __device__ __forceinline__ void group64_body(const nka_rbm& m, const SweepArgs& 
         lhs = rhs = 1.0;
         x = pw * (A + log_call(P / P0));
       }
-      const bool acc = u * lhs * (double)n_new < exp_f64(x) * rhs * (double)n_diff;
+      // (both sides carry a few roundings of the products; the exponential's is one more)
+      const bool acc = u * lhs * (double)n_new < exp_f64<false>(x) * rhs * (double)n_diff;
       if (valid && acc) {
 #pragma unroll
         for (int jj = 0; jj < JG; ++jj) th[jj] = t[jj];
@@ -351,7 +352,7 @@ __device__ __forceinline__ void pair64_body(const nka_rbm& m, const SweepArgs& s
         lhs = rhs = 1.0;
         x = pw * (A + log_call(P / Pe));
       }
-      const uint64_t acc = __ballot(uniform01<double>(rnd) * lhs < exp_f64(x) * rhs);
+      const uint64_t acc = __ballot(uniform01<double>(rnd) * lhs < exp_f64<false>(x) * rhs);
       const bool acc0 = acc & 1ull;
       const bool acc1 = two && (acc >> (acc0 ? 32 : 16) & 1ull);
       if (acc0) {

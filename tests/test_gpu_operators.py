@@ -267,3 +267,60 @@ def test_activations_of_wide_models(gpu, N, M, ns, dtype):
     tol = 1e-13 if dtype == np.float64 else 1e-5  # sums of up to 1056 terms of about 0.02, |theta| < 3
     np.testing.assert_allclose(t.cpu().numpy(), ref, rtol=0, atol=tol)
     np.testing.assert_array_equal(tT.cpu().numpy(), t.cpu().numpy().T)
+
+
+def test_exponential_of_amplitude_ratios(gpu):
+    # all weights zero but the visible bias of site 0: a flip of that site has the
+    # ratio exp(-2 x_0 a_0), and nothing else is rounded on the way
+    print("case exponential of ratios", flush=True)
+    from netket_amd import _engine as eng
+    N = 4
+    model = nk.models.RBM(alpha=1, param_dtype=np.float64)
+    lay = model.layout(N)
+    op = nk.operator.LocalOperator(nk.hilbert.Spin(0.5, N=N), [np.array([[0.0, 1.0], [1.0, 0.0]])], [[0]])
+    x = torch.tensor([[1, 1, 1, 1], [-1, 1, 1, 1]], dtype=torch.int8, device="cuda")
+    args = np.concatenate([np.random.default_rng(5).uniform(-20, 20, 300), [0.0, 0.5, 300.0, -700.0]])
+    got = []
+    for v in args:
+        flat = torch.zeros(lay["n_params"], dtype=torch.float64)
+        flat[lay["visible_bias"][0]] = v / 2
+        got.append(eng.local_energies(model, flat.cuda(), op, x))
+    got = torch.stack(got).cpu().numpy()
+    ref = np.exp(np.stack([-args, args], 1).astype(np.longdouble))
+    ulp = np.abs(got - ref) / np.spacing(ref.astype(np.float64))
+    print(f"largest error {float(ulp.max()):.3f} ulp, rms {float(np.sqrt((ulp ** 2).mean())):.3f}", flush=True)
+    # 0.78 for arguments up to 700, doubled where the power is taken in halves (|x| > 600)
+    assert ulp[np.abs(args) <= 600].max() <= 0.85 and ulp.max() <= 3
+
+
+@pytest.mark.parametrize("N,M", [(10, 20), (14, 28), (16, 64), (33, 70), (64, 128)])
+def test_fp64_ratios_no_further_off_than_log_cosh_sums(gpu, N, M):
+    # the sum of all single flips' ratios, against extended precision: no further off than
+    # the same sum from FP64 log_cosh differences
+    print(f"case fp64 ratios N={N} M={M}", flush=True)
+    from netket_amd import _engine as eng
+    model, flat, p = _rbm_state(N, (M + 0.5) / N, np.float64, 60 + N, scale=0.6 / np.sqrt(M))
+    assert p.W.shape == (N, M)
+    x = _states(N, 1500, 61)
+    op = nk.operator.Ising(nk.hilbert.Spin(0.5, N=N), nk.graph.Chain(N), h=1.0, J=0.0)
+    e = eng.local_energies(model, flat, op, torch.as_tensor(x, device="cuda")).cpu().numpy()
+
+    def flips(f, log2):
+        W, b, a = p.W.astype(f), p.b.astype(f), p.a.astype(f)
+        xf = x.astype(f)
+        th = np.repeat(b[None], len(x), 0)
+        for i in range(N):
+            th = th + xf[:, i:i + 1] * W[i]
+        lc = lambda t: np.abs(t) + np.log1p(np.exp(-2 * np.abs(t))) - log2
+        l0 = lc(th)
+        out = np.zeros(len(x), f)
+        for i in range(N):
+            t = th - 2 * xf[:, i:i + 1] * W[i]
+            out -= np.exp((lc(t) - l0).sum(1) - 2 * xf[:, i] * a[i])
+        return out
+
+    exact = flips(np.longdouble, np.log(np.longdouble(2)))
+    off = lambda v: float(np.linalg.norm((v - exact).astype(np.float64)) / np.linalg.norm(exact.astype(np.float64)))
+    mine, plain = off(e), off(flips(np.float64, np.log(2.0)))
+    print(f"error {mine:.2e}, from log_cosh sums {plain:.2e}", flush=True)
+    assert mine <= plain
