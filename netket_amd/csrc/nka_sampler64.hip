@@ -499,11 +499,12 @@ static size_t group64_lds(const nka_rbm& m, const SweepArgs& sa, int waves, int 
 bool launch_group64(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, double* lp, int8_t* smp, double* lps,
                     int64_t* nacc, const nka_sweep_job* jobs, int n_jobs, hipStream_t s) {
   if (sa.weights) return false;
-  // two proposals per step while every chain has a SIMD of its own and its units fit
-  // four a lane (16 units: 1.30x at 16 chains, 1.16x at 1024, 0.97x at 2048; 64
-  // units: 1.07x, 1.01x, 0.75x)
-  const int64_t chains = (int64_t)sa.C * (jobs ? n_jobs : 1);
-  if (sa.rule == NKA_RULE_LOCAL && m.n_hidden <= 64 && m.n_visible <= 32 * NKA_WAVE && chains <= 4 * device_cus()) {
+  // two proposals per step while every chain of a job has a SIMD of its own and its
+  // units fit four a lane (16 units: 1.30x at 16 chains, 1.16x at 1024, 0.97x at 2048;
+  // 64 units: 1.07x, 1.01x, 0.75x).  The kernels add a chain's units in different
+  // orders, so the choice looks at one job alone: a batched job's chains are those that
+  // it has by itself.
+  if (sa.rule == NKA_RULE_LOCAL && m.n_hidden <= 64 && m.n_visible <= 32 * NKA_WAVE && sa.C <= 4 * device_cus()) {
     const size_t lds = pad16((size_t)m.n_visible * m.n_hidden * sizeof(double)) +
                        pad16((size_t)m.n_visible * sizeof(double));
     if (lds <= 156 * 1024) {

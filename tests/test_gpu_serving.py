@@ -153,3 +153,54 @@ def test_report_latencies_and_accuracy(gpu):
     for a in rep.accuracy:
         assert a["exact_e0"] == pytest.approx(serving.tfim_chain_exact_energy(a["L"], a["h"]))
         assert a["energy"] >= a["exact_e0"] - 0.05 * abs(a["exact_e0"])  # variational, up to noise
+
+
+@pytest.mark.parametrize("rule,M,chains,n_jobs", [
+    ("local", 16, 400, 3), ("local", 40, 400, 3), ("local", 64, 1024, 2), ("local", 128, 400, 3), ("local", 300, 9, 2),
+    ("exchange", 16, 64, 3), ("exchange", 40, 1100, 2), ("exchange", 128, 64, 3)])
+def test_batched_fp64_chains_equal_single_launches(gpu, rule, M, chains, n_jobs):
+    # FP64 jobs that share a launch, fewer chains than SIMDs each and more together:
+    # chains, counts and log-probabilities of every job bit for bit as by itself
+    import netket_amd as nk
+    from netket_amd import _ops
+
+    print(f"case batched fp64 {rule} M={M} chains={chains} jobs={n_jobs}", flush=True)
+    N = 12
+    hi = nk.hilbert.Spin(0.5, N=N, total_sz=0 if rule == "exchange" else None)
+    g = nk.graph.Chain(N)
+    model = nk.models.RBM(alpha=(M + 0.5) / N, param_dtype=np.float64)
+    rng = np.random.default_rng(M)
+    flats = [torch.as_tensor(rng.normal(scale=0.6 / np.sqrt(M), size=model.layout(N)["n_params"]), device="cuda")
+             for _ in range(n_jobs)]
+    if rule == "local":
+        sa = nk.sampler.MetropolisLocal(hi, n_chains=chains)
+        kind, cl, ncl = nat.RULE_LOCAL, None, 0
+    else:
+        sa = nk.sampler.MetropolisExchange(hi, graph=g, n_chains=chains)
+        kind, cl, ncl = nat.RULE_EXCHANGE, _ops.ptr(sa.rule.device_clusters()), len(sa.rule.clusters)
+    single, states = [], []
+    for k, f in enumerate(flats):
+        (s, lps), st = sa.sample_fused(model, f, sa.init_state(model, f, seed=10 + k), 2, 3,
+                                       return_log_probabilities=True)
+        single.append((s.reshape(chains, 3, N), lps.reshape(chains, 3), st.sigma, st.log_prob, st.n_accepted_proc))
+    jobs, batched = (nat.NkaSweepJob * n_jobs)(), []
+    for k, f in enumerate(flats):
+        st = sa.init_state(model, f, seed=10 + k)
+        states.append(st)
+        out = (torch.empty((chains, 3, N), dtype=torch.int8, device="cuda"),
+               torch.empty((chains, 3), dtype=torch.float64, device="cuda"), st.sigma,
+               torch.empty(chains, dtype=torch.float64, device="cuda"), st.n_accepted_proc)
+        batched.append(out)
+        jobs[k].model = model.native(f, N)
+        jobs[k].sigma, jobs[k].log_prob = st.sigma.data_ptr(), out[3].data_ptr()
+        jobs[k].samples, jobs[k].log_prob_samples = out[0].data_ptr(), out[1].data_ptr()
+        jobs[k].n_accepted = st.n_accepted_proc.data_ptr()
+        jobs[k].seed, jobs[k].counter, jobs[k].counter_dev = st.seed, st.counter, st.counter_dev.data_ptr()
+    jd = torch.frombuffer(bytearray(bytes(jobs)), dtype=torch.uint8).cuda()
+    shape = model.native(flats[0], N)
+    nat.call("nka_rbm_metropolis_batched", _ops.ptr(jd), n_jobs, C.byref(shape), kind, cl, ncl, chains, sa.sweep_size,
+             2, 3, 2.0, _ops.stream())
+    torch.cuda.synchronize()
+    for one, many in zip(single, batched):
+        for a, b in zip(one, many):
+            np.testing.assert_array_equal(a.cpu().numpy(), b.cpu().numpy())
