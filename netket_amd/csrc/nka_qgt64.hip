@@ -122,6 +122,7 @@ __device__ inline void bytes4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, 
 // integer I = rint(q 2^(54 - e)), e = e_j + e_l, in seven planes of balanced
 // base-256 digits: I + 0x80..80 has the bytes d + 128, and a byte's digit is
 // its value with the top bit flipped.  |I| <= 2^54 fits the seven digits.
+// (A product below 2^-55 of 2^e is lost, 2^-53 of the product of its units' largest.)
 // rscale[r] = 2^(e - 54).  Plane d, row r, sample s is Q[(d rows + r) ldk + s];
 // zero past ns.  One workgroup per row, 4 samples per thread and step: the
 // loads of a wavefront then cover whole lines, and its stores 256 bytes per
@@ -169,9 +170,10 @@ __global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* 
       uint32_t lo[4], hi[4];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const double v = s0 + q < ns ? f[q] * up : 0.0;
+        // v is a whole number, so its low word is in [0, 2^32)
+        const double v = s0 + q < ns ? rint(f[q] * up) : 0.0;
         const double vh = floor(v * 0x1p-32);
-        const uint32_t vl = (uint32_t)(fma(vh, -0x1p32, v) + 0.5);
+        const uint32_t vl = (uint32_t)fma(vh, -0x1p32, v);
         const uint64_t I = ((uint64_t)(uint32_t)(int32_t)vh << 32) + vl + 0x0080808080808080ull;
         lo[q] = (uint32_t)I ^ 0x80808080u;
         hi[q] = (uint32_t)(I >> 32) ^ 0x00808080u;

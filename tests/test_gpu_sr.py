@@ -737,3 +737,31 @@ def test_gemm_fp64_tiles(gpu, m, n, k):
     c = c0.clone()
     nat.call("nka_gemm_nt_f64", _ops.ptr(a), k, _ops.ptr(b), k, _ops.ptr(c), n, m, n, k, -1.0, 1.0, _ops.stream())
     assert (c - (c0 - a @ b.T)).abs().max().item() < 1e-13 * k
+
+
+def test_rbm_qgt_structured_fp64_small_products_beside_outliers(gpu):
+    # two units with a pair of large activations each, which set their rows' scale, and
+    # products of +-0.3 units of the digits elsewhere: every product rounds to zero, and
+    # the sum is zero as it is in exact arithmetic
+    print("case rbm_qgt fp64 outliers", flush=True)
+    N, ns = 8, 4096
+    model = nk.models.RBM(alpha=1, param_dtype=np.float64)
+    lay = model.layout(N)
+    rng = np.random.default_rng(8)
+    fl = torch.as_tensor(rng.normal(scale=0.3, size=lay["n_params"]), device="cuda")
+    x = rng.choice(np.array([-1, 1], dtype=np.int8), size=(ns, N))
+    t = rng.uniform(-0.5, 0.5, size=(N, ns))
+    small = np.sqrt(0.3 * 2.0 ** -54)
+    t[0] = small * np.tile([1, -1], ns // 2)
+    t[1] = small * np.tile([1, -1, -1, 1], ns // 4)
+    t[0, 0], t[0, 3] = 0.9, -0.9
+    t[1, 5], t[1, 6] = 0.9, -0.9
+    S = eng.qgt_structured(model, fl, torch.as_tensor(x, device="cuda"), torch.as_tensor(t, device="cuda"), 1.0 / ns,
+                           0.0).cpu().numpy()
+    tl = t.astype(np.longdouble)
+    tl -= tl.mean(axis=1, keepdims=True)
+    b = lay["bias"][0]
+    exact = float((tl[0] * tl[1]).sum() / ns)
+    print(f"S {S[b + 1, b]:.3e} exact {exact:.3e}", flush=True)
+    # the few products with an outlier round to half a unit each
+    assert abs(S[b + 1, b] - exact) <= 4 * 2.0 ** -54 / ns
