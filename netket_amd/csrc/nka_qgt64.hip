@@ -373,7 +373,8 @@ __global__ void __launch_bounds__(512) qgt64_unpack_kernel(nka_rbm m, const doub
     auto cov = [&](int w, int x) {
       return row[qgt_hidden_row(w, x, M)] - rowh[w + 1] * (rowl[x + 1] * rns);
     };
-    const double k00 = cov(-1, -1);
+    // (sums of signs: whole numbers below 2^22, so one rounding)
+    const double k00 = (row[0] * ns - rowh[0] * rowl[0]) * rns;
     auto entry = [&](int w, int64_t p, double cw, double kw, int x) {
       const int64_t q = qgt_param(ul, x, m);
       if (q < 0 || (uh == ul && p < q)) return;  // the symmetric diagonal pair: each entry once

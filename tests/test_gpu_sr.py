@@ -765,3 +765,26 @@ def test_rbm_qgt_structured_fp64_small_products_beside_outliers(gpu):
     print(f"S {S[b + 1, b]:.3e} exact {exact:.3e}", flush=True)
     # the few products with an outlier round to half a unit each
     assert abs(S[b + 1, b] - exact) <= 4 * 2.0 ** -54 / ns
+
+
+def test_rbm_qgt_structured_fp64_spins_nearly_aligned(gpu):
+    # spins that flip in a few samples only: the visible biases' covariances are small
+    # differences of large whole numbers, and come out to the last bit or two
+    print("case rbm_qgt fp64 aligned spins", flush=True)
+    N, ns = 8, 4099
+    model = nk.models.RBM(alpha=1, param_dtype=np.float64)
+    lay = model.layout(N)
+    rng = np.random.default_rng(9)
+    fl = torch.as_tensor(rng.normal(scale=0.3, size=lay["n_params"]), device="cuda")
+    x = np.ones((ns, N), dtype=np.int8)
+    for i in range(N):
+        x[rng.choice(ns, 1 + 3 * i, replace=False), i] = -1
+    sig = torch.as_tensor(x, device="cuda")
+    _, tT = eng.prepare(model, fl, sig, row_major=False, transposed=True)
+    S = eng.qgt_structured(model, fl, sig, tT, 1.0 / ns, 0.0).cpu().numpy()
+    v = lay["visible_bias"][0]
+    xi = x.astype(np.int64)
+    m = xi.sum(axis=0)
+    exact = (ns * (xi.T @ xi) - np.outer(m, m)) / (float(ns) * ns)
+    low = np.tril_indices(N)
+    np.testing.assert_allclose(S[v:v + N, v:v + N][low], exact[low], rtol=1e-15, atol=0)
