@@ -367,9 +367,11 @@ int nka_rbm_qgt(const nka_rbm* m, const int8_t* sigma, const void* tT, int64_t n
 
 /* The same S for an FP64 model (arguments as nka_rbm_qgt, tT FP64): P is +-1 in
  * int8, Q 55-bit fixed point with a power-of-two scale per row in seven int8
- * digit planes, and P Q^T exact int32 products on the matrix cores, so C is
- * rounded once per entry.  At most 2^22 samples (the workspace query returns
- * 0 for sizes it does not take). */
+ * digit planes, and P Q^T exact int32 products on the matrix cores.  Small
+ * models take the samples in up to 16 slices side by side, and samples whose
+ * planes would exceed the FP64 Jacobian's memory (and 256 MB) go through in
+ * chunks: C is a sum of slices and chunks, each rounded once per entry.  At most
+ * 2^22 samples (the workspace query returns 0 for sizes it does not take). */
 int64_t nka_rbm_qgt_f64_workspace(const nka_rbm* m, int64_t ns);
 int nka_rbm_qgt_f64(const nka_rbm* m, const int8_t* sigma, const double* tT, int64_t ns, double scale, double shift,
                     double* out, int64_t ldo, void* workspace, void* stream);

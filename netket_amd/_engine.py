@@ -165,17 +165,22 @@ def gram(bufs: JacobianBuffers, shift: float, offset: float = 0.0,
     return out
 
 
+# scratch that the FP64 structured S may take beyond a Jacobian's memory, and that is
+# kept between calls
+_QGT_SPARE = 256 << 20
+
+
 def qgt_structured_available(model, flat, n_sites: int, n_samples: int) -> bool:
     """Whether the dense S of ``model`` is formed from its layer structure
     (RBM: spin-pair x activation-pair products; FP32 models in bf16 planes,
     FP64 models in exact int8 digit planes).
 
-    The FP64 form holds 7 bytes per activation pair and sample, against the
-    8 bytes per parameter and sample of the Jacobian (their ratio grows like
-    alpha / 2), and a product C of about a quarter of S.  Models that would
-    need more than three Jacobians and one more S (alpha above about 6) keep
-    the Jacobian and its FP64 product, as do batches past the entry point's
-    sample limit."""
+    The FP64 form goes through the samples in chunks whose digit planes, with a
+    product C of a quarter of S, fit the memory that the Jacobian would take.
+    Where C alone is larger (more parameters than about four times the samples,
+    past 256 MB), and past the entry point's sample limit, the Jacobian and its
+    FP64 product are kept: but for 256 MB, no program needs more memory than
+    with the Jacobian."""
     if model.kind != "rbm":
         return False
     if flat.dtype == torch.float32:
@@ -183,7 +188,7 @@ def qgt_structured_available(model, flat, n_sites: int, n_samples: int) -> bool:
     m = model.native(flat, n_sites)
     need = nat.lib().nka_rbm_qgt_f64_workspace(C.byref(m), n_samples)
     np_ = model.layout(n_sites)["n_params"]
-    return 0 < need <= 8 * np_ * (3 * _ld(n_samples) + np_) + (64 << 20)
+    return 0 < need <= 8 * np_ * _ld(n_samples) + _QGT_SPARE
 
 
 def qgt_structured(model, flat, sigma2d: torch.Tensor, tT: torch.Tensor, scale: float, shift: float,
@@ -198,7 +203,12 @@ def qgt_structured(model, flat, sigma2d: torch.Tensor, tT: torch.Tensor, scale: 
         out = torch.empty((np_, np_), dtype=torch.float64, device=sigma2d.device)
     m = model.native(flat, N)
     name = "nka_rbm_qgt" if flat.dtype == torch.float32 else "nka_rbm_qgt_f64"
-    ws = _ops.WORKSPACE.get("rbm_qgt", getattr(nat.lib(), name + "_workspace")(C.byref(m), n))
+    need = getattr(nat.lib(), name + "_workspace")(C.byref(m), n)
+    if flat.dtype == torch.float32 or need <= _QGT_SPARE:
+        ws = _ops.WORKSPACE.get("rbm_qgt", need)
+    else:
+        # given back after the call, as the Jacobian that it stands for would be
+        ws = torch.empty(need, dtype=torch.uint8, device=sigma2d.device)
     with _ops.TIMER.region("qgt_structured"):
         nat.call(name, C.byref(m), _ops.ptr(sigma2d), _ops.ptr(tT), n, float(scale), float(shift),
                  _ops.ptr(out), out.stride(0), _ops.ptr(ws), _ops.stream())

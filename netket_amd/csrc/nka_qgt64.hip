@@ -8,8 +8,8 @@
 // 55-bit fixed point with one power-of-two scale per row, in seven planes of
 // balanced base-256 digits (int8), so that P Q_d^T is an exact int32 product
 // on v_mfma_i32_32x32x32_i8 for each digit plane d and C comes out with a
-// single rounding: the sums over the samples carry no rounding error at all,
-// where an FP64 product of the Jacobian rounds at every accumulation.
+// single rounding per entry and slice or chunk of the samples (usually one of
+// each), where an FP64 product of the Jacobian rounds at every accumulation.
 //
 // Seven int8 products of Na Nb Ns (Na Nb about Np^2 / 4) replace Ns Np^2
 // FP64 operations; the int8 rate is 64 times the FP64 one.  64 sites, 128
@@ -126,13 +126,14 @@ __device__ inline void bytes4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, 
 // rscale[r] = 2^(e - 54).  Plane d, row r, sample s is Q[(d rows + r) ldk + s];
 // zero past ns.  One workgroup per row, 4 samples per thread and step: the
 // loads of a wavefront then cover whole lines, and its stores 256 bytes per
-// plane.  Bound by the 7 bytes written per entry.
-__global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* __restrict__ tT, int64_t ns, int M,
+// plane.  Bound by the 7 bytes written per entry.  (t of unit j: tT + j ldt.)
+__global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* __restrict__ tT, int64_t ldt,
+                                                                  int64_t ns, int M,
                                                                   const double* __restrict__ cmean,
                                                                   const double* __restrict__ ex, int64_t ldk,
                                                                   int64_t rows, uint8_t* __restrict__ Q,
                                                                   double* __restrict__ rscale) {
-  const bool vec = (ns % 2) == 0 && (((uintptr_t)tT) % 16) == 0;
+  const bool vec = (ldt % 2) == 0 && (((uintptr_t)tT) % 16) == 0;
   for (int64_t r = blockIdx.x; r < rows; r += gridDim.x) {
     int64_t j, l;
     qgt_hidden_pair(r, M, j, l);
@@ -157,12 +158,12 @@ __global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* 
 #pragma unroll
         for (int q = 0; q < 4; ++q) f[q] = 1.0;
       } else {
-        load4(tT + j * ns, f);
+        load4(tT + j * ldt, f);
 #pragma unroll
         for (int q = 0; q < 4; ++q) f[q] -= cj;
         if (l >= 0) {
           double h[4];
-          load4(tT + l * ns, h);
+          load4(tT + l * ldt, h);
 #pragma unroll
           for (int q = 0; q < 4; ++q) f[q] *= h[q] - cl;
         }
@@ -202,12 +203,14 @@ __global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* 
 // 2.40 ms at 2081 x 8385 x 16384 (1.67e15 int8 operations/s).  With the loads
 // and LDS reads issued ahead of a step's products instead of between them it
 // took 3.07 ms (34% busy); two buffers instead of four made 3.15 ms.
-// blockIdx.y: slice of K (whole K steps); slice y writes C + y * slab.
+// blockIdx.y: slice of K (whole K steps); slice y writes C + y * slab, or with `add`
+// (a further chunk of the samples) adds to it.
 __global__ void __launch_bounds__(256, 1) qgt64_gemm_kernel(const int8_t* __restrict__ P, int64_t ma,
                                                          const uint8_t* __restrict__ Q, int64_t nb,
                                                          const double* __restrict__ rscale, int64_t ldk,
                                                          double* __restrict__ C, int64_t ldc, int64_t slab,
-                                                         int64_t tiles_m, int64_t n_tiles, int64_t steps_per_slice) {
+                                                         int64_t tiles_m, int64_t n_tiles, int64_t steps_per_slice,
+                                                         int add) {
   constexpr int A_BYTES = Q8_TA * Q8_K, B_BYTES = Q8_D * Q8_TB * Q8_K;
   constexpr int LOADS = (A_BYTES + B_BYTES) / 1024 / 4;   // 16-row wavefront loads per wavefront and K step
   static_assert((A_BYTES + B_BYTES) % 4096 == 0, "whole loads per wavefront");
@@ -317,7 +320,8 @@ __global__ void __launch_bounds__(256, 1) qgt64_gemm_kernel(const int8_t* __rest
           const int64_t lo = (int64_t)acc[0][x][e] + ((int64_t)acc[1][x][e] << 8) + ((int64_t)acc[2][x][e] << 16) +
                              ((int64_t)acc[3][x][e] << 24);
           const int64_t hi = (int64_t)acc[4][x][e] + ((int64_t)acc[5][x][e] << 8) + ((int64_t)acc[6][x][e] << 16);
-          out[gi * ldc + gj] = fma((double)hi, 0x1p32, (double)lo) * rs;
+          const double v = fma((double)hi, 0x1p32, (double)lo) * rs;
+          out[gi * ldc + gj] = add ? out[gi * ldc + gj] + v : v;
         }
       }
   }
@@ -411,23 +415,43 @@ __global__ void __launch_bounds__(512) qgt64_unpack_kernel(nka_rbm m, const doub
   }
 }
 
+constexpr int64_t kQ8Spare = 256 << 20;
+static int64_t q8_ldc(const nka_rbm& m) { return (qgt_rows_q(m) + 31) / 32 * 32; }
+static int64_t q8_np(const nka_rbm& m) {
+  return (m.bias_off >= 0 ? m.n_hidden : 0) + (int64_t)m.n_visible * m.n_hidden +
+         (m.visible_off >= 0 ? m.n_visible : 0);
+}
+// The samples go through in chunks (all of them at once where that fits) whose planes,
+// with C, take no more than the FP64 Jacobian that they stand for and 256 MB: 7 bytes
+// per activation pair and sample are 0.44 alpha Jacobians, and C is a quarter of S.  A
+// chunk holds 512 samples at least.
 // Slices of K: enough workgroups for the chip when the tiles alone are few,
 // with at least 8 K steps each.
 struct Q8Plan {
+  int64_t chunk;        // samples of a chunk, padded
   int64_t tiles_m, tiles, slices, steps_per_slice;
+  int64_t fixed;        // bytes of C, the scales and the means
 };
 static Q8Plan q8_plan(const nka_rbm& m, int64_t ns) {
   Q8Plan p;
-  p.tiles_m = (qgt_rows_p(m) + Q8_TA - 1) / Q8_TA;
-  p.tiles = p.tiles_m * ((qgt_rows_q(m) + Q8_TB - 1) / Q8_TB);
-  const int64_t steps = qgt_ldk(ns) / Q8_K;
-  int64_t sl = std::min<int64_t>(std::min<int64_t>(256 / p.tiles, steps / 8), 16);
-  if (sl < 1) sl = 1;
+  const int64_t rp = qgt_rows_p(m), rq = qgt_rows_q(m);
+  const int64_t ldk = qgt_ldk(ns);
+  p.tiles_m = (rp + Q8_TA - 1) / Q8_TA;
+  p.tiles = p.tiles_m * ((rq + Q8_TB - 1) / Q8_TB);
+  const int64_t wanted = std::min<int64_t>(256 / p.tiles, 16);
+  p.fixed = qgt_round(std::max<int64_t>(wanted, 1) * rp * q8_ldc(m) * 8) + qgt_round(rq * 8) +
+            2 * qgt_round((int64_t)m.n_hidden * 8);
+  const int64_t per_sample = m.n_visible + rp + Q8_D * rq, room = 8 * q8_np(m) * ldk + kQ8Spare - p.fixed - 1024;
+  const int64_t fits = std::max<int64_t>(room > 0 ? room / per_sample : 0, 512);
+  const int64_t chunks = (ldk + fits - 1) / fits;
+  p.chunk = std::min<int64_t>(ldk, ((ldk + chunks - 1) / chunks + Q8_K - 1) / Q8_K * Q8_K);
+  if (p.chunk > fits) p.chunk = fits / Q8_K * Q8_K;
+  const int64_t steps = p.chunk / Q8_K;
+  const int64_t sl = std::max<int64_t>(std::min<int64_t>(wanted, steps / 8), 1);
   p.steps_per_slice = (steps + sl - 1) / sl;
   p.slices = (steps + p.steps_per_slice - 1) / p.steps_per_slice;
   return p;
 }
-static int64_t q8_ldc(const nka_rbm& m) { return (qgt_rows_q(m) + 31) / 32 * 32; }
 // 128 ns per digit sum has to stay below 2^31
 constexpr int64_t kQ8MaxSamples = 1 << 22;
 
@@ -439,10 +463,9 @@ extern "C" {
 
 int64_t nka_rbm_qgt_f64_workspace(const nka_rbm* m, int64_t ns) {
   if (!m || ns <= 0 || ns > kQ8MaxSamples || m->n_visible < 1 || m->n_hidden < 1) return 0;
-  const int64_t ldk = qgt_ldk(ns), rp = qgt_rows_p(*m), rq = qgt_rows_q(*m);
-  return qgt_round((int64_t)m->n_visible * ldk) + qgt_round(rp * ldk) + qgt_round(Q8_D * rq * ldk) +
-         qgt_round(q8_plan(*m, ns).slices * rp * q8_ldc(*m) * 8) + qgt_round(rq * 8) +
-         2 * qgt_round((int64_t)m->n_hidden * 8);
+  const Q8Plan p = q8_plan(*m, ns);
+  return qgt_round((int64_t)m->n_visible * p.chunk) + qgt_round(qgt_rows_p(*m) * p.chunk) +
+         qgt_round(Q8_D * qgt_rows_q(*m) * p.chunk) + p.fixed;
 }
 
 int nka_rbm_qgt_f64(const nka_rbm* m, const int8_t* sigma, const double* tT, int64_t ns, double scale, double shift,
@@ -452,20 +475,19 @@ int nka_rbm_qgt_f64(const nka_rbm* m, const int8_t* sigma, const double* tT, int
   NKA_CHECK_ARG(ns <= kQ8MaxSamples, "nka_rbm_qgt_f64: too many samples");
   NKA_CHECK_ARG(m->n_visible >= 1 && m->n_hidden >= 1, "nka_rbm_qgt_f64: empty model");
   const int N = m->n_visible, M = m->n_hidden;
-  const int64_t np = (m->bias_off >= 0 ? M : 0) + (int64_t)N * M + (m->visible_off >= 0 ? N : 0);
-  NKA_CHECK_ARG(ldo >= np, "nka_rbm_qgt_f64: ldo < n_params");
+  NKA_CHECK_ARG(ldo >= q8_np(*m), "nka_rbm_qgt_f64: ldo < n_params");
   const Q8Plan pl = q8_plan(*m, ns);
   NKA_CHECK_ARG((int64_t)(N + 1) * (N + 2) / 2 < (1LL << 31) && pl.tiles < (1LL << 31),
                 "nka_rbm_qgt_f64: too many units");
   hipStream_t s = (hipStream_t)stream;
-  const int64_t ldk = qgt_ldk(ns), rp = qgt_rows_p(*m), rq = qgt_rows_q(*m), ldc = q8_ldc(*m);
+  const int64_t rp = qgt_rows_p(*m), rq = qgt_rows_q(*m), ldc = q8_ldc(*m);
   unsigned char* w = (unsigned char*)workspace;
   int8_t* sT = (int8_t*)w;
-  w += qgt_round((int64_t)N * ldk);
+  w += qgt_round((int64_t)N * pl.chunk);
   int8_t* P = (int8_t*)w;
-  w += qgt_round(rp * ldk);
+  w += qgt_round(rp * pl.chunk);
   uint8_t* Q = (uint8_t*)w;
-  w += qgt_round(Q8_D * rq * ldk);
+  w += qgt_round(Q8_D * rq * pl.chunk);
   double* C = (double*)w;
   w += qgt_round(pl.slices * rp * ldc * 8);
   double* rscale = (double*)w;
@@ -473,18 +495,23 @@ int nka_rbm_qgt_f64(const nka_rbm* m, const int8_t* sigma, const double* tT, int
   double* cmean = (double*)w;
   w += qgt_round((int64_t)M * 8);
   double* ex = (double*)w;
-  launch_qgt_spins_t(sigma, ns, N, ldk, sT, s);
-  hipLaunchKernelGGL(qgt64_spin_pairs_kernel, dim3((unsigned)std::min<int64_t>(rp, 65536)), dim3(256), 0, s,
-                     (const int8_t*)sT, N, ldk, rp, P);
   hipLaunchKernelGGL(qgt64_means_kernel, dim3((unsigned)std::min<int64_t>(M, 65536)), dim3(256), 0, s, tT, ns, M,
                      cmean, ex);
-  hipLaunchKernelGGL(qgt64_hidden_digits_kernel, dim3((unsigned)std::min<int64_t>(rq, 65536)), dim3(256), 0, s, tT,
-                     ns, M, (const double*)cmean, (const double*)ex, ldk, rq, Q, rscale);
   const unsigned grid = (unsigned)((pl.tiles + 7) / 8 * 8);
   const int64_t slab = rp * ldc;
-  hipLaunchKernelGGL(qgt64_gemm_kernel, dim3(grid, (unsigned)pl.slices), dim3(256), 0, s, (const int8_t*)P, rp,
-                     (const uint8_t*)Q, rq, (const double*)rscale, ldk, C, ldc, slab, pl.tiles_m, pl.tiles,
-                     pl.steps_per_slice);
+  for (int64_t s0 = 0; s0 < ns; s0 += pl.chunk) {
+    // (each slice has the first steps_per_slice K steps of the chunk, so all of them
+    // are written: a last chunk keeps the length, zero past its samples)
+    const int64_t nc = std::min<int64_t>(pl.chunk, ns - s0), ldk = pl.chunk;
+    launch_qgt_spins_t(sigma + s0 * N, nc, N, ldk, sT, s);
+    hipLaunchKernelGGL(qgt64_spin_pairs_kernel, dim3((unsigned)std::min<int64_t>(rp, 65536)), dim3(256), 0, s,
+                       (const int8_t*)sT, N, ldk, rp, P);
+    hipLaunchKernelGGL(qgt64_hidden_digits_kernel, dim3((unsigned)std::min<int64_t>(rq, 65536)), dim3(256), 0, s,
+                       tT + s0, ns, nc, M, (const double*)cmean, (const double*)ex, ldk, rq, Q, rscale);
+    hipLaunchKernelGGL(qgt64_gemm_kernel, dim3(grid, (unsigned)pl.slices), dim3(256), 0, s, (const int8_t*)P, rp,
+                       (const uint8_t*)Q, rq, (const double*)rscale, ldk, C, ldc, slab, pl.tiles_m, pl.tiles,
+                       pl.steps_per_slice, s0 > 0 ? 1 : 0);
+  }
   if (pl.slices > 1)
     hipLaunchKernelGGL(qgt64_reduce_kernel, dim3((unsigned)std::min<int64_t>((slab + 255) / 256, 4096)), dim3(256), 0,
                        s, C, slab, slab, (int)pl.slices);

@@ -13,8 +13,8 @@ from the product of the spin-pair and activation-pair tables over the samples
 nka_rbm_qgt_f64, exact int8 digit products).  Other FP32 models store O_L
 parameter-major (X = O_L^T, Np x Ns) as a bf16 hi/lo split and form S with
 three BF16 MFMA products per tile (FP32 accumulate); other FP64 models, and
-RBMs with many more hidden than visible units, keep O_L and S in FP64 (FP64
-MFMA).  S is built on demand and not kept after a Cholesky
+RBMs with more than about four times as many parameters as samples, keep O_L
+and S in FP64 (FP64 MFMA).  S is built on demand and not kept after a Cholesky
 solve consumed it.
 """
 

@@ -767,6 +767,63 @@ def test_rbm_qgt_structured_fp64_small_products_beside_outliers(gpu):
     assert abs(S[b + 1, b] - exact) <= 4 * 2.0 ** -54 / ns
 
 
+@pytest.mark.parametrize("ns", [700, 2050])
+def test_rbm_qgt_structured_fp64_chunks_of_samples(gpu, ns):
+    # many hidden units per site: the digit planes of all samples would not fit the
+    # Jacobian's memory and go through in chunks, the last one shorter
+    import ctypes as C
+    assert nat.lib().nka_rbm_qgt_f64_workspace(C.byref(nk.models.RBM(alpha=50, param_dtype=np.float64).native(
+        torch.zeros(1, dtype=torch.float64), 8)), ns) < 7 * 80601 * ns
+    N, alpha = 8, 50
+    print(f"case rbm_qgt fp64 chunks ns={ns}", flush=True)
+    M = alpha * N
+    model = nk.models.RBM(alpha=alpha, param_dtype=np.float64)
+    rng = np.random.default_rng(ns)
+    n_par = model.layout(N)["n_params"]
+    flat = rng.normal(scale=0.2, size=n_par)
+    x = rng.choice(np.array([-1, 1], dtype=np.int8), size=(ns, N))
+    sig, fl = torch.as_tensor(x, device="cuda"), torch.as_tensor(flat, device="cuda")
+    _, tT = eng.prepare(model, fl, sig, row_major=False, transposed=True)
+    S = eng.qgt_structured(model, fl, sig, tT, 1.0 / ns, 1e-2).cpu().numpy()
+    Ou = orbm.jacobian(orbm.RBMParams(flat, N, M, hidden_bias=True, visible_bias=True), x)
+    Ol = Ou.astype(np.longdouble)
+    Ol -= Ol.sum(axis=0) / ns
+    rows = np.unique(np.concatenate([[0, M - 1, n_par - 1], rng.integers(0, n_par, 30)]))
+    ref = np.dot(Ol[:, rows].T, Ol) / ns
+    ref[np.arange(len(rows)), rows] += 1e-2
+    du = np.sqrt(np.sum(Ou * Ou, axis=0) / ns)
+    bound = 32 * 2.0 ** -53 * np.outer(du[rows], du) + 1e-17   # as for all samples at once
+    keep = np.arange(n_par)[None, :] <= rows[:, None]
+    assert np.all((np.abs(S[rows] - ref.astype(np.float64)) <= bound)[keep])
+
+
+def test_fp64_s_from_the_jacobian_where_planes_are_not_taken(gpu, monkeypatch):
+    # the other side of the rule: S and an SR step of an FP64 RBM through the Jacobian and
+    # its FP64 product against the digit planes
+    print("case fp64 S from the Jacobian", flush=True)
+    N = 12
+    hi = nk.hilbert.Spin(0.5, N=N)
+    H = nk.operator.Ising(hi, nk.graph.Chain(N), h=1.0)
+    out = {}
+    for planes in (True, False):
+        if not planes:
+            monkeypatch.setattr(eng, "qgt_structured_available", lambda *a: False)
+        sa = nk.sampler.MetropolisLocal(hi, n_chains=64)
+        vs = nk.vqs.MCState(sa, nk.models.RBM(alpha=2, param_dtype=np.float64), n_samples=1024, seed=3)
+        q = nk.optimizer.QGTJacobianDense(vs, diag_shift=0.01)
+        assert (q.X is None) == planes
+        S = q.to_dense().cpu().numpy()
+        drv = nk.VMC_SR(H, nk.optimizer.Sgd(0.02), diag_shift=0.01, variational_state=vs, use_ntk=False,
+                        linear_solver=nk.optimizer.solver.cholesky)
+        drv.run(1)
+        out[planes] = (S, vs.parameters_flat.cpu().numpy())
+    d = np.sqrt(np.diag(out[True][0]))
+    # both centre and sum FP64 values: a few n eps against the diagonal, times the condition
+    # of the shifted system (below 1e4) in the step
+    assert np.max(np.abs(out[True][0] - out[False][0]) / np.outer(d, d)) < 1e-12
+    np.testing.assert_allclose(out[False][1], out[True][1], rtol=0, atol=1e-9)
+
+
 def test_rbm_qgt_structured_fp64_spins_nearly_aligned(gpu):
     # spins that flip in a few samples only: the visible biases' covariances are small
     # differences of large whole numbers, and come out to the last bit or two

@@ -152,3 +152,38 @@ def test_structured_s_catches_a_dropped_centring_term():
     finally:
         _hidden_row = orig
     assert np.abs(bad[lo] - ref[lo]).max() > 1e-3
+
+
+@pytest.mark.parametrize("N,alpha", [(8, 1), (16, 4), (64, 2), (64, 8), (100, 1), (144, 4), (8, 50)])
+def test_fp64_structured_s_takes_no_more_memory_than_the_jacobian(N, alpha):
+    # the rule between digit planes and Jacobian, and the planes' scratch, on both sides
+    # of its limits (host code only)
+    import ctypes as C
+
+    import torch
+
+    import netket_amd as nk
+    from netket_amd import _engine as eng
+    from netket_amd import _native as nat
+
+    model = nk.models.RBM(alpha=alpha, param_dtype=np.float64)
+    flat = torch.zeros(1, dtype=torch.float64)
+    m = model.native(flat, N)
+    n_par = model.layout(N)["n_params"]
+    M = alpha * N
+    c_bytes = 8 * (1 + N + N * (N - 1) // 2) * (1 + M + M * (M + 1) // 2)
+    for ns in (1, 64, 1000, 4096, n_par // 4 + 1, 2 * n_par, 16384, 1 << 20, 1 << 22):
+        need = nat.lib().nka_rbm_qgt_f64_workspace(C.byref(m), ns)
+        jac = 8 * n_par * ((ns + 63) // 64 * 64)
+        ok = eng.qgt_structured_available(model, flat, N, ns)
+        assert need > 0
+        if ok:
+            assert need <= jac + (256 << 20)
+        # with room for C and 512 samples of planes the rule always takes them
+        if c_bytes * 1.05 + 512 * (7 * (M + 1) * (M + 2) // 2 + N * N) + (40 << 20) <= jac + (256 << 20):
+            assert ok
+        if c_bytes > jac + (256 << 20):
+            assert not ok
+    assert nat.lib().nka_rbm_qgt_f64_workspace(C.byref(m), (1 << 22) + 1) == 0
+    assert not eng.qgt_structured_available(model, flat, N, (1 << 22) + 1)
+    assert eng.qgt_structured_available(model, torch.zeros(1), N, (1 << 22) + 1)  # FP32: bf16 planes
