@@ -429,9 +429,16 @@ int nka_potrf_f64(double* a, int64_t n, int64_t lda, void* workspace, int32_t* i
 /* cho_solve: b <- A^{-1} b from the factor of nka_potrf_f64 (same workspace, as
  * nka_potrf_f64 or the last nka_potrs_f64 left it; its solve buffers are used
  * and left in their starting state, so solves from one workspace are ordered,
- * never concurrent); b is set to NaN when the factorisation failed (info != 0). */
+ * never concurrent); b is set to NaN when the factorisation failed (info != 0) or
+ * a wait between the blocks ran out. */
 int nka_potrs_f64(const double* a, int64_t n, int64_t lda, const void* workspace, double* b,
                   const int32_t* info, void* stream);
+
+/* nka_potrs_f64 whose waits between the blocks of a solve end after `polls` polls
+ * (about a second's worth there).  When one runs out, b is NaN as a whole and the
+ * workspace is fit for another solve. */
+int nka_potrs_f64_bounded(const double* a, int64_t n, int64_t lda, const void* workspace, double* b,
+                          const int32_t* info, int64_t polls, void* stream);
 
 /* Cholesky factorisation and solve in one call with no allocation and no
  * caller workspace: a = L L^T in place (lower triangle) and b <- A^{-1} b, as

@@ -161,6 +161,7 @@ SIGNATURES = {
     "nka_potrf_workspace": (i64, [i64]),
     "nka_potrf_f64": (i32, [vp, i64, i64, vp, vp, vp]),
     "nka_potrs_f64": (i32, [vp, i64, i64, vp, vp, vp, vp]),
+    "nka_potrs_f64_bounded": (i32, [vp, i64, i64, vp, vp, vp, i64, vp]),
     "nka_symmetrize_f64": (i32, [vp, i64, i64, vp]),
     "nka_check_finite": (i32, [vp, i64, vp, vp]),
     "nka_cholesky_solve_noalloc_max_n": (i64, []),

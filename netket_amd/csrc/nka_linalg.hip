@@ -967,32 +967,41 @@ __global__ void zero_u32_kernel(uint32_t* __restrict__ p, int64_t n) {
 // Triangular solves with the blocked factor, one launch each.  Workgroup k
 // owns the 64-row block k; it waits (bounded spin in global memory) for every
 // block it depends on, and only ever on blocks with a smaller workgroup id,
-// which the hardware dispatched earlier, so the wait always ends.  A wait
-// that exceeds the spin bound sets *err and the workgroup proceeds (the
-// result is then invalid and reported as such by the caller).
+// which the hardware dispatched earlier, so the wait always ends.
 //
 // The solved entries are their own flags: the output vector holds kUnsolved
 // before the launch, each entry is written once, as a 64-bit atomic store, and a
 // reader polls the entries it needs with 64-bit atomic loads until none holds
 // kUnsolved.  One memory round trip per dependency, and no ordering between
 // different entries is needed.
+//
+// A wait that exceeds its bound takes the entry for NaN, which then reaches every
+// entry that depends on it: after a forward solve that ran out, the whole solution.
+// In the backward solve the entries above it are not reached, so a wait that runs out
+// there sets *err (zeroed by the forward launch) before its rows are published, and
+// two parties turn the rest into NaN: the workgroup of the last block to be solved,
+// which depends on all others and so has waited for them or run out itself, fills the
+// vector if it sees *err; and a wavefront that publishes later than that sees *err
+// after its rows are out and takes them back.
 // ---------------------------------------------------------------------------
 constexpr int64_t kSpinLimit = 1LL << 26;
 
 // The entry *p (lanes with active), polled with relaxed agent-scope loads
-// (they read the L2 copy); inactive lanes get 0.  Wave-uniform loop.
-__device__ inline double poll_entry(const double* p, bool active, int32_t* err) {
+// (they read the L2 copy); inactive lanes get 0.  Wave-uniform loop; `late` is set when
+// `limit` polls were not enough.
+__device__ inline double poll_entry(const double* p, bool active, int64_t limit, bool& late) {
   uint64_t u = 0;
   int64_t spins = 0;
   while (true) {
     if (active) u = __hip_atomic_load((const uint64_t*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (!__any(active && u == kUnsolved)) break;
     __builtin_amdgcn_s_sleep(1);
-    if (++spins > kSpinLimit) {
-      if (lane_id() == 0) atomicOr(err, 1);
+    if (++spins > limit) {
+      late = true;
       break;
     }
   }
+  if (u == kUnsolved) u = kDefaultNaN;
   return active ? __longlong_as_double((long long)u) : 0.0;
 }
 
@@ -1046,8 +1055,10 @@ __device__ __forceinline__ double sum_rows(double v) {
 template <bool BWD>
 __global__ void __launch_bounds__(256, 2) trsv_lookback(const double* __restrict__ A, int64_t lda, int64_t n,
                                                         const double* __restrict__ inv, double* rhs, double* out,
-                                                        const int32_t* __restrict__ info, int32_t* err) {
+                                                        const int32_t* __restrict__ info, int32_t* err,
+                                                        int64_t limit) {
   __shared__ double ts[CH_NB];
+  bool late = false;
   const int nblk = gridDim.x;
   const int kb = BWD ? nblk - 1 - (int)blockIdx.x : (int)blockIdx.x;
   const int64_t k0 = (int64_t)kb * CH_NB;
@@ -1061,6 +1072,7 @@ __global__ void __launch_bounds__(256, 2) trsv_lookback(const double* __restrict
     if (BWD && tid < nb) out[k0 + tid] = __longlong_as_double((long long)kDefaultNaN);
     return;
   }
+  if (!BWD && kb == 0 && tid == 0) *err = 0;
   const double* invk = inv + (int64_t)kb * CH_NB * CH_NB;
   const int m = BWD ? nblk - 1 - kb : kb;      // blocks before this one
   // the t-th of them, in the order in which they are solved
@@ -1118,7 +1130,7 @@ __global__ void __launch_bounds__(256, 2) trsv_lookback(const double* __restrict
     for (int u = 0; u < 4; ++u) {
       if (t0 + u + 1 >= m) break;
       const int64_t j = first(t0 + u) + cl;
-      const double x = poll_entry(out + j, j < n, err);
+      const double x = poll_entry(out + j, j < n, limit, late);
       row_dot16(s0, s1, x, L[u]);
       if (t0 + u + 5 < m) load(t0 + u + 4, L[u]);
     }
@@ -1132,20 +1144,25 @@ __global__ void __launch_bounds__(256, 2) trsv_lookback(const double* __restrict
   if (g == 0 && r < nb) ((uint64_t*)rhs)[k0 + r] = kUnsolved;
   if (m > 0) {
     const int64_t j = first(m - 1) + 4 * i + g;   // W's order of columns
-    const double x = poll_entry(out + j, j < n, err);
+    const double x = poll_entry(out + j, j < n, limit, late);
     s0 = s1 = 0.0;
     row_dot16(s0, s1, x, W);
     v -= sum_rows(s0 + s1);
   }
+  if (BWD && late) {
+    if (lane == 0) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __threadfence();  // *err before the rows that it belongs to
+  }
   if (g == 0 && r < nb) publish_entry(out + k0 + r, v);
-  if (BWD && kb == 0) {
-    // the last block to be solved: a wait that ran out anywhere leaves NaN
-    __syncthreads();
-    const bool failed = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
-    __syncthreads();
-    if (failed) {
-      for (int64_t q = tid; q < n; q += 256) out[q] = __longlong_as_double((long long)kDefaultNaN);
-      if (tid == 0) *err = 0;
+  if constexpr (BWD) {
+    if (kb == 0) __syncthreads();
+    __threadfence();  // the rows (and, in the last block, the entries it waited for) before the look at *err
+    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+      if (kb == 0) {
+        for (int64_t q = tid; q < n; q += 256) publish_entry(out + q, __longlong_as_double((long long)kDefaultNaN));
+      } else if (g == 0 && r < nb) {
+        publish_entry(out + k0 + r, __longlong_as_double((long long)kDefaultNaN));
+      }
     }
   }
 }
@@ -1651,7 +1668,7 @@ static void potrf_run(double* a, int64_t n, int64_t lda, void* workspace, double
     }
   }
   hipLaunchKernelGGL(trtri_blocks_kernel, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, ws_vec(workspace, nblk),
-                     (int32_t*)(ws_flags(workspace, n, nblk) + nblk), info);
+                     info);
 }
 
 int nka_potrf_f64(double* a, int64_t n, int64_t lda, void* workspace, int32_t* info,
@@ -1665,26 +1682,33 @@ int nka_potrf_f64(double* a, int64_t n, int64_t lda, void* workspace, int32_t* i
   return NKA_OK;
 }
 
-// The launches of the two triangular solves.
+// The launches of the two triangular solves, whose waits end after `limit` polls.
 static void potrs_run(const double* a, int64_t n, int64_t lda, void* ws, double* b, const int32_t* info,
-                      hipStream_t s) {
+                      hipStream_t s, int64_t limit) {
   const int64_t nblk = (n + CH_NB - 1) / CH_NB;
   const double* inv = ws_inv(ws);
   double* y = ws_vec(ws, nblk);
   int32_t* err = (int32_t*)(ws_flags(ws, n, nblk) + nblk);
-  // (y and err are as the factorisation or the last solve left them: unsolved, 0)
-  hipLaunchKernelGGL(trsv_lookback<false>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, b, y, info, err);
-  hipLaunchKernelGGL(trsv_lookback<true>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, y, b, info, err);
+  // (y is as the factorisation or the last solve left it: unsolved)
+  hipLaunchKernelGGL(trsv_lookback<false>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, b, y, info, err,
+                     limit);
+  hipLaunchKernelGGL(trsv_lookback<true>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, y, b, info, err,
+                     limit);
+}
+
+int nka_potrs_f64_bounded(const double* a, int64_t n, int64_t lda, const void* workspace, double* b,
+                          const int32_t* info, int64_t polls, void* stream) {
+  NKA_CHECK_ARG(n >= 0 && lda >= n && a && workspace && b && info && polls >= 0, "nka_potrs_f64: bad arguments");
+  if (n == 0) return NKA_OK;
+  NKA_CHECK_ARG((n + CH_NB - 1) / CH_NB < (1LL << 31), "nka_potrs_f64: too large");
+  potrs_run(a, n, lda, (void*)workspace, b, info, (hipStream_t)stream, polls);
+  NKA_CHECK_LAUNCH("nka_potrs_f64");
+  return NKA_OK;
 }
 
 int nka_potrs_f64(const double* a, int64_t n, int64_t lda, const void* workspace, double* b,
                   const int32_t* info, void* stream) {
-  NKA_CHECK_ARG(n >= 0 && lda >= n && a && workspace && b && info, "nka_potrs_f64: bad arguments");
-  if (n == 0) return NKA_OK;
-  NKA_CHECK_ARG((n + CH_NB - 1) / CH_NB < (1LL << 31), "nka_potrs_f64: too large");
-  potrs_run(a, n, lda, (void*)workspace, b, info, (hipStream_t)stream);
-  NKA_CHECK_LAUNCH("nka_potrs_f64");
-  return NKA_OK;
+  return nka_potrs_f64_bounded(a, n, lda, workspace, b, info, kSpinLimit, stream);
 }
 
 }  // extern "C"
@@ -1788,7 +1812,7 @@ int nka_cholesky_solve_f64_noalloc(double* a, int64_t n, int64_t lda, double* b,
     return NKA_OK;
   }
   potrf_run(a, n, lda, ws, nullptr, 0, info, s);
-  potrs_run(a, n, lda, ws, b, info, s);
+  potrs_run(a, n, lda, ws, b, info, s, kSpinLimit);
   NKA_CHECK_LAUNCH("nka_cholesky_solve_f64_noalloc");
   return NKA_OK;
 }

@@ -596,7 +596,6 @@ __device__ __forceinline__ void substitute16(const double (&l)[16], double (&E)[
 // block.
 __global__ void __launch_bounds__(256) trtri_blocks_kernel(double* __restrict__ A, int64_t lda, int64_t n,
                                                            double* __restrict__ inv, double* __restrict__ y,
-                                                           int32_t* __restrict__ err,
                                                            const int32_t* __restrict__ info) {
   if (*info != 0) return;
   __shared__ double Lo[6][4][64], Mi[4][4][64];
@@ -607,7 +606,6 @@ __global__ void __launch_bounds__(256) trtri_blocks_kernel(double* __restrict__ 
   double* blk = inv + (int64_t)blockIdx.x * CH_NB * CH_NB;
   // what the solves start from
   if (tid < nb) ((uint64_t*)y)[k0 + tid] = kUnsolved;
-  if (blockIdx.x == 0 && tid == 0) *err = 0;
   double v[16], l[16], E[16];
 #pragma unroll
   for (int q = 0; q < 16; ++q) l[q] = blk[(16 * w + i) * CH_NB + 16 * w + q];

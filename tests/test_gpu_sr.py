@@ -845,3 +845,40 @@ def test_rbm_qgt_structured_fp64_spins_nearly_aligned(gpu):
     exact = (ns * (xi.T @ xi) - np.outer(m, m)) / (float(ns) * ns)
     low = np.tril_indices(N)
     np.testing.assert_allclose(S[v:v + N, v:v + N][low], exact[low], rtol=1e-15, atol=0)
+
+
+@pytest.mark.parametrize("n", [64, 65, 200, 1680, 4200])
+def test_triangular_solves_whose_waits_run_out(gpu, n):
+    # waits of a few polls between the blocks: the solution is right or NaN as a whole,
+    # and the next solve from the same workspace is right
+    print(f"case solve waits n={n}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(n)
+    X = torch.randn(n, n, dtype=torch.float64, device="cuda", generator=g)
+    A = (X @ X.T) / n + 0.1 * torch.eye(n, dtype=torch.float64, device="cuda")
+    a = torch.tril(A)
+    info = torch.zeros(1, dtype=torch.int32, device="cuda")
+    ws = _ops.potrf_(a, info)
+    ran_out = 0
+    for k, polls in enumerate([0, 0, 0, 1, 2, 3, 5, 8, 12, 20, 35, 60, 100, 200, 400, 0, 1 << 26]):
+        b = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+        x = b.clone()
+        nat.call("nka_potrs_f64_bounded", _ops.ptr(a), n, n, _ops.ptr(ws), _ops.ptr(x), _ops.ptr(info), polls,
+                 _ops.stream())
+        bad = int(torch.isnan(x).sum())
+        ran_out += bad > 0
+        assert bad in (0, n), f"{bad} of {n} entries are NaN after {polls} polls"
+        if not bad:
+            assert (A @ x - b).abs().max().item() < 1e-9 * b.abs().max().item()
+        if k % 2:
+            x = b.clone()
+            _ops.potrs_(a, ws, x, info)
+            assert (A @ x - b).abs().max().item() < 1e-9 * b.abs().max().item()
+    print(f"{ran_out} solves ran out", flush=True)
+    assert ran_out > 0 or n <= 200
+    assert bad == 0
+
+
+def test_bounded_solve_refuses_a_negative_bound(gpu):
+    t = torch.zeros(4096, dtype=torch.float64, device="cuda")
+    with pytest.raises(RuntimeError):
+        nat.call("nka_potrs_f64_bounded", _ops.ptr(t), 1, 1, _ops.ptr(t), _ops.ptr(t), _ops.ptr(t), -1, _ops.stream())
