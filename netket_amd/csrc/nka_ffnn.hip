@@ -38,18 +38,21 @@ constexpr int FF_MAXH = 1024;
 // Workgroup sizes.  The second layer is a chain of dependent matrix products
 // per 32-column block; several wavefronts per SIMD cover each other's operand
 // loads (L2 for W2, LDS for the activations), the first layer's gathers and the
-// row sums.  Forward pass: two workgroups of 512 per CU.  Sampler: one of 1024
-// (32 chains per CU are all there is), of 512 where a thread's state does not
-// fit 128 registers (FP64; weighted exchange).  J1-J2 10x10 with layers 100-400-
-// 400 in FP32, against workgroups of 256: the sampler (8192 chains, 700
+// row sums.  Forward pass: two workgroups of 512 per CU (FP64: see forward_small).
+// Sampler: one of 1024 (32 chains per CU are all there is), of 512 where a thread's
+// state does not fit 128 registers (FP64; weighted exchange).  J1-J2 10x10 with layers
+// 100-400-400 in FP32, against workgroups of 256: the sampler (8192 chains, 700
 // proposals) 42.4 -> 20.3 ms (matrix products 60% of it), the local energies of 16384
-// samples 23.2 -> 12.5 ms (58%; the rest is vector work and its latencies; with the connected elements taken as a list of
-// flipped sites instead of as configurations, 3.0 ms of that).
+// samples 23.2 -> 12.5 ms (58%; the rest is vector work and its latencies; with the
+// connected elements taken as a list of flipped sites instead of as configurations, 3.0
+// ms of that).  Layers of 8 to 100 units, 16 to 8192 chains, all rules: the sampler 1.0
+// (8-8 units, FP64) to 2.6 times as fast as with 256.
 constexpr int FF_FWD = 512;
 constexpr int FF_BACK = 256;
 constexpr int FF_MAXBLK = FF_MAXH / 32;  // column blocks of the second layer
 constexpr int FF_MAXD = 4;               // sites a connected configuration differs at (a term acts on at most 4)
 
+int device_cus();  // nka_sampler.hip
 // nka_conn.hip
 int launch_conn_list(int op_kind, const void* op, const int8_t* x, int64_t B, int N, int K, void* mels, int* rows,
                      uint64_t* sites, int* count, hipStream_t s);
@@ -273,15 +276,15 @@ __device__ inline T theta1_full(const FfnnView<T>& v, const int8_t* x, int a) {
 // differs from x[s].  Outputs log psi per row (MODE 1: at the row's own
 // index); g2_out (rows x H2), when set, receives tanh(z2).
 // ---------------------------------------------------------------------------
-template <class T, int MODE>
-__global__ void __launch_bounds__(FF_FWD) ffnn_forward_kernel(nka_ffnn m, const int8_t* __restrict__ xr, int Kc,
+template <class T, int MODE, int NT>
+__global__ void __launch_bounds__(NT) ffnn_forward_kernel(nka_ffnn m, const int8_t* __restrict__ xr, int Kc,
                                                                  const T* __restrict__ th_base, int64_t rows,
                                                                  T* __restrict__ logpsi, T* __restrict__ th_out,
                                                                  T* __restrict__ g2_out, const int* __restrict__ ridx,
                                                                  const uint64_t* __restrict__ rsites,
                                                                  const int* __restrict__ rcount) {
   extern __shared__ unsigned char smem[];
-  constexpr int FWD_G = FF_FWD / FF_ROWS;  // threads per row in the first layer
+  constexpr int FWD_G = NT / FF_ROWS;  // threads per row in the first layer
   const FfnnView<T> v = ffnn_view<T>(m);
   const int N = v.N, H1 = v.H1, H2 = v.H2;
   const int lda = lda_of(H1);
@@ -303,7 +306,7 @@ __global__ void __launch_bounds__(FF_FWD) ffnn_forward_kernel(nka_ffnn m, const 
   const int r = threadIdx.x / FWD_G, g = threadIdx.x % FWD_G;
   const int64_t gr = row_of(r);
   if (MODE == 0) {
-    for (int idx = threadIdx.x; idx < FF_ROWS * N; idx += FF_FWD) {
+    for (int idx = threadIdx.x; idx < FF_ROWS * N; idx += NT) {
       const int64_t ri = row_of(idx / N);
       xl[idx] = ri >= 0 ? xr[ri * N + idx % N] : (int8_t)1;
     }
@@ -369,7 +372,7 @@ __global__ void __launch_bounds__(FF_FWD) ffnn_forward_kernel(nka_ffnn m, const 
     if (g2_out && r0 + rr < rows) g2_out[(r0 + rr) * H2 + c] = tanh_t<T>(zz);
     return log_cosh<T>(zz);
   };
-  rows_gemm<FF_FWD / 64>(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
+  rows_gemm<NT / 64>(hA, lda, H1, H2, W2, H2, 1, epi, part, rowsum, rbuf);
   if (threadIdx.x < FF_ROWS) {
     const int64_t go = row_of(threadIdx.x);
     if (go >= 0) logpsi[go] = rowsum[threadIdx.x];
@@ -1127,7 +1130,8 @@ static void dispatch_ffnn_sweep(const nka_ffnn& m, const FfSweepArgs& sa, int8_t
                                 void* lps, int64_t* nacc, hipStream_t s) {
   constexpr int MAXH = FF_MAXH / (NT / FF_ROWS);
   const int need = (m.n_hidden1 + NT / FF_ROWS - 1) / (NT / FF_ROWS);
-  if (need <= MAXH / 8) launch_ffnn_sweep<T, NT, MAXH / 8, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
+  if (need <= MAXH / 32) launch_ffnn_sweep<T, NT, MAXH / 32, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
+  else if (need <= MAXH / 8) launch_ffnn_sweep<T, NT, MAXH / 8, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
   else if (need <= MAXH / 4) launch_ffnn_sweep<T, NT, MAXH / 4, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
   else if (need <= MAXH / 2) launch_ffnn_sweep<T, NT, MAXH / 2, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
   else launch_ffnn_sweep<T, NT, MAXH, WEIGHTED>(m, sa, sigma, lp, smp, lps, nacc, s);
@@ -1154,14 +1158,32 @@ inline int64_t ffnn_np(const nka_ffnn& m) {
          (m.b2_off >= 0 ? m.n_hidden2 : 0) + (int64_t)m.n_hidden1 * m.n_hidden2;
 }
 
+// FP64 rows on workgroups of 256 where there are many: past 16 workgroups per CU, and
+// from two per CU on with small layers.  The second layer is a plain sum per thread and
+// column there, and more small workgroups cover each other's barriers better than few
+// large ones.  Local energies of 16384 samples of the 6x6 Ising lattice, layers 8-8, 24-24,
+// 64-64: 344, 508, 1442 us against 446, 641, 1487 with 512; of 1024 samples (4.6 workgroups
+// per CU): 58, 77, 169 against 64, 82, 164; log psi of 32 rows, layers 64-64: 48 against 42.
+static bool forward_small(const nka_ffnn& m, int64_t workgroups) {
+  return workgroups >= 16 * device_cus() || (workgroups >= 2 * device_cus() && m.n_hidden1 * m.n_hidden2 <= 2048);
+}
+
 template <class T>
 static void launch_forward0(const nka_ffnn& m, const int8_t* x, int64_t rows, T* lp, T* th, T* g2, hipStream_t s) {
   if (rows <= 0) return;
   const unsigned g = (unsigned)((rows + FF_ROWS - 1) / FF_ROWS);
-  allow_lds(ffnn_forward_kernel<T, 0>, (int64_t)forward_lds<T>(m));
-  hipLaunchKernelGGL((ffnn_forward_kernel<T, 0>), dim3(g), dim3(FF_FWD), forward_lds<T>(m), s, m, x, 1,
-                     (const T*)nullptr, rows, lp, th, g2, (const int*)nullptr, (const uint64_t*)nullptr,
-                     (const int*)nullptr);
+  auto launch = [&](auto kernel, int threads) {
+    allow_lds(kernel, (int64_t)forward_lds<T>(m));
+    hipLaunchKernelGGL(kernel, dim3(g), dim3(threads), forward_lds<T>(m), s, m, x, 1, (const T*)nullptr, rows, lp, th,
+                       g2, (const int*)nullptr, (const uint64_t*)nullptr, (const int*)nullptr);
+  };
+  if constexpr (sizeof(T) == 8) {
+    if (forward_small(m, g)) {
+      launch(ffnn_forward_kernel<T, 0, FF_FWD / 2>, FF_FWD / 2);
+      return;
+    }
+  }
+  launch(ffnn_forward_kernel<T, 0, FF_FWD>, FF_FWD);
 }
 
 static int op_rows(int op_kind, const void* op, int N, int* K, int* mel_dtype) {
@@ -1224,10 +1246,18 @@ static int ffnn_eloc_impl(const nka_ffnn& m, int op_kind, const void* op, const 
     launch_forward0<T>(m, x, cs, lp0, th, nullptr, s);
     const int64_t rows = cs * K;
     const unsigned g = (unsigned)((rows + FF_ROWS - 1) / FF_ROWS);
-    allow_lds(ffnn_forward_kernel<T, 1>, (int64_t)forward_lds<T>(m));
-    hipLaunchKernelGGL((ffnn_forward_kernel<T, 1>), dim3(g), dim3(FF_FWD), forward_lds<T>(m), s, m,
-                       (const int8_t*)nullptr, K, (const T*)th, rows, lp, (T*)nullptr, (T*)nullptr, (const int*)ridx,
-                       (const uint64_t*)rsites, (const int*)rcount);
+    auto launch = [&](auto kernel, int threads) {
+      allow_lds(kernel, (int64_t)forward_lds<T>(m));
+      hipLaunchKernelGGL(kernel, dim3(g), dim3(threads), forward_lds<T>(m), s, m, (const int8_t*)nullptr, K,
+                         (const T*)th, rows, lp, (T*)nullptr, (T*)nullptr, (const int*)ridx, (const uint64_t*)rsites,
+                         (const int*)rcount);
+    };
+    bool half = false;
+    if constexpr (sizeof(T) == 8) {
+      half = forward_small(m, g);
+      if (half) launch(ffnn_forward_kernel<T, 1, FF_FWD / 2>, FF_FWD / 2);
+    }
+    if (!half) launch(ffnn_forward_kernel<T, 1, FF_FWD>, FF_FWD);
     const unsigned gr = (unsigned)((cs + 3) / 4);
     if (md == NKA_F32)
       hipLaunchKernelGGL((ffnn_eloc_reduce_kernel<T, float>), dim3(gr), dim3(256), 0, s, (const float*)mels,

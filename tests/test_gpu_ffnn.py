@@ -324,3 +324,49 @@ def test_fp32_chains_carry_their_own_log_prob(gpu, rule, H1, H2, n_chains):
         assert np.all(x.sum(axis=1) == 0)
     ref = 2 * of.log_psi(p, x)
     np.testing.assert_allclose(st.log_prob.cpu().numpy(), ref, rtol=0, atol=2e-5 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("N,H1,H2,n", [(6, 5, 9, 16500), (5, 45, 45, 16385), (4, 46, 45, 16384), (4, 50, 48, 131100)])
+def test_fp64_many_rows(gpu, N, H1, H2, n):
+    # both workgroup sizes of the FP64 forward pass, on both sides of the rule between them
+    # (two and sixteen workgroups of 32 rows per CU), as log psi and as local energies
+    print(f"case ffnn fp64 rows N={N} H=({H1},{H2}) n={n}", flush=True)
+    model, flat, p = _model(N, H1, H2, np.float64, 4, 0.2)
+    rng = np.random.default_rng(n)
+    x = rng.choice(np.array([-1, 1], dtype=np.int8), size=(n, N))
+    xt = torch.as_tensor(x, device="cuda")
+    every = np.array([[1 - 2 * (k >> i & 1) for i in range(N)] for k in range(2**N)], dtype=np.int8)
+    index = ((x < 0) * (1 << np.arange(N))).sum(1)
+    lp_ref = of.log_psi(p, every)
+    lp = model.apply(flat, xt).cpu().numpy()
+    tol = _rtol(np.float64) * np.abs(lp_ref).max()
+    np.testing.assert_allclose(lp, lp_ref[index], rtol=0, atol=tol)
+    op = nk.operator.Ising(nk.hilbert.Spin(0.5, N=N), nk.graph.Chain(N), h=0.7, J=1.0)
+    m = n // 3
+    e = eng.local_energies(model, flat, op, xt[:m]).cpu().numpy()
+    ref = of.local_energy(p, every, lambda z: O.ising_conn(z, op.edges, 0.7, 1.0))
+    np.testing.assert_allclose(e, ref[index[:m]], rtol=1e-10, atol=1e-10 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("rule", ["local", "exchange", "exchange-weighted"])
+@pytest.mark.parametrize("H1,H2,n_chains", [(1, 8, 33), (16, 3, 5), (32, 40, 32), (33, 8, 40), (129, 8, 7)])
+def test_small_layers_carry_their_own_log_prob(gpu, rule, H1, H2, n_chains, dtype):
+    # first layers of one unit up to a few per thread, at the edges of the sampler's instances
+    print(f"case ffnn sampler {rule} H=({H1},{H2}) chains={n_chains} {np.dtype(dtype)}", flush=True)
+    N = 10
+    model, flat, p = _model(N, H1, H2, dtype, 8, 0.2)
+    if rule == "local":
+        sa = nk.sampler.MetropolisLocal(nk.hilbert.Spin(0.5, N=N), n_chains=n_chains)
+    else:
+        sa = nk.sampler.MetropolisExchange(nk.hilbert.Spin(0.5, N=N, total_sz=0), graph=nk.graph.Chain(N), d_max=2,
+                                           probabilities=[0.4, 1.0] if rule.endswith("weighted") else None,
+                                           n_chains=n_chains)
+    st = sa.init_state(model, flat, seed=6)
+    samples, st = sa.sample_fused(model, flat, st, 2, 4)
+    x = st.sigma.cpu().numpy()
+    np.testing.assert_array_equal(x, samples.cpu().numpy()[:, -1])
+    assert st.n_accepted > 0 if hasattr(st, "n_accepted") else int(st.n_accepted_proc.sum()) > 0
+    ref = 2 * of.log_psi(p, x)
+    tol = 1e-12 if dtype == np.float64 else 2e-5
+    np.testing.assert_allclose(st.log_prob.cpu().numpy(), ref, rtol=0, atol=tol * np.abs(ref).max())
