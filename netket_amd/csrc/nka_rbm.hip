@@ -11,8 +11,6 @@
 //                       (netket/jax/_jacobian/logic.py:356-373)
 #include "nka_rbm.hpp"
 
-#include <type_traits>
-
 namespace nka {
 
 // ---------------------------------------------------------------------------
@@ -885,21 +883,110 @@ static void launch_eloc_f64(const nka_rbm& m, const OpArgs& op, const int8_t* sg
   launch_eloc<JL, double>(m, op, sg, n, e, (double*)lp, s, jobs, n_jobs);
 }
 
-// theta = sigma W + b for models whose W does not fit in LDS, as a tiled
-// matrix product without operand staging: 128 units x 128 samples per workgroup,
-// 64 x 64 per wavefront (W^T as the row operand, so that a lane's results are
-// samples side by side and the transposed output is written in whole lines).
-// FP32 on v_mfma_f32_32x32x2f32, FP64 on v_mfma_f64_16x16x4f64, k ascending.  The W
-// fragments come straight from the caches (16 bytes of it per product at most, 32
-// sites' loads in flight; rows past the last site read zero), the spins from a bit
-// set per sample in LDS.  The epilogue writes t = tanh(theta) to t (ns, M) and/or
-// tT (M, ns); RAW: theta itself to tT.
-// Bound by the matrix cores: FP32, 32768 samples x 400 sites x 3200 units, RAW,
-// 0.76 ms with its packed spins made by spin_bits_kernel (0.02 ms; 110 TFLOP/s, of
-// 149 for a large product), 1.18 ms as a product with both operands staged and the
-// samples as rows, 1.09 ms with every workgroup packing its own spins, which is
-// how the calls without a workspace run.
+// t = tanh(sigma W + b) for models whose W does not fit in LDS, as a tiled
+// matrix product: 64 samples x 64 hidden units per workgroup, K = N in steps
+// of 16 through LDS (sigma as exact +-1), so W is read once per 64 samples
+// instead of once per sample.  FP32 on v_mfma_f32_32x32x2f32 (one 32x32
+// block per wave), FP64 on v_mfma_f64_16x16x4f64 (2x2 blocks per wave).
+// The epilogue writes t to t (ns, M) and/or tT (M, ns).  Bound by the latency of
+// its K steps with few samples, which is what keeps it beside rbm_theta_kernel: packed
+// spins, made by every workgroup for itself, take 60 to 95 us where this takes 25 to 38
+// (up to 4096 samples, 64 to 144 sites), and 1.09 ms against 1.18 at 32768 x 400 x 3200.
 typedef float ffx16 __attribute__((ext_vector_type(16)));
+constexpr int PR_T = 64, PR_K = 16;   // samples and units; sites per step
+
+template <class T>
+__global__ void __launch_bounds__(256) rbm_prepare_gemm_kernel(nka_rbm m, const int8_t* __restrict__ sigma,
+                                                               int64_t ns, T* __restrict__ t, T* __restrict__ tT) {
+  __shared__ T sA[PR_T][PR_K + 1];
+  __shared__ T sB[PR_K][PR_T + 1];
+  const RbmView<T> v = rbm_view<T>(m);
+  const int N = v.N, M = v.M;
+  const int64_t s0 = (int64_t)blockIdx.x * PR_T;
+  const int j0 = blockIdx.y * PR_T;
+  const int tid = threadIdx.x, wid = tid >> 6, lane = lane_id();
+  const int wm = (wid >> 1) * 32, wn = (wid & 1) * 32;
+  ffx16 accf;
+  ddx4 accd[2][2];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) accf[e] = 0.0f;
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) accd[a][b] = (ddx4){0.0, 0.0, 0.0, 0.0};
+  for (int k0 = 0; k0 < N; k0 += PR_K) {
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+      const int idx = tid + it * 256;
+      const int r = idx >> 4, kc = idx & 15;            // A: 64 rows x 16 k
+      const int kk = k0 + kc;
+      T va = (T)0;
+      if (s0 + r < ns && kk < N) va = sigma[(s0 + r) * N + kk] > 0 ? (T)1 : (T)-1;
+      sA[r][kc] = va;
+      const int kr = idx >> 6, c = idx & 63;            // B: 16 k x 64 cols
+      T vb = (T)0;
+      if (k0 + kr < N && j0 + c < M) vb = v.W[(int64_t)(k0 + kr) * M + j0 + c];
+      sB[kr][c] = vb;
+    }
+    __syncthreads();
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int k = 0; k < PR_K; k += 2) {
+        const float a = sA[wm + (lane & 31)][k + (lane >> 5)];
+        const float b = sB[k + (lane >> 5)][wn + (lane & 31)];
+        accf = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, accf, 0, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < PR_K; k += 4) {
+        double av[2], bv[2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a) av[a] = sA[wm + a * 16 + (lane & 15)][k + (lane >> 4)];
+#pragma unroll
+        for (int b = 0; b < 2; ++b) bv[b] = sB[k + (lane >> 4)][wn + b * 16 + (lane & 15)];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+            accd[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], accd[a][b], 0, 0, 0);
+      }
+    }
+  }
+  auto store = [&](int64_t sr, int j, T th) {
+    if (sr < ns && j < M) {
+      const T tv = tanh_t<T>(th + (v.b ? v.b[j] : (T)0));
+      if (t) t[sr * M + j] = tv;
+      if (tT) tT[(int64_t)j * ns + sr] = tv;
+    }
+  };
+  if constexpr (sizeof(T) == 4) {
+    // element e of lane l: row (e/4)*8 + (l/32)*4 + e%4, col l%32
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      store(s0 + wm + (e >> 2) * 8 + (lane >> 5) * 4 + (e & 3), j0 + wn + (lane & 31), (T)accf[e]);
+  } else {
+    // element e of lane l in a 16x16 block: row l/16 + 4e, col l%16
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          store(s0 + wm + a * 16 + (lane >> 4) + 4 * e, j0 + wn + b * 16 + (lane & 15), (T)accd[a][b][e]);
+  }
+}
+
+// theta = sigma W + b of FP32 models whose W does not fit in LDS, for the tiled local
+// energies: 128 units x 128 samples per workgroup, 64 x 64 per wavefront on
+// v_mfma_f32_32x32x2f32, k ascending (W^T as the row operand, so that a lane's results
+// are samples side by side and the transposed output is written in whole lines).  The W
+// fragments come straight from the caches, a batch of 8 sites ahead (rows past the last
+// site read zero); the spins are bits, made by spin_bits_kernel, in LDS.  Writes theta to
+// tT (Mp, ns), the rows from M up to the next multiple of 64 zero.
+// Bound by the matrix cores: 32768 samples x 400 sites x 3200 units 0.76 ms with the
+// packed spins made (0.02 ms; 110 TFLOP/s, of 149 for a large product), 1.18 ms as a
+// product with both operands staged and the samples as rows.
 constexpr int PG_T = 128, PG_K = 1024;    // samples, units; sites whose spins are in LDS at once
 
 // bits[w][sample]: bit k of word w = (x_{32 w + k} > 0); 64 samples x 64 sites
@@ -921,90 +1008,62 @@ __global__ void __launch_bounds__(256) spin_bits_kernel(const int8_t* __restrict
   if (wid < 2 && 32 * word < N && s0 + lane < ns) bits[(int64_t)word * ns + s0 + lane] = w[wid][lane];
 }
 
-template <class T, bool RAW>
-__global__ void __launch_bounds__(256, sizeof(T) == 8 ? 1 : 3) rbm_theta_kernel(
-    nka_rbm m, const int8_t* __restrict__ sigma, const uint32_t* __restrict__ bits, int64_t ns, T* __restrict__ t,
-    T* __restrict__ tT) {
+__global__ void __launch_bounds__(256, 3) rbm_theta_kernel(nka_rbm m, const uint32_t* __restrict__ bits, int64_t ns,
+                                                           float* __restrict__ tT) {
   __shared__ uint32_t sbits[PG_K / 32 * PG_T];  // [word][sample]: bit k % 32 of word k / 32 = (x_k > 0)
-  constexpr bool F64 = sizeof(T) == 8;
-  constexpr int E = F64 ? 16 : 32;        // block edge
-  constexpr int KS = F64 ? 4 : 2;         // sites per product
-  constexpr int NB = 64 / E;              // blocks per wavefront edge
-  constexpr int ACC = F64 ? 4 : 16;
-  using acc_t = typename std::conditional<F64, ddx4, ffx16>::type;
-  const RbmView<T> v = rbm_view<T>(m);
-  const int N = v.N, M = v.M;
+  constexpr int E = 32, KS = 2, NB = 64 / E;    // block edge, sites per product, blocks per wavefront edge
+  const RbmView<float> v = rbm_view<float>(m);
+  const int N = v.N, M = v.M, Mp = (M + 63) / 64 * 64;
   const int64_t s0 = (int64_t)blockIdx.x * PG_T;
   const int j0 = blockIdx.y * PG_T;
   const int tid = threadIdx.x, wid = tid >> 6, lane = tid & 63;
   const int wu = (wid >> 1) * 64, ws = (wid & 1) * 64;
-  const bool active = s0 + ws < ns && j0 + wu < (RAW ? (M + 63) / 64 * 64 : M);
+  const bool active = s0 + ws < ns && j0 + wu < Mp;
   const int lc = lane % E, kh = lane / E;
   int woff[NB];
 #pragma unroll
-  for (int a = 0; a < NB; ++a) woff[a] = (kh * M + min(j0 + wu + a * E + lc, M - 1)) * (int)sizeof(T);
-  acc_t acc[NB][NB];
+  for (int a = 0; a < NB; ++a) woff[a] = (kh * M + min(j0 + wu + a * E + lc, M - 1)) * 4;
+  ffx16 acc[NB][NB];
 #pragma unroll
   for (int a = 0; a < NB; ++a)
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
-      for (int e = 0; e < ACC; ++e) acc[a][b][e] = (T)0;
+      for (int e = 0; e < 16; ++e) acc[a][b][e] = 0.0f;
   constexpr int KB = 8;                   // sites per batch of W loads
   constexpr int Q = KB / KS;
-  T wv[2][Q][NB];
-  auto load = [&](const __amdgpu_buffer_rsrc_t Wb, int k0, T (&w)[Q][NB]) __attribute__((always_inline)) {
+  float wv[2][Q][NB];
+  auto load = [&](const __amdgpu_buffer_rsrc_t Wb, int k0, float (&w)[Q][NB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < Q; ++q)
 #pragma unroll
-      for (int a = 0; a < NB; ++a) {
-        const int soff = (k0 + q * KS) * M * (int)sizeof(T);
-        if constexpr (F64) {
-          const auto x = __builtin_amdgcn_raw_buffer_load_b64(Wb, woff[a], soff, 0);
-          w[q][a] = __builtin_bit_cast(double, x);
-        } else {
-          w[q][a] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(Wb, woff[a], soff, 0));
-        }
-      }
+      for (int a = 0; a < NB; ++a)
+        w[q][a] = __builtin_bit_cast(
+            float, __builtin_amdgcn_raw_buffer_load_b32(Wb, woff[a], (k0 + q * KS) * M * 4, 0));
   };
-  auto group = [&](int k0, const uint32_t (&word)[NB], const T (&w)[Q][NB]) __attribute__((always_inline)) {
+  auto group = [&](int k0, const uint32_t (&word)[NB], const float (&w)[Q][NB]) __attribute__((always_inline)) {
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-      T sg[NB];
+      float sg[NB];
 #pragma unroll
-      for (int b = 0; b < NB; ++b) sg[b] = (word[b] >> ((k0 & 31) + q * KS + kh)) & 1u ? (T)1 : (T)-1;
+      for (int b = 0; b < NB; ++b) sg[b] = (word[b] >> ((k0 & 31) + q * KS + kh)) & 1u ? 1.0f : -1.0f;
 #pragma unroll
       for (int a = 0; a < NB; ++a)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-          if constexpr (F64) acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(w[q][a], sg[b], acc[a][b], 0, 0, 0);
-          else acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[q][a], sg[b], acc[a][b], 0, 0, 0);
-        }
+        for (int b = 0; b < NB; ++b)
+          acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(w[q][a], sg[b], acc[a][b], 0, 0, 0);
     }
   };
   for (int c0 = 0; c0 < N; c0 += PG_K) {
     const int nk = min(PG_K, N - c0);
     if (c0) __syncthreads();
-    if (RAW) {
-      const int nwc = (nk + 31) >> 5;
-      for (int e = tid; e < nwc * PG_T; e += 256)
-        sbits[e] = bits[(int64_t)(c0 / 32 + e / PG_T) * ns + min(s0 + e % PG_T, ns - 1)];
-    } else {
-      // 64 sites of a sample per load, one per lane; eight loads in flight
-      for (int k = 0; k < nk; k += 64) {
-        const bool in = k + lane < nk;
-        const int8_t* col = sigma + c0 + (in ? k + lane : 0);
-#pragma unroll 8
-        for (int r = wid; r < PG_T; r += 4) {
-          const uint64_t up = __ballot(in && s0 + r < ns && col[min(s0 + r, ns - 1) * N] > 0);
-          if (lane < 2) sbits[((k >> 5) + lane) * PG_T + r] = (uint32_t)(up >> (32 * lane));
-        }
-      }
-    }
+    const int nwc = (nk + 31) >> 5;
+    for (int e = tid; e < nwc * PG_T; e += 256)
+      sbits[e] = bits[(int64_t)(c0 / 32 + e / PG_T) * ns + min(s0 + e % PG_T, ns - 1)];
     __syncthreads();
     if (!active) continue;
     const __amdgpu_buffer_rsrc_t Wb = __builtin_amdgcn_make_buffer_rsrc(
-        (void*)(v.W + (size_t)c0 * M), 0, nk * M * (int)sizeof(T), 0x00020000);
+        (void*)(v.W + (size_t)c0 * M), 0, nk * M * 4, 0x00020000);
     load(Wb, 0, wv[0]);
     for (int k1 = 0; k1 < nk; k1 += 32) {
       uint32_t word[NB];
@@ -1019,26 +1078,17 @@ __global__ void __launch_bounds__(256, sizeof(T) == 8 ? 1 : 3) rbm_theta_kernel(
     }
   }
   if (!active) return;
-  // element e of lane l: FP32 row (e/4)*8 + (l/32)*4 + e%4, FP64 row l/16 + 4e;
-  // col (sample) l % E.  RAW also writes the rows up to the next multiple of 64
-  // (zero beyond M).
-  const int Mp = (M + 63) / 64 * 64;
+  // element e of lane l: row (e/4)*8 + (l/32)*4 + e%4; col (sample) l % 32
 #pragma unroll
   for (int a = 0; a < NB; ++a)
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
       const int64_t sr = s0 + ws + b * E + lc;
 #pragma unroll
-      for (int e = 0; e < ACC; ++e) {
-        const int j = j0 + wu + a * E + (F64 ? kh + 4 * e : (e >> 2) * 8 + kh * 4 + (e & 3));
-        const T th = acc[a][b][e] + (v.b && j < M ? v.b[j] : (T)0);
-        if (RAW) {
-          if (sr < ns && j < Mp) tT[(int64_t)j * ns + sr] = j < M ? th : (T)0;
-        } else if (sr < ns && j < M) {
-          const T tv = tanh_t<T>(th);
-          if (t) t[sr * M + j] = tv;
-          if (tT) tT[(int64_t)j * ns + sr] = tv;
-        }
+      for (int e = 0; e < 16; ++e) {
+        const int j = j0 + wu + a * E + (e >> 2) * 8 + kh * 4 + (e & 3);
+        const float th = acc[a][b][e] + (v.b && j < M ? v.b[j] : 0.0f);
+        if (sr < ns && j < Mp) tT[(int64_t)j * ns + sr] = j < M ? th : 0.0f;
       }
     }
 }
@@ -1053,8 +1103,8 @@ static void launch_prepare(const nka_rbm& m, const int8_t* sigma, int64_t ns, T*
   const int waves = 4;
   const bool stage = stage_fits<T>(m, waves);
   if (!stage) {
-    hipLaunchKernelGGL((rbm_theta_kernel<T, false>), theta_grid(ns, m.n_hidden), dim3(256), 0, s,
-                       m, sigma, (const uint32_t*)nullptr, ns, t, tT);
+    dim3 grid((unsigned)((ns + PR_T - 1) / PR_T), (unsigned)((m.n_hidden + PR_T - 1) / PR_T));
+    hipLaunchKernelGGL(rbm_prepare_gemm_kernel<T>, grid, dim3(256), 0, s, m, sigma, ns, t, tT);
     return;
   }
   const size_t lds = (stage ? pad16((size_t)m.n_visible * m.n_hidden * sizeof(T)) : 0) +
@@ -1293,8 +1343,7 @@ static int ising_tiled_eloc(const nka_rbm& m, const nka_ising& is, const int8_t*
     uint32_t* bits = (uint32_t*)part;
     hipLaunchKernelGGL(spin_bits_kernel, dim3((unsigned)((nc + 63) / 64), (unsigned)((N + 63) / 64)), dim3(256), 0, s,
                        sigma + c0 * N, nc, N, bits);
-    hipLaunchKernelGGL((rbm_theta_kernel<float, true>), theta_grid(nc, tl.Mp), dim3(256), 0, s, m,
-                       (const int8_t*)nullptr, bits, nc, (float*)nullptr, thT);
+    hipLaunchKernelGGL(rbm_theta_kernel, theta_grid(nc, tl.Mp), dim3(256), 0, s, m, bits, nc, thT);
     dim3 gf((unsigned)((nc + 63) / 64), (unsigned)tl.n_jt);
     hipLaunchKernelGGL(ising_flip_tile_kernel, gf, dim3(256), bits_lds, s, thT, Wp, sigma + c0 * N, nc, N,
                        tl.Mp, v.a, is, log_psi ? 1 : 0, part, diag);
