@@ -1217,7 +1217,8 @@ static int ffnn_eloc_impl(const nka_ffnn& m, int op_kind, const void* op, const 
   }
   const int N = m.n_visible, H1 = m.n_hidden1;
   const int64_t per = eloc_bytes_per_sample(m, K);
-  const int64_t chunk = std::min<int64_t>(n, (ws_bytes - 4096) / per);
+  // (rows are numbered in 32 bits; a larger workspace is used in part)
+  const int64_t chunk = std::min<int64_t>(std::min<int64_t>(n, (ws_bytes - 4096) / per), ((1LL << 31) - 1) / std::max(K, 1));
   NKA_CHECK_ARG(chunk >= 1, "nka_ffnn_local_energy: workspace too small");
   unsigned char* p = ws;
   auto take = [&](int64_t bytes) {
@@ -1232,7 +1233,6 @@ static int ffnn_eloc_impl(const nka_ffnn& m, int op_kind, const void* op, const 
   T* lp0own = (T*)take(chunk * sizeof(T));
   int* ridx = (int*)take(chunk * K * (int64_t)sizeof(int));
   int* rcount = (int*)take(16);
-  NKA_CHECK_ARG(chunk * (int64_t)K < (1LL << 31), "nka_ffnn_local_energy: too many connected rows per chunk");
   for (int64_t s0 = 0; s0 < n; s0 += chunk) {
     const int64_t cs = std::min<int64_t>(chunk, n - s0);
     const int8_t* x = sigma + s0 * N;

@@ -370,3 +370,35 @@ def test_small_layers_carry_their_own_log_prob(gpu, rule, H1, H2, n_chains, dtyp
     ref = 2 * of.log_psi(p, x)
     tol = 1e-12 if dtype == np.float64 else 2e-5
     np.testing.assert_allclose(st.log_prob.cpu().numpy(), ref, rtol=0, atol=tol * np.abs(ref).max())
+
+
+def test_local_energy_workspace_of_more_rows_than_32_bits_hold(gpu):
+    # a workspace for 2^31 connected rows and more: taken in part, in two chunks.  Aligned
+    # spins have no connected elements, so that the rows are counted and not evaluated
+    N, K = 400, 401
+    n = (1 << 31) // K + 2
+    need = 25 * K * n + (1 << 20)
+    free = torch.cuda.mem_get_info()[0]
+    if free < need + n * (N + 64):
+        pytest.skip("needs 60 GB of device memory")
+    print(f"case ffnn eloc rows past 32 bits n={n}", flush=True)
+    import ctypes as C
+    from netket_amd import _ops
+    g = nk.graph.Chain(N)
+    H = nk.operator.Heisenberg(nk.hilbert.Spin(0.5, N=N), g)
+    model, flat, p = _model(N, 1, 1, np.float32, 5, 0.05)
+    m = model.native(flat, N)
+    kind, op_ptr, keep = _ops.op_struct(H)
+    assert H.max_conn_size == K
+    x = torch.ones((n, N), dtype=torch.int8, device="cuda")
+    x[-1, 3] = -1   # one sample of the second chunk with two connected elements
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    eloc = torch.full((n,), float("nan"), dtype=torch.float64, device="cuda")
+    nat.call("nka_ffnn_local_energy", C.byref(m), kind, op_ptr, _ops.ptr(x), n, _ops.ptr(eloc), None, _ops.ptr(ws),
+             ws.numel(), _ops.stream())
+    assert torch.all(eloc[:-1] == float(N))
+    terms = dict(zip([tuple(a) for a in H.acting_on], H.operators))
+    ref = of.local_energy(p, x[-1:].cpu().numpy(), lambda z: O.local_conn(z, terms))
+    np.testing.assert_allclose(eloc[-1:].cpu().numpy(), ref, rtol=1e-5)
+    del keep, ws, x
+    torch.cuda.empty_cache()
