@@ -335,6 +335,7 @@ int launch_conn_list(int op_kind, const void* op, const int8_t* x, int64_t B, in
     NKA_CHECK_ARG(o->max_conn_size >= 1, "nka_localop_conn: max_conn_size must be >= 1");
     NKA_CHECK_ARG(o->mel_dtype == NKA_F32 || o->mel_dtype == NKA_F64, "nka_localop_conn: bad dtype");
     const size_t lds = 4 * (size_t)((N + 15) & ~15);
+    // (the operators that nka_localop_conn takes, whose LDS holds the elements as well)
     NKA_CHECK_ARG(lds + 16 * (size_t)K <= 64 * 1024, "nka_localop_conn: N or max_conn_size too large");
     if (o->mel_dtype == NKA_F64)
       hipLaunchKernelGGL(localop_list_kernel<double>, dim3(g), dim3(256), lds, s, x, B, N, *o, (double*)mels, rows,

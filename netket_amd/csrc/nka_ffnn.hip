@@ -12,18 +12,13 @@
 // depend on scheduling.
 //
 // Callers of the tile kernel: log psi, the local energies (connected
-// configurations from the conn kernels, first layer updated from the
+// elements as a list from the conn kernels, first layer updated from the
 // sample's theta1 by the differing sites), the per-sample quantities of the
 // Jacobian (h1, tanh z2, back-propagated d1) and the Metropolis sampler
 // (32 chains per workgroup stepping in lock step).
 #include "nka_common.hpp"
 #include "netket_amd.h"
 
-extern "C" int nka_ising_conn(const int8_t* x, int64_t n_batch, int n_sites, const int32_t* edges,
-                              int n_edges, double h, double J, int mel_dtype, int n_rows, int8_t* xp,
-                              void* mels, void* stream);
-extern "C" int nka_localop_conn(const int8_t* x, int64_t n_batch, int n_sites, const nka_localop* op,
-                                int8_t* xp, void* mels, int32_t* n_conn, void* stream);
 extern "C" int nka_gemm_nt_f64(const double* a, int64_t lda, const double* b, int64_t ldb, double* c,
                                int64_t ldc, int64_t m, int64_t n, int64_t k, double alpha, double beta,
                                void* stream);
@@ -730,14 +725,14 @@ __global__ void ffnn_jacobian_kernel(nka_ffnn m, const int8_t* __restrict__ x, c
 }
 
 // ---------------------------------------------------------------------------
-// Metropolis sampler: 32 chains per workgroup in lock step.  Thread t holds
-// theta1 of chain t / 8 for the units a = t % 8 + 8 j in registers; the chain
-// spins live in LDS.  Each proposal: wave w draws the proposals of chains
-// 8w .. 8w+7 (same rules and Philox stream layout as the RBM sampler:
-// counter q, chain id, TAG_METROPOLIS; x word picks the site / cluster, the
-// uniform of the acceptance comes from the same draw); theta1' and
-// h1' = log_cosh(theta1') are formed, the second layer gives log psi'; a
-// chain accepts when u < exp(machine_pow (log psi' - log psi) + corr).
+// Metropolis sampler: 32 chains per workgroup of NT threads in lock step.  With
+// GR = NT / 32 threads per chain, thread t holds theta1 of chain t / GR for the units
+// a = t % GR + GR j in registers; the chain spins live in LDS.  Each proposal: a
+// wavefront draws those of its CPW = 2048 / NT chains, 64 / CPW lanes each (same rules
+// and Philox stream layout as the RBM sampler: counter q, chain id, TAG_METROPOLIS; x
+// word picks the site / cluster, the uniform of the acceptance comes from the same
+// draw); theta1' and h1' = log_cosh(theta1') are formed, the second layer gives log psi';
+// a chain accepts when u < exp(machine_pow (log psi' - log psi) + corr).
 // ---------------------------------------------------------------------------
 struct FfSweepArgs {
   int rule;

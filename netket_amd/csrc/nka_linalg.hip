@@ -586,10 +586,9 @@ __global__ void __launch_bounds__(256, 4) gemm_exact_a_small_kernel(const uint16
 
 // ---------------------------------------------------------------------------
 // FP64 NT GEMM: C = beta C + alpha A B^T (+ shift on the diagonal),
-// 64x64 tile per workgroup, 4 waves of 32x32, K step 16.  lower_only skips
-// tiles above the diagonal and elements with j > i.  A and C may alias when
-// beta == 0 and the grid has a single column tile (in-place panel solve):
-// every workgroup reads all of its A rows before it writes them.
+// 64x64 tile per workgroup, 4 waves of 32x32, K step 16, for K that is no multiple
+// of the K step (the kernel below takes the others).  lower_only skips tiles above
+// the diagonal and elements with j > i.
 // ---------------------------------------------------------------------------
 constexpr int GD_T = 64;
 constexpr int GD_K = 16;
@@ -1300,8 +1299,9 @@ __device__ inline double group_var(const double* d, const GroupSpec& g, double* 
 }
 
 // One workgroup; bound by the latency of its passes over data that fits the caches,
-// so a thread's loads are in flight together and each group's mean is formed once
-// (16 chains of 63 and of 1000: 22.8 -> 11.5 us, 242 -> 33 us).
+// so a thread's loads are in flight together, and the mean of a thread's first group is
+// kept for the second pass (all of them up to 1024 groups; 16 chains of 63 and of 1000:
+// 22.8 -> 11.5 us, 242 -> 33 us).
 __global__ void __launch_bounds__(1024) stats_kernel(const double* __restrict__ d, int C, int L,
                                                      double* __restrict__ out) {
   __shared__ double red[16];
@@ -1561,34 +1561,31 @@ int nka_gemm_nt_f64(const double* a, int64_t lda, const double* b, int64_t ldb, 
   return NKA_OK;
 }
 
-// Workspace: 64x64 inverses of the diagonal blocks, the intermediate vector
-// of the solves, one flag per block and one error word, and the K-slices of
-// the trailing products' split tail tiles (up to kMaxSplitUnits raw 128x128
-// tiles, fewer for small n).
+// Workspace: 64x64 inverses of the diagonal blocks, the intermediate vector and the
+// error word of the solves, and the K-slices of the trailing products' split tail tiles
+// (up to kMaxSplitUnits raw 128x128 tiles, fewer for small n).
 static int64_t split_units(int64_t n) {
   const int64_t t = (n + G2_T - 1) / G2_T;
   return std::min<int64_t>(kMaxSplitUnits, 2 * t * (t + 1) / 2);
 }
+static constexpr int64_t ws_head(int64_t n, int64_t nblk) {
+  return (nblk * CH_NB * CH_NB * (int64_t)sizeof(double) + (n + 64) * (int64_t)sizeof(double) + 256 + 255) / 256 * 256;
+}
 
 int64_t nka_potrf_workspace(int64_t n) {
   if (n <= 0) return 0;
-  const int64_t nblk = (n + CH_NB - 1) / CH_NB;
-  const int64_t head = nblk * CH_NB * CH_NB * (int64_t)sizeof(double) + (n + 64) * (int64_t)sizeof(double) +
-                       (nblk + 64) * (int64_t)sizeof(uint32_t);
-  return ((head + 255) / 256) * 256 + split_units(n) * G2_T * G2_T * (int64_t)sizeof(double);
+  return ws_head(n, (n + CH_NB - 1) / CH_NB) + split_units(n) * G2_T * G2_T * (int64_t)sizeof(double);
 }
 
 static inline double* ws_inv(void* ws) { return (double*)ws; }
 static inline double* ws_vec(void* ws, int64_t nblk) {
   return (double*)ws + nblk * CH_NB * CH_NB;
 }
-static inline uint32_t* ws_flags(void* ws, int64_t n, int64_t nblk) {
-  return (uint32_t*)(ws_vec(ws, nblk) + n + 64);
+static inline int32_t* ws_err(void* ws, int64_t n, int64_t nblk) {
+  return (int32_t*)(ws_vec(ws, nblk) + n + 64);
 }
 static inline double* ws_split(void* ws, int64_t n, int64_t nblk) {
-  const int64_t head = nblk * CH_NB * CH_NB * (int64_t)sizeof(double) + (n + 64) * (int64_t)sizeof(double) +
-                       (nblk + 64) * (int64_t)sizeof(uint32_t);
-  return (double*)((char*)ws + ((head + 255) / 256) * 256);
+  return (double*)((char*)ws + ws_head(n, nblk));
 }
 
 // Right-looking Cholesky with up to three levels of blocking.  An outer
@@ -1688,7 +1685,7 @@ static void potrs_run(const double* a, int64_t n, int64_t lda, void* ws, double*
   const int64_t nblk = (n + CH_NB - 1) / CH_NB;
   const double* inv = ws_inv(ws);
   double* y = ws_vec(ws, nblk);
-  int32_t* err = (int32_t*)(ws_flags(ws, n, nblk) + nblk);
+  int32_t* err = ws_err(ws, n, nblk);
   // (y is as the factorisation or the last solve left it: unsolved)
   hipLaunchKernelGGL(trsv_lookback<false>, dim3((unsigned)nblk), dim3(256), 0, s, a, lda, n, inv, b, y, info, err,
                      limit);
@@ -1715,8 +1712,8 @@ int nka_potrs_f64(const double* a, int64_t n, int64_t lda, const void* workspace
 
 // ---------------------------------------------------------------------------
 // Factor and solve with no allocation and no caller workspace.  The scratch
-// (inverses of the diagonal blocks, the intermediate vector, the flags and
-// the error word of the solves) is a static device array of a fixed size;
+// (inverses of the diagonal blocks, the intermediate vector and the error word
+// of the solves) is a static device array of a fixed size;
 // host code reaches it only through the address hipGetSymbolAddress returns
 // for the current device.  Trailing products run unsplit here (the split of
 // tail tiles would need up to 128 MiB more), so the last bits can differ from
@@ -1724,10 +1721,7 @@ int nka_potrs_f64(const double* a, int64_t n, int64_t lda, const void* workspace
 // ---------------------------------------------------------------------------
 constexpr int64_t kNoAllocMaxN = 32768;
 constexpr int64_t kNoAllocNblk = (kNoAllocMaxN + CH_NB - 1) / CH_NB;
-constexpr int64_t kNoAllocHead = kNoAllocNblk * CH_NB * CH_NB * (int64_t)sizeof(double) +
-                                 (kNoAllocMaxN + 64) * (int64_t)sizeof(double) +
-                                 (kNoAllocNblk + 64) * (int64_t)sizeof(uint32_t);
-constexpr int64_t kNoAllocBytes = (kNoAllocHead + 255) / 256 * 256;
+constexpr int64_t kNoAllocBytes = ws_head(kNoAllocMaxN, kNoAllocNblk);
 
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 

@@ -188,13 +188,12 @@ __global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* 
   }
 }
 
-// C = P Q^T (FP64), one 192 x 64 tile per workgroup: four wavefronts of 96 x 32
-// with one int32 accumulator per digit plane and 32 x 32 block (3 x 7), so a
-// K sub-step of 32 samples reads 3 + 7 operand fragments from LDS for 21
-// products.  Operands go from global memory straight into LDS
-// (global_load_lds, 16 bytes per lane) into the buffer of the next K step while
-// the current one is multiplied, which leaves the registers to the 336
-// accumulators.  A row's four 16-byte chunks of a K step are stored in the
+// C = P Q^T (FP64), one 128 x 64 tile per workgroup: four wavefronts of 64 x 32
+// with one int32 accumulator per digit plane and 32 x 32 block (2 x 7), so a
+// K sub-step of 32 samples reads 2 + 7 operand fragments from LDS for 14
+// products.  Operands go from global memory straight into LDS (16 bytes per lane),
+// three K steps ahead of the one that is multiplied, which leaves the registers to
+// the 224 accumulators.  A row's four 16-byte chunks of a K step are stored in the
 // order chunk ^ (row / 4 % 4), which makes the fragment reads (32 consecutive
 // rows, one chunk) free of bank conflicts over the 64 banks.
 // Tiles are numbered down the columns, so the workgroups that share a panel of

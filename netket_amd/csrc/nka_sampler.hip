@@ -280,38 +280,29 @@ __global__ void __launch_bounds__(256) rbm_metropolis_kernel_batched(const nka_s
 // add the same two operands, so every lane of a group holds the identical sum.
 // Same random streams, rules and acceptance as rbm_metropolis_kernel.
 // ---------------------------------------------------------------------------
-// log of a small positive integer count: hardware log2 for FP32, log for FP64.
-template <class T> __device__ inline T log_fast(T x);
-template <> __device__ inline float log_fast<float>(float x) {
-  return 0.69314718055994531f * __builtin_amdgcn_logf(x);
-}
-template <> __device__ inline double log_fast<double>(double x) { return log(x); }
+// log of a small positive integer count, from the hardware log2.
+__device__ inline float log_fast(float x) { return 0.69314718055994531f * __builtin_amdgcn_logf(x); }
 
-template <class T, int G, int JG, int RSG, bool STAGE>
-__device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& m, const SweepArgs& sa, int8_t* __restrict__ sigma, T* __restrict__ log_prob, int8_t* __restrict__ samples, T* __restrict__ lp_samples, int64_t* __restrict__ n_accepted, int bx) {
+template <int G, int JG, int RSG>
+__device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& m, const SweepArgs& sa, int8_t* __restrict__ sigma, float* __restrict__ log_prob, int8_t* __restrict__ samples, float* __restrict__ lp_samples, int64_t* __restrict__ n_accepted, int bx) {
   constexpr int LPC = NKA_WAVE / G;
   constexpr uint64_t GMASK = (LPC == 64) ? ~0ull : ((1ull << LPC) - 1ull);
   extern __shared__ unsigned char smem[];
-  const RbmView<T> v = rbm_view<T>(m);
+  const RbmView<float> v = rbm_view<float>(m);
   const int N = v.N, M = v.M;
   const int wid = threadIdx.x / NKA_WAVE, waves = blockDim.x / NKA_WAVE;
   const int lane = lane_id(), g = lane / LPC, gl = lane % LPC;
-  const size_t wbytes = STAGE ? pad16((size_t)N * M * sizeof(T)) : 0;
-  // LDS: [W (staged)] [visible bias a] [cluster pairs] [spins of each chain]
-  T* a_s = (T*)(smem + wbytes);
-  int32_t* cl_s = (int32_t*)(smem + wbytes + pad16((size_t)N * sizeof(T)));
-  int8_t* xs = (int8_t*)(smem + wbytes + pad16((size_t)N * sizeof(T)) +
+  const size_t wbytes = pad16((size_t)N * M * sizeof(float));
+  // LDS: [W] [visible bias a] [cluster pairs] [spins of each chain]
+  float* a_s = (float*)(smem + wbytes);
+  int32_t* cl_s = (int32_t*)(smem + wbytes + pad16((size_t)N * sizeof(float)));
+  int8_t* xs = (int8_t*)(smem + wbytes + pad16((size_t)N * sizeof(float)) +
                          pad16((size_t)2 * sa.n_clusters * sizeof(int32_t))) +
                (wid * G + g) * pad16(N);
-  const T* W = v.W;
-  for (int i = threadIdx.x; i < N; i += blockDim.x) a_s[i] = v.a ? v.a[i] : (T)0;
+  const float* W = (const float*)smem;
+  for (int i = threadIdx.x; i < N; i += blockDim.x) a_s[i] = v.a ? v.a[i] : (float)0;
   for (int i = threadIdx.x; i < 2 * sa.n_clusters; i += blockDim.x) cl_s[i] = sa.clusters[i];
-  if (STAGE) {
-    stage_w<T>((T*)smem, v.W, N, M);  // ends with a workgroup barrier
-    W = (const T*)smem;
-  } else {
-    __syncthreads();
-  }
+  stage_w<float>((float*)smem, v.W, N, M);  // ends with a workgroup barrier
   const int c_raw = (bx * waves + wid) * G + g;
   if ((bx * waves + wid) * G >= sa.C) return;  // whole wavefront past the last chain
   const bool live = c_raw < sa.C;                        // groups past the last chain repeat it
@@ -322,27 +313,27 @@ __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& 
   // register slot jj of a lane holds hidden unit gl + LPC * ((jj + g) mod JG):
   // the rotation by the group index makes the groups of a wavefront read
   // different LDS bank ranges of their W rows in the same instruction
-  T th[JG], lc[JG];
-  T part = (T)0;
+  float th[JG], lc[JG];
+  float part = (float)0;
 #pragma unroll
   for (int jj = 0; jj < JG; ++jj) {
     const int j = gl + LPC * ((jj + g) & (JG - 1));
-    th[jj] = (T)0;
-    lc[jj] = (T)0;
+    th[jj] = (float)0;
+    lc[jj] = (float)0;
     if (j < M) {
-      T acc = v.b ? v.b[j] : (T)0;
+      float acc = v.b ? v.b[j] : (float)0;
       for (int i = 0; i < N; ++i) {
-        const T w = W[(size_t)i * M + j];
+        const float w = W[(size_t)i * M + j];
         acc += (xs[i] > 0) ? w : -w;
       }
       th[jj] = acc;
-      lc[jj] = log_cosh<T>(acc);
+      lc[jj] = log_cosh<float>(acc);
       part += lc[jj];
     }
   }
   for (int i = gl; i < N; i += LPC) part += (xs[i] > 0) ? a_s[i] : -a_s[i];
-  const T pw = (T)sa.machine_pow;
-  T lp = pw * group_sum<LPC, T>(part);
+  const float pw = (float)sa.machine_pow;
+  float lp = pw * group_sum<LPC>(part);
 
   // cluster slots of this lane: cl = gl + LPC * r, r < RSG (RSG * LPC >= n_clusters)
   const bool exch = sa.rule == NKA_RULE_EXCHANGE;
@@ -375,7 +366,7 @@ __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& 
       const u32x4 rnd = rnd_next;
       rnd_next = draws.at(q + 1, (uint32_t)c, sa.k0, sa.k1);
       int s0, s1 = 0, nf;
-      T corr = (T)0;
+      float corr = (float)0;
       bool valid = true;
       if (!exch) {
         s0 = (int)bounded(rnd.x, (uint32_t)N);
@@ -384,36 +375,36 @@ __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& 
         int n_diff, n_new;
         valid = group_exchange<LPC, RSG>(xs, cl_s, sa.n_clusters, cu, cv, g, rnd.x, s0, s1, n_diff, n_new);
         nf = 2;
-        corr = valid ? log_fast<T>((T)n_diff) - log_fast<T>((T)n_new) : (T)0;
+        corr = valid ? log_fast((float)n_diff) - log_fast((float)n_new) : (float)0;
       }
       // change of log psi with the new theta / log_cosh kept for a commit
       const int8_t x0 = xs[s0], x1 = xs[s1];
-      T nth[JG], nlc[JG];
-      T dpart = (T)0;
+      float nth[JG], nlc[JG];
+      float dpart = (float)0;
 #pragma unroll
       for (int jj = 0; jj < JG; ++jj) {
         const int j = gl + LPC * ((jj + g) & (JG - 1));
         nth[jj] = th[jj];
         nlc[jj] = lc[jj];
         if (j < M) {
-          const T w0 = W[(size_t)s0 * M + j];
-          T d = (x0 > 0) ? -2 * w0 : 2 * w0;
+          const float w0 = W[(size_t)s0 * M + j];
+          float d = (x0 > 0) ? -2 * w0 : 2 * w0;
           if (nf == 2) {
-            const T w1 = W[(size_t)s1 * M + j];
+            const float w1 = W[(size_t)s1 * M + j];
             d += (x1 > 0) ? -2 * w1 : 2 * w1;
           }
-          const T t = th[jj] + d;
-          const T l = log_cosh<T>(t);
+          const float t = th[jj] + d;
+          const float l = log_cosh<float>(t);
           nth[jj] = t;
           nlc[jj] = l;
           dpart += l - lc[jj];
         }
       }
-      T delta = group_sum<LPC, T>(dpart);
+      float delta = group_sum<LPC>(dpart);
       delta += (x0 > 0) ? -2 * a_s[s0] : 2 * a_s[s0];
       if (nf == 2) delta += (x1 > 0) ? -2 * a_s[s1] : 2 * a_s[s1];
-      const T u = uniform01<T>(rnd);
-      const bool acc = valid && (u < exp_t<T>(pw * delta + corr));
+      const float u = uniform01<float>(rnd);
+      const bool acc = valid && (u < exp_t<float>(pw * delta + corr));
       if (acc) {
 #pragma unroll
         for (int jj = 0; jj < JG; ++jj) {
@@ -445,14 +436,14 @@ __device__ __forceinline__ void rbm_metropolis_group_kernel_body(const nka_rbm& 
   }
 }
 
-template <class T, int G, int JG, int RSG, bool STAGE>
-__global__ void __launch_bounds__(256) rbm_metropolis_group_kernel(nka_rbm m, SweepArgs sa, int8_t* __restrict__ sigma, T* __restrict__ log_prob, int8_t* __restrict__ samples, T* __restrict__ lp_samples, int64_t* __restrict__ n_accepted) {
-  rbm_metropolis_group_kernel_body<T, G, JG, RSG, STAGE>(m, sa, sigma, log_prob, samples, lp_samples, n_accepted, blockIdx.x);
+template <int G, int JG, int RSG>
+__global__ void __launch_bounds__(256) rbm_metropolis_group_kernel(nka_rbm m, SweepArgs sa, int8_t* __restrict__ sigma, float* __restrict__ log_prob, int8_t* __restrict__ samples, float* __restrict__ lp_samples, int64_t* __restrict__ n_accepted) {
+  rbm_metropolis_group_kernel_body<G, JG, RSG>(m, sa, sigma, log_prob, samples, lp_samples, n_accepted, blockIdx.x);
 }
 
 // The same sweeps for a batch of jobs of one shape: blockIdx.y selects the job
 // (its parameters, chains, outputs and random stream); the shape arguments are shared.
-template <class T, int G, int JG, int RSG, bool STAGE>
+template <int G, int JG, int RSG>
 __global__ void __launch_bounds__(256) rbm_metropolis_group_kernel_batched(const nka_sweep_job* __restrict__ jobs, SweepArgs sa) {
   const nka_sweep_job& j = jobs[blockIdx.y];
   SweepArgs s = sa;
@@ -460,7 +451,7 @@ __global__ void __launch_bounds__(256) rbm_metropolis_group_kernel_batched(const
   s.k1 = (uint32_t)(j.seed >> 32);
   s.counter = j.counter;
   s.counter_dev = j.counter_dev;
-  rbm_metropolis_group_kernel_body<T, G, JG, RSG, STAGE>(j.model, s, j.sigma, (T*)j.log_prob, j.samples, (T*)j.log_prob_samples, j.n_accepted, blockIdx.x);
+  rbm_metropolis_group_kernel_body<G, JG, RSG>(j.model, s, j.sigma, (float*)j.log_prob, j.samples, (float*)j.log_prob_samples, j.n_accepted, blockIdx.x);
 }
 
 // counter += inc (one thread), after the sweep that consumed the counter
@@ -488,9 +479,8 @@ static bool stage_fits_s(const nka_rbm& m, int waves) {
          kLdsBudget;
 }
 
-template <class T>
 static size_t group_lds(const nka_rbm& m, const SweepArgs& sa, int waves, int G) {
-  return pad16((size_t)m.n_visible * m.n_hidden * sizeof(T)) + pad16((size_t)m.n_visible * sizeof(T)) +
+  return pad16((size_t)m.n_visible * m.n_hidden * sizeof(float)) + pad16((size_t)m.n_visible * sizeof(float)) +
          pad16((size_t)2 * sa.n_clusters * sizeof(int32_t)) + (size_t)waves * G * pad16(m.n_visible);
 }
 
@@ -498,7 +488,6 @@ static size_t group_lds(const nka_rbm& m, const SweepArgs& sa, int waves, int G)
 // 4 chains of 16 lanes when M <= 128 and there are chains enough for two such
 // wavefronts per SIMD, else 2 of 32 lanes when M <= 256, provided the clusters
 // fit the per-lane slots and W is staged in LDS.
-template <class T>
 static int pick_group(const nka_rbm& m, const SweepArgs& sa, int waves) {
   // four chains per wavefront only when that still leaves two wavefronts per
   // SIMD (the chains are latency-bound): measured on MI355X with 4096 chains,
@@ -510,7 +499,7 @@ static int pick_group(const nka_rbm& m, const SweepArgs& sa, int waves) {
     const int lpc = NKA_WAVE / G;
     if (m.n_hidden > 8 * lpc) continue;
     if (sa.rule == NKA_RULE_EXCHANGE && sa.n_clusters > kMaxClusterSlots * lpc) continue;
-    if (group_lds<T>(m, sa, waves, G) > kLdsBudget) continue;
+    if (group_lds(m, sa, waves, G) > kLdsBudget) continue;
     return G;
   }
   return 0;
@@ -519,33 +508,33 @@ static int pick_group(const nka_rbm& m, const SweepArgs& sa, int waves) {
 // Every launch helper takes an optional batch: with jobs != nullptr the
 // kernel runs once per job of the batch (grid y), each job's parameters,
 // chains and random stream read from jobs[] (device memory), the shape from m.
-template <class T, int G, int JG, int RSG>
-static void launch_group_rs(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, T* lp, int8_t* smp,
-                            T* lps, int64_t* nacc, int waves, const nka_sweep_job* jobs, int n_jobs,
+template <int G, int JG, int RSG>
+static void launch_group_rs(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, float* lp, int8_t* smp,
+                            float* lps, int64_t* nacc, int waves, const nka_sweep_job* jobs, int n_jobs,
                             hipStream_t s) {
-  const size_t lds = group_lds<T>(m, sa, waves, G);
+  const size_t lds = group_lds(m, sa, waves, G);
   const int per_block = waves * G;
   const unsigned g = (unsigned)((sa.C + per_block - 1) / per_block);
   if (jobs)
-    hipLaunchKernelGGL((rbm_metropolis_group_kernel_batched<T, G, JG, RSG, true>), dim3(g, n_jobs),
+    hipLaunchKernelGGL((rbm_metropolis_group_kernel_batched<G, JG, RSG>), dim3(g, n_jobs),
                        dim3(64 * waves), lds, s, jobs, sa);
   else
-    hipLaunchKernelGGL((rbm_metropolis_group_kernel<T, G, JG, RSG, true>), dim3(g), dim3(64 * waves), lds, s,
+    hipLaunchKernelGGL((rbm_metropolis_group_kernel<G, JG, RSG>), dim3(g), dim3(64 * waves), lds, s,
                        m, sa, sigma, lp, smp, lps, nacc);
 }
 
 // cluster slots per lane rounded up to a power of two (1 for the local rule)
-template <class T, int G, int JG>
-static void launch_group(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, T* lp, int8_t* smp,
-                         T* lps, int64_t* nacc, int waves, const nka_sweep_job* jobs, int n_jobs,
+template <int G, int JG>
+static void launch_group(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, float* lp, int8_t* smp,
+                         float* lps, int64_t* nacc, int waves, const nka_sweep_job* jobs, int n_jobs,
                          hipStream_t s) {
   const int lpc = NKA_WAVE / G;
   const int need = sa.rule == NKA_RULE_EXCHANGE ? (sa.n_clusters + lpc - 1) / lpc : 1;
-  if (need <= 1) launch_group_rs<T, G, JG, 1>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
-  else if (need <= 2) launch_group_rs<T, G, JG, 2>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
-  else if (need <= 4) launch_group_rs<T, G, JG, 4>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
-  else if (need <= 8) launch_group_rs<T, G, JG, 8>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
-  else launch_group_rs<T, G, JG, 16>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
+  if (need <= 1) launch_group_rs<G, JG, 1>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
+  else if (need <= 2) launch_group_rs<G, JG, 2>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
+  else if (need <= 4) launch_group_rs<G, JG, 4>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
+  else if (need <= 8) launch_group_rs<G, JG, 8>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
+  else launch_group_rs<G, JG, 16>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);
 }
 
 template <int JL, class T>
@@ -554,13 +543,13 @@ static void launch_sweep(const nka_rbm& m, const SweepArgs& sa, int8_t* sigma, T
   const int waves = 4;
   if constexpr (sizeof(T) == 8) {
     if (launch_group64(m, sa, sigma, lp, smp, lps, nacc, jobs, n_jobs, s)) return;
-  } else if (const int G = pick_group<T>(m, sa, waves)) {
+  } else if (const int G = pick_group(m, sa, waves)) {
     const int lpc = NKA_WAVE / G;
     const int need = (m.n_hidden + lpc - 1) / lpc;
     const int jg = need <= 1 ? 1 : need <= 2 ? 2 : need <= 4 ? 4 : 8;
 #define NKA_GROUP_CASE(GG, JJ)                                                                  \
     if (G == GG && jg == JJ) {                                                                  \
-      launch_group<T, GG, JJ>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);        \
+      launch_group<GG, JJ>(m, sa, sigma, lp, smp, lps, nacc, waves, jobs, n_jobs, s);        \
       return;                                                                                   \
     }
     NKA_GROUP_CASE(4, 1) NKA_GROUP_CASE(4, 2) NKA_GROUP_CASE(4, 4) NKA_GROUP_CASE(4, 8)
