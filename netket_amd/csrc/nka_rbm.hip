@@ -57,6 +57,11 @@ __device__ inline double load_mel(const void* p, int64_t i, int dtype) {
 // many as the registers of a CU hold (16 of up to 128, 8 of up to 256).
 template <class T, int JL, bool STAGE>
 constexpr int eloc_waves = sizeof(T) == 8 && STAGE && JL < 16 ? (JL <= 4 ? 16 : 8) : 4;
+// Wavefronts per SIMD that the registers have to leave room for.  With W from the cache
+// they cover its latency (FP64, 121 sites x 484 units, 14445 samples: 1.51 ms at three a
+// SIMD, 1.84 at two); two units a lane leave room for four.
+template <class T, int JL, bool STAGE>
+constexpr int eloc_occupancy = sizeof(T) == 8 && !STAGE && JL <= 8 ? (JL == 2 ? 4 : 3) : 1;
 
 // Up to 64 connected elements of one sample, one per lane: the sites that flip
 // (16 bits each, site | (x'_site > 0) << 15, 0xffff for none, in order), the matrix
@@ -111,7 +116,7 @@ __device__ inline void wave_prod_rest(double& v, double& rest) {
 // sample's 1 / prod (1 + e^{-2|theta|}); with more than 15 units per lane `rpr` is the
 // lane's and the logarithms of the lanes' quotients are added.  One exponential per unit.
 //
-// Bound by the vector units (78% busy in FP64).  Heisenberg, 64 sites, 128 units,
+// Bound by the vector units (71% busy in FP64).  Heisenberg, 64 sites, 128 units,
 // 16384 samples, FP64: 0.18 ms; an element at a time, each with its own reduction
 // over the wavefront, its logarithms and W from the cache, 0.46 ms.  FP32: 0.12 and
 // 0.40 ms.
@@ -392,7 +397,7 @@ __device__ __forceinline__ void rbm_eloc_body(const nka_rbm& m, const OpArgs& op
 }
 
 template <class T, int JL, bool STAGE>
-__global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64)) rbm_eloc_kernel(nka_rbm m, OpArgs op,
+__global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64), (eloc_occupancy<T, JL, STAGE>)) rbm_eloc_kernel(nka_rbm m, OpArgs op,
                                                                                const int8_t* __restrict__ sigma,
                                                                                int64_t n, double* __restrict__ eloc,
                                                                                T* __restrict__ log_psi) {
@@ -402,7 +407,7 @@ __global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64)) rbm_eloc_kern
 // The local energies of a batch of jobs of one shape (Ising operators on the
 // same lattice, each with its own couplings): blockIdx.y selects the job.
 template <class T, int JL, bool STAGE>
-__global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64)) rbm_eloc_kernel_batched(
+__global__ void __launch_bounds__((eloc_waves<T, JL, STAGE> * 64), (eloc_occupancy<T, JL, STAGE>)) rbm_eloc_kernel_batched(
     const nka_eloc_job* __restrict__ jobs, int64_t n) {
   const nka_eloc_job& j = jobs[blockIdx.y];
   OpArgs op{};
