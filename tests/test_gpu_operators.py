@@ -116,6 +116,17 @@ def test_log_psi(gpu, N, alpha, dtype):
         np.testing.assert_allclose(lp, ref, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("N,M", [(5, 2048), (7, 2049), (12, 2111), (30, 4096)])
+def test_log_psi_fp64_wide(gpu, N, M):
+    """The last size that keeps a lane's units in registers and those that do not.  Both
+    sums add M terms in another order: relative error at most a few M 2^-53 / 64 lanes."""
+    print(f"case log_psi N={N} M={M} float64", flush=True)
+    model, flat, p = _rbm_state(N, (M + 0.5) / N, np.float64, 12)
+    assert p.M == M
+    x = _states(N, 131, 13)
+    np.testing.assert_allclose(model.apply(flat, x).cpu().numpy(), orbm.log_psi(p, x), rtol=1e-12, atol=1e-12)
+
+
 @pytest.mark.parametrize("kind,N,alpha,dtype", [
     ("ising", 16, 1, np.float64), ("ising", 40, 2, np.float32),
     ("heis", 22, 1, np.float64), ("heis", 64, 2, np.float32),
