@@ -14,7 +14,7 @@
 // Seven int8 products of Na Nb Ns (Na Nb about Np^2 / 4) replace Ns Np^2
 // FP64 operations; the int8 rate is 64 times the FP64 one.  64 sites, 128
 // hidden units, 16384 samples (S 8384^2, mirrored): 47.7 ms as the FP64
-// product of the Jacobian, 2.9 ms here, and the error of S against extended
+// product of the Jacobian, 3.0 ms here, and the error of S against extended
 // precision fell from 3.5e-15 to 1.0e-15 (relative norms).
 #include "nka_common.hpp"
 #include "nka_qgt.hpp"
@@ -198,10 +198,10 @@ __global__ void __launch_bounds__(256) qgt64_hidden_digits_kernel(const double* 
 // rows, one chunk) free of bank conflicts over the 64 banks.
 // Tiles are numbered down the columns, so the workgroups that share a panel of
 // Q (the larger operand) run on one XCD and read it through one L2.
-// Bound by the matrix cores (46% busy at the 2.0 GHz the card holds here):
-// 2.40 ms at 2081 x 8385 x 16384 (1.67e15 int8 operations/s).  With the loads
-// and LDS reads issued ahead of a step's products instead of between them it
-// took 3.07 ms (34% busy); two buffers instead of four made 3.15 ms.
+// Bound by the matrix cores (48% busy at the clock the card holds here): 2.36 to
+// 2.56 ms over cards at 2081 x 8385 x 16384 (1.6e15 int8 operations/s).  Where it took
+// 2.40 ms, it took 3.07 (34% busy) with the loads and LDS reads issued ahead of a
+// step's products instead of between them, and 3.15 with two buffers instead of four.
 // blockIdx.y: slice of K (whole K steps); slice y writes C + y * slab, or with `add`
 // (a further chunk of the samples) adds to it.
 __global__ void __launch_bounds__(256, 1) qgt64_gemm_kernel(const int8_t* __restrict__ P, int64_t ma,

@@ -15,7 +15,9 @@
 // local rule's site does not depend on the state, so its W row and bias are read
 // one proposal ahead.
 //
-// Bound by the FP64 issue rate with many chains, by the serial latency of a
+// Bound by the vector units with many chains (79% busy; 333 instructions per proposal
+// of two chains with four units a lane, a third of them exponentials, the rest the
+// choice of the exchange, the draws and the reductions), by the serial latency of a
 // proposal (about 800 cycles) with few.  Measured, against one exponential and
 // one log1p of the library per unit and a draw per proposal: 4096 chains, 64
 // sites, 128 hidden units, exchange, 576 proposals: 5.22 -> 0.81 ms (W, 64 KB, now

@@ -15,9 +15,9 @@
 // A row is read through a buffer descriptor of its M values: lanes past the last
 // unit read zero, so no unit needs a bounds check, and the slots' offsets are
 // scalar.  Units per lane come in steps of two (a slot past the last unit costs as
-// much as a real one).  Bound by the vector unit: five instructions per unit, one of
+// much as a real one).  Bound by the vector unit (92% busy): five instructions per unit, one of
 // them an exp2.  8192 chains, 400 sites, 3200 units, 3600
-// proposals: 45.3 -> 22.6 ms, against a bounds check per load, one row buffer copied to the
+// proposals: 45.3 -> 22.6 to 25.1 ms over cards, against a bounds check per load, one row buffer copied to the
 // other after each proposal, a draw per lane and units in steps of eight.
 #include "nka_sampler.hpp"
 
