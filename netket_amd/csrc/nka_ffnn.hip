@@ -38,7 +38,7 @@ constexpr int FF_MAXH = 1024;
 // state does not fit 128 registers (FP64; weighted exchange).  J1-J2 10x10 with layers
 // 100-400-400 in FP32, against workgroups of 256: the sampler (8192 chains, 700
 // proposals) 42.4 -> 20.3 ms (matrix products 60% of it), the local energies of 16384
-// samples 23.2 -> 12.5 ms (58%; the rest is vector work and its latencies; with the
+// samples 23.2 -> 12.4 ms (59%; the rest is vector work and its latencies; with the
 // connected elements taken as a list of flipped sites instead of as configurations, 3.0
 // ms of that).  Layers of 8 to 100 units, 16 to 8192 chains, all rules: the sampler 1.0
 // (8-8 units, FP64) to 2.6 times as fast as with 256.
