@@ -235,20 +235,28 @@ __device__ __forceinline__ void rows_gemm(const float* As, int lda, int K, int n
 template <int NW, class Epi>
 __device__ __forceinline__ void rows_gemm(const double* As, int lda, int K, int ncols, const double* __restrict__ Bp, int sk,
                           int sc, Epi epi, double* part, double* rowsum, double* rbuf = nullptr) {
-  constexpr int G = NW * 64 / FF_ROWS;  // threads per row
-  static_assert(G <= FF_MAXBLK, "one partial sum per thread of a row");
+  // 16 sums of every 16th column per row, whichever the number of threads, so that a row's
+  // value does not depend on its batch (which chooses the workgroups' size): a thread has
+  // one of them, or two for its columns in turn
+  constexpr int G = NW * 64 / FF_ROWS, S = 16;  // threads of a row, sums of a row
+  static_assert((S == G || S == 2 * G) && S <= FF_MAXBLK, "one or two sums per thread");
   const int r = threadIdx.x & 31, g = threadIdx.x >> 5;
-  double s = 0.0;
-  for (int c = g; c < ncols; c += G) {
+  double s = 0.0, other = 0.0;
+  int c = g;
+  for (; c < ncols; c += G) {
     double z = 0.0;
     for (int k = 0; k < K; ++k) z += As[r * lda + k] * Bp[(int64_t)k * sk + (int64_t)c * sc];
-    s += epi(r, c, z);
+    const double sum = s + epi(r, c, z);
+    s = S == G ? sum : other;
+    other = sum;
   }
-  part[r * FF_MAXBLK + g] = s;
+  // (c, past the end now, is the next column that s would have taken)
+  part[r * FF_MAXBLK + c % S] = s;
+  if constexpr (S != G) part[r * FF_MAXBLK + (c + G) % S] = other;
   __syncthreads();
   if (threadIdx.x < FF_ROWS) {
     double t = 0.0;
-    for (int q = 0; q < G; ++q) t += part[threadIdx.x * FF_MAXBLK + q];
+    for (int q = 0; q < S; ++q) t += part[threadIdx.x * FF_MAXBLK + q];
     rowsum[threadIdx.x] = t;
   }
   __syncthreads();

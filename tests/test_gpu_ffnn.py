@@ -348,6 +348,18 @@ def test_fp64_many_rows(gpu, N, H1, H2, n):
     np.testing.assert_allclose(e, ref[index[:m]], rtol=1e-10, atol=1e-10 * np.abs(ref).max())
 
 
+@pytest.mark.parametrize("N,H1,H2,n", [(6, 5, 33, 16500), (7, 40, 50, 16500), (6, 50, 70, 131100)])
+def test_fp64_log_psi_is_the_same_in_any_batch(gpu, N, H1, H2, n):
+    """Workgroups of 256 (many rows) and of 512 (few) add a row's columns in one order."""
+    print(f"case ffnn fp64 batches N={N} H=({H1},{H2}) n={n}", flush=True)
+    model, flat, p = _model(N, H1, H2, np.float64, 31, 0.3)
+    x = torch.as_tensor(np.random.default_rng(5).choice(np.array([-1, 1], dtype=np.int8), size=(n, N)), device="cuda")
+    few = x[:64].contiguous()
+    assert torch.equal(model.apply(flat, x)[:64], model.apply(flat, few))
+    H = nk.operator.Ising(nk.hilbert.Spin(0.5, N=N), nk.graph.Chain(N), h=0.7, J=1.1)
+    assert torch.equal(eng.local_energies(model, flat, H, x)[:64], eng.local_energies(model, flat, H, few))
+
+
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("rule", ["local", "exchange", "exchange-weighted"])
 @pytest.mark.parametrize("H1,H2,n_chains", [(1, 8, 33), (16, 3, 5), (32, 40, 32), (33, 8, 40), (129, 8, 7)])
