@@ -1161,14 +1161,19 @@ inline int64_t ffnn_np(const nka_ffnn& m) {
          (m.b2_off >= 0 ? m.n_hidden2 : 0) + (int64_t)m.n_hidden1 * m.n_hidden2;
 }
 
-// FP64 rows on workgroups of 256 where there are many: past 16 workgroups per CU, and
-// from two per CU on with small layers.  The second layer is a plain sum per thread and
-// column there, and more small workgroups cover each other's barriers better than few
-// large ones.  Local energies of 16384 samples of the 6x6 Ising lattice, layers 8-8, 24-24,
-// 64-64: 344, 508, 1442 us against 446, 641, 1487 with 512; of 1024 samples (4.6 workgroups
-// per CU): 58, 77, 169 against 64, 82, 164; log psi of 32 rows, layers 64-64: 48 against 42.
-static bool forward_small(const nka_ffnn& m, int64_t workgroups) {
-  return workgroups >= 16 * device_cus() || (workgroups >= 2 * device_cus() && m.n_hidden1 * m.n_hidden2 <= 2048);
+// FP64 rows on workgroups of 256 where there are many: from 4 workgroups per CU on for
+// whole configurations, 16 for connected elements (whose first layer has at most FF_MAXD
+// sites to add, and many of whose workgroups are past the end of the list), and from two
+// with small layers or a second layer no wider than the first one's `sites`.  The layers
+// are plain sums per thread there, and more small workgroups cover each other's barriers
+// better than few large ones.  Local energies of 16384 samples of the 6x6 Ising lattice,
+// layers 8-8, 24-24, 64-64: 344, 508, 1442 us against 446, 641, 1487 with 512; of 1024
+// samples (4.6 workgroups per CU): 58, 77, 169 against 64, 82, 164.  Log psi of 32768 rows
+// (4 per CU), 100 sites, layers 24-100, 100-24: 79, 188 us against 88, 196; of 24576 (3),
+// 16 sites, layers 100-100, 200-200: 133, 500 against 127, 452.
+static bool forward_small(const nka_ffnn& m, int64_t workgroups, int sites) {
+  return workgroups >= (sites > FF_MAXD ? 4 : 16) * device_cus() ||
+         (workgroups >= 2 * device_cus() && (m.n_hidden1 * m.n_hidden2 <= 2048 || m.n_hidden2 <= sites));
 }
 
 template <class T>
@@ -1181,7 +1186,7 @@ static void launch_forward0(const nka_ffnn& m, const int8_t* x, int64_t rows, T*
                        g2, (const int*)nullptr, (const uint64_t*)nullptr, (const int*)nullptr);
   };
   if constexpr (sizeof(T) == 8) {
-    if (forward_small(m, g)) {
+    if (forward_small(m, g, m.n_visible)) {
       launch(ffnn_forward_kernel<T, 0, FF_FWD / 2>, FF_FWD / 2);
       return;
     }
@@ -1257,7 +1262,7 @@ static int ffnn_eloc_impl(const nka_ffnn& m, int op_kind, const void* op, const 
     };
     bool half = false;
     if constexpr (sizeof(T) == 8) {
-      half = forward_small(m, g);
+      half = forward_small(m, g, FF_MAXD);
       if (half) launch(ffnn_forward_kernel<T, 1, FF_FWD / 2>, FF_FWD / 2);
     }
     if (!half) launch(ffnn_forward_kernel<T, 1, FF_FWD>, FF_FWD);
